@@ -63,6 +63,27 @@ struct DevBuf {
   }
 };
 
+// Pinned host memory that kernels write directly.
+template <class T>
+struct PinBuf {
+  T* p = nullptr;
+  size_t n = 0;
+  PinBuf() = default;
+  PinBuf(const PinBuf&) = delete;
+  PinBuf& operator=(const PinBuf&) = delete;
+  ~PinBuf() { reset(); }
+  void reset() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  hipError_t alloc(size_t count) {
+    reset();
+    n = count;
+    return hipHostMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocDefault);
+  }
+};
+
 struct PointHost {
   cvf_params prm;
   uint32_t L, N, woff, loff, shell_off;
@@ -175,7 +196,6 @@ struct cvf_sim {
   DevBuf<PointState> pst;
   DevBuf<float> dist;
   DevBuf<int32_t> freq;
-  DevBuf<unsigned long long> counters;
   DevBuf<uint64_t> cur_steps;          // one slot per group
   DevBuf<BlockEnt> tab_cell_all;       // every point's cells, for observables
   DevBuf<unsigned long long> hist;     // sigma histogram of one point (6 counters)
@@ -192,7 +212,13 @@ struct cvf_sim {
   int64_t steps = 0;
   int64_t obs_at = -1;
   bool sw_labels = false;  // the labels hold a Swendsen-Wang step's (all zero before the first)
-  std::vector<unsigned long long> obs_counters;
+  // the sample of step obs_at: written by k_observe, the partial sums added
+  // up per point
+  PinBuf<uint2> obs_part;
+  PinBuf<PointState> obs_ps;
+  PinBuf<uint32_t> obs_status;
+  std::vector<int32_t> obs_point;  // point of each k_observe workgroup (-1: padding)
+  std::vector<int64_t> obs_nhb2, obs_nsig;
 
   void drop_graphs() {
     for (auto& g : groups) g->drop_graphs();
@@ -381,14 +407,17 @@ void init_words(const PointHost& P, std::vector<uint32_t>& w) {
 
 // The resident kernel's abort flag: a neighbour wait that timed out leaves
 // the lattice invalid.  Call after the handle's stream has been synchronised.
-int check_resident(cvf_sim* s) {
-  if (!s->resident_used) return CVF_OK;
-  uint32_t v = 0;
-  HIPC(hipMemcpy(&v, s->rstatus.p, sizeof v, hipMemcpyDeviceToHost));
+int resident_status(uint32_t v) {
   if (v)
     return fail(CVF_EDEVICE, "resident kernel: a workgroup's wait for its neighbour slab timed out; "
                              "the lattice state is invalid");
   return CVF_OK;
+}
+int check_resident(cvf_sim* s) {
+  if (!s->resident_used) return CVF_OK;
+  uint32_t v = 0;
+  HIPC(hipMemcpy(&v, s->rstatus.p, sizeof v, hipMemcpyDeviceToHost));
+  return resident_status(v);
 }
 
 int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
@@ -1032,10 +1061,16 @@ int build_groups(cvf_sim* s) {
   if (rc0) return rc0;
   std::vector<int> all(s->npts);
   for (int i = 0; i < s->npts; ++i) all[i] = i;
-  const auto ta = make_table(s->ph, all, kObserveSpan, cells_all);
-  int rc = upload_vec(s->tab_cell_all, ta);
-  if (rc) return rc;
-  s->nb_cell_all = (uint32_t)ta.size();
+  if (!s->obs_part.p) {  // the observables' table does not depend on the tuning
+    const auto ta = make_table(s->ph, all, observe_span(s->total_cells), cells_all);
+    int rc = upload_vec(s->tab_cell_all, ta);
+    if (rc) return rc;
+    s->nb_cell_all = (uint32_t)ta.size();
+    for (const BlockEnt& en : ta) s->obs_point.push_back(en.point);
+    HIPC(s->obs_ps.alloc(s->npts));
+    HIPC(s->obs_status.alloc(1));
+    HIPC(s->obs_part.alloc(ta.size()));
+  }
   HIPC(hipDeviceSynchronize());
   return CVF_OK;
 }
@@ -1068,7 +1103,7 @@ void enqueue_lattice(cvf_sim* s, int gi, hipStream_t st, uint32_t step_off, Time
     // one step of the resident kernel, in place on `words`
     timed(CVF_KCLASS_RESIDENT, [&] {
       launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                      s->words.p, g.rings.p, g.rver.p, stepp, step_off, 1, s->rstatus.p, g.r_fine);
+                      s->words.p, g.rings.p, g.rver.p, stepp, step_off, 1, nullptr, s->rstatus.p, g.r_fine);
     });
   } else if (s->sched == CVF_SCHED_FAST) {
     // eta cube sweep, then n_metropolis x the two colour passes (in place,
@@ -1129,8 +1164,6 @@ constexpr uint32_t kHistSpan = 4096;  // per-step histograms per copy back
 // state in `words`.
 int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = false) {
   Group& g = *s->groups[gi];
-  const int nsteps_all = nsteps;
-  if (g.resident) s->resident_used = true;
   const bool ok = g.fused && s->nm > 0;
   bool variant_ok = false;
   int flips = 0;  // word-array swaps of one variant step
@@ -1142,30 +1175,6 @@ int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = fal
     flips = 1;
   }
   int par = 0;
-  if (g.resident && s->nc == 0 && !rec) {
-    if (s->vol_device) {
-      // every step of the sequence in one resident launch, the volume
-      // chain of the same steps beside it (it never reads the lattice, and
-      // takes the volume state only from its own last run); the group
-      // counter moves on once both have read it
-      HIPC(hipEventRecord(g.fork, st));
-      HIPC(hipStreamWaitEvent(g.side, g.fork, 0));
-      launch_vol_chain(g.side, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, nullptr,
-                       (uint32_t)nsteps_all, s->dist.p, s->freq.p, s->precision, 1);
-      HIPC(hipEventRecord(g.join, g.side));
-      launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                      s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)nsteps, s->rstatus.p,
-                      g.r_fine);
-      HIPC(hipStreamWaitEvent(st, g.join, 0));
-      launch_vol_chain(st, s->pts.p, g.plist.p, 0, s->pst.p, s->cur_steps.p + gi, (uint32_t)nsteps_all, s->dist.p,
-                       s->freq.p, s->precision, 0);
-      return CVF_OK;
-    }
-    // every step of the sequence in one resident launch
-    launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                    s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)nsteps, s->rstatus.p, g.r_fine);
-    nsteps = 0;
-  }
   for (int i = 0; i < nsteps; ++i) {
     const bool variant = variant_ok && (i < nsteps - 1 || (par ^ flips) == 0);
     enqueue_lattice(s, gi, st, (uint32_t)i, Untimed{}, par, variant);
@@ -1176,7 +1185,37 @@ int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = fal
     }
   }
   launch_vol_chain(st, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,
-                   (uint32_t)nsteps_all, s->dist.p, s->freq.p, s->precision, s->vol_device);
+                   (uint32_t)nsteps, s->dist.p, s->freq.p, s->precision, s->vol_device);
+  return CVF_OK;
+}
+
+// Group g runs whole sequences of steps in single resident launches: nothing
+// reads the lattice between its steps.
+bool resident_sequences(const cvf_sim* s, const Group& g) { return g.resident && s->nc == 0; }
+
+// nsteps MC steps of a resident group (resident_sequences) from step s->steps
+// on, as one resident launch on st.  One launch takes any number of steps, so
+// no graph is captured for it: a captured sequence of fixed length cut a
+// 10-step call into launches of 8 and 2 steps, each with its own staging and
+// counter kernel (L = 32, 10 steps and a sample: 266 us; as one launch, with
+// the sample in one kernel, 175).  The device volume chain of the same steps
+// runs beside it on the group's second stream: it never reads the lattice,
+// and takes the volume state only from its own last run.
+int enqueue_resident(cvf_sim* s, int gi, hipStream_t st, int nsteps) {
+  Group& g = *s->groups[gi];
+  s->resident_used = true;
+  if (s->vol_device) {
+    HIPC(hipEventRecord(g.fork, st));
+    HIPC(hipStreamWaitEvent(g.side, g.fork, 0));
+    launch_vol_chain(g.side, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, nullptr, (uint32_t)nsteps,
+                     s->dist.p, s->freq.p, s->precision, 1);
+    HIPC(hipEventRecord(g.join, g.side));
+  }
+  launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
+                  s->words.p, g.rings.p, g.rver.p, nullptr, (uint64_t)s->steps, (uint32_t)nsteps,
+                  s->cur_steps.p + gi, s->rstatus.p, g.r_fine);
+  if (s->vol_device) HIPC(hipStreamWaitEvent(st, g.join, 0));
+  HIPC(hipGetLastError());
   return CVF_OK;
 }
 
@@ -1252,6 +1291,16 @@ void host_volume_moves(cvf_sim* s) {
     const double te =
         vdw_energy_fp64(trial, P.prm.r_cutoff, P.dist.data(), P.freq.data(), (int)P.dist.size());
     volume_accept(P.vol, P.vp, trial, te, u2);
+  }
+}
+
+// The handle moves on by n steps.  The volume chain does not read the
+// lattice: in host-volume mode the host advances it while the device runs
+// the lattice steps just enqueued.
+void host_moves(cvf_sim* s, int n) {
+  for (int j = 0; j < n; ++j) {
+    if (!s->vol_device) host_volume_moves(s);
+    ++s->steps;
   }
 }
 
@@ -1401,7 +1450,6 @@ int create_impl(const cvf_params* pts, int32_t n, cvf_sim** out) {
   HIPC(s->cov.alloc(s->total_cells));
   HIPC(s->pts.alloc(n));
   HIPC(s->pst.alloc(n));
-  HIPC(s->counters.alloc(2 * (size_t)n));
   const uint32_t maxN = maxL * maxL * maxL;
   HIPC(s->csize.alloc(6 * (size_t)maxN));
   HIPC(s->slot.alloc(6 * (size_t)maxN));
@@ -1537,32 +1585,38 @@ int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
   return CVF_OK;
 }
 
-// n_steps MC steps as graph launches; group rec_gi (if >= 0) replays its
-// recording sequences.
+// n_steps MC steps as resident launches or graph launches; group rec_gi (if
+// >= 0) replays its recording sequences.
 int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
+  if (rec_gi < 0 && s->groups.size() == 1 && resident_sequences(s, *s->groups[0])) {
+    for (int64_t i = 0; i < n_steps;) {
+      const int k = (int)std::min<int64_t>(s->tune.graph_steps, n_steps - i);
+      if (int rc = enqueue_resident(s, 0, s->stream, k)) return rc;
+      host_moves(s, k);
+      i += k;
+    }
+    return CVF_OK;
+  }
   int rc = capture_step_graphs(s);
   if (rc) return rc;
   if (s->nc > 0 && n_steps > 0) s->sw_labels = true;
   if (rec_gi >= 0 && (rc = capture_rec_graphs(s, rec_gi))) return rc;
-  if ((rc = fork_groups(s))) return rc;
+  // one group's graphs go to the main stream itself
+  const bool fork = s->groups.size() > 1;
+  if (fork && (rc = fork_groups(s))) return rc;
   const std::vector<int>& sizes = s->groups[0]->gsteps;  // the same for every group
   for (int64_t i = 0; i < n_steps;) {
     size_t c = 0;
     while (sizes[c] > n_steps - i) ++c;  // the last size is 1
     for (size_t gi = 0; gi < s->groups.size(); ++gi) {
       Group& g = *s->groups[gi];
-      HIPC(hipGraphLaunch((int)gi == rec_gi ? g.rgexecs[c] : g.gexecs[c], g.stream));
+      if (g.resident) s->resident_used = true;
+      HIPC(hipGraphLaunch((int)gi == rec_gi ? g.rgexecs[c] : g.gexecs[c], fork ? g.stream : s->stream));
     }
-    const int64_t k = sizes[c];
-    // the volume chain does not read the lattice: in host-volume mode the
-    // host advances it while the device runs the lattice steps
-    for (int64_t j = 0; j < k; ++j) {
-      if (!s->vol_device) host_volume_moves(s);
-      ++s->steps;
-    }
-    i += k;
+    host_moves(s, sizes[c]);
+    i += sizes[c];
   }
-  return join_groups(s);
+  return fork ? join_groups(s) : CVF_OK;
 }
 
 int cvf_step(cvf_sim* s, int64_t n_steps) {
@@ -1603,22 +1657,26 @@ int cvf_observe(cvf_sim* s, int32_t pt, cvf_obs* o) {
   if (!o) return fail(CVF_EINVAL, "null output");
   HIPC(hipSetDevice(s->device));
   if (s->obs_at != s->steps) {
-    launch_zero_u32(s->stream, (uint32_t*)s->counters.p, 4 * (size_t)s->npts);
-    launch_observe(s->stream, Launch{s->tab_cell_all.p, s->nb_cell_all, 256, nullptr, 0}, s->words.p,
-                   s->counters.p);
-    s->obs_counters.resize(2 * (size_t)s->npts);
-    HIPC(hipMemcpyAsync(s->obs_counters.data(), s->counters.p, 16 * (size_t)s->npts,
-                        hipMemcpyDeviceToHost, s->stream));
+    launch_observe(s->stream, s->tab_cell_all.p, s->nb_cell_all, s->words.p, observe_span(s->total_cells), s->pst.p,
+                   s->rstatus.p, ObsOut{s->obs_part.p, s->obs_ps.p, s->obs_status.p});
+    HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
-    if ((rc = check_resident(s))) return rc;
+    if ((rc = resident_status(*s->obs_status.p))) return rc;
+    s->obs_nhb2.assign(s->npts, 0);
+    s->obs_nsig.assign(s->npts, 0);
+    for (size_t b = 0; b < s->obs_point.size(); ++b)
+      if (s->obs_point[b] >= 0) {
+        s->obs_nhb2[s->obs_point[b]] += s->obs_part.p[b].x;
+        s->obs_nsig[s->obs_point[b]] += s->obs_part.p[b].y;
+      }
     s->obs_at = s->steps;
   }
-  double r_cell, V, E_vdw;
-  rc = cvf_get_volume(s, pt, &r_cell, &V, &E_vdw);
-  if (rc) return rc;
+  // the volume chain as of the same step
+  const VolState& vol = s->vol_device ? s->obs_ps.p[pt].vol : s->ph[pt].vol;
+  const double r_cell = vol.r_cell, E_vdw = vol.E_vdw;
   const PointHost& P = s->ph[pt];
-  int64_t nhb2 = (int64_t)s->obs_counters[2 * pt];
-  const int64_t nsig = (int64_t)s->obs_counters[2 * pt + 1];
+  int64_t nhb2 = s->obs_nhb2[pt];
+  const int64_t nsig = s->obs_nsig[pt];
   if (!P.prm.flag_chessboard) {
     // the capped count is sequential over cells: taken on the host
     std::vector<uint32_t> w;
@@ -1839,6 +1897,7 @@ int cvf_set_shells(cvf_sim* s, int32_t pt, const float* dist, const int32_t* fre
   HIPC(hipMemcpy(&st, s->pst.p + pt, sizeof st, hipMemcpyDeviceToHost));
   st.vol.E_vdw = vdw_energy_fp64(st.vol.r_cell, P.prm.r_cutoff, P.dist.data(), P.freq.data(), nshell);
   HIPC(hipMemcpy(s->pst.p + pt, &st, sizeof st, hipMemcpyHostToDevice));
+  s->obs_at = -1;
   return CVF_OK;
 }
 
@@ -1896,7 +1955,7 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     s->resident_used = true;
     timed(CVF_KCLASS_RESIDENT, [&] {
       launch_resident(g.stream, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p,
-                      s->pts.p, s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)n_steps,
+                      s->pts.p, s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)n_steps, nullptr,
                       s->rstatus.p, g.r_fine);
     });
     timed(CVF_KCLASS_BEGIN, [&] {

@@ -52,7 +52,6 @@ constexpr uint32_t kEntNoChess = 1;
 
 constexpr int kChunk = 6;      // half-sweeps per fused kernel (default)
 constexpr int kMaxChunk = 12;  // half-sweeps per fused kernel at most: a whole Metropolis pass
-constexpr uint32_t kObserveSpan = 4096;  // cells per k_observe workgroup (256 threads)
 constexpr int kMaxSlab = 16;  // planes per slab of the fused kernel
 
 struct Launch {
@@ -87,7 +86,20 @@ void launch_chunk(hipStream_t st, Launch ln, const PointDev* pts, const uint32_t
 uint32_t chunk_lds_limit();
 void launch_zero_u32(hipStream_t st, uint32_t* p, size_t n);
 void launch_zero3_u32(hipStream_t st, uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc);
-void launch_observe(hipStream_t st, Launch ln, const uint32_t* words, unsigned long long* counters);
+// Cells per k_observe workgroup (a multiple of 1024): small handles spread
+// over more workgroups (L = 32: 32 of them), large ones keep the host's sum of
+// the partial results short.
+constexpr uint32_t observe_span(size_t total_cells) { return total_cells < (1u << 20) ? 1024 : 4096; }
+// A sample's results in host memory (pinned, device-visible): per workgroup
+// of the table the pair (2 N_HB, N_sigma) of its cells, every point's
+// mutable state and the resident kernel's abort flag.
+struct ObsOut {
+  uint2* part;
+  PointState* ps;
+  uint32_t* status;
+};
+void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
+                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out);
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc);
 void launch_sw_union(hipStream_t st, Launch ln, uint32_t* parent, const uint8_t* cov);
@@ -174,8 +186,11 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 // per lane (one, below 64 quads), cube families whose cubes fit the lanes one cube per lane, and
 // z half-sweeps one cell per lane where that fits, else two where that
 // does, instead of one quad (one four-cube item) per lane
+// The launch's first step is *stepp + step_off, or step_off itself without
+// stepp; with step_out (then no stepp) the step after its last goes there.
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                     const uint64_t* stepp, uint32_t step_off, uint32_t nsteps, uint32_t* status, bool fine);
+                     const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                     bool fine);
 
 }  // namespace cvf

@@ -690,60 +690,74 @@ __global__ void k_zero3_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, uint
   }
 }
 
-// One workgroup of 256 threads per kObserveSpan cells of a point: each
-// thread sums kObserveSpan / 256 cells, the workgroup reduces through LDS,
-// and one pair of 64-bit atomics per workgroup adds to the point's totals
-// (one pair per wavefront serialised on the same address at large L).
+// Equal-sigma arm pairs of a cell (the cell's share of N_sigma): over the
+// five arm distances k, the fields of w ^ (w >> 3k) that are zero; the
+// zero-field test is sigma_thr_index's.  15 pairs minus the unequal ones.
+__device__ __forceinline__ uint32_t equal_pairs(uint32_t w) {
+  constexpr uint32_t kLo2 = 0x1B6DBu, kHi = 0x24924u;
+  uint32_t ne = 0;
+#pragma unroll
+  for (int k = 1; k < 6; ++k) {
+    const uint32_t y = (w ^ (w >> (3 * k))) & (kSigmaBits >> (3 * k));
+    ne += (uint32_t)popc32((((y & kLo2) + kLo2) | y) & kHi);
+  }
+  return 15u - ne;
+}
+
+// 2 N_HB of the forward bond of axis AX between a cell and its neighbour.
+template <int AX>
+__device__ __forceinline__ uint32_t bond_nhb2(uint32_t w, uint32_t wn) {
+  return sigma_of(w, 2 * AX) == sigma_of(wn, 2 * AX + 1) ? eta_of(w, 2 * AX) + eta_of(wn, 2 * AX + 1) : 0u;
+}
+
+// One sample of a handle in one launch: a workgroup of 256 threads sums
+// `span` cells of a point (four cells along x per thread and round: three
+// 16-byte loads and the next word of the row) and stores the pair of sums
+// at its own place in host memory; a point's first workgroup copies the
+// point's mutable state there and workgroup 0 the resident kernel's abort
+// flag.  The host adds the partial sums after the stream has drained, so a
+// sample needs no counters to clear, no atomics and no copy.  Bound by the
+// latency of one launch: the word-at-a-time form with its clearing kernel
+// and copies took 4.6 + 16.2 + 2 x 3.8 us of GPU time at L = 32 and 40 us
+// for the kernel alone at L = 160.
 __global__ __launch_bounds__(256) void k_observe(const BlockEnt* __restrict__ tab, uint32_t nb,
-                                                const uint32_t* __restrict__ words,
-                                                unsigned long long* __restrict__ counters) {
-  const BlockEnt e = tab[xcd_logical_block(blockIdx.x, nb)];
+                                                const uint32_t* __restrict__ words, uint32_t span,
+                                                const PointState* __restrict__ ps,
+                                                const uint32_t* __restrict__ rstatus, uint2* __restrict__ part,
+                                                PointState* __restrict__ ps_out, uint32_t* __restrict__ status_out) {
+  const uint32_t lb = xcd_logical_block(blockIdx.x, nb);
+  const BlockEnt e = tab[lb];
+  if (lb == 0 && threadIdx.x == 0) *status_out = *rstatus;
   if (e.point < 0) return;
-  const uint32_t L = e.L;
+  if (e.start == 0 && threadIdx.x == 0) ps_out[e.point] = ps[e.point];
+  const uint32_t L = e.L, LL = L * L;
   const uint32_t* W = words + e.woff;
   uint32_t nhb2 = 0, nsig = 0;
-  for (uint32_t k = 0; k < kObserveSpan / 256; ++k) {
-    const uint32_t t = e.start + k * 256 + threadIdx.x;
+  for (uint32_t k = 0; k < span; k += 1024) {
+    const uint32_t t = e.start + k + 4 * threadIdx.x;
     if (t >= e.N) break;
     uint32_t x, y, z;
     cell_coords(e, t, x, y, z);
-    const uint32_t w = W[t];
-    const uint32_t nbs[3] = {neighbor_up(t, x, 1, L), neighbor_up(t, y, L, L),
-                             neighbor_up(t, z, L * L, L)};
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-      const uint32_t wn = W[nbs[ax]];
-      if (sigma_of(w, 2 * ax) == sigma_of(wn, 2 * ax + 1))
-        nhb2 += eta_of(w, 2 * ax) + eta_of(wn, 2 * ax + 1);
-    }
-    uint32_t pairs = 0;
-#pragma unroll
-    for (int a = 0; a < 6; ++a) pairs += (uint32_t)count_eq(w, sigma_of(w, a)) - 1;
-    nsig += pairs / 2;
+    // L is a multiple of 4: the four cells share their row
+    const uint4 c = *reinterpret_cast<const uint4*>(W + t);
+    const uint32_t xn = W[neighbor_up(t + 3, x + 3, 1, L)];
+    const uint4 yn = *reinterpret_cast<const uint4*>(W + neighbor_up(t, y, L, L));
+    const uint4 zn = *reinterpret_cast<const uint4*>(W + neighbor_up(t, z, LL, L));
+    nhb2 += bond_nhb2<0>(c.x, c.y) + bond_nhb2<0>(c.y, c.z) + bond_nhb2<0>(c.z, c.w) + bond_nhb2<0>(c.w, xn);
+    nhb2 += bond_nhb2<1>(c.x, yn.x) + bond_nhb2<1>(c.y, yn.y) + bond_nhb2<1>(c.z, yn.z) + bond_nhb2<1>(c.w, yn.w);
+    nhb2 += bond_nhb2<2>(c.x, zn.x) + bond_nhb2<2>(c.y, zn.y) + bond_nhb2<2>(c.z, zn.z) + bond_nhb2<2>(c.w, zn.w);
+    nsig += equal_pairs(c.x) + equal_pairs(c.y) + equal_pairs(c.z) + equal_pairs(c.w);
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
     nhb2 += __shfl_xor(nhb2, m, 64);
     nsig += __shfl_xor(nsig, m, 64);
   }
-  __shared__ uint32_t part[2][4];
-  const uint32_t wv = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    part[0][wv] = nhb2;
-    part[1][wv] = nsig;
-  }
+  __shared__ uint2 sh[4];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = make_uint2(nhb2, nsig);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long a = 0, b = 0;
-    for (int i = 0; i < 4; ++i) {
-      a += part[0][i];
-      b += part[1][i];
-    }
-    if (a | b) {
-      atomicAdd(&counters[2 * e.point], a);
-      atomicAdd(&counters[2 * e.point + 1], b);
-    }
-  }
+  if (threadIdx.x == 0)
+    part[lb] = make_uint2(sh[0].x + sh[1].x + sh[2].x + sh[3].x, sh[0].y + sh[1].y + sh[2].y + sh[3].y);
 }
 
 // Counts of the six sigma values over the 6N arms of one point, as
@@ -1368,8 +1382,9 @@ void launch_zero3_u32(hipStream_t st, uint32_t* a, size_t na, uint32_t* b, size_
   if (blocks == 0) blocks = 1;
   launch(k_zero3_u32, dim3((unsigned)blocks), dim3(256), st, a, na, b, nb, c, nc);
 }
-void launch_observe(hipStream_t st, Launch ln, const uint32_t* words, unsigned long long* counters) {
-  launch(k_observe, dim3(ln.nblocks), dim3(ln.block), st, ln.tab, ln.nblocks, words, counters);
+void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
+                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out) {
+  launch(k_observe, dim3(nblocks), dim3(256), st, tab, nblocks, words, span, ps, rstatus, out.part, out.ps, out.status);
 }
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc) {

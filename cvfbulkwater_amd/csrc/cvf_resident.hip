@@ -474,8 +474,9 @@ template <bool FINE>
 __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__ grp, const RSlab* __restrict__ slabs,
                                                     const PointDev* __restrict__ pts, uint32_t* __restrict__ words,
                                                     uint32_t* __restrict__ rings, uint64_t* __restrict__ ver,
-                                                    const uint64_t* __restrict__ stepp, uint32_t step_off,
-                                                    uint32_t nsteps, uint32_t* __restrict__ status) {
+                                                    const uint64_t* __restrict__ stepp, uint64_t step_off,
+                                                    uint32_t nsteps, uint64_t* __restrict__ step_out,
+                                                    uint32_t* __restrict__ status) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ RSlab Ssh[kMaxRSlabs];
   __shared__ uint32_t thr_s[kMaxRSlabs][33];
@@ -547,7 +548,10 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
     }
   }
   __syncthreads();
-  const uint64_t step0 = *stepp + step_off;
+  const uint64_t step0 = (stepp ? *stepp : 0) + step_off;
+  // (a launch that moves the counter on takes its first step by value, so
+  // no workgroup of it reads the counter)
+  if (step_out && blockIdx.x == 0 && tid == 0) *step_out = step0 + nsteps;
   for (uint32_t si = 0; si < nsteps; ++si) {
     const uint64_t step = step0 + si;
     const uint32_t half = (uint32_t)(step & 1u) * kRingHalf;
@@ -950,17 +954,18 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                     const uint64_t* stepp, uint32_t step_off, uint32_t nsteps, uint32_t* status, bool fine) {
+                     const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                     bool fine) {
   set_resident_attribute();
   hipEvent_t t0, t1;
   get_launch_timing(&t0, &t1);
   auto* k = fine ? k_resident<true> : k_resident<false>;
   if (t0)
     hipExtLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, rings, ver,
-                          stepp, step_off, nsteps, status);
+                          stepp, step_off, nsteps, step_out, status);
   else
     hipLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, grp, slabs, pts, words, rings, ver, stepp,
-                       step_off, nsteps, status);
+                       step_off, nsteps, step_out, status);
 }
 
 }  // namespace cvf

@@ -150,7 +150,7 @@ typedef struct cvf_tuning {
   int32_t block_sigma;  /* workgroup size of the sigma half-sweep (64..1024, power of 2) */
   int32_t block_eta;    /* workgroup size of the eta cube sweep */
   int32_t block_cell;   /* workgroup size of the per-cell kernels (SW, observables) */
-  int32_t graph_steps;  /* MC steps per replayed hipGraph (1..64) */
+  int32_t graph_steps;  /* MC steps per replayed hipGraph, or per resident launch (1..64) */
   int32_t fused;        /* 1: eta sweep + 6 half-sweeps per kernel on LDS-staged z-slabs
                            where the slab fits in LDS; 0: one kernel per half-sweep;
                            2: the resident kernel (every step of a graph in one launch, the
