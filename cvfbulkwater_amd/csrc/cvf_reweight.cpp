@@ -168,6 +168,13 @@ double ising_peak(double (*f)(double), bool by_x) {
   }
 }
 
+// the maxima of the two universal distributions, found once
+void ising_peaks(double* peak2d, double* peak3d) {
+  static const double p2 = ising_peak(cvf_rw_ising2d, true), p3 = ising_peak(cvf_rw_ising3d, false);
+  *peak2d = p2;
+  *peak3d = p3;
+}
+
 // The order-parameter histogram p of nm bins of width w from xmin, as
 // Calcula_Histograma_Rotado_normX has it after binning (f90:1466-1617):
 // bin centres into x, norm / mean / variance, the sine stretch, the same
@@ -235,29 +242,83 @@ struct cvf_reweight {
   bool have_ctes = false;
 
   hipStream_t stream = nullptr;
-  DMem<double> en, vn, lh, c0, c1, logp, pmax, mx, ps, lz, norm;
+  DMem<double> en, vn, lh, used, dens, sum, pmax, mx, ps, lz, norm;
   DMem<uint32_t> dcell;  // the occupied cells as i << 16 | w, for the projections
+  DMem<uint8_t> mixed;
+  DMem<RwMixed> mix;
+  DMem<uint32_t> plow, low;
   DMem<RwSim> sims;
-  DMem<double2> tgt;
   int32_t cap_t = 0, n_t = 0;
+  size_t cap_dens = 0;
   HMem<double> dist;  // [target][cell] densities of the last reweighting (pinned)
+  // a call's inputs (constants, targets, angles) go down in one copy
+  HMem<double> hin;
+  DMem<double> din;
+  size_t cap_in = 0;
+  // buffers and results of a scan, kept for the next one
+  DMem<double2> srange, sbin;
+  DMem<double> shist;
+  DMem<uint32_t> scode, scbin;
+  HMem<double> sout;
+  int32_t cap_pairs = 0, cap_angles = 0;
 
-  int32_t nblk() const { return (int32_t)((cell.size() + kRwBlock - 1) / kRwBlock); }
   RwCells cells() const { return RwCells{en.p, vn.p, lh.p, (int64_t)cell.size()}; }
-  RwWork work() const { return RwWork{logp.p, pmax.p, mx.p, ps.p, lz.p, norm.p, nblk()}; }
+  RwWork work(int32_t n) const {
+    RwWork w{sum.p, mixed.p, mix.p, pmax.p, mx.p, ps.p, plow.p, low.p, lz.p, norm.p, 0, 0, 0};
+    rw_shape((int64_t)cell.size(), n, &w);
+    return w;
+  }
   RwGeom geom() const { return RwGeom{dcell.p, (int64_t)cell.size(), nb, nm, e_min, de, rho_min, drho}; }
+  const double* dev_ctes() const { return din.p; }
+  RwTargets targets(int32_t n) const {
+    return RwTargets{reinterpret_cast<const double2*>(din.p + in_targets()), n};
+  }
+  const double2* dev_angles(int32_t n) const {
+    return reinterpret_cast<const double2*>(din.p + in_targets() + 2 * (size_t)n);
+  }
+  size_t in_targets() const { return ((size_t)n_sim + 1) & ~(size_t)1; }  // 16-byte aligned
 
   int reserve_targets(int32_t n) {
     if (n <= cap_t) return CVF_OK;
-    const size_t nc = cell.size(), b = (size_t)nblk();
-    HIPR(logp.alloc((size_t)n * nc));
-    HIPR(pmax.alloc((size_t)n * b));
-    HIPR(ps.alloc((size_t)n * b * 2));
+    const size_t nc = cell.size(), b = kRwMaxBlocks, rows = ((size_t)n + kRwRow - 1) / kRwRow;
+    cap_t = 0;
+    HIPR(sum.alloc(rows * nc));
+    HIPR(mixed.alloc(rows * nc));
+    HIPR(pmax.alloc(rows * kRwRow * b));
+    HIPR(ps.alloc(rows * kRwRow * b * kRwScanSums));
+    HIPR(plow.alloc((size_t)n * b));
+    HIPR(low.alloc(n));
     HIPR(mx.alloc(n));
     HIPR(lz.alloc(n));
     HIPR(norm.alloc(n));
-    HIPR(tgt.alloc(n));
     cap_t = n;
+    return CVF_OK;
+  }
+
+  // constants (null: zero), (beta, p) of the targets and (sin, cos) of the
+  // angles to the device
+  int upload_inputs(const double* c, int32_t n, const double* T_K, const double* P_bar, int32_t n_a = 0,
+                    const double* alpha = nullptr) {
+    const size_t m = in_targets() + 2 * (size_t)n + 2 * (size_t)n_a;
+    if (m > cap_in) {
+      cap_in = 0;
+      HIPR(hin.resize(m));
+      HIPR(din.alloc(m));
+      cap_in = m;
+    }
+    double* h = hin.data();
+    for (size_t j = 0; j < in_targets(); ++j) h[j] = c && j < (size_t)n_sim ? c[j] : 0.0;
+    h += in_targets();
+    for (int32_t t = 0; t < n; ++t) {
+      h[2 * t] = 1000. / (sl(0.2293f) * T_K[t]);
+      h[2 * t + 1] = P_bar[t] * 100.0;
+    }
+    h += 2 * (size_t)n;
+    for (int32_t a = 0; a < n_a; ++a) {
+      h[2 * a] = sin(alpha[a]);  // as Rotate's sin / cos
+      h[2 * a + 1] = cos(alpha[a]);
+    }
+    HIPR(hipMemcpyAsync(din.p, hin.data(), m * sizeof(double), hipMemcpyHostToDevice, stream));
     return CVF_OK;
   }
 
@@ -392,8 +453,8 @@ int cvf_rw_create(int32_t L, int32_t n_sim, const double* T_hat, const double* P
   HIPR(rw->en.alloc(nc));
   HIPR(rw->vn.alloc(nc));
   HIPR(rw->lh.alloc(nc));
-  HIPR(rw->c0.alloc(n_sim));
-  HIPR(rw->c1.alloc(n_sim));
+  HIPR(rw->used.alloc(n_sim));
+  HIPR(rw->mix.alloc(nc));
   HIPR(rw->sims.alloc(n_sim));
   HIPR(rw->dcell.alloc(nc));
   {
@@ -443,23 +504,22 @@ int cvf_rw_solve_constants(cvf_reweight* rw, int32_t steps, double* ctes, double
   if (steps < 0) return set_error(CVF_EINVAL, "negative step count");
   HIPR(hipSetDevice(rw->device));
   if (int rc = rw->reserve_targets(rw->n_sim)) return rc;
-  // the targets of a sweep are the simulations themselves
-  std::vector<double2> bp(rw->n_sim);
-  for (int j = 0; j < rw->n_sim; ++j) bp[j] = double2{1000. / (sl(0.2293f) * rw->T[j]), rw->P[j] * 100.0};
-  HIPR(hipMemcpyAsync(rw->tgt.p, bp.data(), bp.size() * sizeof(double2), hipMemcpyHostToDevice, rw->stream));
-  HIPR(hipMemsetAsync(rw->c0.p, 0, rw->n_sim * sizeof(double), rw->stream));
-  HIPR(hipMemsetAsync(rw->c1.p, 0, rw->n_sim * sizeof(double), rw->stream));
-  double *cur = rw->c0.p, *nxt = rw->c1.p;
-  const RwTargets tg{rw->tgt.p, rw->n_sim};
-  for (int s = 0; s < steps; ++s) {
-    HIPR(launch_rw_pass(rw->cells(), rw->sims.p, cur, rw->n_sim, tg, rw->work(), rw->de, rw->drho, nxt, false,
-                        rw->stream));
-    std::swap(cur, nxt);
+  // the targets of a sweep are the simulations themselves; each sweep's
+  // first launch takes its constants from the partial sums of the one before
+  if (int rc = rw->upload_inputs(nullptr, rw->n_sim, rw->T.data(), rw->P.data())) return rc;
+  const RwTargets tg = rw->targets(rw->n_sim);
+  for (int s = 0; s < steps; ++s)
+    HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), rw->geom(), kRwSweep,
+                        s > 0, rw->used.p, rw->stream));
+  std::vector<double> z(rw->n_sim, 0.0), prev(rw->n_sim, 0.0);
+  if (steps > 0) {
+    HIPR(launch_rw_finish(tg, rw->work(tg.n), rw->geom(), kRwSweep, nullptr, rw->stream));
+    HIPR(hipMemcpyAsync(z.data(), rw->lz.p, rw->n_sim * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
+    if (steps > 1)  // the first sweep starts from zero
+      HIPR(hipMemcpyAsync(prev.data(), rw->used.p, rw->n_sim * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
   }
-  std::vector<double> prev(rw->n_sim);
-  HIPR(hipMemcpyAsync(ctes, cur, rw->n_sim * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
-  HIPR(hipMemcpyAsync(prev.data(), nxt, rw->n_sim * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
   HIPR(hipStreamSynchronize(rw->stream));
+  for (int j = 0; j < rw->n_sim; ++j) ctes[j] = z[j] - z[0];
   if (ctes_prev) std::copy(prev.begin(), prev.end(), ctes_prev);
   rw->ctes.assign(ctes, ctes + rw->n_sim);
   rw->have_ctes = true;
@@ -479,17 +539,22 @@ int cvf_rw_reweight(cvf_reweight* rw, int32_t n_targets, const double* T_K, cons
     if (!(T_K[t] > 0)) return set_error(CVF_EINVAL, "target %d: T = %g K", t, T_K[t]);
   HIPR(hipSetDevice(rw->device));
   if (int rc = rw->reserve_targets(n_targets)) return rc;
-  std::vector<double2> bp(n_targets);
-  for (int t = 0; t < n_targets; ++t) bp[t] = double2{1000. / (sl(0.2293f) * T_K[t]), P_bar[t] * 100.0};
-  HIPR(hipMemcpyAsync(rw->tgt.p, bp.data(), bp.size() * sizeof(double2), hipMemcpyHostToDevice, rw->stream));
-  HIPR(hipMemcpyAsync(rw->c0.p, rw->ctes.data(), rw->n_sim * sizeof(double), hipMemcpyHostToDevice, rw->stream));
-  HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->c0.p, rw->n_sim, RwTargets{rw->tgt.p, n_targets}, rw->work(),
-                      rw->de, rw->drho, nullptr, true, rw->stream));
   const size_t nc = rw->cell.size();
+  if ((size_t)n_targets * nc > rw->cap_dens) {
+    rw->cap_dens = 0;
+    HIPR(rw->dens.alloc((size_t)n_targets * nc));
+    rw->cap_dens = (size_t)n_targets * nc;
+  }
+  if (int rc = rw->upload_inputs(rw->ctes.data(), n_targets, T_K, P_bar)) return rc;
+  const RwTargets tg = rw->targets(n_targets);
+  HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), rw->geom(), kRwDensity,
+                      false, nullptr, rw->stream));
+  HIPR(launch_rw_finish(tg, rw->work(tg.n), rw->geom(), kRwDensity, nullptr, rw->stream));
+  HIPR(launch_rw_dist(rw->cells(), tg, rw->work(tg.n), rw->dens.p, rw->stream));
   rw->n_t = 0;
   HIPR(rw->dist.resize((size_t)n_targets * nc));
   rw->n_t = n_targets;
-  HIPR(hipMemcpyAsync(rw->dist.data(), rw->logp.p, rw->dist.size() * sizeof(double), hipMemcpyDeviceToHost,
+  HIPR(hipMemcpyAsync(rw->dist.data(), rw->dens.p, rw->dist.size() * sizeof(double), hipMemcpyDeviceToHost,
                       rw->stream));
   std::vector<double> z(n_targets);
   HIPR(hipMemcpyAsync(z.data(), rw->lz.p, n_targets * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
@@ -584,75 +649,53 @@ int cvf_rw_scan(cvf_reweight* rw, int32_t n_targets, const double* T_K, const do
     if (!(T_K[t] > 0)) return set_error(CVF_EINVAL, "target %d: T = %g K", t, T_K[t]);
   HIPR(hipSetDevice(rw->device));
   if (int rc = rw->reserve_targets(n_targets)) return rc;
-  // densities of every target, left on the device
-  std::vector<double2> bp(n_targets);
-  for (int t = 0; t < n_targets; ++t) bp[t] = double2{1000. / (sl(0.2293f) * T_K[t]), P_bar[t] * 100.0};
-  HIPR(hipMemcpyAsync(rw->tgt.p, bp.data(), bp.size() * sizeof(double2), hipMemcpyHostToDevice, rw->stream));
-  HIPR(hipMemcpyAsync(rw->c0.p, rw->ctes.data(), rw->n_sim * sizeof(double), hipMemcpyHostToDevice, rw->stream));
-  HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->c0.p, rw->n_sim, RwTargets{rw->tgt.p, n_targets}, rw->work(),
-                      rw->de, rw->drho, nullptr, true, rw->stream));
-  rw->n_t = 0;  // the host copy of the densities no longer matches the device
+  rw->n_t = 0;  // no densities are kept for the per-target calls
+  if (nta > rw->cap_pairs || n_angles > rw->cap_angles) {
+    const size_t pairs = (size_t)std::max(nta, rw->cap_pairs), ang = (size_t)std::max(n_angles, rw->cap_angles);
+    rw->cap_pairs = rw->cap_angles = 0;
+    HIPR(rw->srange.alloc((ang + pairs) * kRwProjBlocks));
+    HIPR(rw->sbin.alloc(pairs + ang));
+    HIPR(rw->scbin.alloc(ang * rw->cell.size()));  // at most a group per angle
+    HIPR(rw->shist.alloc(pairs * kRwProjBlocks * nm));
+    HIPR(rw->scode.alloc(pairs));
+    // 2 cumulants per target (at most one target per pair), 2 nm + 9 numbers
+    // and a code per pair
+    HIPR(rw->sout.resize(pairs * (2 * (size_t)nm + 12)));
+    rw->cap_pairs = (int32_t)pairs;
+    rw->cap_angles = (int32_t)ang;
+  }
+  if (int rc = rw->upload_inputs(rw->ctes.data(), n_targets, T_K, P_bar, n_angles, alpha)) return rc;
+  const RwTargets tg = rw->targets(n_targets);
   const RwGeom g = rw->geom();
-  std::vector<double2> sc(n_angles);
-  for (int a = 0; a < n_angles; ++a) sc[a] = double2{sin(alpha[a]), cos(alpha[a])};  // as Rotate's sin / cos
-  DMem<double2> dsc, dbin;
-  DMem<double> pm, px, ph;
-  DMem<uint32_t> derr;
-  const int B = kRwProjBlocks;
-  HIPR(dsc.alloc(n_angles));
-  HIPR(dbin.alloc(nta));
-  HIPR(pm.alloc((size_t)n_targets * B * 5));
-  HIPR(px.alloc((size_t)nta * B * 2));
-  HIPR(ph.alloc((size_t)nta * B * nm));
-  HIPR(derr.alloc(1));
-  HIPR(hipMemcpyAsync(dsc.p, sc.data(), sc.size() * sizeof(double2), hipMemcpyHostToDevice, rw->stream));
-  HIPR(launch_rw_moments(g, rw->logp.p, n_targets, pm.p, rw->stream));
-  HIPR(launch_rw_xrange(g, rw->logp.p, n_targets, n_angles, dsc.p, px.p, rw->stream));
-  std::vector<double> hm((size_t)n_targets * B * 5), hx((size_t)nta * B * 2);
-  HIPR(hipMemcpyAsync(hm.data(), pm.p, hm.size() * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
-  HIPR(hipMemcpyAsync(hx.data(), px.p, hx.size() * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
+  RwScanOut out;
+  out.binder_ed = rw->sout.data();
+  out.x = out.binder_ed + 2 * (size_t)n_targets;
+  out.p = out.x + (size_t)nta * nm;
+  out.stats3 = out.p + (size_t)nta * nm;
+  out.scores6 = out.stats3 + 3 * (size_t)nta;
+  out.code = reinterpret_cast<uint32_t*>(out.scores6 + 6 * (size_t)nta);
+  HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), g, kRwScan, false, nullptr,
+                      rw->stream));
+  HIPR(launch_rw_finish(tg, rw->work(tg.n), g, kRwScan, out.binder_ed, rw->stream));
+  const RwScan sc{rw->dev_angles(n_targets), n_angles, rw->srange.p, rw->sbin.p + n_angles, rw->sbin.p,
+                  rw->scbin.p, rw->shist.p, rw->scode.p};
+  double peak2d, peak3d;
+  ising_peaks(&peak2d, &peak3d);
+  HIPR(launch_rw_project(rw->cells(), tg, rw->work(tg.n), g, sc, peak2d, peak3d, out, rw->stream));
   HIPR(hipStreamSynchronize(rw->stream));
-  // Binder cumulants of the marginals: <x^2> = sum v x^2 / sum v
-  for (int t = 0; t < n_targets; ++t) {
-    double m[5] = {0, 0, 0, 0, 0};
-    for (int b = 0; b < B; ++b)
-      for (int k = 0; k < 5; ++k) m[k] += hm[((size_t)t * B + b) * 5 + k];
-    binder_ed[2 * t] = 1.0 - (m[2] / m[0]) / (3.0 * (m[1] / m[0]) * (m[1] / m[0]));
-    binder_ed[2 * t + 1] = 1.0 - (m[4] / m[0]) / (3.0 * (m[3] / m[0]) * (m[3] / m[0]));
-  }
-  // bins: the range over the occupied cells, two empty bins each side
-  std::vector<double2> bins(nta);
+  for (int ta = 0; ta < nta; ++ta)
+    if (out.code[ta] & kRwNoCell) return set_error(CVF_ERANGE, "target %d: no cell of positive density", ta / n_angles);
+  for (int ta = 0; ta < nta; ++ta)
+    if (out.code[ta] & kRwOutside) return set_error(CVF_ERANGE, "an order parameter fell outside its histogram");
   for (int ta = 0; ta < nta; ++ta) {
-    double xmin = sl(1E12f), xmax = sl(-1E12f);
-    for (int b = 0; b < B; ++b) {
-      xmin = std::min(xmin, hx[2 * ((size_t)ta * B + b)]);
-      xmax = std::max(xmax, hx[2 * ((size_t)ta * B + b) + 1]);
-    }
-    if (!(xmax >= xmin)) return set_error(CVF_ERANGE, "target %d: no cell of positive density", ta / n_angles);
-    double range = xmax - xmin, w = range / nm;
-    range = range + 4 * w;
-    xmin = xmin - 2 * w;
-    w = range / nm;
-    bins[ta] = double2{xmin, w};
+    if (out.code[ta] & kRwMoments) return set_error(CVF_ERANGE, "order-parameter moments off");
+    if (out.code[ta] & kRwStretched) return set_error(CVF_ERANGE, "stretched order-parameter moments off");
   }
-  HIPR(hipMemcpyAsync(dbin.p, bins.data(), bins.size() * sizeof(double2), hipMemcpyHostToDevice, rw->stream));
-  HIPR(hipMemsetAsync(derr.p, 0, sizeof(uint32_t), rw->stream));
-  HIPR(launch_rw_xhist(g, rw->logp.p, n_targets, n_angles, dsc.p, dbin.p, ph.p, derr.p, rw->stream));
-  // the workgroups' partial histograms summed on the device, in workgroup order
-  DMem<double> phs;
-  HIPR(phs.alloc((size_t)nta * nm));
-  HIPR(launch_rw_xhist_sum(ph.p, nta, nm, phs.p, rw->stream));
-  uint32_t err = 0;
-  HIPR(hipMemcpyAsync(p, phs.p, (size_t)nta * nm * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
-  HIPR(hipMemcpyAsync(&err, derr.p, sizeof err, hipMemcpyDeviceToHost, rw->stream));
-  HIPR(hipStreamSynchronize(rw->stream));
-  if (err) return set_error(CVF_ERANGE, "an order parameter fell outside its histogram");
-  for (int ta = 0; ta < nta; ++ta) {
-    double* xo = x + (size_t)ta * nm;
-    double* po = p + (size_t)ta * nm;
-    if (int rc = finish_order_parameter(bins[ta].x, bins[ta].y, nm, xo, po, stats3 + 3 * ta)) return rc;
-    if (int rc = cvf_rw_ising_scores(xo, po, nm, scores6 + 6 * ta)) return rc;
-  }
+  std::copy_n(out.binder_ed, 2 * (size_t)n_targets, binder_ed);
+  std::copy_n(out.x, (size_t)nta * nm, x);
+  std::copy_n(out.p, (size_t)nta * nm, p);
+  std::copy_n(out.stats3, 3 * (size_t)nta, stats3);
+  std::copy_n(out.scores6, 6 * (size_t)nta, scores6);
   return CVF_OK;
 }
 
@@ -672,7 +715,8 @@ double cvf_rw_ising3d(double z) {
 
 int cvf_rw_ising_scores(const double* x, const double* p, int32_t n, double* out6) {
   if (!x || !p || !out6 || n < 1) return set_error(CVF_EINVAL, "bad arguments");
-  static const double peak2d = ising_peak(cvf_rw_ising2d, true), peak3d = ising_peak(cvf_rw_ising3d, false);
+  double peak2d, peak3d;
+  ising_peaks(&peak2d, &peak3d);
   double kl2 = 0, kl3 = 0, liu2 = 0, liu3 = 0;
   int n_liu = 0;
   for (int i = 0; i < n; ++i) {

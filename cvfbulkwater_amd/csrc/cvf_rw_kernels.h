@@ -1,5 +1,6 @@
 // Device side of the histogram reweighting (include/cvf_reweight.h): the
-// per-cell log-sum over simulations and the per-target reductions.
+// per-cell log-sum over simulations, the per-target reductions and the
+// projections of a scan.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -8,6 +9,12 @@
 namespace cvf {
 
 constexpr int kRwBlock = 256;
+constexpr int kRwRow = 16;          // targets that share one pass over the cells' simulation sums
+constexpr int kRwProjBlocks = 64;   // workgroups per target (or pair) of a projection
+// what a pass is for: a sweep of the constants (log_Z alone), densities
+// (and the normalization), a scan (and the moments of the marginals)
+enum { kRwSweep = 0, kRwDensity = 1, kRwScan = 2 };
+constexpr int kRwScanSums = 6;
 
 // One simulation of the reweighting sums: beta_j = 1000/(0.2293 T_j) in
 // mol/kJ, p_j = 100 P_j in kPa, lm_j = log(real(medidas_j)).
@@ -28,23 +35,25 @@ struct RwTargets {
   int32_t n;
 };
 
-// Buffers of one reweighting pass over n targets.
-struct RwWork {
-  double* logp;  // [target][cell]: log_P, then (with dist) the density
-  double* pmax;  // [target][block] partial maxima
-  double* mx;    // [target] max log_P
-  double* ps;    // [target][block][2] partial sums (truncated, full)
-  double* lz;    // [target] log_Z
-  double* norm;  // [target] sum of exp(log_P - log_Z) * de * drho
-  int32_t nblk;
+// Both sums of a cell and the bounds that pick one.
+struct RwMixed {
+  double near, all, umax, umin;
 };
 
-// log_P and log_Z of every target (Calcula_Histograma over all targets);
-// with ctes_out, also writes log_Z(t) - log_Z(0) there (one Jacobi sweep
-// of the constants); with dist, replaces log_P by the normalized density.
-hipError_t launch_rw_pass(const RwCells& cells, const RwSim* sims, const double* ctes, int32_t n_sim,
-                          const RwTargets& tg, const RwWork& w, double de, double drho, double* ctes_out,
-                          bool dist, hipStream_t stream);
+// Buffers of one reweighting pass over n targets.
+struct RwWork {
+  double* sum;     // [row][cell]: the simulation sum that the row's targets use
+  uint8_t* mixed;  // [row][cell]: the row's targets use different ones (mix[cell])
+  RwMixed* mix;    // [cell], written where mixed
+  double* pmax;    // [row][block][target of the row] partial maxima of log_P
+  double* mx;      // [target] max log_P
+  double* ps;      // [sum][row][block][target of the row] partial sums
+  uint32_t* plow;  // [target][block] of a scan: a density may have underflowed
+  uint32_t* low;   // [target] the same
+  double* lz;      // [target] log_Z
+  double* norm;    // [target] sum of exp(log_P - log_Z) * de * drho
+  int32_t rows, nblk, threads;  // rows of targets; launch shape (rw_shape)
+};
 
 // Grid geometry for the projections: cell = i << 16 | w (nb < 2^16), energy
 // e_min + (i + 1/2) de (kJ/mol), density rho_min + (w + 1/2) drho (kg/m^3).
@@ -55,28 +64,45 @@ struct RwGeom {
   double e_min, de, rho_min, drho;
 };
 
-constexpr int kRwProjBlocks = 64;  // workgroups per target (or target x angle) of a projection
+// Buffers of a scan's projections; pair ta = target * n_a + angle.
+struct RwScan {
+  const double2* angle;  // (sin, cos) per angle
+  int32_t n_a;
+  double2* range;  // [n_a + pairs][kRwProjBlocks]: min and max of x
+  double2* bin;    // [pair]: first bin's lower edge, bin width
+  double2* gbin;   // [n_a]: the same over all the grid's cells
+  uint32_t* cbin;  // [group of up to 4 angles][cell]: the cell's bins, a byte per angle
+  double* hist;    // [pair][kRwProjBlocks][nm]
+  uint32_t* code;  // [pair]: kRwNoCell, kRwOutside
+};
+// What went wrong with a pair: no cell of positive density, an x outside its
+// bins, moments off before or after the axis stretch.
+enum : uint32_t { kRwNoCell = 1, kRwOutside = 2, kRwMoments = 4, kRwStretched = 8 };
+// A scan's results, written straight to pinned host memory.
+struct RwScanOut {
+  double *binder_ed, *x, *p, *stats3, *scores6;
+  uint32_t* code;
+};
 
-// Per target t (density dens[t][cell]): partial sums over each workgroup's
-// cells of {v, v e^2, v e^4, v rho^2, v rho^4} -> part[t][block][5]
-// (kRwProjBlocks blocks), for the Binder cumulants of the marginals.
-hipError_t launch_rw_moments(const RwGeom& g, const double* dens, int32_t n_t, double* part, hipStream_t st);
+// Fills in the launch shape of a pass over n_cells cells.
+constexpr int kRwMaxBlocks = 256;  // workgroups per row of targets
+void rw_shape(int64_t n_cells, int32_t n_targets, RwWork* w);
 
-// Per (target, angle) pair ta = t * n_a + a: the min and max of
-// x = e sin(a) + rho cos(a) over the cells with density > 0 ->
-// part[ta][block][2].  sc holds (sin, cos) per angle.
-hipError_t launch_rw_xrange(const RwGeom& g, const double* dens, int32_t n_t, int32_t n_a, const double2* sc,
-                            double* part, hipStream_t st);
-
-// Per pair ta, the histogram of x over nm bins of width w from x0
-// (binfo[ta] = (x0, w)), weighted by the density: part[ta][block][nm],
-// summed in a fixed order (reproducible).  A cell with density > 0 outside
-// the bins (and not within 1e-10 of x0, which goes to bin 0) sets *err.
-hipError_t launch_rw_xhist(const RwGeom& g, const double* dens, int32_t n_t, int32_t n_a, const double2* sc,
-                           const double2* binfo, double* part, uint32_t* err, hipStream_t st);
-
-// out[ta][k] = sum over the kRwProjBlocks workgroups b, in order, of
-// part[ta][b][k] (n_ta pairs, nm bins).
-hipError_t launch_rw_xhist_sum(const double* part, int32_t n_ta, int32_t nm, double* out, hipStream_t st);
+// One pass over the cells for every target (Calcula_Histograma over all
+// targets): the cells' sums, then the partial sums of `mode`.  chain: the
+// constants are log_Z(t) - log_Z(0) of the pass before (a kRwSweep pass over
+// the same targets, the simulations themselves), written to `used`.
+hipError_t launch_rw_pass(const RwCells& cells, const RwSim* sims, const double* ctes, int32_t n_sim,
+                          const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, bool chain, double* used,
+                          hipStream_t stream);
+// log_Z, norm and (kRwScan) the Binder cumulants {energy, density} per target
+hipError_t launch_rw_finish(const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, double* binder_ed,
+                            hipStream_t st);
+// dens[target][cell] = exp(log_P - log_Z) / norm
+hipError_t launch_rw_dist(const RwCells& cells, const RwTargets& tg, const RwWork& w, double* dens, hipStream_t st);
+// The order parameter of every pair (Calcula_Histograma_Rotado_normX, binder,
+// ConfrontIsing, ZeroTest, HeightTest) after a finished kRwScan pass.
+hipError_t launch_rw_project(const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwGeom& g,
+                             const RwScan& sc, double peak2d, double peak3d, const RwScanOut& out, hipStream_t st);
 
 }  // namespace cvf

@@ -17,15 +17,39 @@
 //  - log_Z drops cells more than 10 below the largest log_P (1106-1118).
 // Factoring t1 out rounds differently from the reference's left-to-right
 // sum: log_P moves by about |t1| x 1e-16 (1e-10 for L = 8).
+//
+// No kernel stores log_P: it is a few flops from the cell's sum, so every
+// pass forms it again from 33 bytes per cell (which stay in the caches)
+// instead of writing and reading 8 bytes per cell and target.  At the
+// production shape (710,000 cells, 11 simulations) a constants' sweep went
+// from three launches of 31.8 + 17.8 + 6.0 us to two of 26.0 + 17.7, and a
+// scan of 64 targets x 3 angles from 1.17 ms of kernels over 363 MB of
+// densities to 0.57 ms.
 #include <math.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "cvf_rw_kernels.h"
 
 namespace cvf {
 namespace {
 
-constexpr int kTargetsPerBlock = 16;  // targets served per k_rw_logp block
-constexpr int kSumBlocks = 128;       // k_rw_sum blocks per target (grid-stride)
+constexpr double kUnderflow = -700.0;  // log densities above it are positive doubles, see k_rw_sum
+
+// max and min of doubles, one instruction each (fmax and fmin put a
+// canonicalizing one before it where an operand's origin is unknown); a NaN
+// operand gives the other one
+__device__ inline double max1(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline double min1(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 
 __device__ inline double wave_max(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
@@ -37,149 +61,455 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-// block-wide reduction of kRwBlock threads, result in every thread
+// block-wide reduction, result in every thread (red: one entry per wave)
 template <bool kMax>
 __device__ inline double block_reduce(double v, double* red) {
   v = kMax ? wave_max(v) : wave_sum(v);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
   if (lane == 0) red[wave] = v;
   __syncthreads();
   double r = red[0];
-  for (int i = 1; i < kRwBlock / 64; ++i) r = kMax ? fmax(r, red[i]) : r + red[i];
+  for (int i = 1; i < nw; ++i) r = kMax ? fmax(r, red[i]) : r + red[i];
   __syncthreads();
   return r;
+}
+
+// exp(d) for d <= 0 (or NaN): d = k ln2 + r, |r| <= ln2 / 2, and the degree-11
+// Chebyshev interpolant of e^r there (1.6e-17 relative; coefficients computed
+// for this file to 60 digits).  Seven instructions fewer than the library's
+// exp, which also serves large arguments: a third of a pass is exponentials.
+__device__ inline double exp_le0(double d) {
+  const double k = __builtin_rint(d * 0x1.71547652b82fep+0);
+  double r = __builtin_fma(k, -0x1.62e42fefa39efp-1, d);
+  r = __builtin_fma(k, -0x1.abc9e3b39803fp-56, r);
+  double p = 0x1.af632a0f7e2cep-26;
+  p = __builtin_fma(p, r, 0x1.28b4101c77212p-22);
+  p = __builtin_fma(p, r, 0x1.71ddf56d8deb5p-19);
+  p = __builtin_fma(p, r, 0x1.a01991a10d9aep-16);
+  p = __builtin_fma(p, r, 0x1.a01a01b1461c5p-13);
+  p = __builtin_fma(p, r, 0x1.6c16c1880029fp-10);
+  p = __builtin_fma(p, r, 0x1.111111110f21ep-7);
+  p = __builtin_fma(p, r, 0x1.555555554f0bap-5);
+  p = __builtin_fma(p, r, 0x1.555555555555ap-3);
+  p = __builtin_fma(p, r, 0x1.0000000000011p-1);
+  p = __builtin_fma(p, r, 1.0);
+  p = __builtin_fma(p, r, 1.0);
+  // below -745.14 the result is zero (and k may be no int)
+  return d < -746.0 ? 0.0 : __builtin_ldexp(p, (int)k);
+}
+
+// (a & m) | (b & ~m) of the bits of two doubles, m all ones or all zeros (a
+// conditional between two elements of an array would become an indexed read
+// of it, a chain of selects over all its elements)
+__device__ inline double pick_bits(uint32_t m, double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const uint32_t lo = ((uint32_t)x & m) | ((uint32_t)y & ~m);
+  const uint32_t hi = ((uint32_t)(x >> 32) & m) | ((uint32_t)(y >> 32) & ~m);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// Sums (or maxima) of N values over the wavefront, N a power of two: value i
+// ends in the lanes whose bits 5, 4, ... spell i from its highest bit on.
+// Each step halves the values that a lane still carries, so N values cost
+// N - 1 + log2(64 / N) exchanges and not 6 N.
+template <int N, bool kMax>
+__device__ inline void wave_reduce(double (&v)[N]) {
+  int m = 32;
+#pragma unroll
+  for (int n = N; n > 1; n /= 2, m /= 2) {
+    const uint32_t up = (threadIdx.x & m) ? ~0u : 0u;
+#pragma unroll
+    for (int i = 0; i < n / 2; ++i) {
+      const double keep = pick_bits(up, v[i + n / 2], v[i]), give = pick_bits(up, v[i], v[i + n / 2]);
+      const double got = __shfl_xor(give, m);
+      v[i] = kMax ? max1(keep, got) : keep + got;
+    }
+  }
+#pragma unroll
+  for (; m > 0; m /= 2) {
+    const double got = __shfl_xor(v[0], m);
+    v[0] = kMax ? max1(v[0], got) : v[0] + got;
+  }
+}
+// the value that a lane holds after wave_reduce<N>, and whether it is the
+// first lane of those that hold it
+template <int N>
+__device__ inline int reduced_index() {
+  int i = 0;
+  for (int n = N, m = 32; n > 1; n /= 2, m /= 2) i += (threadIdx.x & m) ? n / 2 : 0;
+  return i;
+}
+template <int N>
+__device__ inline bool reduced_first() {
+  return (threadIdx.x & (64 / N - 1)) == 0;
+}
+
+// The wavefronts' results red[slot][wave] of a workgroup combined, four lanes
+// per slot: valid in the threads 4 slot .. 4 slot + 3 that the call covers.
+template <bool kMax>
+__device__ inline double combine_waves(const double (*red)[16]) {
+  const int nw = blockDim.x >> 6, slot = threadIdx.x >> 2, q = threadIdx.x & 3;
+  double v = kMax ? -INFINITY : 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int wv = 4 * i + q;
+    const double x = red[slot][wv < nw ? wv : q];  // (q < nw: at least four wavefronts)
+    if (wv < nw) v = kMax ? fmax(v, x) : v + x;
+  }
+  for (int m = 1; m < 4; m *= 2) {
+    const double x = __shfl_xor(v, m);
+    v = kMax ? fmax(v, x) : v + x;
+  }
+  return v;
+}
+
+// T partial results of nblk workgroups each, kRwRow apart (p[i * kRwRow + k]):
+// their sums or maxima into out[0..T), all threads loading at once (one
+// latency, not one per result).  red: 16 x 16 of LDS; out(k, result) runs in
+// one thread per result.
+template <int T, bool kMax, class Out>
+__device__ inline void reduce_partials(const double* p, int nblk, double (*red)[16], Out&& out) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double v = kMax ? -INFINITY : 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x / T; i < nblk; i += blockDim.x / T) {
+    const double x = p[i * kRwRow + (threadIdx.x & (T - 1))];
+    v = kMax ? fmax(v, x) : v + x;
+  }
+#pragma unroll
+  for (int m = T; m < 64; m *= 2) {
+    const double x = __shfl_xor(v, m);
+    v = kMax ? fmax(v, x) : v + x;
+  }
+  if (lane < T) red[lane][wave] = v;
+  __syncthreads();
+  if ((int)threadIdx.x < 4 * T) {
+    v = combine_waves<kMax>(red);
+    if ((threadIdx.x & 3) == 0) out((int)(threadIdx.x >> 2), v);
+  }
 }
 
 // u_j = -beta_j (E + p_j V) - c_j + lm_j; s = {beta, p, c, lm}
 __device__ inline double rw_u(double E, double V, const double* s) { return -(s[0] * (E + s[1] * V)) - s[2] + s[3]; }
 
-__global__ __launch_bounds__(kRwBlock) void k_rw_logp(RwCells cells, const RwSim* __restrict__ sims,
-                                                      const double* __restrict__ ctes, int32_t n_sim,
-                                                      RwTargets tg, double* __restrict__ logp,
-                                                      double* __restrict__ pmax, int32_t nblk) {
-  extern __shared__ double sl[];  // 4 per simulation: beta, p, c, lm
-  __shared__ double red[kTargetsPerBlock][kRwBlock / 64];
-  for (int j = threadIdx.x; j < n_sim; j += kRwBlock) {
+// log_P of a cell for one target: t1 shifts the cell's sum, and picks it
+// where the targets of a row disagree (a mixed cell).
+__device__ inline double rw_t1(double E, double V, double2 bp) { return bp.x * (E + bp.y * V); }
+__device__ inline bool rw_cut(double t1, double umax, double umin) { return t1 + umax > 10.0 || t1 + umin < -10.0; }
+
+// 0, unknown to the compiler: an LDS index that includes it is read where it
+// stands, in each round of the loop, instead of all targets' values being
+// held in registers across it (which spills)
+__device__ inline int opaque_zero() {
+  int z = 0;
+  asm volatile("" : "+v"(z));
+  return z;
+}
+
+// A thread's first cell of the grid-stride walk: a wavefront's 64 cells
+// together, the workgroups' first wavefronts before their second ones, so
+// that the last, partial round is spread over all CUs.
+__device__ inline int64_t first_cell() {
+  return ((int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * 64 + (threadIdx.x & 63);
+}
+
+struct CellIn {
+  double E, V, lh, S;
+  bool mixed;
+};
+__device__ inline CellIn cell_in(const RwCells& c, const RwWork& w, int row, int64_t b) {
+  return CellIn{c.en[b], c.vn[b], c.lh[b], w.sum[(int64_t)row * c.n + b], w.mixed[(int64_t)row * c.n + b] != 0};
+}
+__device__ inline double cell_sum(const CellIn& c, const RwWork& w, int64_t b, double t1) {
+  if (!c.mixed) return c.S;
+  const RwMixed m = w.mix[b];
+  return rw_cut(t1, m.umax, m.umin) ? m.near : m.all;
+}
+__device__ inline double cell_logp(const CellIn& c, const RwWork& w, int64_t b, double2 bp) {
+  const double t1 = rw_t1(c.E, c.V, bp);
+  return c.lh - (t1 + cell_sum(c, w, b, t1));
+}
+
+// The cells' sums over the simulations for a row of kRwRow targets
+// (blockIdx.y), and the row's partial maxima of log_P.  A sweep of the
+// constants takes them from the previous sweep's partial sums (`ps`, not
+// null), each workgroup reducing them for itself, so that no launch lies
+// between two sweeps but k_rw_sum; workgroup 0 writes them to `used`.
+// Bound by FP64 issue (n_sim exponentials per cell); a thread takes several
+// cells, so that the maxima are reduced across lanes once per workgroup and
+// not once per cell (those shuffles cost as much as the exponentials).
+template <int R>
+__global__ __launch_bounds__(1024) void k_rw_cells(RwCells cells, const RwSim* __restrict__ sims,
+                                                   const double* __restrict__ ctes, int32_t n_sim, RwTargets tg,
+                                                   RwWork w, const double* __restrict__ ps,
+                                                   const double* __restrict__ mx, double* __restrict__ used) {
+  extern __shared__ double sl[];  // 4 per simulation: beta, p, c, lm; then log_Z of each
+  __shared__ double red[16][16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int j = threadIdx.x; j < n_sim; j += blockDim.x) {
     sl[4 * j] = sims[j].beta;
     sl[4 * j + 1] = sims[j].pres;
-    sl[4 * j + 2] = ctes[j];
+    sl[4 * j + 2] = ps ? 0.0 : ctes[j];
     sl[4 * j + 3] = sims[j].lm;
   }
+  // the row's targets, the last one repeated to fill it: the loop over them
+  // below then has no branch, and no global load stalls it
+  const int row = blockIdx.y, t0 = row * kRwRow, nt = min(tg.n - t0, kRwRow);
+  __shared__ double2 bps[R];
+  if ((int)threadIdx.x < R) bps[threadIdx.x] = tg.bp[t0 + min((int)threadIdx.x, nt - 1)];
+  if (ps) {
+    double* lz = sl + 4 * n_sim;  // log_Z of the sweep before
+    for (int j0 = 0; j0 < n_sim; j0 += kRwRow) {
+      reduce_partials<kRwRow, false>(ps + (int64_t)j0 * w.nblk, w.nblk, red, [&](int k, double st) {
+        if (j0 + k < n_sim) lz[j0 + k] = (st != 0 ? log(st) : 0.0) + mx[j0 + k];
+      });
+      __syncthreads();
+    }
+    for (int j = threadIdx.x; j < n_sim; j += blockDim.x) {
+      const double c = lz[j] - lz[0];
+      sl[4 * j + 2] = c;
+      if (blockIdx.x == 0 && blockIdx.y == 0) used[j] = c;
+    }
+  }
   __syncthreads();
-  const int64_t b = (int64_t)blockIdx.x * kRwBlock + threadIdx.x;
-  const bool live = b < cells.n;
-  double E = 0, V = 0, lh = 0, umax = -INFINITY, umin = INFINITY, all = 0, near = 0;
-  if (live) {
-    E = cells.en[b];
-    V = cells.vn[b];
-    lh = cells.lh[b];
+  double top[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) top[k] = -INFINITY;
+  const int64_t lanes = (int64_t)gridDim.x * blockDim.x, b0 = first_cell();
+  double En = 0, Vn = 0, lhn = 0;  // the next cell, loaded a round ahead
+  if (b0 < cells.n) En = cells.en[b0], Vn = cells.vn[b0], lhn = cells.lh[b0];
+  for (int64_t b = b0; b < cells.n; b += lanes) {
+    const double E = En, V = Vn, lh = lhn;
+    if (b + lanes < cells.n) En = cells.en[b + lanes], Vn = cells.vn[b + lanes], lhn = cells.lh[b + lanes];
+    double umax = -INFINITY, umin = INFINITY, sa = 0, st = 0;
+    const double* sp = sl + opaque_zero();
     for (int j = 0; j < n_sim; ++j) {
-      const double u = rw_u(E, V, sl + 4 * j);
+      const double u = rw_u(E, V, sp + 4 * j);
       umax = fmax(umax, u);
       umin = fmin(umin, u);
     }
-    double sa = 0, st = 0;
-    for (int j = 0; j < n_sim; ++j) {
-      const double d = rw_u(E, V, sl + 4 * j) - umax;
-      const double e = exp(d);
+    // four at a time, so that four chains interleave, then the rest
+    int j = 0;
+    for (; j + 4 <= n_sim; j += 4) {
+      double d[4], e[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] = rw_u(E, V, sp + 4 * (j + i)) - umax;
+        e[i] = exp_le0(d[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sa = sa + e[i];
+        if (-d[i] < 10.0) st = st + e[i];
+      }
+    }
+    for (; j < n_sim; ++j) {
+      const double d = rw_u(E, V, sp + 4 * j) - umax;
+      const double e = exp_le0(d);
       sa = sa + e;
       if (-d < 10.0) st = st + e;
     }
-    all = log(sa) + umax;   // log sum_j exp(u_j)
-    near = log(st) + umax;  // the same over the terms within 10 of the largest
-  }
-  // every target's wave maxima into LDS, then one barrier for all of them
-  const int t0 = blockIdx.y * kTargetsPerBlock, nt = min(tg.n - t0, kTargetsPerBlock);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int k = 0; k < nt; ++k) {
-    const int t = t0 + k;
-    double lp = -INFINITY;
-    if (live) {
-      const double2 bp = tg.bp[t];
-      const double t1 = bp.x * (E + bp.y * V);
-      const bool cut = t1 + umax > 10.0 || t1 + umin < -10.0;
-      lp = lh - (t1 + (cut ? near : all));
-      logp[(int64_t)t * cells.n + b] = lp;
+    const double near = log(st) + umax;  // log sum_j exp(u_j) over the terms within 10 of the largest
+    // (each target's t1, and its log_P with the sum that the cell's targets
+    // mostly use; a cell whose targets may not all be cut, as a bound of t1
+    // says, is looked at again target by target)
+    double all = near;  // log sum_j exp(u_j); not needed by a cell whose targets are all cut
+    bool any_cut = true, any_all = false;
+    const double2* bp = bps + opaque_zero();
+    double t_lo = INFINITY;
+#pragma unroll
+    for (int k0 = 0; k0 < R; k0 += 4)
+      if (k0 < nt) {
+#pragma unroll
+        for (int k = k0; k < k0 + 4; ++k) t_lo = fmin(t_lo, rw_t1(E, V, bp[k]));
+      }
+    if (__ballot(!(t_lo + umax > 10.0))) {
+      all = log(sa) + umax;
+      any_cut = false;
+      for (int k = 0; k < nt; ++k) {
+        const bool cut = rw_cut(rw_t1(E, V, bp[k]), umax, umin);
+        any_cut = any_cut || cut;
+        any_all = any_all || !cut;
+      }
     }
-    lp = wave_max(lp);
-    if (lane == 0) red[k][wave] = lp;
+    const double S = any_cut ? near : all;
+    if (__ballot(any_cut && any_all)) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const double t1 = rw_t1(E, V, bp[k]);
+        top[k] = fmax(top[k], lh - (t1 + (rw_cut(t1, umax, umin) ? near : all)));
+      }
+    } else {
+#pragma unroll
+      for (int k0 = 0; k0 < R; k0 += 4)
+        if (k0 < nt) {
+#pragma unroll
+          for (int k = k0; k < k0 + 4; ++k) top[k] = fmax(top[k], lh - (rw_t1(E, V, bp[k]) + S));
+        }
+    }
+    w.sum[(int64_t)row * cells.n + b] = S;
+    w.mixed[(int64_t)row * cells.n + b] = any_cut && any_all;
+    if (any_cut && any_all) w.mix[b] = RwMixed{near, all, umax, umin};  // the same in every row
+  }
+  wave_reduce<R, true>(top);
+  if (reduced_first<R>()) red[reduced_index<R>()][wave] = top[0];
+  __syncthreads();
+  if ((int)threadIdx.x < 4 * R) {
+    const double m = combine_waves<true>(red);
+    const int k = threadIdx.x >> 2;
+    if ((threadIdx.x & 3) == 0 && k < nt) w.pmax[((int64_t)row * w.nblk + blockIdx.x) * kRwRow + k] = m;
+  }
+}
+
+__device__ inline void cell_er(const RwGeom& g, uint32_t c, double& e, double& r) {
+  const uint32_t i = c >> 16, w = c & 0xFFFFu;
+  e = g.e_min + ((int)(i + 1) - 0.5) * g.de;
+  r = g.rho_min + ((int)(w + 1) - 0.5) * g.drho;
+}
+
+// For a tile of T targets (blockIdx.y): their max log_P m from the partial
+// maxima, then over the workgroup's cells the partial sums of
+// x = exp(log_P - m): over the cells within 10 of the max (for log_Z); with
+// kMode >= kRwDensity over all cells (for the normalization); with kRwScan
+// also of x e^2, x e^4, x rho^2, x rho^4 (the Binder cumulants are ratios, so
+// any scale serves).  A scan's workgroup also says which targets have a
+// cell with log_P - m <= -700 (or not a number): for the others every
+// density exp(log_P - log_Z) / norm is surely positive (0 <= log_Z - m <=
+// log of the cell count, and the norm is that sum times the cell's area), so
+// the order parameter's range is that of the grid's cells, whatever the
+// target.  T: what the accumulators leave of the registers at four waves
+// per SIMD.
+template <int T, int kMode>
+__global__ __launch_bounds__(1024) void k_rw_sum(RwCells cells, RwTargets tg, RwWork w, RwGeom g) {
+  constexpr int V = kMode == kRwSweep ? 1 : kMode == kRwDensity ? 2 : kRwScanSums;
+  constexpr int kRed = V * T > 16 ? V * T : 16;
+  __shared__ double red[kRed][16];
+  __shared__ double ms[T];
+  __shared__ double2 bps[T];
+  __shared__ uint32_t low_s;
+  const int wave = threadIdx.x >> 6;
+  const int t0 = blockIdx.y * T, nt = min(tg.n - t0, T), row = t0 / kRwRow;
+  if (threadIdx.x == 0) low_s = 0;
+  if ((int)threadIdx.x < T) bps[threadIdx.x] = tg.bp[t0 + min((int)threadIdx.x, nt - 1)];
+  reduce_partials<T, true>(w.pmax + (int64_t)row * w.nblk * kRwRow + (t0 - row * kRwRow), w.nblk, red,
+                           [&](int k, double m) {
+                             ms[k] = k < nt ? m : 0.0;
+                             if (blockIdx.x == 0 && k < nt) w.mx[t0 + k] = m;
+                           });
+  __syncthreads();
+  double s[V][T];
+#pragma unroll
+  for (int k = 0; k < T; ++k)
+#pragma unroll
+    for (int v = 0; v < V; ++v) s[v][k] = 0;
+  uint32_t low = 0;
+  const int64_t lanes = (int64_t)gridDim.x * blockDim.x, b0 = first_cell();
+  // the cells whose targets all use one sum, then (if there are any) the
+  // mixed ones, so that the usual loop has no branch between its exponentials
+  int saw_mixed = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int64_t b = b0; b < cells.n; b += lanes) {
+      CellIn c = cell_in(cells, w, row, b);
+      if (pass == 0) saw_mixed |= c.mixed;
+      if (c.mixed != (pass != 0)) continue;
+      RwMixed m{c.S, c.S, 0, 0};
+      if (pass) m = w.mix[b];
+      double e2 = 0, r2 = 0, e4 = 0, r4 = 0;
+      if (kMode == kRwScan) {
+        double e, r;
+        cell_er(g, g.cell[b], e, r);
+        e2 = e * e;
+        r2 = r * r;
+        e4 = e2 * e2;
+        r4 = r2 * r2;
+      }
+      // four targets at a time: their chains interleave, and a last tile of
+      // few targets skips the groups that hold none (the spare members of a
+      // group repeat its last target and are not stored)
+#pragma unroll
+      for (int k0 = 0; k0 < T; k0 += 4)
+        if (k0 < nt) {
+          const int z = opaque_zero();
+#pragma unroll
+          for (int k = k0; k < k0 + 4; ++k) {
+            const double t1 = rw_t1(c.E, c.V, bps[k + z]);
+            double S = c.S;
+            if (pass) S = rw_cut(t1, m.umax, m.umin) ? m.near : m.all;
+            const double d = (c.lh - (t1 + S)) - ms[k + z];
+            const double x = exp_le0(d);
+            if (-d < 10.0) s[0][k] = s[0][k] + x;
+            if (kMode >= kRwDensity) s[1 % V][k] = s[1 % V][k] + x;
+            if (kMode == kRwScan) {
+              if (!(d > kUnderflow)) low |= 1u << k;
+              s[2 % V][k] = s[2 % V][k] + e2 * x;
+              s[3 % V][k] = s[3 % V][k] + e4 * x;
+              s[4 % V][k] = s[4 % V][k] + r2 * x;
+              s[5 % V][k] = s[5 % V][k] + r4 * x;
+            }
+          }
+        }
+    }
+    if (pass == 0 && !__syncthreads_or(saw_mixed)) break;
+  }
+  if (kMode == kRwScan && low) atomicOr(&low_s, low);
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    wave_reduce<T, false>(s[v]);
+    if (reduced_first<T>()) red[reduced_index<T>() * V + v][wave] = s[v][0];
   }
   __syncthreads();
-  if (threadIdx.x < nt) {
-    double m = red[threadIdx.x][0];
-    for (int w = 1; w < kRwBlock / 64; ++w) m = fmax(m, red[threadIdx.x][w]);
-    pmax[(int64_t)(t0 + threadIdx.x) * nblk + blockIdx.x] = m;
+  if ((int)threadIdx.x < 4 * nt * V) {
+    const double x = combine_waves<false>(red);
+    const int k = (threadIdx.x >> 2) / V, v = (threadIdx.x >> 2) - k * V;
+    if ((threadIdx.x & 3) == 0) w.ps[(((int64_t)v * w.rows + row) * w.nblk + blockIdx.x) * kRwRow + (t0 + k - row * kRwRow)] = x;
+  }
+  if (kMode == kRwScan && (int)threadIdx.x < nt)
+    w.plow[(int64_t)(t0 + threadIdx.x) * w.nblk + blockIdx.x] = (low_s >> threadIdx.x) & 1u;
+}
+
+// One wavefront per target: log_Z = log(truncated sum) + max; with kMode >=
+// kRwDensity the normalization sum exp(log_P - log_Z) de drho; of a scan the
+// Binder cumulants 1 - <x^4> / (3 <x^2>^2) of the marginals and whether
+// some cell's density may have underflowed.
+template <int kMode>
+__global__ __launch_bounds__(64) void k_rw_finish(RwWork w, double de, double drho,
+                                                  double* __restrict__ binder_ed) {
+  constexpr int V = kMode == kRwSweep ? 1 : kMode == kRwDensity ? 2 : kRwScanSums;
+  const int t = blockIdx.x, lane = threadIdx.x;
+  double s[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const double* p = w.ps + ((int64_t)v * w.rows + t / kRwRow) * w.nblk * kRwRow + t % kRwRow;
+    double x = 0;
+    for (int i = lane; i < w.nblk; i += 64) x += p[i * kRwRow];
+    s[v] = wave_sum(x);
+  }
+  uint32_t low = 0;
+  if (kMode == kRwScan) {
+    for (int i = lane; i < w.nblk; i += 64) low |= w.plow[(int64_t)t * w.nblk + i];
+    low = __ballot(low != 0) != 0;
+  }
+  if (lane) return;
+  const double z = (s[0] != 0 ? log(s[0]) : 0.0) + w.mx[t];
+  w.lz[t] = z;
+  if (kMode >= kRwDensity) w.norm[t] = s[1 % V] * exp(w.mx[t] - z) * de * drho;
+  if (kMode == kRwScan) {
+    const double m0 = s[1 % V], e2 = s[2 % V] / m0, r2 = s[4 % V] / m0;
+    binder_ed[2 * t] = 1.0 - (s[3 % V] / m0) / (3.0 * e2 * e2);
+    binder_ed[2 * t + 1] = 1.0 - (s[5 % V] / m0) / (3.0 * r2 * r2);
+    w.low[t] = low;
   }
 }
 
-// per target: the max of log_P from the k_rw_logp partials, then partial
-// sums of exp(log_P - max) over the cells within 10 of the max (for log_Z)
-// and over all cells (for the normalization), grid-stride over the cells
-__global__ __launch_bounds__(kRwBlock) void k_rw_sum(const double* __restrict__ logp, int64_t n,
-                                                     const double* __restrict__ pmax, int32_t nblk,
-                                                     double* __restrict__ mx, double* __restrict__ ps) {
-  __shared__ double red[kRwBlock / 64];
-  const int t = blockIdx.y;
-  const double* pm = pmax + (int64_t)t * nblk;
-  double m = -INFINITY;
-  for (int i = threadIdx.x; i < nblk; i += kRwBlock) m = fmax(m, pm[i]);
-  m = block_reduce<true>(m, red);
-  const double* lp = logp + (int64_t)t * n;
-  double st = 0, sa = 0;
-  for (int64_t b = (int64_t)blockIdx.x * kRwBlock + threadIdx.x; b < n; b += (int64_t)gridDim.x * kRwBlock) {
-    const double v = lp[b];
-    const double e = exp(v - m);
-    sa = sa + e;
-    if (m - v < 10.0) st = st + e;
-  }
-  st = block_reduce<false>(st, red);
-  sa = block_reduce<false>(sa, red);
-  if (threadIdx.x == 0) {
-    ps[2 * ((int64_t)t * gridDim.x + blockIdx.x)] = st;
-    ps[2 * ((int64_t)t * gridDim.x + blockIdx.x) + 1] = sa;
-    if (blockIdx.x == 0) mx[t] = m;
-  }
-}
-
-// one wave per target: log_Z = log(truncated sum) + max, the
-// normalization sum exp(log_P - log_Z) de drho, and with ctes_out the
-// constants' update log_Z(t) - log_Z(0)
-__global__ __launch_bounds__(kRwBlock) void k_rw_finish(const double* __restrict__ ps, int32_t sblk, int32_t n_t,
-                                                        const double* __restrict__ mx, double de, double drho,
-                                                        double* __restrict__ lz, double* __restrict__ norm,
-                                                        double* __restrict__ ctes_out) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int t = wave; t < n_t; t += kRwBlock / 64) {
-    double st = 0, sa = 0;
-    for (int i = lane; i < sblk; i += 64) {
-      st += ps[2 * ((int64_t)t * sblk + i)];
-      sa += ps[2 * ((int64_t)t * sblk + i) + 1];
-    }
-    st = wave_sum(st);
-    sa = wave_sum(sa);
-    if (lane == 0) {
-      const double z = (st != 0 ? log(st) : 0.0) + mx[t];
-      lz[t] = z;
-      norm[t] = sa * exp(mx[t] - z) * de * drho;
-    }
-  }
-  __syncthreads();
-  if (ctes_out)
-    for (int t = threadIdx.x; t < n_t; t += kRwBlock) ctes_out[t] = lz[t] - lz[0];
-}
-
-__global__ __launch_bounds__(kRwBlock) void k_rw_dist(double* __restrict__ logp, int64_t n,
-                                                      const double* __restrict__ lz,
-                                                      const double* __restrict__ norm) {
+// densities exp(log_P - log_Z) / norm, one target per blockIdx.y
+__global__ __launch_bounds__(kRwBlock) void k_rw_dist(RwCells cells, RwTargets tg, RwWork w,
+                                                      double* __restrict__ dens) {
   const int t = blockIdx.y;
   const int64_t b = (int64_t)blockIdx.x * kRwBlock + threadIdx.x;
-  if (b < n) {
-    double* p = logp + (int64_t)t * n + b;
-    *p = exp(*p - lz[t]) / norm[t];
-  }
+  if (b >= cells.n) return;
+  const double lp = cell_logp(cell_in(cells, w, t / kRwRow, b), w, b, tg.bp[t]);
+  dens[(int64_t)t * cells.n + b] = exp(lp - w.lz[t]) / w.norm[t];
 }
-
-int32_t rw_sum_blocks(int32_t nblk) { return nblk < kSumBlocks ? nblk : kSumBlocks; }
 
 // ------------------------------------------------------------ projections
 // Each workgroup of a projection takes one contiguous range of cells, so
@@ -190,204 +520,448 @@ __device__ inline void block_range(int64_t n, int64_t& lo, int64_t& hi) {
   hi = lo + per < n ? lo + per : n;
 }
 
-__device__ inline void cell_er(const RwGeom& g, uint32_t c, double& e, double& r) {
-  const uint32_t i = c >> 16, w = c & 0xFFFFu;
-  e = g.e_min + ((int)(i + 1) - 0.5) * g.de;
-  r = g.rho_min + ((int)(w + 1) - 0.5) * g.drho;
-}
-
-constexpr int kRwBatch = 8;  // cells per thread whose loads a projection issues together
-
-__global__ __launch_bounds__(kRwBlock) void k_rw_moments(RwGeom g, const double* __restrict__ dens,
-                                                         double* __restrict__ part) {
+// Min and max of x = e sin(a) + rho cos(a) over a workgroup's cells: with
+// blockIdx.y < n_a over all cells at angle blockIdx.y, the range of every
+// target whose densities are all positive; beyond that, for target and
+// angle blockIdx.y - n_a, over its cells of positive density, left out for
+// the targets that the first kind serves.
+__global__ __launch_bounds__(kRwBlock) void k_rw_xrange(RwGeom g, RwCells cells, RwTargets tg, RwWork w,
+                                                        RwScan sc) {
   __shared__ double red[kRwBlock / 64];
-  const int t = blockIdx.y;
-  const double* v = dens + (int64_t)t * g.n;
-  int64_t lo, hi;
-  block_range(g.n, lo, hi);
-  double s[5] = {0, 0, 0, 0, 0};
-  // kRwBatch cells per thread per trip, their loads issued first, then
-  // added in cell order
-  for (int64_t b0 = lo + threadIdx.x; b0 < hi; b0 += kRwBlock * kRwBatch) {
-    double xs[kRwBatch];
-    uint32_t cs[kRwBatch];
-#pragma unroll
-    for (int u = 0; u < kRwBatch; ++u) {
-      const int64_t bb = b0 + kRwBlock * u, bc = bb < hi ? bb : hi - 1;
-      xs[u] = v[bc];
-      cs[u] = g.cell[bc];
-    }
-#pragma unroll
-    for (int u = 0; u < kRwBatch; ++u) {
-      if (b0 + kRwBlock * u >= hi) break;
-      double e, r;
-      cell_er(g, cs[u], e, r);
-      const double x = xs[u], e2 = e * e, r2 = r * r;
-      s[0] += x;
-      s[1] += e2 * x;
-      s[2] += e2 * e2 * x;
-      s[3] += r2 * x;
-      s[4] += r2 * r2 * x;
-    }
-  }
-  for (int k = 0; k < 5; ++k) {
-    const double m = block_reduce<false>(s[k], red);
-    if (threadIdx.x == 0) part[((int64_t)t * gridDim.x + blockIdx.x) * 5 + k] = m;
-  }
-}
-
-__global__ __launch_bounds__(kRwBlock) void k_rw_xrange(RwGeom g, const double* __restrict__ dens, int32_t n_a,
-                                                        const double2* __restrict__ sc,
-                                                        double* __restrict__ part) {
-  __shared__ double red[kRwBlock / 64];
-  const int ta = blockIdx.y, t = ta / n_a, a = ta - t * n_a;
-  const double* v = dens + (int64_t)t * g.n;
-  const double2 q = sc[a];
+  const int y = blockIdx.y;
+  const bool own = y >= sc.n_a;
+  const int t = own ? (y - sc.n_a) / sc.n_a : 0, a = own ? (y - sc.n_a) - t * sc.n_a : y;
+  if (own && !w.low[t]) return;
+  const double2 q = sc.angle[a], bp = own ? tg.bp[t] : double2{0, 0};
   int64_t lo, hi;
   block_range(g.n, lo, hi);
   double mn = INFINITY, mx = -INFINITY;
-  for (int64_t b0 = lo + threadIdx.x; b0 < hi; b0 += kRwBlock * kRwBatch) {
-    double xs[kRwBatch];
-    uint32_t cs[kRwBatch];
-#pragma unroll
-    for (int u = 0; u < kRwBatch; ++u) {
-      const int64_t bb = b0 + kRwBlock * u, bc = bb < hi ? bb : hi - 1;
-      xs[u] = v[bc];
-      cs[u] = g.cell[bc];
+  for (int64_t b = lo + threadIdx.x; b < hi; b += kRwBlock) {
+    if (own) {
+      const double lp = cell_logp(cell_in(cells, w, t / kRwRow, b), w, b, bp);
+      if (!(exp(lp - w.lz[t]) / w.norm[t] > 0)) continue;
     }
-#pragma unroll
-    for (int u = 0; u < kRwBatch; ++u) {
-      if (b0 + kRwBlock * u >= hi || !(xs[u] > 0)) continue;
-      double e, r;
-      cell_er(g, cs[u], e, r);
-      const double x = e * q.x + r * q.y;
-      mn = fmin(mn, x);
-      mx = fmax(mx, x);
-    }
+    double e, r;
+    cell_er(g, g.cell[b], e, r);
+    const double x = e * q.x + r * q.y;
+    mn = fmin(mn, x);
+    mx = fmax(mx, x);
   }
   mn = -block_reduce<true>(-mn, red);
   mx = block_reduce<true>(mx, red);
-  if (threadIdx.x == 0) {
-    part[2 * ((int64_t)ta * gridDim.x + blockIdx.x)] = mn;
-    part[2 * ((int64_t)ta * gridDim.x + blockIdx.x) + 1] = mx;
-  }
+  if (threadIdx.x == 0) sc.range[(int64_t)y * gridDim.x + blockIdx.x] = double2{mn, mx};
 }
 
-// One wavefront per workgroup; every lane adds its cells (lane, lane + 64,
-// ... of the workgroup's contiguous range) into its own LDS row of nm bins,
-// and lane k then sums column k over the 64 rows in lane order.  Every sum
-// runs in an order fixed by the launch shape, with one LDS read-modify-write
-// per cell and no cross-lane traffic.
-constexpr int kRwXhistBatch = 16;
+// Bins from the range of x over the occupied cells, two empty ones on each
+// side (f90:1420-1429): of the grid's cells at angle blockIdx.x < n_a (gbin),
+// then of pair blockIdx.x - n_a, which are the grid's where all its
+// densities are positive; one wavefront each.
+__global__ __launch_bounds__(64) void k_rw_bins(RwWork w, RwScan sc, int32_t nm) {
+  const bool pair = (int)blockIdx.x >= sc.n_a;
+  const int ta = (int)blockIdx.x - sc.n_a, t = pair ? ta / sc.n_a : 0;
+  const int at = pair && !w.low[t] ? ta - t * sc.n_a : (int)blockIdx.x;  // whose range
+  const double2* r = sc.range + (int64_t)at * kRwProjBlocks;
+  double xmin = (double)1E12f, xmax = (double)-1E12f;
+  for (int i = threadIdx.x; i < kRwProjBlocks; i += 64) {
+    xmin = fmin(xmin, r[i].x);
+    xmax = fmax(xmax, r[i].y);
+  }
+  xmin = -wave_max(-xmin);
+  xmax = wave_max(xmax);
+  if (threadIdx.x) return;
+  if (pair) sc.code[ta] = xmax >= xmin ? 0u : kRwNoCell;
+  double range = xmax - xmin, width = range / nm;
+  range = range + 4 * width;
+  xmin = xmin - 2 * width;
+  width = range / nm;
+  (pair ? sc.bin[ta] : sc.gbin[blockIdx.x]) = double2{xmin, width};
+}
 
-__global__ __launch_bounds__(64) void k_rw_xhist(RwGeom g, const double* __restrict__ dens, int32_t n_a,
-                                                 const double2* __restrict__ sc,
-                                                 const double2* __restrict__ binfo, double* __restrict__ part,
-                                                 uint32_t* __restrict__ err) {
-  extern __shared__ double hl[];  // [64 lanes][nm]
-  const int ta = blockIdx.y, t = ta / n_a, a = ta - t * n_a;
-  const int lane = threadIdx.x, nm = g.nm;
-  double* h = hl + lane * nm;
-  for (int k = 0; k < nm; ++k) h[k] = 0;
-  const double* v = dens + (int64_t)t * g.n;
-  const double2 q = sc[a], bi = binfo[ta];
+// Bin of X: (int)((X - x0) / w) (f90:1440-1452), kRwNoBin outside the bins.
+constexpr uint32_t kRwNoBin = 255;  // n_bin_mixed <= 215
+__device__ inline uint32_t order_bin(double X, double2 bi, int nm) {
+  const double y = X - bi.x, d = y / bi.y;
+  if (fabs(d) < 1073741824.0 && (int)d >= 0 && (int)d < nm) return (uint32_t)(int)d;
+  return fabs(y) < (double)1E-10f ? 0u : kRwNoBin;
+}
+
+// The cells' bins at NA angles, a byte each, for every target whose bins
+// are the grid's (blockIdx.y: group of angles).
+template <int NA>
+__device__ inline uint32_t cell_bins(const RwGeom& g, uint32_t id, const RwScan& sc, const double2* bin, int a0, int na) {
+  double e, r;
+  cell_er(g, id, e, r);
+  uint32_t v = 0;
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+    if (a < na) {
+      const double2 q = sc.angle[a0 + a];
+      v |= order_bin(e * q.x + r * q.y, bin[a0 + a], g.nm) << (8 * a);
+    }
+  return v;
+}
+template <int NA>
+__global__ __launch_bounds__(kRwBlock) void k_rw_cell_bins(RwGeom g, RwScan sc) {
+  const int64_t b = (int64_t)blockIdx.x * kRwBlock + threadIdx.x;
+  if (b >= g.n) return;
+  const int a0 = blockIdx.y * NA;
+  sc.cbin[(int64_t)blockIdx.y * g.n + b] = cell_bins<NA>(g, g.cell[b], sc, sc.gbin, a0, min(NA, sc.n_a - a0));
+}
+
+// Histograms of x over the bins of NA angles (blockIdx.y = target and group
+// of NA angles), weighted by the density, one wavefront per workgroup.  A
+// cell's exponential serves all NA angles.  kRwRows lanes apart share a row
+// of the wavefront's histogram and add to it one group of kRwRows lanes
+// after the other, so every sum runs in an order fixed by the launch shape:
+// LDS additions of one wavefront are done in order, and no two lanes of a
+// group share a row.  The densities are left unnormalized unless some
+// underflow: the histogram is normalized after.
+// Bound by FP64 issue and those additions.  A row per lane and angle (30 KB
+// at 59 bins) with each lane reading, adding and writing back: 489 us for 64
+// targets x 3 angles at 710,000 cells; 275 us in this form, with its exponentials.
+constexpr int kRwXhistBatch = 4;  // cells per lane whose loads are issued together
+constexpr int kRwRows = 16;
+
+template <int NA>
+__global__ __launch_bounds__(64) void k_rw_xhist(RwGeom g, RwCells cells, RwTargets tg, RwWork w, RwScan sc) {
+  extern __shared__ double hl[];  // [NA][kRwRows][stride]
+  const int ng = (sc.n_a + NA - 1) / NA, t = blockIdx.y / ng, a0 = (blockIdx.y - t * ng) * NA;
+  const int na = min(NA, sc.n_a - a0), lane = threadIdx.x, nm = g.nm, stride = nm | 1;
+  for (int i = lane; i < NA * kRwRows * stride; i += 64) hl[i] = 0;
+  __syncthreads();
+  const double2 bp = tg.bp[t];
+  const double lz = w.lz[t], norm = w.norm[t];
+  const bool own = w.low[t] != 0;  // the target has its own bins
+  double* row = hl + (lane & (kRwRows - 1)) * stride;
+  const uint32_t* cb = sc.cbin + (int64_t)(a0 / NA) * g.n;
   int64_t lo, hi;
   block_range(g.n, lo, hi);
-  // kRwXhistBatch cells per lane per trip, all their loads issued first
-  // (clamped indices), then added in cell order
-  for (int64_t b0 = lo + lane; b0 < hi; b0 += 64 * kRwXhistBatch) {
-    double xs[kRwXhistBatch];
-    uint32_t cs[kRwXhistBatch];
+  uint32_t bad = 0;
+  for (int64_t b0 = lo; b0 < hi; b0 += 64 * kRwXhistBatch) {
+    // the batch's loads first (an index past the end re-reads the last cell)
+    CellIn c[kRwXhistBatch];
+    uint32_t kb[kRwXhistBatch];
+    double x[kRwXhistBatch];
 #pragma unroll
     for (int u = 0; u < kRwXhistBatch; ++u) {
-      const int64_t bb = b0 + 64 * u, bc = bb < hi ? bb : hi - 1;
-      xs[u] = v[bc];
-      cs[u] = g.cell[bc];
+      const int64_t b = b0 + 64 * u + lane, bc = b < hi ? b : hi - 1;
+      c[u] = cell_in(cells, w, t / kRwRow, bc);
+      kb[u] = own ? cell_bins<NA>(g, g.cell[bc], sc, sc.bin + t * sc.n_a, a0, na) : cb[bc];
     }
 #pragma unroll
     for (int u = 0; u < kRwXhistBatch; ++u) {
-      const double x = xs[u];
-      if (b0 + 64 * u >= hi || !(x > 0)) continue;
-      double e, r;
-      cell_er(g, cs[u], e, r);
-      const double X = e * q.x + r * q.y, d = (X - bi.x) / bi.y;
-      int k;
-      if (fabs(d) < 1073741824.0 && (int)d >= 0 && (int)d < nm)
-        k = (int)d;
-      else if (fabs(X - bi.x) < (double)1E-10f)
-        k = 0;
-      else {
-        atomicOr(err, 1u);
-        continue;
+      const int64_t b = b0 + 64 * u + lane, bc = b < hi ? b : hi - 1;
+      x[u] = exp_le0(cell_logp(c[u], w, bc, bp) - lz);  // log_Z is at least the largest log_P
+      if (own) x[u] = x[u] / norm;
+      if (b >= hi) x[u] = 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kRwXhistBatch; ++u) {
+      const bool on = x[u] > 0;
+      double* h[NA];
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        const uint32_t k = (kb[u] >> (8 * a)) & 255u;
+        if (on && k == kRwNoBin) bad |= 1u << a;
+        h[a] = row + a * kRwRows * stride + (k == kRwNoBin ? 0u : k);
       }
-      h[k] += x;
+#pragma unroll
+      for (int s = 0; s < 64 / kRwRows; ++s) {
+        if (on && lane / kRwRows == s) {
+#pragma unroll
+          for (int a = 0; a < NA; ++a)
+            __hip_atomic_fetch_add(h[a], x[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        asm volatile("" ::: "memory");  // the groups' turns stay apart
+      }
     }
   }
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+    if (a < na && ((bad >> a) & 1u)) atomicOr(&sc.code[t * sc.n_a + a0 + a], kRwOutside);
   __syncthreads();
-  for (int k = lane; k < nm; k += 64) {
+  for (int i = lane; i < na * nm; i += 64) {
+    const int a = i / nm, k = i - a * nm;
     double s = 0;
-    for (int l = 0; l < 64; ++l) s += hl[l * nm + k];
-    part[((int64_t)ta * gridDim.x + blockIdx.x) * nm + k] = s;
+    for (int l = 0; l < kRwRows; ++l) s += hl[(a * kRwRows + l) * stride + k];
+    sc.hist[((int64_t)(t * sc.n_a + a0 + a) * gridDim.x + blockIdx.x) * nm + k] = s;
   }
 }
 
-__global__ void k_rw_xhist_sum(const double* __restrict__ part, int32_t nm, double* __restrict__ out) {
-  const int ta = blockIdx.x;
-  for (int k = threadIdx.x; k < nm; k += blockDim.x) {
-    double v = 0;
-    for (int b = 0; b < kRwProjBlocks; ++b) v += part[((int64_t)ta * kRwProjBlocks + b) * nm + k];
-    out[(int64_t)ta * nm + k] = v;
+// ---------------------------------------------------- order parameter
+// The rest of a pair's order parameter on its own wavefront, lane l taking
+// bins l, l + 64, ... (kRwBinsPerLane of them: n_bin_mixed <= 215): the
+// workgroups' histograms added in order, then Calcula_Histograma_Rotado_normX
+// after binning (f90:1466-1617), binder (2580-2608) and the Ising scores
+// (2042-2182), the steps of finish_order_parameter and cvf_rw_ising_scores on
+// the host with sums taken across the lanes.  On the host the 192 pairs of a
+// 64 x 3 scan took about 0.4 ms.
+constexpr int kRwBinsPerLane = 4;
+struct Bins {
+  double x[kRwBinsPerLane], p[kRwBinsPerLane], w[kRwBinsPerLane];
+};
+template <class F>
+__device__ inline double bins_sum(int nm, F f) {
+  double s = 0;
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i)
+    if ((int)threadIdx.x + 64 * i < nm) s += f(i);
+  return wave_sum(s);
+}
+// norm 1, mean 0, variance 1; the mean removed and the scale applied
+__device__ inline void bins_standardize(Bins& h, int nm, double& mean, double& a1) {
+  const double norma = bins_sum(nm, [&](int i) { return h.p[i] * h.w[i]; });
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) h.p[i] = h.p[i] / norma;
+  mean = bins_sum(nm, [&](int i) { return h.x[i] * h.p[i] * h.w[i]; });
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) h.x[i] = h.x[i] - mean;
+  const double n2 = bins_sum(nm, [&](int i) { return h.p[i] > 0 ? h.p[i] * h.w[i] : 0.0; });
+  const double var = bins_sum(nm, [&](int i) { return h.p[i] > 0 ? h.x[i] * h.x[i] * h.p[i] * h.w[i] : 0.0; });
+  a1 = sqrt(n2 / var);
+  const double a2 = 1 / (n2 * a1);
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    h.x[i] = h.x[i] * a1;
+    h.w[i] = h.w[i] * a1;
+    h.p[i] = h.p[i] * a2;
   }
+}
+// the reference's own check (f90:1510-1533)
+__device__ inline bool bins_standard(const Bins& h, int nm) {
+  const auto pos = [&](int i, double v) { return h.p[i] > 0 ? v : 0.0; };
+  const double norma = bins_sum(nm, [&](int i) { return pos(i, h.p[i] * h.w[i]); });
+  const double mean = bins_sum(nm, [&](int i) { return pos(i, h.x[i] * h.p[i] * h.w[i]); });
+  const double var = bins_sum(nm, [&](int i) { return pos(i, h.x[i] * h.x[i] * h.p[i] * h.w[i]); }) - mean * mean;
+  const double tol = (double)1E-10f;
+  return !(fabs(mean) > tol || fabs(norma - 1) > tol || fabs(var - 1) > tol);
+}
+__device__ inline double ising2d(double z) {
+  const double a = (double)0.058137f, b = (double)-2.68949f, c = (double)-0.11235f, d = (double)2.884162f;
+  const double z2 = z * z, z4 = z2 * z2, z8 = z4 * z4, z16 = z8 * z8;
+  return exp(-(a * z16 + b * z * z + c * fabs(z) + d));
+}
+__device__ inline double ising3d(double z) {
+  const double a = (double)0.196f, c = (double)0.807f, M0 = (double)1.141059404f, A0 = (double)0.436591191f;
+  const double q = z * z / (M0 * M0) - 1;
+  return A0 * exp(-q * q * (a * z * z / (M0 * M0) + c));
+}
+// the first bin in order with the largest key (v, then lowest index): its
+// index, or -1 where no lane has one (i < 0)
+__device__ inline int wave_first_max(double v, int i) {
+  for (int o = 32; o > 0; o >>= 1) {
+    const double v2 = __shfl_xor(v, o);
+    const int i2 = __shfl_xor(i, o);
+    if (i2 >= 0 && (i < 0 || v2 > v || (v2 == v && i2 < i))) v = v2, i = i2;
+  }
+  return i;
+}
+// the bin's value from the lane that holds it
+__device__ inline double bin_value(const double (&v)[kRwBinsPerLane], int k) {
+  double r = 0;
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) r = k >> 6 == i ? v[i] : r;
+  return __shfl(r, k & 63);
+}
+
+__global__ __launch_bounds__(64) void k_rw_order(RwScan sc, int32_t nm, double peak2d, double peak3d, RwScanOut out) {
+  __shared__ double xs[64 * kRwBinsPerLane];
+  const int ta = blockIdx.x, lane = threadIdx.x;
+  const double2 bin = sc.bin[ta];
+  Bins h;
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    const int k = lane + 64 * i;
+    double s = 0;
+    if (k < nm)
+      for (int b = 0; b < kRwProjBlocks; ++b) s += sc.hist[((int64_t)ta * kRwProjBlocks + b) * nm + k];
+    h.p[i] = s;
+    h.x[i] = bin.x + ((k + 1) - 0.5) * bin.y;
+    h.w[i] = k < nm ? bin.y : 0.0;
+  }
+  double media, a1, unused;
+  bins_standardize(h, nm, media, a1);
+  uint32_t code = sc.code[ta];
+  if (!bins_standard(h, nm)) code |= kRwMoments;
+  // sine stretch of the axis (f90:1530-1534), then norm / mean / variance
+  // again with the stretched bin widths (1538-1617)
+  const double b = (double)1.53f, pi = (double)3.14159f;
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    h.x[i] = b * b * sin(pi * h.x[i] / b) / (pi * pi) + h.x[i];
+    xs[lane + 64 * i] = h.x[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    const int k = lane + 64 * i;
+    h.w[i] = k >= nm ? 0.0 : k == 0 ? xs[1] - xs[0] : k == nm - 1 ? xs[k] - xs[k - 1] : (xs[k + 1] - xs[k - 1]) / 2.0;
+  }
+  bins_standardize(h, nm, unused, a1);
+  if (!bins_standard(h, nm)) code |= kRwStretched;
+  // cumulant of M = x / a1 + media
+  const double s = bins_sum(nm, [&](int i) { return h.p[i]; });
+  const auto m2 = [&](int i) {
+    const double m = (h.x[i] / a1) + media;
+    return m * m;
+  };
+  const double u2 = bins_sum(nm, [&](int i) { return m2(i) * h.p[i] / s; });
+  const double u4 = bins_sum(nm, [&](int i) { return m2(i) * m2(i) * h.p[i] / s; });
+  // Ising scores
+  double f2[kRwBinsPerLane], f3[kRwBinsPerLane];
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    f2[i] = ising2d(h.x[i]);
+    f3[i] = ising3d(h.x[i]);
+  }
+  const auto on = [&](int i, double v) { return h.p[i] == 0 ? 0.0 : v; };
+  const double n_liu = bins_sum(nm, [&](int i) { return on(i, 1.0); });
+  const double kl2 = bins_sum(nm, [&](int i) { return on(i, f2[i] > 0 ? (log(f2[i]) - log(h.p[i])) * f2[i] : 0.0); });
+  const double kl3 = bins_sum(nm, [&](int i) { return on(i, f3[i] > 0 ? (log(f3[i]) - log(h.p[i])) * f3[i] : 0.0); });
+  const double liu2 = bins_sum(nm, [&](int i) { return on(i, sqrt(h.p[i]) * fabs(h.p[i] - f2[i])); });
+  const double liu3 = bins_sum(nm, [&](int i) { return on(i, sqrt(h.p[i]) * fabs(h.p[i] - f3[i])); });
+  // ZeroTest: the lowest bin with |x| < 1; HeightTest: the highest bin of
+  // each side (the first of equals)
+  double zv = 0, v1 = 0, v2 = 0;
+  int zi = -1, i1 = -1, i2 = -1;
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    const int k = lane + 64 * i;
+    if (k >= nm) continue;
+    const double x = h.x[i], p = h.p[i];
+    if (x > -1 && x < 1 && p < (double)1E12f && (zi < 0 || -p > zv)) zv = -p, zi = k;
+    if (x < 0 && p > -10 && (i1 < 0 || p > v1)) v1 = p, i1 = k;
+    if (!(x < 0) && p > -10 && (i2 < 0 || p > v2)) v2 = p, i2 = k;
+  }
+  zi = wave_first_max(zv, zi);
+  i1 = wave_first_max(v1, i1);
+  i2 = wave_first_max(v2, i2);
+  const double k = (double)(6.0f / 0.8f);
+  double zero = (double)1E3f, height = (double)1E3f;
+  if (zi >= 0) {
+    const double d = bin_value(h.p, zi) - ising3d(0.0), x = bin_value(h.x, zi);
+    zero = d * d;
+    zero = zero * k * k;
+    zero = zero + x * x;
+  }
+  if (i1 >= 0 && i2 >= 0) {
+    const double x1 = (double)-1.14f, x2 = (double)1.14f;
+    const double d1 = bin_value(h.p, i1) - ising3d(x1), d2 = bin_value(h.p, i2) - ising3d(x2);
+    const double y1 = bin_value(h.x, i1) - x1, y2 = bin_value(h.x, i2) - x2;
+    height = d1 * d1 * k * k;
+    height = height + d2 * d2 * k * k;
+    height = height + y1 * y1;
+    height = height + y2 * y2;
+  }
+#pragma unroll
+  for (int i = 0; i < kRwBinsPerLane; ++i) {
+    const int kk = lane + 64 * i;
+    if (kk < nm) {
+      out.x[(int64_t)ta * nm + kk] = h.x[i];
+      out.p[(int64_t)ta * nm + kk] = h.p[i];
+    }
+  }
+  if (lane) return;
+  out.code[ta] = code;
+  double *stats3 = out.stats3, *scores6 = out.scores6;
+  stats3[3 * ta] = media;
+  stats3[3 * ta + 1] = a1;
+  stats3[3 * ta + 2] = 1.0 - u4 / (3.0 * u2 * u2);
+  scores6[6 * ta] = kl2;
+  scores6[6 * ta + 1] = kl3;
+  scores6[6 * ta + 2] = liu2 / ((peak2d - ising2d(0.0)) * n_liu);
+  scores6[6 * ta + 3] = liu3 / ((peak3d - ising3d(0.0)) * n_liu);
+  scores6[6 * ta + 4] = zero;
+  scores6[6 * ta + 5] = height;
+}
+
+template <int T, int kMode>
+void sum_launch(const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwGeom& g, hipStream_t st) {
+  hipLaunchKernelGGL((k_rw_sum<T, kMode>), dim3((unsigned)w.nblk, (unsigned)((tg.n + T - 1) / T)), dim3(w.threads), 0,
+                     st, cells, tg, w, g);
+}
+
+template <int NA>
+hipError_t xhist_launch(const RwGeom& g, const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwScan& sc,
+                        hipStream_t st) {
+  const unsigned groups = (unsigned)((sc.n_a + NA - 1) / NA);
+  hipLaunchKernelGGL(k_rw_cell_bins<NA>, dim3((unsigned)((g.n + kRwBlock - 1) / kRwBlock), groups), dim3(kRwBlock), 0,
+                     st, g, sc);
+  const size_t lds = sizeof(double) * NA * kRwRows * (size_t)(g.nm | 1);
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rw_xhist<NA>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_rw_xhist<NA>, dim3(kRwProjBlocks, (unsigned)tg.n * groups), dim3(64), lds, st, g,
+                     cells, tg, w, sc);
+  return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_rw_xhist_sum(const double* part, int32_t n_ta, int32_t nm, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_rw_xhist_sum, dim3((unsigned)n_ta), dim3(64), 0, st, part, nm, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_rw_moments(const RwGeom& g, const double* dens, int32_t n_t, double* part, hipStream_t st) {
-  hipLaunchKernelGGL(k_rw_moments, dim3(kRwProjBlocks, (unsigned)n_t), dim3(kRwBlock), 0, st, g, dens, part);
-  return hipGetLastError();
-}
-
-hipError_t launch_rw_xrange(const RwGeom& g, const double* dens, int32_t n_t, int32_t n_a, const double2* sc,
-                            double* part, hipStream_t st) {
-  hipLaunchKernelGGL(k_rw_xrange, dim3(kRwProjBlocks, (unsigned)(n_t * n_a)), dim3(kRwBlock), 0, st, g, dens, n_a,
-                     sc, part);
-  return hipGetLastError();
-}
-
-hipError_t launch_rw_xhist(const RwGeom& g, const double* dens, int32_t n_t, int32_t n_a, const double2* sc,
-                           const double2* binfo, double* part, uint32_t* err, hipStream_t st) {
-  // 64 rows of nm <= 215 bins (n_bin2D <= 46340): up to 110 KB of LDS
-  const size_t lds = sizeof(double) * 64 * (size_t)g.nm;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rw_xhist),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(k_rw_xhist, dim3(kRwProjBlocks, (unsigned)(n_t * n_a)), dim3(64), lds, st, g, dens, n_a, sc,
-                     binfo, part, err);
-  return hipGetLastError();
+// At most 256 workgroups per row of targets, since every workgroup of the
+// next launch reduces their partial results for itself, and at most one of
+// 1024 threads per CU; small grids take smaller workgroups, so that they
+// spread over the CUs.  With several rows each takes its share of the CUs
+// and a thread more cells: the reductions at the end of a workgroup cost as
+// much as about four cells.
+void rw_shape(int64_t n_cells, int32_t n_targets, RwWork* w) {
+  w->rows = (n_targets + kRwRow - 1) / kRwRow;
+  w->threads = n_cells > 131072 ? 1024 : n_cells > 65536 ? 512 : 256;
+  const int64_t need = (n_cells + w->threads - 1) / w->threads;
+  w->nblk = (int32_t)std::min<int64_t>(need, std::max<int64_t>(kRwMaxBlocks / w->rows, 32));
 }
 
 hipError_t launch_rw_pass(const RwCells& cells, const RwSim* sims, const double* ctes, int32_t n_sim,
-                          const RwTargets& tg, const RwWork& w, double de, double drho, double* ctes_out,
-                          bool dist, hipStream_t stream) {
-  const unsigned rows = (unsigned)((tg.n + kTargetsPerBlock - 1) / kTargetsPerBlock);
-  const size_t lds = sizeof(double) * 4 * (size_t)n_sim;
-  hipLaunchKernelGGL(k_rw_logp, dim3((unsigned)w.nblk, rows), dim3(kRwBlock), lds, stream, cells, sims, ctes,
-                     n_sim, tg, w.logp, w.pmax, w.nblk);
-  const int32_t sblk = rw_sum_blocks(w.nblk);
-  hipLaunchKernelGGL(k_rw_sum, dim3((unsigned)sblk, (unsigned)tg.n), dim3(kRwBlock), 0, stream, w.logp, cells.n,
-                     w.pmax, w.nblk, w.mx, w.ps);
-  hipLaunchKernelGGL(k_rw_finish, dim3(1), dim3(kRwBlock), 0, stream, w.ps, sblk, tg.n, w.mx, de, drho, w.lz,
-                     w.norm, ctes_out);
-  if (dist)
-    hipLaunchKernelGGL(k_rw_dist, dim3((unsigned)w.nblk, (unsigned)tg.n), dim3(kRwBlock), 0, stream, w.logp,
-                       cells.n, w.lz, w.norm);
+                          const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, bool chain, double* used,
+                          hipStream_t stream) {
+  const unsigned rows = (unsigned)((tg.n + kRwRow - 1) / kRwRow);
+  const size_t lds = sizeof(double) * 5 * (size_t)n_sim;
+  // (the last row of many may hold fewer targets: it repeats one)
+  auto* k = tg.n <= 4 ? k_rw_cells<4> : tg.n <= 8 ? k_rw_cells<8> : k_rw_cells<kRwRow>;
+  hipLaunchKernelGGL(k, dim3((unsigned)w.nblk, rows), dim3(w.threads), lds, stream, cells, sims, ctes, n_sim, tg, w,
+                     chain ? w.ps : nullptr, w.mx, used);
+  if (mode == kRwSweep)
+    tg.n <= 4   ? sum_launch<4, kRwSweep>(cells, tg, w, g, stream)
+    : tg.n <= 8 ? sum_launch<8, kRwSweep>(cells, tg, w, g, stream)
+                : sum_launch<kRwRow, kRwSweep>(cells, tg, w, g, stream);
+  else if (mode == kRwDensity)
+    sum_launch<8, kRwDensity>(cells, tg, w, g, stream);
+  else
+    sum_launch<4, kRwScan>(cells, tg, w, g, stream);
+  return hipGetLastError();
+}
+
+hipError_t launch_rw_finish(const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, double* binder_ed,
+                            hipStream_t st) {
+  auto* k = mode == kRwSweep ? k_rw_finish<kRwSweep> : mode == kRwDensity ? k_rw_finish<kRwDensity>
+                                                                          : k_rw_finish<kRwScan>;
+  hipLaunchKernelGGL(k, dim3((unsigned)tg.n), dim3(64), 0, st, w, g.de, g.drho, binder_ed);
+  return hipGetLastError();
+}
+
+hipError_t launch_rw_dist(const RwCells& cells, const RwTargets& tg, const RwWork& w, double* dens, hipStream_t st) {
+  const unsigned nb = (unsigned)((cells.n + kRwBlock - 1) / kRwBlock);
+  hipLaunchKernelGGL(k_rw_dist, dim3(nb, (unsigned)tg.n), dim3(kRwBlock), 0, st, cells, tg, w, dens);
+  return hipGetLastError();
+}
+
+hipError_t launch_rw_project(const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwGeom& g,
+                             const RwScan& sc, double peak2d, double peak3d, const RwScanOut& out, hipStream_t st) {
+  const unsigned nta = (unsigned)(tg.n * sc.n_a);
+  hipLaunchKernelGGL(k_rw_xrange, dim3(kRwProjBlocks, (unsigned)sc.n_a + nta), dim3(kRwBlock), 0, st, g, cells, tg, w,
+                     sc);
+  hipLaunchKernelGGL(k_rw_bins, dim3((unsigned)sc.n_a + nta), dim3(64), 0, st, w, sc, g.nm);
+  // angles per wavefront: as many (up to 4) as keep five wavefronts on a CU
+  const int fit = (int)(32 * 1024 / (sizeof(double) * kRwRows * (size_t)(g.nm | 1)));
+  const int na = fit < sc.n_a ? fit : sc.n_a;
+  const hipError_t e = na >= 4   ? xhist_launch<4>(g, cells, tg, w, sc, st)
+                       : na == 3 ? xhist_launch<3>(g, cells, tg, w, sc, st)
+                       : na == 2 ? xhist_launch<2>(g, cells, tg, w, sc, st)
+                                 : xhist_launch<1>(g, cells, tg, w, sc, st);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_rw_order, dim3(nta), dim3(64), 0, st, sc, g.nm, peak2d, peak3d, out);
   return hipGetLastError();
 }
 

@@ -1,0 +1,133 @@
+"""The launch forms of a reweighting pass: target rows of 4, 8 and 16 and
+several rows, simulation counts that leave a group of four part filled, grids
+on either side of the workgroup sizes, cells whose targets use different sums
+over the simulations, and targets whose densities underflow on part of the
+grid.  Bars as in test_gpu_reweight.py: 1e-9 against the oracle (constants
+absolute, densities relative), 1e-8 on what is derived from histograms."""
+import numpy as np
+import pytest
+
+from cvfbulkwater_amd import CVFError
+from cvfbulkwater_amd.reweight import Reweighting, ising_scores
+from oracle import rw
+import rw_synth
+
+pytestmark = pytest.mark.gpu
+
+
+def isobar(n_sim, n):
+    Ts = [0.1058 + 0.001 * k / max(n_sim - 1, 1) for k in range(n_sim)]
+    return Ts, rw_synth.samples(Ts, n, seed=40 + n_sim)
+
+
+@pytest.mark.parametrize("n_sim", [1, 2, 4, 5, 8, 9, 13, 16, 17, 35])
+def test_constants_for_any_number_of_simulations(n_sim):
+    Ts, data = isobar(n_sim, 400)
+    ora = rw.OraGrid.from_samples(8, Ts, [0.5] * n_sim, [400] * n_sim, np.concatenate(data), 0.5)
+    with Reweighting(8, Ts, [0.5] * n_sim, data, 0.5) as eng:
+        for steps in (0, 1, 2, 7):
+            c, prev, ok = eng.solve_constants(steps)
+            co, po, rc = ora.constants(steps)
+            np.testing.assert_allclose(c, co, rtol=0, atol=1e-9)
+            np.testing.assert_allclose(prev, po, rtol=0, atol=1e-9)
+            assert ok == (rc == 0)
+    ora.close()
+
+
+def scan_matches_targets(eng, T, P, angles):
+    s = eng.scan(T, P, angles)
+    again = eng.scan(T, P, angles)
+    assert all(np.array_equal(s[k], again[k], equal_nan=True) for k in s)  # a fixed order of summation
+    eng.reweight(T, P)
+    for t in range(len(T)):
+        np.testing.assert_allclose(s["binder_ed"][t], eng.binder_ed(t), rtol=1e-9)
+        for a, alpha in enumerate(angles):
+            x, p, st = eng.order_parameter(t, alpha)
+            np.testing.assert_allclose(s["x"][t, a], x, rtol=1e-9, atol=1e-12)
+            np.testing.assert_allclose(s["p"][t, a], p, rtol=1e-9, atol=1e-12)
+            np.testing.assert_allclose(s["stats"][t, a], st, rtol=1e-8)
+            np.testing.assert_allclose(s["scores"][t, a], ising_scores(x, p), rtol=1e-8, atol=1e-12)
+
+
+# rows of targets, groups of angles; n_sim = 1 and 2 at 3000 samples have
+# arguments on both sides of the cut at 10 (mixed cells)
+@pytest.mark.parametrize("n_sim,n_t,n_a", [(1, 3, 1), (2, 9, 2), (6, 1, 3), (6, 4, 4), (6, 5, 5), (3, 17, 6), (6, 36, 1)])
+def test_scan_matches_the_targets_one_by_one(n_sim, n_t, n_a):
+    Ts, data = isobar(n_sim, 3000)
+    with Reweighting(8, Ts, [0.5] * n_sim, data, 1.0) as eng:
+        eng.solve_constants(100)
+        T = np.array([(0.1055 + 0.0015 * k / n_t) * 140.5678 + 185.4676 for k in range(n_t)])
+        P = np.array([(0.5 + 0.001 * (k % 3)) * 4694.59 - 2111.5552 for k in range(n_t)])
+        scan_matches_targets(eng, T, P, [0.4 + 0.31 * a for a in range(n_a)])
+
+
+def test_densities_of_mixed_cells_match_oracle():
+    Ts, data = isobar(2, 3000)
+    ora = rw.OraGrid.from_samples(8, Ts, [0.5] * 2, [3000] * 2, np.concatenate(data), 1.0)
+    c = ora.constants(100)[0]
+    with Reweighting(8, Ts, [0.5] * 2, data, 1.0) as eng:
+        eng.set_constants(c)
+        T = [(0.1056 + 0.0002 * k) * 140.5678 + 185.4676 for k in range(9)]
+        P = [0.5 * 4694.59 - 2111.5552] * 9
+        lz = eng.reweight(T, P)
+        for t in range(9):
+            assert lz[t] == pytest.approx(ora.calcula(c, T[t], P[t])[2], rel=0, abs=1e-9)
+            np.testing.assert_allclose(eng.density(t), ora.distribution(c, T[t], P[t]), rtol=1e-9, atol=1e-300)
+    ora.close()
+
+
+def test_scan_with_underflowing_densities():
+    """Targets far from the simulations, where part of the grid's densities
+    are zero and the order parameter's range is that of the other cells, beside
+    near ones.  beta = 1000 / (0.2293 T) is 21.8 at the simulations' 200.4 K,
+    so at 160 K the exponents of cells 1 kJ/mol apart differ by
+    512 (27.3 - 21.8) = 2800, well over the 745 that a double's exponent
+    spans; at 200.35 K by 3."""
+    Ts, data = isobar(4, 3000)
+    with Reweighting(8, Ts, [0.5] * 4, data, 1.0) as eng:
+        eng.solve_constants(100)
+        T = np.array([200.35, 160.0, 250.0, 200.4])
+        P = np.array([235.0, 235.0, 236.0, 236.0])
+        eng.reweight(T, P)
+        zero = [int((eng.density(t) > 0).sum()) < eng.info()["n_occupied"] for t in range(4)]
+        assert zero == [False, True, True, False]
+        # a distribution that has shrunk to one bin is refused by the checks
+        # on its moments, on both paths; all others are compared
+        compared = 0
+        for t in range(4):
+            for alpha in (0.0, 0.05, 1.2, 1.55):
+                eng.reweight(T[t:t + 1], P[t:t + 1])
+                try:
+                    eng.order_parameter(0, alpha)
+                except CVFError:
+                    with pytest.raises(CVFError):
+                        eng.scan(T[t:t + 1], P[t:t + 1], [alpha])
+                    continue
+                scan_matches_targets(eng, T[t:t + 1], P[t:t + 1], [alpha])
+                compared += zero[t]
+        assert compared > 0
+
+
+# cells below 65,536, below 131,072 and above
+@pytest.mark.parametrize("n_sim,n,bf", [(3, 9000, 1.0), (3, 40000, 1.0), (3, 60000, 2.0)])
+def test_grid_sizes_of_the_launch_shapes(n_sim, n, bf):
+    Ts, data = isobar(n_sim, n)
+    with Reweighting(8, Ts, [0.5] * n_sim, data, bf) as eng:
+        c, _, ok = eng.solve_constants(150)
+        assert ok
+        T, P = eng.sim_points()
+        lz = eng.reweight(T, P)
+        np.testing.assert_allclose(lz - lz[0], c, rtol=0, atol=1e-7)  # the converged fixed point
+        scan_matches_targets(eng, T, P, [1.55])
+
+
+@pytest.mark.parametrize("ctes,P", [([0.0, -np.inf], 235.0), ([np.inf, np.inf], 235.0), ([0.0, 0.0], np.nan),
+                                    ([0.0, 0.0], np.inf)])
+def test_scan_refuses_what_has_no_density(ctes, P):
+    Ts, data = isobar(2, 1000)
+    with Reweighting(8, Ts, [0.5] * 2, data, 0.5) as eng:
+        eng.set_constants(ctes)
+        with pytest.raises(CVFError, match="positive density"):
+            eng.scan([200.4], [P], [1.5])
+        assert not np.any(eng.reweight([200.4], [P]) == 0.0)
+        assert not np.any(eng.density(0) > 0)
