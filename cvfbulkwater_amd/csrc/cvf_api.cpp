@@ -188,7 +188,8 @@ struct cvf_sim {
   cvf_tuning tune{};
 
   DevBuf<uint32_t> words, words2, parent, cover, nslot_nperc;  // words2: ping-pong partner
-  DevBuf<uint8_t> cov;
+  DevBuf<uint8_t> cov, cfg_bytes;
+  DevBuf<uint32_t> cfg_res;                 // first value out of range, inconsistent cubes
   DevBuf<int32_t> csize, slot, cclusters;  // cluster sizes by label, percolation slots, compacted sizes
   DevBuf<uint32_t> cblock;                  // per-workgroup cluster counts of the compaction, then the total
   DevBuf<uint64_t> cmom;                    // per-workgroup size moments, then their total (4 words each)
@@ -258,14 +259,6 @@ int validate(const cvf_params& p) {
   return CVF_OK;
 }
 
-// ---------------------------------------------------------- packing
-inline uint32_t pack_cell(const uint8_t* s6, const uint8_t* e6) {
-  uint32_t w = 0;
-  for (int a = 0; a < 6; ++a) w |= (uint32_t)s6[a] << (3 * a);
-  for (int a = 0; a < 6; ++a) w |= (uint32_t)(e6[a] & 1) << (kEtaShift + a);
-  return w;
-}
-
 // corner cell of the cube with origin (ox,oy,oz) at local corner b
 inline uint32_t corner_cell(uint32_t L, uint32_t ox, uint32_t oy, uint32_t oz, int b) {
   const uint32_t x = (ox + (b & 1)) % L, y = (oy + ((b >> 1) & 1)) % L, z = (oz + ((b >> 2) & 1)) % L;
@@ -284,41 +277,6 @@ void set_cube_eta(std::vector<uint32_t>& w, uint32_t L, uint32_t ox, uint32_t oy
                           (((M >> corner_edge(b, 2)) & 1u) << (4 + bz));
     w[c] = (w[c] & ~(own << kEtaShift)) | (bits << kEtaShift);
   }
-}
-
-// gpu_Chessboard_set_state decision tree (gpu_water3D.cu:3350-3368) on the
-// packed words: v1=b0, v2=b1, v3=b2, v6=b6, v7=b5, v8=b3.
-uint32_t cube_state_from_words(const std::vector<uint32_t>& w, uint32_t L, uint32_t ox, uint32_t oy,
-                               uint32_t oz) {
-  auto eta = [&](int b, int arm) { return eta_of(w[corner_cell(L, ox, oy, oz, b)], arm); };
-  if (eta(0, 0) == 0) {
-    if (eta(6, 0) == 0) return 2;
-    if (eta(2, 4) == 0) return 3;
-    return 8;
-  } else if (eta(0, 2) == 0) {
-    if (eta(1, 4) == 0) return 4;
-    if (eta(5, 2) == 0) return 5;
-    return 7;
-  }
-  if (eta(2, 0) == 0) return 0;
-  if (eta(3, 4) == 0) return 1;
-  return 6;
-}
-
-// 12-bit active-edge mask of a cube as stored in the words
-uint32_t cube_mask_from_words(const std::vector<uint32_t>& w, uint32_t L, uint32_t ox, uint32_t oy,
-                              uint32_t oz, bool* consistent) {
-  uint32_t m = 0;
-  bool ok = true;
-  for (int j = 0; j < kEdges; ++j) {
-    const int A = edge_start(j), ax = edge_axis(j), B = A | (1 << ax);
-    const uint32_t ea = eta_of(w[corner_cell(L, ox, oy, oz, A)], 2 * ax);
-    const uint32_t eb = eta_of(w[corner_cell(L, ox, oy, oz, B)], 2 * ax + 1);
-    if (ea != eb) ok = false;
-    m |= ea << j;
-  }
-  *consistent = ok;
-  return m;
 }
 
 template <class F>
@@ -426,6 +384,14 @@ int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
                       s->stream));
   HIPC(hipStreamSynchronize(s->stream));
   s->obs_at = -1;
+  return CVF_OK;
+}
+
+// Device copy of a point's sigma and eta bytes, kept for the next call
+// (sized for the largest point that asked).
+int reserve_config(cvf_sim* s, size_t n6) {
+  if (!s->cfg_res.p) HIPC(s->cfg_res.alloc(2));
+  if (2 * n6 > s->cfg_bytes.n) HIPC(s->cfg_bytes.alloc(2 * n6));
   return CVF_OK;
 }
 
@@ -1527,61 +1493,42 @@ int cvf_set_config(cvf_sim* s, int32_t pt, const uint8_t* sigma6N, const uint8_t
   if (!sigma6N || !eta6N) return fail(CVF_EINVAL, "null config buffer");
   HIPC(hipSetDevice(s->device));
   const PointHost& P = s->ph[pt];
-  const uint32_t N = P.N, L = P.L;
-  for (uint32_t i = 0; i < 6 * N; ++i) {
-    if (sigma6N[i] > 5)
-      return fail(CVF_ERANGE, "Unexpected value for spin (%d) appeared in line %u", sigma6N[i], i % N);
-    if (eta6N[i] > 1)
-      return fail(CVF_ERANGE, "Unexpected value for active_bond (%d) appeared in line %u", eta6N[i],
-                  i % N);
+  const size_t n6 = 6 * (size_t)P.N;
+  if ((rc = reserve_config(s, n6))) return rc;
+  // words2 is free between steps: the packed input, decoded into words
+  uint32_t* res = s->cfg_res.p;
+  HIPC(hipMemcpyAsync(s->cfg_bytes.p, sigma6N, n6, hipMemcpyHostToDevice, s->stream));
+  HIPC(hipMemcpyAsync(s->cfg_bytes.p + n6, eta6N, n6, hipMemcpyHostToDevice, s->stream));
+  HIPC(hipMemsetAsync(res, 0xFF, 2 * sizeof(uint32_t), s->stream));
+  launch_config_in(s->stream, s->cfg_bytes.p, s->cfg_bytes.p + n6, P.L, P.prm.flag_chessboard, s->words2.p + P.woff,
+                   s->words.p + P.woff, res, res + 1);
+  HIPC(hipGetLastError());
+  uint32_t out[2];
+  HIPC(hipMemcpyAsync(out, res, sizeof out, hipMemcpyDeviceToHost, s->stream));
+  HIPC(hipStreamSynchronize(s->stream));
+  if (out[0] != 0xFFFFFFFFu) {
+    const uint32_t i = out[0] / 2;
+    if (out[0] & 1u)
+      return fail(CVF_ERANGE, "Unexpected value for active_bond (%d) appeared in line %u", eta6N[i], i % P.N);
+    return fail(CVF_ERANGE, "Unexpected value for spin (%d) appeared in line %u", sigma6N[i], i % P.N);
   }
-  std::vector<uint32_t> w(N);
-  for (uint32_t c = 0; c < N; ++c) {
-    uint8_t s6[6], e6[6];
-    for (int a = 0; a < 6; ++a) {
-      s6[a] = sigma6N[a * N + c];
-      e6[a] = eta6N[a * N + c];
-    }
-    w[c] = pack_cell(s6, e6);
-  }
-  if (!P.prm.flag_chessboard) {
-    // eta kept as read, no cube decoding (gpu_water3D.cu:794)
-    set_nhb(L, w);
-    return upload_point_words(s, pt, w);
-  }
-  int bad = 0;
-  std::vector<uint32_t> masks;
-  std::vector<uint32_t> org;
-  for_each_cube(L, [&](uint32_t ox, uint32_t oy, uint32_t oz, uint32_t) {
-    bool ok = true;
-    const uint32_t st = cube_state_from_words(w, L, ox, oy, oz);
-    const uint32_t cur = cube_mask_from_words(w, L, ox, oy, oz, &ok);
-    const uint32_t M = sol_mask(st);
-    if (!ok || cur != M) ++bad;
-    masks.push_back(M);
-    org.push_back(ox | (oy << 8) | (oz << 16));
-  });
-  // rewrite after all decisions are taken (each decision reads the input eta)
-  for (size_t k = 0; k < masks.size(); ++k)
-    set_cube_eta(w, L, org[k] & 0xFF, (org[k] >> 8) & 0xFF, org[k] >> 16, masks[k]);
-  rc = upload_point_words(s, pt, w);
-  if (rc) return rc;
-  return bad;
+  s->obs_at = -1;
+  return (int)(out[1] + 1u);  // counted from all ones; without the chessboard nothing is counted
 }
 
 int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
   int rc = check_pt(s, pt);
   if (rc) return rc;
   HIPC(hipSetDevice(s->device));
-  std::vector<uint32_t> w;
-  rc = download_point_words(s, pt, w);
-  if (rc) return rc;
-  const uint32_t N = s->ph[pt].N;
-  for (uint32_t c = 0; c < N; ++c)
-    for (int a = 0; a < 6; ++a) {
-      if (sigma6N) sigma6N[a * N + c] = (uint8_t)sigma_of(w[c], a);
-      if (eta6N) eta6N[a * N + c] = (uint8_t)eta_of(w[c], a);
-    }
+  const PointHost& P = s->ph[pt];
+  const size_t n6 = 6 * (size_t)P.N;
+  if ((rc = reserve_config(s, n6))) return rc;
+  launch_config_out(s->stream, s->words.p + P.woff, P.N, s->cfg_bytes.p, s->cfg_bytes.p + n6);
+  HIPC(hipGetLastError());
+  HIPC(hipStreamSynchronize(s->stream));
+  if ((rc = check_resident(s))) return rc;
+  if (sigma6N) HIPC(hipMemcpy(sigma6N, s->cfg_bytes.p, n6, hipMemcpyDeviceToHost));
+  if (eta6N) HIPC(hipMemcpy(eta6N, s->cfg_bytes.p + n6, n6, hipMemcpyDeviceToHost));
   return CVF_OK;
 }
 

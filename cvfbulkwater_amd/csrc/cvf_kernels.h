@@ -100,6 +100,13 @@ struct ObsOut {
 };
 void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
                     const PointState* ps, const uint32_t* rstatus, const ObsOut& out);
+// The words W of a point (N cells) as sigma and eta arrays (6N bytes each).
+void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* sigma, uint8_t* eta);
+// sigma and eta arrays to the words W through `scratch` (L^3 words): *first
+// (all ones before) tells the first value out of range, then W is not
+// written; *inconsistent counts up the cubes whose eta was not a solution.
+void launch_config_in(hipStream_t st, const uint8_t* sigma, const uint8_t* eta, uint32_t L, int chessboard,
+                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent);
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc);
 void launch_sw_union(hipStream_t st, Launch ln, uint32_t* parent, const uint8_t* cov);

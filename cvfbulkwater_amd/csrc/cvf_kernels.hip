@@ -760,6 +760,111 @@ __global__ __launch_bounds__(256) void k_observe(const BlockEnt* __restrict__ ta
     part[lb] = make_uint2(sh[0].x + sh[1].x + sh[2].x + sh[3].x, sh[0].y + sh[1].y + sh[2].y + sh[3].y);
 }
 
+// ------------------------------------------------- configuration in and out
+// sigma and eta arrays (arm-major bytes, index arm N + cell) to and from the
+// packed words, four cells per thread: twelve 4-byte pieces on the byte side,
+// one 16-byte piece on the word side.  Done on the host, the two directions
+// and the decoding below took 3.3 ms at L = 48; here they are bound by the
+// copies over the link.
+__global__ __launch_bounds__(256) void k_config_out(const uint32_t* __restrict__ W, uint32_t N,
+                                                   uint8_t* __restrict__ sigma, uint8_t* __restrict__ eta) {
+  const uint32_t t = 4 * (blockIdx.x * 256 + threadIdx.x);
+  if (t >= N) return;  // N is a multiple of 4
+  const uint4 v = *reinterpret_cast<const uint4*>(W + t);
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    *reinterpret_cast<uint32_t*>(sigma + (size_t)a * N + t) =
+        sigma_of(v.x, a) | sigma_of(v.y, a) << 8 | sigma_of(v.z, a) << 16 | sigma_of(v.w, a) << 24;
+    *reinterpret_cast<uint32_t*>(eta + (size_t)a * N + t) =
+        eta_of(v.x, a) | eta_of(v.y, a) << 8 | eta_of(v.z, a) << 16 | eta_of(v.w, a) << 24;
+  }
+}
+
+// The first value out of range (sigma above 5, eta above 1) in the order of
+// the arrays, sigma before eta at one index: *first = 2 i, or 2 i + 1.
+__global__ __launch_bounds__(256) void k_config_in(const uint8_t* __restrict__ sigma, const uint8_t* __restrict__ eta,
+                                                  uint32_t N, uint32_t* __restrict__ W, uint32_t* __restrict__ first) {
+  const uint32_t t = 4 * (blockIdx.x * 256 + threadIdx.x);
+  if (t >= N) return;
+  uint32_t w[4] = {0, 0, 0, 0}, bad = 0xFFFFFFFFu;
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    const uint32_t s = *reinterpret_cast<const uint32_t*>(sigma + (size_t)a * N + t);
+    const uint32_t e = *reinterpret_cast<const uint32_t*>(eta + (size_t)a * N + t);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const uint32_t sv = (s >> (8 * m)) & 255u, ev = (e >> (8 * m)) & 255u, i = a * N + t + m;
+      if (sv > 5) bad = min(bad, 2 * i);
+      if (ev > 1) bad = min(bad, 2 * i + 1);
+      w[m] |= (sv & 7u) << (3 * a) | (ev & 1u) << (kEtaShift + a);
+    }
+  }
+  if (bad != 0xFFFFFFFFu) atomicMin(first, bad);
+  *reinterpret_cast<uint4*>(W + t) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// State of the cube with origin (ox, oy, oz) by the decision tree of
+// gpu_Chessboard_set_state (gpu_water3D.cu:3350-3368): v1 = b0, v2 = b1,
+// v3 = b2, v6 = b6, v7 = b5, v8 = b3.
+template <class Eta>
+__device__ __forceinline__ uint32_t cube_state(Eta&& eta) {
+  if (eta(0, 0) == 0) return eta(6, 0) == 0 ? 2u : eta(2, 4) == 0 ? 3u : 8u;
+  if (eta(0, 2) == 0) return eta(1, 4) == 0 ? 4u : eta(5, 2) == 0 ? 5u : 7u;
+  return eta(2, 0) == 0 ? 0u : eta(3, 4) == 0 ? 1u : 6u;
+}
+
+// The packed input in src to the state in dst, unless a value was out of
+// range.  With the chessboard each cell takes the eta bits that its two
+// cubes' solutions give it, the states read from the input's eta; the cell at
+// a cube's origin counts the cube into *inconsistent when its eta was not a
+// solution.  Without it eta stays as read and the cell's HB counter is set
+// (gpu_water3D.cu:845-862).
+__global__ __launch_bounds__(256) void k_config_decode(const uint32_t* __restrict__ src, uint32_t L, FastDiv dL,
+                                                      int chessboard, uint32_t* __restrict__ dst,
+                                                      const uint32_t* __restrict__ first,
+                                                      uint32_t* __restrict__ inconsistent) {
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x, N = L * L * L;
+  if (t >= N || *first != 0xFFFFFFFFu) return;
+  const uint32_t r1 = fdiv(t, dL), x = t - r1 * L, z = fdiv(r1, dL), y = r1 - z * L;
+  const uint32_t w = src[t];
+  if (!chessboard) {
+    const uint32_t up[3] = {neighbor_up(t, x, 1, L), neighbor_up(t, y, L, L), neighbor_up(t, z, L * L, L)};
+    const uint32_t dn[3] = {x ? t - 1 : t + L - 1, y ? t - L : t + (L - 1) * L, z ? t - L * L : t + (L - 1) * L * L};
+    uint32_t n = 0;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+      n += eta_of(w, 2 * ax) & (uint32_t)(sigma_of(w, 2 * ax) == sigma_of(src[up[ax]], 2 * ax + 1));
+      n += eta_of(w, 2 * ax + 1) & (uint32_t)(sigma_of(w, 2 * ax + 1) == sigma_of(src[dn[ax]], 2 * ax));
+    }
+    dst[t] = (w & kLowBits) | n << kNhbShift;
+    return;
+  }
+  uint32_t bits = 0;
+#pragma unroll
+  for (uint32_t fam = 0; fam < 2; ++fam) {
+    const uint32_t bx = (x & 1u) != fam, by = (y & 1u) != fam, bz = (z & 1u) != fam;  // the cell's corner
+    const uint32_t ox = bx ? (x ? x - 1 : L - 1) : x, oy = by ? (y ? y - 1 : L - 1) : y, oz = bz ? (z ? z - 1 : L - 1) : z;
+    const uint32_t x1 = ox + 1 == L ? 0 : ox + 1, y1 = oy + 1 == L ? 0 : oy + 1, z1 = oz + 1 == L ? 0 : oz + 1;
+    const auto eta = [&](int b, int arm) {
+      return eta_of(src[((b & 1) ? x1 : ox) + L * (((b & 2) ? y1 : oy) + L * ((b & 4) ? z1 : oz))], arm);
+    };
+    const uint32_t M = sol_mask(cube_state(eta));
+    const int b = (int)(bx + 2 * by + 4 * bz);
+    bits |= ((M >> corner_edge(b, 0)) & 1u) << bx | ((M >> corner_edge(b, 1)) & 1u) << (2 + by) |
+            ((M >> corner_edge(b, 2)) & 1u) << (4 + bz);
+    if (b == 0) {
+      bool ok = true;
+      for (int j = 0; j < kEdges; ++j) {
+        const int A = edge_start(j), ax = edge_axis(j), B = A | (1 << ax);
+        const uint32_t want = (M >> j) & 1u;
+        ok = ok && eta(A, 2 * ax) == want && eta(B, 2 * ax + 1) == want;
+      }
+      if (!ok) atomicAdd(inconsistent, 1u);
+    }
+  }
+  dst[t] = (w & kSigmaBits) | bits << kEtaShift;
+}
+
 // Counts of the six sigma values over the 6N arms of one point, as
 // kHistReplicas partial histograms (counts[r * 6 + s], r = workgroup mod
 // kHistReplicas) that the host sums: spreading the atomics keeps them from
@@ -1385,6 +1490,16 @@ void launch_zero3_u32(hipStream_t st, uint32_t* a, size_t na, uint32_t* b, size_
 void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
                     const PointState* ps, const uint32_t* rstatus, const ObsOut& out) {
   launch(k_observe, dim3(nblocks), dim3(256), st, tab, nblocks, words, span, ps, rstatus, out.part, out.ps, out.status);
+}
+void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* sigma, uint8_t* eta) {
+  launch(k_config_out, dim3((N / 4 + 255) / 256), dim3(256), st, W, N, sigma, eta);
+}
+void launch_config_in(hipStream_t st, const uint8_t* sigma, const uint8_t* eta, uint32_t L, int chessboard,
+                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent) {
+  const uint32_t N = L * L * L;
+  launch(k_config_in, dim3((N / 4 + 255) / 256), dim3(256), st, sigma, eta, N, scratch, first);
+  launch(k_config_decode, dim3((N + 255) / 256), dim3(256), st, (const uint32_t*)scratch, L, make_fastdiv(L),
+         chessboard, W, (const uint32_t*)first, inconsistent);
 }
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc) {
