@@ -315,7 +315,7 @@ class Simulation:
 
     def plan(self, pt: int = 0) -> dict:
         """Launch plan of point pt: stream group, planes per z-slab (0:
-        unfused kernels), sigma half-sweeps per fused launch and the kind of
+        unfused kernels or tiles), sigma half-sweeps per fused launch and the kind of
         Metropolis launch (unfused, fused, resident)."""
         g, t, k, kind = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()
         _check(self._lib, self._lib.cvf_get_plan(self._h, pt, C.byref(g), C.byref(t), C.byref(k), C.byref(kind)),

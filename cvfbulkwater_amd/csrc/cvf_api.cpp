@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <map>
 #include <queue>
 #include <memory>
 #include <string>
@@ -111,6 +112,11 @@ struct Group {
   uint32_t chunk_lds_long = 0;  // the same for kMaxChunk half-sweeps; 0 if that does not fit
   uint32_t chunk_lds_eta = 0;   // the same for the eta sweep alone (fast schedule)
   bool any_nc = false;          // some point runs the non-chessboard rule
+  // fused launches on tiles instead of slabs (chunk_lds, chunk_lds_long hold
+  // their LDS then)
+  bool tiled = false;
+  DevBuf<TileEnt> tab_tile;
+  uint32_t nb_tile = 0;
   size_t sigma_cells = 0;    // cells swept per fused launch
   // resident Metropolis kernel (tuning fused = 2): slabs dealt to at most one
   // workgroup per CU, their neighbour rings and versions
@@ -930,6 +936,169 @@ int upload_group_steps(cvf_sim* s) {
   return CVF_OK;
 }
 
+// Tiles of a set of points: an axis of length d takes ceil(d / edge) tiles of
+// even length, the last one shorter; half-sweeps per launch, workgroup size
+// and modeled length of a Metropolis pass.
+struct TilePlan {
+  uint32_t edge[3] = {0, 0, 0}, nk = 0, block = 0;
+  double us = 0;  // 0: none
+};
+uint32_t even_edge(uint32_t edge, uint32_t d) {
+  const uint32_t n = (d + edge - 1) / edge;
+  return (d + n - 1) / n;
+}
+
+// Modeled length of a pass (cube sweep and 12 half-sweeps) in us, 0 if the
+// windows do not fit.  A launch takes 7.1 us and a workgroup 4.9 us at 1024
+// threads (schedule, tables, window); a half-sweep 0.22 us for each trip of
+// the workgroup over its quads and 0.21 us for each 256 quads on the CU; a cube
+// family 3.8 and 2.8 us likewise.  Fitted to 170 measured shapes of one point
+// of L = 32 .. 200, to 7 % rms; the shape it picks ran within 2 % of the fastest
+// measured one at every L.
+double tile_model(const std::map<uint32_t, uint32_t>& points, const TilePlan& t, uint32_t ncu) {
+  struct Tile {
+    double edge[3], n;
+  };
+  std::vector<Tile> tiles;
+  uint32_t lds = 0;
+  double total = 0;
+  for (const auto& lc : points) {
+    const uint32_t d[3] = {lc.first / 2, lc.first / 2, lc.first};
+    uint32_t c[3];
+    Tile q;
+    q.n = lc.second;
+    for (int a = 0; a < 3; ++a) {
+      c[a] = even_edge(t.edge[a], d[a]);
+      q.edge[a] = c[a];
+      q.n *= (d[a] + c[a] - 1) / c[a];
+    }
+    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], t.nk, true));
+    total += q.n;
+    tiles.push_back(q);
+  }
+  if (lds > tile_lds_limit()) return 0;
+  // tiles of a CU, and how many of them run together
+  const double per_cu = std::ceil(total / ncu);
+  const double co =
+      std::max(1.0, std::min({per_cu, std::floor(160 * 1024.0 / (lds + 3072)), std::floor(2048.0 / t.block)}));
+  const auto box = [](const Tile& q, double more) {
+    return (q.edge[0] + more) * (q.edge[1] + more) * (q.edge[2] + more);
+  };
+  const auto phase = [&](double quads, double trip, double per256) {
+    return trip * std::ceil(quads / t.block) + per256 * co * quads / 256;
+  };
+  double us = 0;
+  for (uint32_t launch = 0; launch < 12 / t.nk; ++launch) {
+    double work = 0;
+    for (const Tile& q : tiles) {
+      double x = 4.9 * co * t.block / 1024;
+      if (launch == 0) x += 2 * phase(box(q, t.nk / 6.0 + 2) / 8, 3.8, 2.8);
+      // a later half-sweep adds 1/6 layer on average to each axis
+      for (uint32_t k = 0; k < t.nk; ++k) {
+        const double quads = box(q, (t.nk - 1 - k) / 6.0) / 2;
+        x += 4 * quads <= t.block ? 0.34 * co * quads / 256 : phase(quads, 0.22, 0.21);
+      }
+      work += q.n * x;
+    }
+    us += 7.1 + std::ceil(per_cu / co) * work / total;
+  }
+  return us;
+}
+
+// The fastest modeled shape with t's launch length and workgroup size: every
+// number of tiles along the axes of the largest point, boxes at most three
+// times as long as thin.
+TilePlan best_tiles(const std::map<uint32_t, uint32_t>& points, uint32_t nk, uint32_t block, uint32_t ncu) {
+  const uint32_t L = points.rbegin()->first;
+  const auto edges = [](uint32_t d) {
+    std::vector<uint32_t> e;
+    for (uint32_t n = 1; n <= d; ++n) {
+      const uint32_t c = (d + n - 1) / n;
+      if (c <= std::min(32u, kMaxTile) && c >= std::min(3u, d) && (e.empty() || e.back() != c)) e.push_back(c);
+    }
+    return e;
+  };
+  TilePlan best;
+  for (uint32_t ex : edges(L / 2))
+    for (uint32_t ey : edges(L / 2))
+      for (uint32_t ez : edges(L)) {
+        if (ey > ex || std::max(ex, ez) > 3 * std::min(ey, ez) + 2) continue;
+        TilePlan t;
+        t.edge[0] = ex, t.edge[1] = ey, t.edge[2] = ez;
+        t.nk = nk;
+        t.block = block;
+        t.us = tile_model(points, t, ncu);
+        if (t.us > 0 && (best.us == 0 || t.us < best.us)) best = t;
+      }
+  return best;
+}
+
+// Fused launches can run on tiles: the chessboard rule's reference schedule,
+// no slab thickness asked for, and the workgroups the kernel's tables need.
+bool tiles_possible(const cvf_sim* s, const cvf_tuning& t) {
+  for (const auto& P : s->ph)
+    if (!P.prm.flag_chessboard) return false;
+  return s->sched == CVF_SCHED_REFERENCE && s->nm > 0 && t.fused != 0 && t.slab_planes == 0 &&
+         t.block_chunk >= 256;
+}
+
+int cu_count(const cvf_sim* s, uint32_t& ncu) {
+  int n = 0;
+  HIPC(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, s->device));
+  ncu = (uint32_t)std::max(n, 1);
+  return CVF_OK;
+}
+
+// Tiles for group g's fused launches, in the place of slabs that do not fit
+// LDS (L > 64; L = 72 / 96 / 128 / 160 / 200 / 252: 27.1 / 33.2 / 47.6 / 75.6 /
+// 142 / 268 us per step, unfused 44.9 / 49.9 / 67.2 / 104 / 162 / 304) or are
+// one plane thick, so that each of them recomputes two planes and more (a step
+// with a cluster sweep at L = 8 / 16 / 32 / 48 / 64: 31.1 / 30.6 / 34.3 / 37.8 /
+// 43.2 us, slabs 32.6 / 30.9 / 36.2 / 49.4 / 57.8).  At two planes the two are even
+// (16 points of L = 32: 30.4 and 29.6).
+int build_tiles(cvf_sim* s, Group& g, uint32_t thickest) {
+  g.tiled = false;
+  if (!tiles_possible(s, s->tune) || (g.fused && thickest > 1)) return CVF_OK;
+  uint32_t ncu = 0;
+  int rc = cu_count(s, ncu);
+  if (rc) return rc;
+  std::map<uint32_t, uint32_t> count;
+  for (int p : g.points) ++count[s->ph[p].L];
+  const uint32_t want = s->tune.chunk_sweeps == kMaxChunk ? kMaxChunk : kChunk;
+  ncu = std::max(1u, ncu / (uint32_t)s->groups.size());
+  TilePlan t = best_tiles(count, want, (uint32_t)s->tune.block_chunk, ncu);
+  if (t.us == 0) t = best_tiles(count, kChunk, (uint32_t)s->tune.block_chunk, ncu);
+  if (t.us == 0) return CVF_OK;
+  std::vector<TileEnt> tab;
+  uint32_t lds = 0, lds_long = 0;
+  g.sigma_cells = 0;
+  for (int p : g.points) {
+    const PointHost& P = s->ph[p];
+    const uint32_t hL = P.L / 2, d[3] = {hL, hL, P.L};
+    uint32_t c[3];
+    for (int a = 0; a < 3; ++a) c[a] = even_edge(t.edge[a], d[a]);
+    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], kChunk, true));
+    lds_long = std::max(lds_long, 16 * tile_window_quads(c[0], c[1], c[2], kMaxChunk, true));
+    g.sigma_cells += P.N;
+    for (uint32_t z = 0; z < d[2]; z += c[2])
+      for (uint32_t y = 0; y < d[1]; y += c[1])
+        for (uint32_t x = 0; x < d[0]; x += c[0])
+          tab.push_back(TileEnt{p, P.L, P.woff, (uint32_t)P.prm.seed, (uint32_t)(P.prm.seed >> 32), x, y, z,
+                                std::min(c[0], d[0] - x), std::min(c[1], d[1] - y), std::min(c[2], d[2] - z), 0});
+  }
+  TileEnt pad;
+  memset(&pad, 0, sizeof pad);
+  pad.point = -1;
+  while (tab.size() % kNumXcd) tab.push_back(pad);
+  if ((rc = upload_vec(g.tab_tile, tab))) return rc;
+  g.nb_tile = (uint32_t)tab.size();
+  g.chunk_lds = lds;
+  g.chunk_lds_long = lds_long <= tile_lds_limit() ? lds_long : 0;
+  g.fused = true;
+  g.tiled = true;
+  return CVF_OK;
+}
+
 // (Re)build the groups for the current tuning: points are dealt to groups
 // largest-first onto the group with the fewest cells.
 int build_groups(cvf_sim* s) {
@@ -999,13 +1168,16 @@ int build_groups(cvf_sim* s) {
       }
     }
     if (!long_fits) g->chunk_lds_long = 0;
+    uint32_t thickest = 0;
+    for (const BlockEnt& en : ts) thickest = std::max(thickest, en.T);
+    if ((rc = build_tiles(s, *g, thickest))) return rc;
     for (int p : g->points) {
       s->ph[p].group = (int32_t)(&g - &s->groups[0]);
       s->ph[p].slab_T = 0;
     }
-    if (g->fused)
+    if (g->fused && !g->tiled)
       for (const BlockEnt& en : ts) s->ph[en.point].slab_T = en.T;
-    if (g->fused) {
+    if (g->fused && !g->tiled) {
       // largest slabs first (the kernel takes entries in launch order, and
       // each XCD's dispatcher hands out its share in that order)
       std::stable_sort(ts.begin(), ts.end(), [](const BlockEnt& a, const BlockEnt& b) {
@@ -1039,6 +1211,18 @@ int build_groups(cvf_sim* s) {
   }
   HIPC(hipDeviceSynchronize());
   return CVF_OK;
+}
+
+// A fused launch of half-sweeps k0 .. k0 + nk - 1 of group g from src to dst.
+void launch_fused(cvf_sim* s, const Group& g, hipStream_t st, const uint64_t* stepp, uint32_t step_off,
+                  const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk, int with_eta) {
+  const uint32_t lds = nk == (uint32_t)kMaxChunk ? g.chunk_lds_long : g.chunk_lds;
+  if (g.tiled)
+    launch_tile(st, g.tab_tile.p, g.nb_tile, (uint32_t)s->tune.block_chunk, stepp, step_off, s->pts.p, src, dst, k0,
+                nk, with_eta, lds);
+  else
+    launch_chunk(st, Launch{g.tab_slab.p, g.nb_slab, (uint32_t)s->tune.block_chunk, stepp, step_off}, s->pts.p, src,
+                 dst, k0, nk, with_eta, lds, g.any_nc);
 }
 
 struct Untimed {
@@ -1089,14 +1273,12 @@ void enqueue_lattice(cvf_sim* s, int gi, hipStream_t st, uint32_t step_off, Time
       timed(CVF_KCLASS_SIGMA, [&] { launch_sigma_f(st, lh, s->pts.p, cur, (uint32_t)pass); });
   } else if (g.fused && s->nm > 0) {
     // 12*n_metropolis half-sweeps in launches of kChunk (kMaxChunk in the variant form)
-    const Launch lz{g.tab_slab.p, g.nb_slab, (uint32_t)s->tune.block_chunk, stepp, step_off};
     const int len = variant ? kMaxChunk : kChunk;
-    const uint32_t lds = variant ? g.chunk_lds_long : g.chunk_lds;
     for (int c = 0; c < 12 * s->nm / len; ++c) {
       const uint32_t* src = par ? s->words2.p : s->words.p;
       uint32_t* dst = par ? s->words.p : s->words2.p;
       timed(CVF_KCLASS_CHUNK, [&] {
-        launch_chunk(st, lz, s->pts.p, src, dst, (uint32_t)(c * len), (uint32_t)len, c == 0, lds, g.any_nc);
+        launch_fused(s, g, st, stepp, step_off, src, dst, (uint32_t)(c * len), (uint32_t)len, c == 0);
       });
       par ^= 1;
     }
@@ -1310,12 +1492,30 @@ cvf_tuning default_tuning(const cvf_sim* s) {
   }
   t.chunk_sweeps = s->total_cells < (1u << 20) && !any_nc ? kMaxChunk : kChunk;
   if (all_wide) {
-    // no fused window fits a plane beyond L = 64: one-plane resident slabs,
-    // one workgroup per CU (49.7 against 59.8 us per step at L = 96 for the
-    // unfused kernels); points that cannot run resident fall back to those
-    t.fused = 2;
-    t.slab_planes = 1;
-    t.block_chunk = 1024;
+    // no slab's window fits a plane beyond L = 64: tiles, at the launch length
+    // and workgroup size that their model gives the shortest pass (L = 68 / 72 /
+    // 96 / 112: 26.3 / 27.1 / 33.2 / 41.8 us per step, one-plane resident slabs
+    // 29.8 / 30.6 / 42.2 / 53.6)
+    TilePlan best;
+    uint32_t ncu = 0;
+    std::map<uint32_t, uint32_t> count;
+    for (const auto& P : s->ph) ++count[P.L];
+    if (tiles_possible(s, t) && cu_count(s, ncu) == CVF_OK)
+      for (uint32_t nk : {(uint32_t)kChunk, (uint32_t)kMaxChunk})
+        for (uint32_t block : {512u, 1024u}) {
+          const TilePlan p = best_tiles(count, nk, block, ncu);
+          if (p.us > 0 && (best.us == 0 || p.us < best.us)) best = p;
+        }
+    if (best.us > 0) {
+      t.chunk_sweeps = (int32_t)best.nk;
+      t.block_chunk = (int32_t)best.block;
+    } else {
+      // one-plane resident slabs, one workgroup per CU; points that cannot
+      // run resident fall back to the unfused kernels
+      t.fused = 2;
+      t.slab_planes = 1;
+      t.block_chunk = 1024;
+    }
   }
   // a small handle of one Metropolis sweep per step, nothing between the
   // steps, whose planes can each have a workgroup: one-plane resident slabs
@@ -1331,7 +1531,7 @@ cvf_tuning default_tuning(const cvf_sim* s) {
     planes += P.L;
     maxL = std::max(maxL, P.L);
   }
-  if (!any_nc && s->sched == CVF_SCHED_REFERENCE && s->nm == 1 && s->nc == 0 && planes <= 256 &&
+  if (!any_nc && !all_wide && s->sched == CVF_SCHED_REFERENCE && s->nm == 1 && s->nc == 0 && planes <= 256 &&
       s->total_cells < (1u << 20)) {
     t.fused = 2;
     t.slab_planes = 1;
@@ -1955,7 +2155,7 @@ int cvf_get_plan(cvf_sim* s, int32_t pt, int32_t* group, int32_t* slab_planes, i
   const PointHost& P = s->ph[pt];
   const Group& g = *s->groups[P.group];
   if (group) *group = P.group;
-  if (kind) *kind = g.resident ? 2 : P.slab_T ? 1 : 0;
+  if (kind) *kind = g.resident ? 2 : P.slab_T || g.tiled ? 1 : 0;
   if (g.resident) {
     if (slab_planes) *slab_planes = (int32_t)P.slab_T;
     if (chunk_sweeps) *chunk_sweeps = 0;
@@ -1967,7 +2167,7 @@ int cvf_get_plan(cvf_sim* s, int32_t pt, int32_t* group, int32_t* slab_planes, i
     // only where every window of the group holds the wider halo
     const bool whole = s->sched == CVF_SCHED_REFERENCE && s->tune.chunk_sweeps == kMaxChunk &&
                        g.chunk_lds_long != 0;
-    const bool none = P.slab_T == 0 || s->nm == 0 || s->sched != CVF_SCHED_REFERENCE;
+    const bool none = (P.slab_T == 0 && !g.tiled) || s->nm == 0 || s->sched != CVF_SCHED_REFERENCE;
     *chunk_sweeps = none ? 0 : whole ? kMaxChunk : kChunk;
   }
   return CVF_OK;

@@ -146,4 +146,76 @@ __device__ __forceinline__ void quad_plane_cells(uint32_t base, uint32_t L, uint
   nb[3] = cell[3] + off_hi;
 }
 
+// A wave-uniform value in a scalar register.
+__device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+
+// Chessboard sigma rule on one word w (facing neighbour word wn, random
+// word rw): the cell's new word, as sigma_quad_regs computes each of four.
+__device__ __forceinline__ uint32_t sigma_cell(uint32_t w, uint32_t wn, const uint32_t* thr, int arm, uint32_t rw) {
+  uint32_t sp, ra;
+  split_word(rw, 6, sp, ra);
+  const uint32_t sa = sigma_of(w, arm);
+  const uint32_t t = thr[sigma_thr_index(w, wn, arm, sa, sp)];
+  const uint32_t nw = (w & ~(7u << (3 * arm))) | (sp << (3 * arm));
+  return sp != sa && ra < t ? nw : w;
+}
+
+// Word h of a Philox block (h lane-dependent).
+__device__ __forceinline__ uint32_t pick4(const U4& r, uint32_t h) {
+  return h == 0 ? r.x : h == 1 ? r.y : h == 2 ? r.z : r.w;
+}
+
+// Chessboard sigma rule on four words held in registers (facing neighbour
+// words wn, one Philox block): the cells' new words.  The four threshold
+// loads are issued together (the index is in range also when the proposal
+// equals the current value), then the four decisions are made.
+__device__ __forceinline__ void sigma_quad_regs(uint32_t (&w)[4], const uint32_t (&wn)[4], const uint32_t* thr,
+                                                int arm, const U4& q) {
+  uint32_t sp[4], ra[4], t[4];
+  bool act[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const uint32_t rw = m == 0 ? q.x : m == 1 ? q.y : m == 2 ? q.z : q.w;
+    split_word(rw, 6, sp[m], ra[m]);
+    const uint32_t sa = sigma_of(w[m], arm);
+    act[m] = sp[m] != sa;
+    t[m] = thr[sigma_thr_index(w[m], wn[m], arm, sa, sp[m])];
+  }
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const uint32_t nw = (w[m] & ~(7u << (3 * arm))) | (sp[m] << (3 * arm));
+    w[m] = act[m] && ra[m] < t[m] ? nw : w[m];
+  }
+}
+
+// The draws of one phase, draw(seed, stream, site, step, sub) for every
+// item's site: the part that does not depend on the site, once per phase
+// (in scalar registers) ...
+__device__ __forceinline__ PhiloxFixed phase_draws(uint64_t seed, uint32_t stream, uint64_t step, uint32_t sub) {
+  return philox_fixed((uint32_t)step, (stream << 24) | sub, (uint32_t)(step >> 32), (uint32_t)seed,
+                      (uint32_t)(seed >> 32));
+}
+// ... and one item's draw.  The round-2 key goes through an empty asm
+// statement, so that the compiler rebuilds the later round keys with
+// scalar adds in each iteration instead of holding all of them in scalar
+// registers across the loop (which spills the phase's other scalars).
+__device__ __forceinline__ U4 draw_site(uint32_t site, const PhiloxFixed& f) {
+  uint32_t k0 = f.k0, k1 = f.k1;
+  asm volatile("" : "+s"(k0), "+s"(k1));
+  return philox_site(site, f, k0, k1);
+}
+
+// The four words of a quad (16-byte aligned window index w).
+__device__ __forceinline__ void quad_load(const uint32_t* lds, uint32_t w, uint32_t (&v)[4]) {
+  const uint4 t = *reinterpret_cast<const uint4*>(lds + w);
+  v[0] = t.x;
+  v[1] = t.y;
+  v[2] = t.z;
+  v[3] = t.w;
+}
+__device__ __forceinline__ void quad_store(uint32_t* lds, uint32_t w, const uint32_t (&v)[4]) {
+  *reinterpret_cast<uint4*>(lds + w) = make_uint4(v[0], v[1], v[2], v[3]);
+}
+
 }  // namespace cvf

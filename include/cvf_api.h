@@ -151,19 +151,21 @@ typedef struct cvf_tuning {
   int32_t block_eta;    /* workgroup size of the eta cube sweep */
   int32_t block_cell;   /* workgroup size of the per-cell kernels (SW, observables) */
   int32_t graph_steps;  /* MC steps per replayed hipGraph, or per resident launch (1..64) */
-  int32_t fused;        /* 1: eta sweep + 6 half-sweeps per kernel on LDS-staged z-slabs
-                           where the slab fits in LDS; 0: one kernel per half-sweep;
+  int32_t fused;        /* 1: eta sweep + 6 half-sweeps per kernel on LDS-staged z-slabs, or
+                           on boxes short along all axes (tiles) where slabs do not fit in
+                           LDS or would be one plane thick; 0: one kernel per half-sweep;
                            2: the resident kernel (every step of a graph in one launch, the
                            lattice held in LDS, one stream group) where the points allow it
                            (reference schedule, one Metropolis sweep per step, chessboard
                            rule), else as 1.  The default is 1, or 2 with one-plane slabs
-                           when every point's L exceeds 64 (no fused window fits) */
+                           for small handles of one Metropolis sweep per step */
   int32_t slab_planes;  /* planes per slab of the fused kernel (<= 16), or the thickest slab
-                           of the resident kernel; 0 = automatic */
+                           of the resident kernel; 0 = automatic (tiles included) */
   int32_t block_chunk;  /* workgroup size of the fused kernel */
   int32_t chunk_sweeps; /* half-sweeps per fused launch: 6, or 12 (a whole Metropolis pass per
                            launch where the wider window still fits in LDS); 0 = 6.  The default
-                           is 12 for handles under 2^20 cells with the chessboard rule, else 6 */
+                           is 12 for handles under 2^20 cells with the chessboard rule, what
+                           the tiles' model gives when every point's L exceeds 64, else 6 */
 } cvf_tuning;
 
 int cvf_get_tuning(cvf_sim *s, cvf_tuning *t);
@@ -171,10 +173,10 @@ int cvf_get_tuning(cvf_sim *s, cvf_tuning *t);
 /* Launch plan of state point pt under the current tuning (no reference
  * counterpart; the reference has one launch shape): its stream group, the
  * planes per z-slab of its fused or resident launches (0 when its group
- * runs the unfused kernels), the sigma half-sweeps per fused launch of the
+ * runs the unfused kernels, or tiles), the sigma half-sweeps per fused launch of the
  * reference schedule (6 or 12; 0 when none run fused) and the kind of
- * Metropolis launch: 0 unfused kernels, 1 fused slab launches, 2 the
- * resident kernel. */
+ * Metropolis launch: 0 unfused kernels, 1 fused launches (slabs, or tiles),
+ * 2 the resident kernel. */
 int cvf_get_plan(cvf_sim *s, int32_t pt, int32_t *group, int32_t *slab_planes, int32_t *chunk_sweeps,
                  int32_t *kind);
 /* Rebuilds the groups, block tables and graphs; synchronises the handle. */
@@ -199,7 +201,7 @@ enum {
   CVF_KCLASS_SW_LOCAL = 3,
   CVF_KCLASS_SW_UNION = 4,
   CVF_KCLASS_SW_FLIP = 5,
-  CVF_KCLASS_CHUNK = 6,   /* fused slab kernel (eta sweep + 6 sigma half-sweeps) */
+  CVF_KCLASS_CHUNK = 6,   /* fused slab or tile kernel (eta sweep + 6 sigma half-sweeps) */
   CVF_KCLASS_RESIDENT = 7, /* resident kernel: all profiled steps in one launch (one step per
                               launch with Swendsen-Wang steps) */
   CVF_KCLASS_COUNT = 8
