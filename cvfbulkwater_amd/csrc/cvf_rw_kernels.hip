@@ -259,8 +259,9 @@ __global__ __launch_bounds__(1024) void k_rw_cells(RwCells cells, const RwSim* _
   if ((int)threadIdx.x < R) bps[threadIdx.x] = tg.bp[t0 + min((int)threadIdx.x, nt - 1)];
   if (ps) {
     double* lz = sl + 4 * n_sim;  // log_Z of the sweep before
-    for (int j0 = 0; j0 < n_sim; j0 += kRwRow) {
-      reduce_partials<kRwRow, false>(ps + (int64_t)j0 * w.nblk, w.nblk, red, [&](int k, double st) {
+    // (a sweep's targets are its simulations: n_sim <= R where R < kRwRow)
+    for (int j0 = 0; j0 < n_sim; j0 += R) {
+      reduce_partials<R, false>(ps + (int64_t)j0 * w.nblk, w.nblk, red, [&](int k, double st) {
         if (j0 + k < n_sim) lz[j0 + k] = (st != 0 ? log(st) : 0.0) + mx[j0 + k];
       });
       __syncthreads();
