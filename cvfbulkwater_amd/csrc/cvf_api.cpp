@@ -224,6 +224,12 @@ struct cvf_sim {
   PinBuf<uint2> obs_part;
   PinBuf<PointState> obs_ps;
   PinBuf<uint32_t> obs_status;
+  // non-chessboard points: their table, bond bytes (one per cell of the
+  // handle) and capped counts (by point)
+  DevBuf<CappedEnt> tab_capped;
+  uint32_t n_capped = 0, capped_L = 0;
+  DevBuf<uint8_t> bonds;
+  PinBuf<uint32_t> obs_capped;
   std::vector<int32_t> obs_point;  // point of each k_observe workgroup (-1: padding)
   std::vector<int64_t> obs_nhb2, obs_nsig;
 
@@ -316,29 +322,6 @@ void set_nhb(uint32_t L, std::vector<uint32_t>& w) {
   for (uint32_t c = 0; c < N; ++c) w[c] = (w[c] & kLowBits) | (n[c] << kNhbShift);
 }
 
-// Capped HB count of measure() without the chessboard (gpu_water3D.cu:
-// 2064-2099): cells in index order, forward x, y, z bonds; a bond counts for
-// both cells while both counters are below NHBMAX = 4.  Returns 2 N_HB.
-int64_t greedy_nhb2(uint32_t L, const std::vector<uint32_t>& w) {
-  const uint32_t N = L * L * L;
-  std::vector<uint8_t> cnt(N, 0);
-  int64_t total = 0;
-  for (uint32_t c = 0; c < N; ++c) {
-    const uint32_t x = c % L, y = (c / L) % L, z = c / (L * L);
-    const uint32_t nb[3] = {(x + 1) % L + L * (y + L * z), x + L * ((y + 1) % L + L * z),
-                            x + L * (y + L * ((z + 1) % L))};
-    for (int ax = 0; ax < 3; ++ax) {
-      const uint32_t j = nb[ax];
-      if (sigma_of(w[c], 2 * ax) == sigma_of(w[j], 2 * ax + 1) && cnt[c] < 4 && cnt[j] < 4) {
-        ++cnt[c];
-        ++cnt[j];
-        total += 2;
-      }
-    }
-  }
-  return total;
-}
-
 // Initial state of one point (gpu_water3D.cu:639-826 with Philox streams).
 void init_words(const PointHost& P, std::vector<uint32_t>& w) {
   const uint32_t L = P.L, N = P.N;
@@ -398,14 +381,6 @@ int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
 int reserve_config(cvf_sim* s, size_t n6) {
   if (!s->cfg_res.p) HIPC(s->cfg_res.alloc(2));
   if (2 * n6 > s->cfg_bytes.n) HIPC(s->cfg_bytes.alloc(2 * n6));
-  return CVF_OK;
-}
-
-int download_point_words(cvf_sim* s, int pt, std::vector<uint32_t>& w) {
-  w.resize(s->ph[pt].N);
-  HIPC(hipStreamSynchronize(s->stream));
-  if (int rc = check_resident(s)) return rc;
-  HIPC(hipMemcpy(w.data(), s->words.p + s->ph[pt].woff, w.size() * 4, hipMemcpyDeviceToHost));
   return CVF_OK;
 }
 
@@ -1208,6 +1183,19 @@ int build_groups(cvf_sim* s) {
     HIPC(s->obs_ps.alloc(s->npts));
     HIPC(s->obs_status.alloc(1));
     HIPC(s->obs_part.alloc(ta.size()));
+    std::vector<CappedEnt> tc;
+    for (int p = 0; p < s->npts; ++p) {
+      const PointHost& P = s->ph[p];
+      if (P.prm.flag_chessboard) continue;
+      tc.push_back(CappedEnt{p, P.L, P.woff, make_fastdiv(P.L / 2).m});
+      s->capped_L = std::max(s->capped_L, P.L);
+    }
+    if (!tc.empty()) {
+      if ((rc = upload_vec(s->tab_capped, tc))) return rc;
+      HIPC(s->bonds.alloc(s->total_cells));
+      HIPC(s->obs_capped.alloc(s->npts));
+      s->n_capped = (uint32_t)tc.size();
+    }
   }
   HIPC(hipDeviceSynchronize());
   return CVF_OK;
@@ -1805,7 +1793,9 @@ int cvf_observe(cvf_sim* s, int32_t pt, cvf_obs* o) {
   HIPC(hipSetDevice(s->device));
   if (s->obs_at != s->steps) {
     launch_observe(s->stream, s->tab_cell_all.p, s->nb_cell_all, s->words.p, observe_span(s->total_cells), s->pst.p,
-                   s->rstatus.p, ObsOut{s->obs_part.p, s->obs_ps.p, s->obs_status.p});
+                   s->rstatus.p, ObsOut{s->obs_part.p, s->obs_ps.p, s->obs_status.p}, s->bonds.p);
+    if (s->n_capped)
+      launch_capped_hb(s->stream, s->tab_capped.p, s->n_capped, s->capped_L, s->bonds.p, s->obs_capped.p);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
     if ((rc = resident_status(*s->obs_status.p))) return rc;
@@ -1822,14 +1812,8 @@ int cvf_observe(cvf_sim* s, int32_t pt, cvf_obs* o) {
   const VolState& vol = s->vol_device ? s->obs_ps.p[pt].vol : s->ph[pt].vol;
   const double r_cell = vol.r_cell, E_vdw = vol.E_vdw;
   const PointHost& P = s->ph[pt];
-  int64_t nhb2 = s->obs_nhb2[pt];
+  const int64_t nhb2 = P.prm.flag_chessboard ? s->obs_nhb2[pt] : (int64_t)s->obs_capped.p[pt];
   const int64_t nsig = s->obs_nsig[pt];
-  if (!P.prm.flag_chessboard) {
-    // the capped count is sequential over cells: taken on the host
-    std::vector<uint32_t> w;
-    if ((rc = download_point_words(s, pt, w))) return rc;
-    nhb2 = greedy_nhb2(P.L, w);
-  }
   // measure(), gpu_water3D.cu:2138-2152
   const double n_hb = 0.5 * (double)nhb2;
   double e = E_vdw + n_hb * (double)(-P.prm.J_hb);

@@ -120,7 +120,16 @@ struct ObsOut {
   uint32_t* status;
 };
 void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
-                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out);
+                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out, uint8_t* bonds);
+// Capped counts of n non-chessboard points (no larger than maxL) from the bond
+// bytes that launch_observe left at `bonds` + woff (null there if the handle
+// has no such point); they are used up.  2 N_HB of a point goes to out[point].
+struct CappedEnt {
+  int32_t point;
+  uint32_t L, woff, mH;  // mH: fast-division multiplier for L / 2
+};
+constexpr uint32_t kCappedLds = 160 * 1024 - 256;
+void launch_capped_hb(hipStream_t st, const CappedEnt* ent, uint32_t n, uint32_t maxL, uint8_t* bonds, uint32_t* out);
 // The words W of a point (N cells) as sigma and eta arrays (6N bytes each).
 void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* sigma, uint8_t* eta);
 // sigma and eta arrays to the words W through `scratch` (L^3 words): *first

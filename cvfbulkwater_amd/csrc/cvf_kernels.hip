@@ -710,6 +710,12 @@ __device__ __forceinline__ uint32_t bond_nhb2(uint32_t w, uint32_t wn) {
   return sigma_of(w, 2 * AX) == sigma_of(wn, 2 * AX + 1) ? eta_of(w, 2 * AX) + eta_of(wn, 2 * AX + 1) : 0u;
 }
 
+// Bits 0-2: the forward x, y, z bonds of a cell whose sigma values agree.
+__device__ __forceinline__ uint32_t bond_bits(uint32_t w, uint32_t wx, uint32_t wy, uint32_t wz) {
+  return (uint32_t)(sigma_of(w, 0) == sigma_of(wx, 1)) | (uint32_t)(sigma_of(w, 2) == sigma_of(wy, 3)) << 1 |
+         (uint32_t)(sigma_of(w, 4) == sigma_of(wz, 5)) << 2;
+}
+
 // One sample of a handle in one launch: a workgroup of 256 threads sums
 // `span` cells of a point (four cells along x per thread and round: three
 // 16-byte loads and the next word of the row) and stores the pair of sums
@@ -724,7 +730,8 @@ __global__ __launch_bounds__(256) void k_observe(const BlockEnt* __restrict__ ta
                                                 const uint32_t* __restrict__ words, uint32_t span,
                                                 const PointState* __restrict__ ps,
                                                 const uint32_t* __restrict__ rstatus, uint2* __restrict__ part,
-                                                PointState* __restrict__ ps_out, uint32_t* __restrict__ status_out) {
+                                                PointState* __restrict__ ps_out, uint32_t* __restrict__ status_out,
+                                                uint8_t* __restrict__ bonds) {
   const uint32_t lb = xcd_logical_block(blockIdx.x, nb);
   const BlockEnt e = tab[lb];
   if (lb == 0 && threadIdx.x == 0) *status_out = *rstatus;
@@ -747,6 +754,10 @@ __global__ __launch_bounds__(256) void k_observe(const BlockEnt* __restrict__ ta
     nhb2 += bond_nhb2<1>(c.x, yn.x) + bond_nhb2<1>(c.y, yn.y) + bond_nhb2<1>(c.z, yn.z) + bond_nhb2<1>(c.w, yn.w);
     nhb2 += bond_nhb2<2>(c.x, zn.x) + bond_nhb2<2>(c.y, zn.y) + bond_nhb2<2>(c.z, zn.z) + bond_nhb2<2>(c.w, zn.w);
     nsig += equal_pairs(c.x) + equal_pairs(c.y) + equal_pairs(c.z) + equal_pairs(c.w);
+    if (e.flags & kEntNoChess)
+      *reinterpret_cast<uint32_t*>(bonds + e.woff + t) =
+          bond_bits(c.x, c.y, yn.x, zn.x) | bond_bits(c.y, c.z, yn.y, zn.y) << 8 |
+          bond_bits(c.z, c.w, yn.z, zn.z) << 16 | bond_bits(c.w, xn, yn.w, zn.w) << 24;
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
@@ -758,6 +769,80 @@ __global__ __launch_bounds__(256) void k_observe(const BlockEnt* __restrict__ ta
   __syncthreads();
   if (threadIdx.x == 0)
     part[lb] = make_uint2(sh[0].x + sh[1].x + sh[2].x + sh[3].x, sh[0].y + sh[1].y + sh[2].y + sh[3].y);
+}
+
+// Capped HB count of a non-chessboard point (measure(), gpu_water3D.cu:
+// 2064-2099): cells in index order, forward x, y, z bonds; a bond counts for
+// both cells while both counters are below NHBMAX = 4.  A cell reads and
+// writes its own counter and those of its three forward neighbours, so two
+// cells touch a common one only if they are one of +-x, +-y, +-z, x - y, x - z,
+// y - z apart, or meet over the periodic boundary, and in each of these
+// cases x + 2y + 4z is the smaller for the one whose index is: the cells of
+// one value of it are independent, and 7 (L - 1) + 1 rounds with a barrier
+// between them give the sequential count.  One workgroup per point; a round's
+// cells have x = 2i + (d & 1), i < L/2, in every plane.  Cell byte: bonds in
+// bits 0-2 (k_observe), counter above.  In LDS where L^3 bytes fit.  Bound by
+// the rounds, one LDS round trip each: the download and the host's loop it
+// replaces took 350 us at L = 32.
+template <bool kLds>
+__global__ __launch_bounds__(1024) void k_capped_hb(const CappedEnt* __restrict__ ent, uint8_t* __restrict__ bonds,
+                                                   uint32_t* __restrict__ out) {
+  extern __shared__ __align__(16) uint8_t cap_lds[];
+  __shared__ uint32_t sums[16];
+  const CappedEnt e = ent[blockIdx.x];
+  const uint32_t L = e.L, N = L * L * L, hL = L / 2, tid = threadIdx.x, nt = blockDim.x;
+  const FastDiv dH{hL, e.mH};
+  uint8_t* g = bonds + e.woff;
+  if (kLds)
+    for (uint32_t i = tid; i < N / 16; i += nt) reinterpret_cast<uint4*>(cap_lds)[i] = reinterpret_cast<uint4*>(g)[i];
+  uint8_t* cell = kLds ? cap_lds : g;
+  __syncthreads();
+  uint32_t n = 0;
+  // rounds d = 2h + p: cell x = 2i + p, y = h - i - 2z
+  const auto visit = [&](uint32_t z, uint32_t i, uint32_t h, uint32_t p) {
+    const uint32_t y = h - i - 2 * z;  // (a large number where there is none)
+    if (y >= L) return;
+    const uint32_t c = 2 * i + p + L * (y + L * z);
+    const uint32_t nx = p && i == hL - 1 ? c + 1 - L : c + 1, ny = y + 1 < L ? c + L : c + L - L * L,
+                   nz = z + 1 < L ? c + L * L : c + L * L - N;
+    uint32_t b = cell[c], vx = cell[nx], vy = cell[ny], vz = cell[nz];
+    // (no other cell of the round touches these four: written back whatever
+    // became of them)
+    const auto bond = [&](uint32_t a, uint32_t& v) {
+      const uint32_t take = ((b >> a) & 1u) & (uint32_t)(b < 32) & (uint32_t)(v < 32);
+      b += 8 * take;
+      v += 8 * take;
+      n += take;
+    };
+    bond(0, vx);
+    bond(1, vy);
+    bond(2, vz);
+    cell[c] = (uint8_t)b;
+    cell[nx] = (uint8_t)vx;
+    cell[ny] = (uint8_t)vy;
+    cell[nz] = (uint8_t)vz;
+  };
+  const uint32_t items = L * hL, z0 = fdiv(tid, dH), i0 = tid - z0 * hL;
+  for (uint32_t h = 0; h <= 7 * (L - 1) / 2; ++h)
+    for (uint32_t p = 0; p < 2; ++p) {
+      if (items <= nt) {
+        if (tid < items) visit(z0, i0, h, p);
+      } else {
+        for (uint32_t it = tid; it < items; it += nt) {
+          const uint32_t z = fdiv(it, dH);
+          visit(z, it - z * hL, h, p);
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) n += __shfl_xor(n, m, 64);
+  if ((tid & 63) == 0) sums[tid >> 6] = n;
+  __syncthreads();
+  if (tid == 0) {
+    for (uint32_t w = 1; w < nt / 64; ++w) n += sums[w];
+    out[e.point] = 2 * n;
+  }
 }
 
 // ------------------------------------------------- configuration in and out
@@ -1488,8 +1573,26 @@ void launch_zero3_u32(hipStream_t st, uint32_t* a, size_t na, uint32_t* b, size_
   launch(k_zero3_u32, dim3((unsigned)blocks), dim3(256), st, a, na, b, nb, c, nc);
 }
 void launch_observe(hipStream_t st, const BlockEnt* tab, uint32_t nblocks, const uint32_t* words, uint32_t span,
-                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out) {
-  launch(k_observe, dim3(nblocks), dim3(256), st, tab, nblocks, words, span, ps, rstatus, out.part, out.ps, out.status);
+                    const PointState* ps, const uint32_t* rstatus, const ObsOut& out, uint8_t* bonds) {
+  launch(k_observe, dim3(nblocks), dim3(256), st, tab, nblocks, words, span, ps, rstatus, out.part, out.ps, out.status,
+         bonds);
+}
+void launch_capped_hb(hipStream_t st, const CappedEnt* ent, uint32_t n, uint32_t maxL, uint8_t* bonds, uint32_t* out) {
+  const uint32_t block = std::min(1024u, (maxL * maxL / 2 + 63) / 64 * 64), bytes = maxL * maxL * maxL;
+  if (bytes > kCappedLds) {
+    hipLaunchKernelGGL(k_capped_hb<false>, dim3(n), dim3(block), 0, st, ent, bonds, out);
+    return;
+  }
+  static std::atomic<uint64_t> attr_set{0};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  const uint64_t bit = 1ull << (dev & 63);
+  if (!(attr_set.load(std::memory_order_acquire) & bit)) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_capped_hb<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCappedLds);
+    attr_set.fetch_or(bit, std::memory_order_acq_rel);
+  }
+  hipLaunchKernelGGL(k_capped_hb<true>, dim3(n), dim3(block), bytes, st, ent, bonds, out);
 }
 void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* sigma, uint8_t* eta) {
   launch(k_config_out, dim3((N / 4 + 255) / 256), dim3(256), st, W, N, sigma, eta);
