@@ -911,9 +911,55 @@ int upload_group_steps(cvf_sim* s) {
   return CVF_OK;
 }
 
+// z-slabs of a set of points, and the dynamic LDS of their launches
+struct SlabTable {
+  std::vector<BlockEnt> ents;  // empty: some point's do not fit
+  uint32_t lds = 0;            // for kChunk half-sweeps
+  uint32_t lds_long = 0;       // for kMaxChunk; 0 if that does not fit
+  uint32_t lds_eta = 0;        // for the eta sweep alone
+  bool any_nc = false;
+};
+SlabTable slab_table(const cvf_sim* s, const std::vector<int>& points, int requested) {
+  const uint64_t slab_cells = auto_slab_cells(s);
+  SlabTable st;
+  bool long_fits = true;
+  for (int p : points) {
+    const PointHost& P = s->ph[p];
+    const bool nc = !P.prm.flag_chessboard;
+    st.any_nc = st.any_nc || nc;
+    const uint32_t T = choose_slab(P.L, requested, slab_cells, nc);
+    if (!T) {
+      SlabTable none;
+      for (int i : points) none.any_nc = none.any_nc || !s->ph[i].prm.flag_chessboard;
+      return none;
+    }
+    st.lds = std::max(st.lds, slab_lds_bytes(P.L, T, kChunk, nc));
+    st.lds_long = std::max(st.lds_long, slab_lds_bytes(P.L, T, kMaxChunk, nc));
+    st.lds_eta = std::max(st.lds_eta, slab_lds_bytes(P.L, T, 0));
+    long_fits = long_fits && slab_lds_bytes(P.L, T, kMaxChunk, nc) <= chunk_lds_limit();
+    for (uint32_t z0 = 0; z0 < P.L; z0 += T) {
+      BlockEnt en = make_entry(P, p, z0);
+      en.T = T;
+      st.ents.push_back(en);
+    }
+  }
+  if (!long_fits) st.lds_long = 0;
+  return st;
+}
+
 // Tiles of a set of points: an axis of length d takes ceil(d / edge) tiles of
 // even length, the last one shorter; half-sweeps per launch, workgroup size
 // and modeled length of a Metropolis pass.
+// (the points: how many there are of each L; nc: some run without the
+// chessboard)
+struct TilePoints {
+  std::map<uint32_t, uint32_t> count;
+  bool nc = false;
+  void add(const PointHost& P) {
+    ++count[P.L];
+    nc = nc || !P.prm.flag_chessboard;
+  }
+};
 struct TilePlan {
   uint32_t edge[3] = {0, 0, 0}, nk = 0, block = 0;
   double us = 0;  // 0: none
@@ -923,21 +969,41 @@ uint32_t even_edge(uint32_t edge, uint32_t d) {
   return (d + n - 1) / n;
 }
 
+// Modeled times, us: what a pass costs besides its launches, a launch, a
+// workgroup of 1024 threads (schedule, tables, window), a half-sweep per trip
+// of the workgroup over its quads and per 256 quads on the CU (few: in the
+// one-cell-per-lane form), a cube family likewise.
+struct TileCost {
+  double pass, launch, group, trip, per256, few_trip, few_per256, cube_trip, cube_per256;
+};
+// fitted to 170 measured shapes of one point of L = 32 .. 200, to 7 % rms, and
+// the chosen shape ran within 2 % of the fastest measured one at every L; without
+// the chessboard to 64 shapes of 1 .. 256 points of L = 8 .. 160, to 8 %
+constexpr TileCost kCost = {0, 7.1, 4.9, 0.22, 0.21, 0, 0.34, 3.8, 2.8};
+constexpr TileCost kCostNc = {14.5, 1.5, 3.0, 0.64, 0.53, 0.2, 0.78, 0, 0};
+
+double sweep_us(const TileCost& c, double quads, double co, uint32_t block) {
+  return c.trip * std::ceil(quads / block) + c.per256 * co * quads / 256;
+}
+double cubes_us(const TileCost& c, double quads, double co, uint32_t block) {
+  return c.cube_trip * std::ceil(quads / block) + c.cube_per256 * co * quads / 256;
+}
+// workgroups of `block` threads and `lds` bytes, per_cu of them to a CU, that
+// run together there
+double together(double per_cu, uint32_t lds, uint32_t block) {
+  return std::max(1.0, std::min({per_cu, std::floor(160 * 1024.0 / (lds + 3072)), std::floor(2048.0 / block)}));
+}
+
 // Modeled length of a pass (cube sweep and 12 half-sweeps) in us, 0 if the
-// windows do not fit.  A launch takes 7.1 us and a workgroup 4.9 us at 1024
-// threads (schedule, tables, window); a half-sweep 0.22 us for each trip of
-// the workgroup over its quads and 0.21 us for each 256 quads on the CU; a cube
-// family 3.8 and 2.8 us likewise.  Fitted to 170 measured shapes of one point
-// of L = 32 .. 200, to 7 % rms; the shape it picks ran within 2 % of the fastest
-// measured one at every L.
-double tile_model(const std::map<uint32_t, uint32_t>& points, const TilePlan& t, uint32_t ncu) {
+// windows do not fit.
+double tile_model(const TilePoints& points, const TilePlan& t, uint32_t ncu) {
   struct Tile {
     double edge[3], n;
   };
   std::vector<Tile> tiles;
   uint32_t lds = 0;
   double total = 0;
-  for (const auto& lc : points) {
+  for (const auto& lc : points.count) {
     const uint32_t d[3] = {lc.first / 2, lc.first / 2, lc.first};
     uint32_t c[3];
     Tile q;
@@ -947,44 +1013,69 @@ double tile_model(const std::map<uint32_t, uint32_t>& points, const TilePlan& t,
       q.edge[a] = c[a];
       q.n *= (d[a] + c[a] - 1) / c[a];
     }
-    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], t.nk, true));
+    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], t.nk, false));
+    if (points.nc) lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], t.nk, true));
     total += q.n;
     tiles.push_back(q);
   }
   if (lds > tile_lds_limit()) return 0;
   // tiles of a CU, and how many of them run together
   const double per_cu = std::ceil(total / ncu);
-  const double co =
-      std::max(1.0, std::min({per_cu, std::floor(160 * 1024.0 / (lds + 3072)), std::floor(2048.0 / t.block)}));
+  const double co = together(per_cu, lds, t.block);
   const auto box = [](const Tile& q, double more) {
     return (q.edge[0] + more) * (q.edge[1] + more) * (q.edge[2] + more);
   };
-  const auto phase = [&](double quads, double trip, double per256) {
-    return trip * std::ceil(quads / t.block) + per256 * co * quads / 256;
-  };
-  double us = 0;
+  const TileCost& cost = points.nc ? kCostNc : kCost;
+  double us = cost.pass;
   for (uint32_t launch = 0; launch < 12 / t.nk; ++launch) {
     double work = 0;
     for (const Tile& q : tiles) {
-      double x = 4.9 * co * t.block / 1024;
-      if (launch == 0) x += 2 * phase(box(q, t.nk / 6.0 + 2) / 8, 3.8, 2.8);
-      // a later half-sweep adds 1/6 layer on average to each axis
+      double x = cost.group * co * t.block / 1024;
+      if (launch == 0 && !points.nc) x += 2 * cubes_us(cost, box(q, t.nk / 6.0 + 2) / 8, co, t.block);
+      // a later half-sweep adds 1/6 layer (1/3) on average to each axis
       for (uint32_t k = 0; k < t.nk; ++k) {
-        const double quads = box(q, (t.nk - 1 - k) / 6.0) / 2;
-        x += 4 * quads <= t.block ? 0.34 * co * quads / 256 : phase(quads, 0.22, 0.21);
+        const double quads = box(q, (t.nk - 1 - k) / (points.nc ? 3.0 : 6.0)) / 2;
+        x += 4 * quads <= t.block ? cost.few_trip + cost.few_per256 * co * quads / 256
+                                  : sweep_us(cost, quads, co, t.block);
       }
       work += q.n * x;
     }
-    us += 7.1 + std::ceil(per_cu / co) * work / total;
+    us += cost.launch + std::ceil(per_cu / co) * work / total;
   }
   return us;
+}
+
+// The same for the slabs of `tab` (windows of at most lds bytes): planes
+// without a halo in the plane, a z half-sweep adding one to each window (two
+// without the chessboard).  0.87: measured against kCost for the chessboard
+// (0.73 - 1.0 over 22 handles of 1 - 128 points of L = 16 .. 64); without it
+// their half-sweeps, word by word, take 2.5 times as long (0.85 - 1.2 over 11).
+double slab_model(const SlabTable& st, uint32_t nk, uint32_t block, uint32_t ncu) {
+  const std::vector<BlockEnt>& tab = st.ents;
+  const bool nc = st.any_nc;
+  const uint32_t lds = nk == (uint32_t)kMaxChunk ? st.lds_long : st.lds;
+  const double per_cu = std::ceil((double)tab.size() / ncu), co = together(per_cu, lds, block);
+  double us = 0;
+  for (uint32_t launch = 0; launch < 12 / nk; ++launch) {
+    double work = 0;
+    for (const BlockEnt& e : tab) {
+      const double plane = e.L * e.L / 4.0;
+      double x = kCost.group * co * block / 1024;
+      if (launch == 0 && !nc) x += 2 * cubes_us(kCost, (e.T + 2 + nk / 3.0) * plane / 8, co, block);
+      for (uint32_t k = 0; k < nk; ++k)
+        x += (nc ? 2.5 : 1) * sweep_us(kCost, (e.T + (nk - 1 - k) * (nc ? 2 : 1) / 3.0) * plane / 2, co, block);
+      work += x;
+    }
+    us += kCost.launch + std::ceil(per_cu / co) * work / (double)tab.size();
+  }
+  return nc ? us : 0.87 * us;
 }
 
 // The fastest modeled shape with t's launch length and workgroup size: every
 // number of tiles along the axes of the largest point, boxes at most three
 // times as long as thin.
-TilePlan best_tiles(const std::map<uint32_t, uint32_t>& points, uint32_t nk, uint32_t block, uint32_t ncu) {
-  const uint32_t L = points.rbegin()->first;
+TilePlan best_tiles(const TilePoints& points, uint32_t nk, uint32_t block, uint32_t ncu) {
+  const uint32_t L = points.count.rbegin()->first;
   const auto edges = [](uint32_t d) {
     std::vector<uint32_t> e;
     for (uint32_t n = 1; n <= d; ++n) {
@@ -1008,11 +1099,9 @@ TilePlan best_tiles(const std::map<uint32_t, uint32_t>& points, uint32_t nk, uin
   return best;
 }
 
-// Fused launches can run on tiles: the chessboard rule's reference schedule,
-// no slab thickness asked for, and the workgroups the kernel's tables need.
+// Fused launches can run on tiles: the reference schedule, no slab thickness
+// asked for, and the workgroups the kernel's tables need.
 bool tiles_possible(const cvf_sim* s, const cvf_tuning& t) {
-  for (const auto& P : s->ph)
-    if (!P.prm.flag_chessboard) return false;
   return s->sched == CVF_SCHED_REFERENCE && s->nm > 0 && t.fused != 0 && t.slab_planes == 0 &&
          t.block_chunk >= 256;
 }
@@ -1024,47 +1113,61 @@ int cu_count(const cvf_sim* s, uint32_t& ncu) {
   return CVF_OK;
 }
 
-// Tiles for group g's fused launches, in the place of slabs that do not fit
-// LDS (L > 64; L = 72 / 96 / 128 / 160 / 200 / 252: 27.1 / 33.2 / 47.6 / 75.6 /
-// 142 / 268 us per step, unfused 44.9 / 49.9 / 67.2 / 104 / 162 / 304) or are
-// one plane thick, so that each of them recomputes two planes and more (a step
-// with a cluster sweep at L = 8 / 16 / 32 / 48 / 64: 31.1 / 30.6 / 34.3 / 37.8 /
-// 43.2 us, slabs 32.6 / 30.9 / 36.2 / 49.4 / 57.8).  At two planes the two are even
-// (16 points of L = 32: 30.4 and 29.6).
-int build_tiles(cvf_sim* s, Group& g, uint32_t thickest) {
+// Tiles for the fused launches of `points` (us = 0: none) where slabs do not
+// fit LDS (L > 64; L = 72 / 96 / 128 / 160 / 200 / 252: 27.1 / 33.2 / 47.6 / 75.6 /
+// 142 / 268 us per step, unfused 44.9 / 49.9 / 67.2 / 104 / 162 / 304) or the
+// models say that they take longer: thin slabs recompute as many planes as they
+// own, and large ones are alone on a CU.  A step with a cluster sweep at L = 8 /
+// 16 / 32 / 48 / 64: 31.1 / 30.6 / 34.3 / 37.8 / 43.2 us, slabs 32.6 / 30.9 / 36.2 /
+// 49.4 / 57.8; 8 / 16 / 32 points of L = 48: 37 / 49 / 74, slabs 66 / 53 / 72;
+// thick slabs of small lattices stay (128 points of L = 16: 22.7, tiles 31).
+// Without the chessboard L = 8 / 16 / 32 / 64: 20.7 / 20.0 / 21.5 / 29.2 us, slabs
+// 24.9 / 25.4 / 30.3 / 46.6; 128 points of L = 16: 39, slabs 30.8.
+TilePlan fused_tiles(const cvf_sim* s, const cvf_tuning& t, const std::vector<int>& points, const SlabTable& slabs,
+                     uint32_t ncu) {
+  if (!tiles_possible(s, t)) return TilePlan();
+  TilePoints count;
+  for (int p : points) count.add(s->ph[p]);
+  const bool whole = t.chunk_sweeps == kMaxChunk;
+  TilePlan best = best_tiles(count, whole ? kMaxChunk : kChunk, (uint32_t)t.block_chunk, ncu);
+  if (best.us == 0) best = best_tiles(count, kChunk, (uint32_t)t.block_chunk, ncu);
+  // (without the chessboard a whole-pass slab launch is no faster than two)
+  const bool whole_slabs = whole && slabs.lds_long && !slabs.any_nc;
+  if (!slabs.ents.empty() &&
+      slab_model(slabs, whole_slabs ? kMaxChunk : kChunk, (uint32_t)t.block_chunk, ncu) <= best.us)
+    return TilePlan();
+  return best;
+}
+
+int build_tiles(cvf_sim* s, Group& g, const SlabTable& slabs) {
   g.tiled = false;
-  if (!tiles_possible(s, s->tune) || (g.fused && thickest > 1)) return CVF_OK;
   uint32_t ncu = 0;
   int rc = cu_count(s, ncu);
   if (rc) return rc;
-  std::map<uint32_t, uint32_t> count;
-  for (int p : g.points) ++count[s->ph[p].L];
-  const uint32_t want = s->tune.chunk_sweeps == kMaxChunk ? kMaxChunk : kChunk;
-  ncu = std::max(1u, ncu / (uint32_t)s->groups.size());
-  TilePlan t = best_tiles(count, want, (uint32_t)s->tune.block_chunk, ncu);
-  if (t.us == 0) t = best_tiles(count, kChunk, (uint32_t)s->tune.block_chunk, ncu);
+  const TilePlan t = fused_tiles(s, s->tune, g.points, slabs, std::max(1u, ncu / (uint32_t)s->groups.size()));
   if (t.us == 0) return CVF_OK;
   std::vector<TileEnt> tab;
   uint32_t lds = 0, lds_long = 0;
-  g.sigma_cells = 0;
   for (int p : g.points) {
     const PointHost& P = s->ph[p];
     const uint32_t hL = P.L / 2, d[3] = {hL, hL, P.L};
     uint32_t c[3];
     for (int a = 0; a < 3; ++a) c[a] = even_edge(t.edge[a], d[a]);
-    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], kChunk, true));
-    lds_long = std::max(lds_long, 16 * tile_window_quads(c[0], c[1], c[2], kMaxChunk, true));
-    g.sigma_cells += P.N;
+    const bool nc = !P.prm.flag_chessboard;
+    lds = std::max(lds, 16 * tile_window_quads(c[0], c[1], c[2], kChunk, nc));
+    lds_long = std::max(lds_long, 16 * tile_window_quads(c[0], c[1], c[2], kMaxChunk, nc));
     for (uint32_t z = 0; z < d[2]; z += c[2])
       for (uint32_t y = 0; y < d[1]; y += c[1])
         for (uint32_t x = 0; x < d[0]; x += c[0])
           tab.push_back(TileEnt{p, P.L, P.woff, (uint32_t)P.prm.seed, (uint32_t)(P.prm.seed >> 32), x, y, z,
-                                std::min(c[0], d[0] - x), std::min(c[1], d[1] - y), std::min(c[2], d[2] - z), 0});
+                                std::min(c[0], d[0] - x), std::min(c[1], d[1] - y), std::min(c[2], d[2] - z),
+                                nc ? 1u : 0u});
   }
   TileEnt pad;
   memset(&pad, 0, sizeof pad);
   pad.point = -1;
   while (tab.size() % kNumXcd) tab.push_back(pad);
+  if (lds > tile_lds_limit()) return CVF_OK;
   if ((rc = upload_vec(g.tab_tile, tab))) return rc;
   g.nb_tile = (uint32_t)tab.size();
   g.chunk_lds = lds;
@@ -1078,7 +1181,6 @@ int build_tiles(cvf_sim* s, Group& g, uint32_t thickest) {
 // largest-first onto the group with the fewest cells.
 int build_groups(cvf_sim* s) {
   HIPC(hipDeviceSynchronize());
-  const uint64_t slab_cells = auto_slab_cells(s);
   s->groups.clear();
   // the resident kernel takes every point in one group (its workgroups must
   // all be resident at once, one per CU at most)
@@ -1115,37 +1217,16 @@ int build_groups(cvf_sim* s) {
     // fused path when every point's slab fits in LDS: the reference
     // schedule's eta sweep and half-sweeps, or the fast schedule's eta sweep
     g->fused = s->tune.fused != 0;  // (fused = 2: the resident kernel where it applies, else fused slabs)
-    std::vector<BlockEnt> ts;
-    g->chunk_lds = 0;
-    g->chunk_lds_long = 0;
-    g->chunk_lds_eta = 0;
-    g->any_nc = false;
-    bool long_fits = true;
+    SlabTable slabs = slab_table(s, g->points, s->tune.slab_planes);
+    std::vector<BlockEnt>& ts = slabs.ents;
+    g->fused = g->fused && !ts.empty();
+    g->chunk_lds = slabs.lds;
+    g->chunk_lds_long = slabs.lds_long;
+    g->chunk_lds_eta = slabs.lds_eta;
+    g->any_nc = slabs.any_nc;
     g->sigma_cells = 0;
-    for (int p : g->points) {
-      const PointHost& P = s->ph[p];
-      const bool nc = !P.prm.flag_chessboard;
-      g->any_nc = g->any_nc || nc;
-      const uint32_t T = choose_slab(P.L, s->tune.slab_planes, slab_cells, nc);
-      if (!T) {
-        g->fused = false;
-        break;
-      }
-      g->chunk_lds = std::max(g->chunk_lds, slab_lds_bytes(P.L, T, kChunk, nc));
-      g->chunk_lds_long = std::max(g->chunk_lds_long, slab_lds_bytes(P.L, T, kMaxChunk, nc));
-      g->chunk_lds_eta = std::max(g->chunk_lds_eta, slab_lds_bytes(P.L, T, 0));
-      long_fits = long_fits && slab_lds_bytes(P.L, T, kMaxChunk, nc) <= chunk_lds_limit();
-      g->sigma_cells += P.N;
-      for (uint32_t z0 = 0; z0 < P.L; z0 += T) {
-        BlockEnt en = make_entry(P, p, z0);
-        en.T = T;
-        ts.push_back(en);
-      }
-    }
-    if (!long_fits) g->chunk_lds_long = 0;
-    uint32_t thickest = 0;
-    for (const BlockEnt& en : ts) thickest = std::max(thickest, en.T);
-    if ((rc = build_tiles(s, *g, thickest))) return rc;
+    for (int p : g->points) g->sigma_cells += s->ph[p].N;
+    if ((rc = build_tiles(s, *g, slabs))) return rc;
     for (int p : g->points) {
       s->ph[p].group = (int32_t)(&g - &s->groups[0]);
       s->ph[p].slab_T = 0;
@@ -1207,7 +1288,7 @@ void launch_fused(cvf_sim* s, const Group& g, hipStream_t st, const uint64_t* st
   const uint32_t lds = nk == (uint32_t)kMaxChunk ? g.chunk_lds_long : g.chunk_lds;
   if (g.tiled)
     launch_tile(st, g.tab_tile.p, g.nb_tile, (uint32_t)s->tune.block_chunk, stepp, step_off, s->pts.p, src, dst, k0,
-                nk, with_eta, lds);
+                nk, with_eta, lds, g.any_nc);
   else
     launch_chunk(st, Launch{g.tab_slab.p, g.nb_slab, (uint32_t)s->tune.block_chunk, stepp, step_off}, s->pts.p, src,
                  dst, k0, nk, with_eta, lds, g.any_nc);
@@ -1479,31 +1560,32 @@ cvf_tuning default_tuning(const cvf_sim* s) {
     all_wide = all_wide && P.L > 64;
   }
   t.chunk_sweeps = s->total_cells < (1u << 20) && !any_nc ? kMaxChunk : kChunk;
-  if (all_wide) {
-    // no slab's window fits a plane beyond L = 64: tiles, at the launch length
-    // and workgroup size that their model gives the shortest pass (L = 68 / 72 /
-    // 96 / 112: 26.3 / 27.1 / 33.2 / 41.8 us per step, one-plane resident slabs
-    // 29.8 / 30.6 / 42.2 / 53.6)
-    TilePlan best;
-    uint32_t ncu = 0;
-    std::map<uint32_t, uint32_t> count;
-    for (const auto& P : s->ph) ++count[P.L];
-    if (tiles_possible(s, t) && cu_count(s, ncu) == CVF_OK)
+  // tiles, where they are the faster fused launches, at the launch length and
+  // workgroup size that their model gives the shortest pass
+  uint32_t ncu = 0;
+  if (tiles_possible(s, t) && cu_count(s, ncu) == CVF_OK) {
+    std::vector<int> all(s->npts);
+    for (int i = 0; i < s->npts; ++i) all[i] = i;
+    const SlabTable slabs = slab_table(s, all, 0);
+    if (fused_tiles(s, t, all, slabs, ncu).us > 0) {
+      TilePoints count;
+      for (int p : all) count.add(s->ph[p]);
+      TilePlan best;
       for (uint32_t nk : {(uint32_t)kChunk, (uint32_t)kMaxChunk})
         for (uint32_t block : {512u, 1024u}) {
           const TilePlan p = best_tiles(count, nk, block, ncu);
           if (p.us > 0 && (best.us == 0 || p.us < best.us)) best = p;
         }
-    if (best.us > 0) {
       t.chunk_sweeps = (int32_t)best.nk;
       t.block_chunk = (int32_t)best.block;
-    } else {
-      // one-plane resident slabs, one workgroup per CU; points that cannot
-      // run resident fall back to the unfused kernels
-      t.fused = 2;
-      t.slab_planes = 1;
-      t.block_chunk = 1024;
+      all_wide = false;
     }
+  }
+  if (all_wide) {
+    // the fast schedule, or no Metropolis sweep, above L = 64
+    t.fused = 2;
+    t.slab_planes = 1;
+    t.block_chunk = 1024;
   }
   // a small handle of one Metropolis sweep per step, nothing between the
   // steps, whose planes can each have a workgroup: one-plane resident slabs
@@ -1519,7 +1601,7 @@ cvf_tuning default_tuning(const cvf_sim* s) {
     planes += P.L;
     maxL = std::max(maxL, P.L);
   }
-  if (!any_nc && !all_wide && s->sched == CVF_SCHED_REFERENCE && s->nm == 1 && s->nc == 0 && planes <= 256 &&
+  if (!any_nc && maxL <= 64 && s->sched == CVF_SCHED_REFERENCE && s->nm == 1 && s->nc == 0 && planes <= 256 &&
       s->total_cells < (1u << 20)) {
     t.fused = 2;
     t.slab_planes = 1;

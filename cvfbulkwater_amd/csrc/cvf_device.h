@@ -106,15 +106,18 @@ __device__ __forceinline__ uint32_t popc_add(uint32_t x, uint32_t acc) {
   return r;
 }
 
-__device__ __forceinline__ uint32_t sigma_thr_index(uint32_t w, uint32_t wn, int arm, uint32_t sa, uint32_t sp) {
+// d + 5 + base
+__device__ __forceinline__ uint32_t sigma_count_index(uint32_t w, uint32_t sa, uint32_t sp, uint32_t base) {
   constexpr uint32_t kLo2 = 0x1B6DBu, kHi = 0x24924u;  // bits 0-1, bit 2 of each field
-  const uint32_t snb = sigma_of(wn, arm ^ 1);
-  const bool eta = (w >> (kEtaShift + arm)) & 1u;
-  const uint32_t h11 = eta && sp == snb ? 22u : eta && sa == snb ? 0u : 11u;
   const uint32_t ya = w ^ (sa * kFieldLsb), yp = w ^ (sp * kFieldLsb);
   const uint32_t ne_a = (((ya & kLo2) + kLo2) | ya) & kHi;
   const uint32_t eq_p = ~(((yp & kLo2) + kLo2) | yp) & kHi;
-  return popc_add(ne_a, popc_add(eq_p, h11));
+  return popc_add(ne_a, popc_add(eq_p, base));
+}
+__device__ __forceinline__ uint32_t sigma_thr_index(uint32_t w, uint32_t wn, int arm, uint32_t sa, uint32_t sp) {
+  const uint32_t snb = sigma_of(wn, arm ^ 1);
+  const bool eta = (w >> (kEtaShift + arm)) & 1u;
+  return sigma_count_index(w, sa, sp, eta && sp == snb ? 22u : eta && sa == snb ? 0u : 11u);
 }
 
 // Cells and facing neighbours (window indices) of the in-plane (x or y arm)
@@ -186,6 +189,24 @@ __device__ __forceinline__ void sigma_quad_regs(uint32_t (&w)[4], const uint32_t
   for (int m = 0; m < 4; ++m) {
     const uint32_t nw = (w[m] & ~(7u << (3 * arm))) | (sp[m] << (3 * arm));
     w[m] = act[m] && ra[m] < t[m] ? nw : w[m];
+  }
+}
+
+// Non-chessboard rule on one word w (facing neighbour word wn, random word rw):
+// both words' new values.  The bond counts in bits 24-31 (4 at most allowed,
+// gpu_water3D.cu:1966-1984, 2004-2007) move with the proposal, and decide whether the
+// bond before and after it counts.
+__device__ __forceinline__ void sigma_cell_nc(uint32_t& w, uint32_t& wn, const uint32_t* thr, int arm, uint32_t rw) {
+  uint32_t sp, ra;
+  split_word(rw, 6, sp, ra);
+  const uint32_t sa = sigma_of(w, arm), snb = sigma_of(wn, arm ^ 1);
+  const bool bp = sp == snb, ba = sa == snb;
+  const int dn = (int)bp - (int)ba, ni = (int)(w >> kNhbShift), nj = (int)(wn >> kNhbShift);
+  const uint32_t up = bp && max(ni, nj) + dn <= 4 ? 11u : 0u, down = ba && max(ni, nj) <= 4 ? 11u : 0u;
+  const uint32_t t = thr[sigma_count_index(w, sa, sp, 11u + up - down)];
+  if (sp != sa && ra < t) {
+    w = (w & kLowBits & ~(7u << (3 * arm))) | (sp << (3 * arm)) | (uint32_t)(ni + dn) << kNhbShift;
+    wn = (wn & kLowBits) | (uint32_t)(nj + dn) << kNhbShift;
   }
 }
 

@@ -92,19 +92,20 @@ uint32_t chunk_lds_limit();
 struct TileEnt {
   int32_t point;
   uint32_t L, woff, seed_lo, seed_hi;
-  uint32_t x0, y0, z0, tx, ty, tz, pad;
+  uint32_t x0, y0, z0, tx, ty, tz, nc;  // nc: runs without the chessboard
 };
 constexpr int kMaxTileWin = 64;  // quads along one axis of a window
-constexpr uint32_t kMaxTile = kMaxTileWin - kMaxChunk - 2;
-// quads of the largest window of a tile for nk half-sweeps (and the cube sweep)
-uint32_t tile_window_quads(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t nk, bool eta);
+constexpr uint32_t kMaxTile = kMaxTileWin - 2 * kMaxChunk - 2;
+// quads of the largest window of a tile for nk half-sweeps (and the cube
+// sweep; nc: of a non-chessboard point)
+uint32_t tile_window_quads(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t nk, bool nc);
 // largest dynamic LDS of a tile workgroup
 constexpr uint32_t tile_lds_limit() { return 160 * 1024 - 4096; }
 // As launch_chunk, on the ntiles (a multiple of kNumXcd) boxes of `tab`;
 // workgroups of at least 3 kMaxTileWin threads.
 void launch_tile(hipStream_t st, const TileEnt* tab, uint32_t ntiles, uint32_t block, const uint64_t* stepp,
                  uint32_t step_off, const PointDev* pts, const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk,
-                 int with_eta, uint32_t lds_bytes);
+                 int with_eta, uint32_t lds_bytes, bool any_nc);
 void launch_zero_u32(hipStream_t st, uint32_t* p, size_t n);
 void launch_zero3_u32(hipStream_t st, uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc);
 // Cells per k_observe workgroup (a multiple of 1024): small handles spread

@@ -12,8 +12,10 @@
 //
 // The halo is found from the launch's own schedule, walking it backwards:
 // a + (-) half-sweep along an axis adds one layer on the upper (lower) side,
-// and only when the outermost layer moves in it (its parity); the cube sweep
-// adds one layer on every side.  That is about half a layer per side for six
+// and only when the outermost layer moves in it (its parity); without the
+// chessboard, whose moves also write the facing cell's bond count, the layer
+// beyond the other end counts likewise.  The cube sweep adds one layer on every
+// side.  That is about half a layer per side for six
 // half-sweeps, where a slab of T full planes recomputes whole planes: an
 // L = 32 point of a 16-point handle has 2-plane slabs whose windows hold 4-5
 // planes, and above L = 64 no slab's window fits LDS at all.
@@ -77,6 +79,8 @@ constexpr uint32_t kFoldMask = 0x0FFFFFFFu;  // site bits of a folded coordinate
 
 }  // namespace
 
+// kAnyNc: the launch may hold non-chessboard points (compiled out otherwise)
+template <bool kAnyNc>
 __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, uint32_t ntiles,
                                                 const uint64_t* __restrict__ stepp, uint32_t step_off,
                                                 const PointDev* __restrict__ pts, const uint32_t* __restrict__ src,
@@ -111,27 +115,28 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   __syncthreads();
   const int L = (int)e.L, hL = L / 2;
   const int org[3] = {(int)e.x0, (int)e.y0, (int)e.z0};
+  const bool nc = kAnyNc && e.nc != 0;
   // the box valid after the last half-sweep, and walking back the boxes
-  // before: grow bit k says that half-sweep k adds a layer
+  // before: bit k of grow_lo, grow_hi says that half-sweep k adds a layer
+  // below, above
   int lo[3] = {0, 0, 0}, hi[3] = {(int)e.tx, (int)e.ty, (int)e.tz};
-  uint32_t grow = 0;
+  uint32_t grow_lo = 0, grow_hi = 0;
   for (int k = (int)nk - 1; k >= 0; --k) {
-    const uint32_t s = uni(sch[k]), arm = s & 7u, q = s >> 3;
+    const uint32_t s = uni(sch[k]), arm = s & 7u, q = s >> 3, down = arm & 1u;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
       if (a == (int)(arm >> 1)) {
-        // the outermost layer on the arm's side moves when its parity is kept
-        const int edge = org[a] + ((arm & 1u) ? lo[a] : hi[a] - 1);
-        if (((uint32_t)edge & 1u) == q) {
-          grow |= 1u << k;
-          if (arm & 1u)
-            --lo[a];
-          else
-            ++hi[a];
-        }
+        // the cell at the arm's end of the box faces one outside, if it moves;
+        // without the chessboard the cell before the other end, if it moves,
+        // changes the counter of the box's first one
+        const bool end = ((uint32_t)(org[a] + (down ? lo[a] : hi[a] - 1)) & 1u) == q;
+        const bool start = nc && ((uint32_t)(org[a] + (down ? hi[a] : lo[a] - 1)) & 1u) == q;
+        if (down ? end : start) grow_lo |= 1u << k, --lo[a];
+        if (down ? start : end) grow_hi |= 1u << k, ++hi[a];
       }
   }
-  const int ext = with_eta ? 1 : 0;
+  const bool cubes = with_eta && !nc;
+  const int ext = cubes ? 1 : 0;
   int wo[3], wn[3];  // window origin relative to the core, window size
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
@@ -184,7 +189,7 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
     }
   }
   __syncthreads();
-  if (with_eta) {
+  if (cubes) {
     for (int fam = 0; fam < 2; ++fam) {
       // origins of the family's parity whose cubes hold a cell of the box
       uint32_t f[3], cnt[3];
@@ -244,17 +249,24 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
     uint32_t f[3], cnt[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      if (a == ax && ((grow >> k) & 1u)) {
-        if (arm & 1)
-          ++lo[a];
-        else
-          --hi[a];
+      int first = lo[a], end = hi[a];
+      if (a == ax) {
+        // without the chessboard every pair within the box before, else the
+        // cells of the box after
+        if (nc) {
+          if (arm & 1)
+            ++first;
+          else
+            --end;
+        }
+        lo[a] += (int)((grow_lo >> k) & 1u);
+        hi[a] -= (int)((grow_hi >> k) & 1u);
+        if (!nc) first = lo[a], end = hi[a];
+        // the layers of the kept parity
+        first += ((uint32_t)(org[a] + first) & 1u) != q;
       }
-      // along the arm's axis the layers of the kept parity
-      const int skip = a == ax ? ((uint32_t)(org[a] + lo[a]) & 1u) != q : 0;
-      f[a] = (uint32_t)(lo[a] + skip - wo[a]);
-      const int len = hi[a] - lo[a] - skip;
-      cnt[a] = (uint32_t)(a == ax ? (len + 1) / 2 : len);
+      f[a] = (uint32_t)(first - wo[a]);
+      cnt[a] = (uint32_t)(a == ax ? (end - first + 1) / 2 : end - first);
     }
     const uint32_t n = cnt[0] * cnt[1] * cnt[2];
     const uint32_t mx = ax == 0 ? 2u : 1u, my = ax == 1 ? 2u : 1u, mz = ax == 2 ? 2u : 1u;
@@ -272,7 +284,15 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
         const uint32_t h = tid & 3u, c = item(tid >> 2, w0);
         const uint32_t w = win[w0 + h], wf = win[w0 + dn + h];
         const U4 r = draw_site(c & kFoldMask, pf);
-        win[w0 + h] = sigma_cell(w, wf, thr_s, arm, pick4(r, h ^ (c >> 28)));
+        const uint32_t rw = pick4(r, h ^ (c >> 28));
+        if (nc) {
+          uint32_t v = w, vf = wf;
+          sigma_cell_nc(v, vf, thr_s, arm, rw);
+          win[w0 + h] = v;
+          win[w0 + dn + h] = vf;
+        } else {
+          win[w0 + h] = sigma_cell(w, wf, thr_s, arm, rw);
+        }
       }
     } else {
       for (uint32_t i = tid; i < n; i += nt) {
@@ -281,7 +301,15 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
         quad_load(win, w0, w);
         quad_load(win, w0 + dn, wf);
         const U4 r = draw_swap(draw_site(c & kFoldMask, pf), c >> 28);
-        sigma_quad_regs(w, wf, thr_s, arm, r);
+        if (nc) {
+          sigma_cell_nc(w[0], wf[0], thr_s, arm, r.x);
+          sigma_cell_nc(w[1], wf[1], thr_s, arm, r.y);
+          sigma_cell_nc(w[2], wf[2], thr_s, arm, r.z);
+          sigma_cell_nc(w[3], wf[3], thr_s, arm, r.w);
+          quad_store(win, w0 + dn, wf);
+        } else {
+          sigma_quad_regs(w, wf, thr_s, arm, r);
+        }
         quad_store(win, w0, w);
       }
     }
@@ -307,40 +335,49 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   }
 }
 
-uint32_t tile_window_quads(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t nk, bool eta) {
-  // every half-sweep can add a layer to one axis: the largest window over how
-  // they may fall on the three
-  const uint32_t e = eta ? 2u : 0u;
+uint32_t tile_window_quads(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t nk, bool nc) {
+  // every half-sweep can add a layer to one axis (two without the chessboard,
+  // which has no cubes): the largest window over how they may fall on the
+  // three
+  const uint32_t e = nc ? 0u : 2u, g = nc ? 2u : 1u;
   uint32_t most = 0;
   for (uint32_t a = 0; a <= nk; ++a)
-    for (uint32_t b = 0; a + b <= nk; ++b) {
-      const uint32_t c = nk - a - b;
-      most = std::max(most, (tx + e + a) * (ty + e + b) * (tz + e + c));
-    }
+    for (uint32_t b = 0; a + b <= nk; ++b)
+      most = std::max(most, (tx + e + g * a) * (ty + e + g * b) * (tz + e + g * (nk - a - b)));
   return most;
 }
 
-void launch_tile(hipStream_t st, const TileEnt* tab, uint32_t ntiles, uint32_t block, const uint64_t* stepp,
-                 uint32_t step_off, const PointDev* pts, const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk,
-                 int with_eta, uint32_t lds_bytes) {
+namespace {
+template <bool kAnyNc>
+void launch_tile_t(hipStream_t st, const TileEnt* tab, uint32_t ntiles, uint32_t block, const uint64_t* stepp,
+                   uint32_t step_off, const PointDev* pts, const uint32_t* src, uint32_t* dst, uint32_t k0,
+                   uint32_t nk, int with_eta, uint32_t lds_bytes) {
   // the dynamic-LDS limit is a per-device function attribute
   static std::atomic<uint64_t> attr_set{0};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const uint64_t bit = 1ull << (dev & 63);
   if (!(attr_set.load(std::memory_order_acquire) & bit)) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)tile_lds_limit());
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile<kAnyNc>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile_lds_limit());
     attr_set.fetch_or(bit, std::memory_order_acq_rel);
   }
   hipEvent_t t0, t1;
   get_launch_timing(&t0, &t1);
   if (t0)
-    hipExtLaunchKernelGGL(k_tile, dim3(ntiles), dim3(block), lds_bytes, st, t0, t1, 0, tab, ntiles, stepp, step_off,
-                          pts, src, dst, k0, nk, with_eta);
+    hipExtLaunchKernelGGL(k_tile<kAnyNc>, dim3(ntiles), dim3(block), lds_bytes, st, t0, t1, 0, tab, ntiles, stepp,
+                          step_off, pts, src, dst, k0, nk, with_eta);
   else
-    hipLaunchKernelGGL(k_tile, dim3(ntiles), dim3(block), lds_bytes, st, tab, ntiles, stepp, step_off, pts, src, dst,
-                       k0, nk, with_eta);
+    hipLaunchKernelGGL(k_tile<kAnyNc>, dim3(ntiles), dim3(block), lds_bytes, st, tab, ntiles, stepp, step_off, pts,
+                       src, dst, k0, nk, with_eta);
+}
+}  // namespace
+
+void launch_tile(hipStream_t st, const TileEnt* tab, uint32_t ntiles, uint32_t block, const uint64_t* stepp,
+                 uint32_t step_off, const PointDev* pts, const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk,
+                 int with_eta, uint32_t lds_bytes, bool any_nc) {
+  (any_nc ? launch_tile_t<true> : launch_tile_t<false>)(st, tab, ntiles, block, stepp, step_off, pts, src, dst, k0, nk,
+                                                        with_eta, lds_bytes);
 }
 
 }  // namespace cvf
