@@ -433,15 +433,15 @@ struct Piece {
 // makes ceil((n - 64 j) / (64 v)) iterations, j its rank in the slab)
 // times the phase's VALU instructions per iteration, summed over the two
 // cube families, eight in-plane and four z half-sweeps (two of each
-// parity): the expected phases of a step.
+// parity), the expected phases of a step, or the fast schedule's two passes.
 struct SlabShape {
   uint32_t L, z0, T;
   bool split;
 };
-double workgroup_step_model(const std::vector<SlabShape>& sl, const std::vector<uint32_t>& nw) {
+double workgroup_step_model(const std::vector<SlabShape>& sl, const std::vector<uint32_t>& nw, bool fast) {
   constexpr double kInPlane = 190, kZ = 176, kCube = 614;  // VALU per iteration
   double total = 0;
-  for (int ph = 0; ph < 5; ++ph) {
+  for (int ph = 0; ph < (fast ? 3 : 5); ++ph) {
     // 0, 1: cube families; 2: in-plane (x8); 3, 4: z of parity 0, 1 (x2)
     double simd[4] = {0, 0, 0, 0};
     uint32_t w0 = 0;
@@ -458,7 +458,7 @@ double workgroup_step_model(const std::vector<SlabShape>& sl, const std::vector<
         cost = kCube;
       } else if (ph == 2) {
         n = (uint64_t)x.T * LL / 8;
-        cost = 8 * kInPlane;
+        cost = (fast ? 12 : 8) * kInPlane;  // (fast: two passes of six arms)
       } else {
         const uint32_t first = (x.z0 & 1u) == (uint32_t)(ph - 3) ? 0u : 1u;
         const uint32_t npl = first < x.T ? (x.T - first + 1) / 2 : 0u;
@@ -505,7 +505,7 @@ bool fill_workgroups(const cvf_sim* s, const std::vector<int>& order, double W, 
           if (used + need > cap) continue;
           cells.push_back((double)t * LL);
           shapes.push_back(SlabShape{L, z, t, t < L});
-          const bool ok = split_waves(cells, wpg, nw) && workgroup_step_model(shapes, nw) <= W;
+          const bool ok = split_waves(cells, wpg, nw) && workgroup_step_model(shapes, nw, s->sched == CVF_SCHED_FAST) <= W;
           cells.pop_back();
           shapes.pop_back();
           if (ok) {
@@ -542,11 +542,11 @@ bool fill_workgroups(const cvf_sim* s, const std::vector<int>& order, double W, 
 // are slabs of at least two planes (one with max_T = 1) and at most max_T
 // planes when max_T > 0.  Each workgroup's waves go to its slabs in
 // proportion to their cells, at least one each.  False when the group's
-// points cannot run resident (fast schedule, several Metropolis sweeps per
-// step, the non-chessboard rule) or do not fit.
+// points cannot run resident (several Metropolis sweeps per step, the
+// non-chessboard rule) or do not fit.
 bool plan_resident(const cvf_sim* s, const Group& g, int nwg, uint32_t wpg, uint32_t cap, uint32_t max_T,
                    RDeal& out) {
-  if (s->sched != CVF_SCHED_REFERENCE || s->nm != 1 || nwg <= 0 || wpg == 0) return false;
+  if (s->nm != 1 || nwg <= 0 || wpg == 0) return false;
   std::vector<int> order = g.points;
   for (int p : order)
     if (!s->ph[p].prm.flag_chessboard) return false;
@@ -736,10 +736,11 @@ int build_resident(cvf_sim* s, Group& g) {
   for (const auto& r : d.slabs) {
     thin = thin && r.T <= 2;
     const uint64_t lanes = std::min<uint64_t>(64ull * r.nw, 512), LL = (uint64_t)r.L * r.L;
-    fine_phase = fine_phase || 2 * (uint64_t)r.T * (LL / 8) <= lanes || 4 * ((r.T + 1) / 2) * (LL / 16) <= lanes;
+    fine_phase = fine_phase || 2 * (uint64_t)r.T * (LL / 8) <= lanes || 4 * ((r.T + 1) / 2) * (LL / 16) <= lanes ||
+                 (s->sched == CVF_SCHED_FAST && r.T * LL / 2 <= 128ull * r.nw);
   }
   const bool fine = thin && fine_phase;
-  HIPC(resident_occupancy(&occ, (uint32_t)s->tune.block_chunk, d.lds_bytes, fine));
+  HIPC(resident_occupancy(&occ, (uint32_t)s->tune.block_chunk, d.lds_bytes, fine, s->sched == CVF_SCHED_FAST));
   if (occ < per_cu) return CVF_OK;
   int rc;
   if ((rc = upload_vec(g.rslabs, d.slabs)) || (rc = upload_vec(g.rgroups, d.groups))) return rc;
@@ -1322,7 +1323,7 @@ void enqueue_lattice(cvf_sim* s, int gi, hipStream_t st, uint32_t step_off, Time
     // one step of the resident kernel, in place on `words`
     timed(CVF_KCLASS_RESIDENT, [&] {
       launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                      s->words.p, g.rings.p, g.rver.p, stepp, step_off, 1, nullptr, s->rstatus.p, g.r_fine);
+                      s->words.p, g.rings.p, g.rver.p, stepp, step_off, 1, nullptr, s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
     });
   } else if (s->sched == CVF_SCHED_FAST) {
     // eta cube sweep, then n_metropolis x the two colour passes (in place,
@@ -1430,7 +1431,7 @@ int enqueue_resident(cvf_sim* s, int gi, hipStream_t st, int nsteps) {
   }
   launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
                   s->words.p, g.rings.p, g.rver.p, nullptr, (uint64_t)s->steps, (uint32_t)nsteps,
-                  s->cur_steps.p + gi, s->rstatus.p, g.r_fine);
+                  s->cur_steps.p + gi, s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
   if (s->vol_device) HIPC(hipStreamWaitEvent(st, g.join, 0));
   HIPC(hipGetLastError());
   return CVF_OK;
@@ -1554,10 +1555,9 @@ cvf_tuning default_tuning(const cvf_sim* s) {
   // small handles are bound by per-launch cost: a whole Metropolis pass per
   // fused launch where the window fits (not with the non-chessboard rule,
   // whose 24-plane halo reserve costs more than the launch it saves)
-  bool any_nc = false, all_wide = true;
+  bool any_nc = false;
   for (const auto& P : s->ph) {
     any_nc = any_nc || !P.prm.flag_chessboard;
-    all_wide = all_wide && P.L > 64;
   }
   t.chunk_sweeps = s->total_cells < (1u << 20) && !any_nc ? kMaxChunk : kChunk;
   // tiles, where they are the faster fused launches, at the launch length and
@@ -1578,14 +1578,7 @@ cvf_tuning default_tuning(const cvf_sim* s) {
         }
       t.chunk_sweeps = (int32_t)best.nk;
       t.block_chunk = (int32_t)best.block;
-      all_wide = false;
     }
-  }
-  if (all_wide) {
-    // the fast schedule, or no Metropolis sweep, above L = 64
-    t.fused = 2;
-    t.slab_planes = 1;
-    t.block_chunk = 1024;
   }
   // a small handle of one Metropolis sweep per step, nothing between the
   // steps, whose planes can each have a workgroup: one-plane resident slabs
@@ -1607,6 +1600,24 @@ cvf_tuning default_tuning(const cvf_sim* s) {
     t.slab_planes = 1;
     t.block_chunk = maxL <= 16 ? 256 : maxL <= 32 ? 512 : 1024;
     t.graph_steps = 64;
+  }
+  // the fast schedule's step of four phases with two exchanges between: the
+  // resident kernel where it holds the points (one-plane slabs while there is
+  // a workgroup per plane), up to L = 64, beyond which it has too few
+  // workgroups (L = 8 / 16 / 32 / 48 / 64 / 80: 8.9 / 9.4 / 10.9 / 16.6 / 21.1 / 33.3 us per
+  // step, the per-pass kernels 19.0 / 20.4 / 20.0 / 20.8 / 22.7 / 21.6; 32 points of
+  // L = 32 17.7 and 28.0, 128 of L = 16 .. 48 58.0 and 69.4).  With a cluster
+  // sweep, a launch per step, only small ones gain (L = 16 / 32 / 64: 29.3 / 31.2 /
+  // 47.3 and 35.4 / 35.0 / 43.0).
+  if (s->sched == CVF_SCHED_FAST && s->nm == 1 && cu_count(s, ncu) == CVF_OK) {
+    const bool planes_fit = planes <= 256, small = maxL <= 32 && s->total_cells < (1u << 21);
+    const uint64_t room = (uint64_t)ncu * resident_lds_limit() / 4;  // words; windows hold ghost planes too
+    if (s->nc == 0 ? maxL <= 64 && s->total_cells <= room / 5 * 4 : maxL <= 32 && planes_fit) {
+      t.fused = 2;
+      t.slab_planes = planes_fit ? 1 : 0;
+      t.block_chunk = small ? 512 : 1024;
+      t.graph_steps = 64;
+    }
   }
   return t;
 }
@@ -2169,7 +2180,7 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     timed(CVF_KCLASS_RESIDENT, [&] {
       launch_resident(g.stream, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p,
                       s->pts.p, s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)n_steps, nullptr,
-                      s->rstatus.p, g.r_fine);
+                      s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
     });
     timed(CVF_KCLASS_BEGIN, [&] {
       launch_vol_chain(g.stream, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,
@@ -2365,8 +2376,23 @@ extern "C" int cvf_autotune(cvf_sim* s, int32_t steps_per_trial, cvf_tuning* cho
             t.streams = streams;
             t.fused = fused;
             t.block_chunk = bc;
+            t.slab_planes = 0;
+            t.graph_steps = 16;
             t.chunk_sweeps = kChunk;  // no half-sweeps in fused launches here
             t.block_sigma = t.block_eta = bs;
+            cand.push_back(t);
+          }
+      // the resident kernel, `streams` workgroups per CU
+      if (streams <= 2)
+        for (int bc : {512, 1024})
+          for (int slab : {0, 1}) {
+            cvf_tuning t = base;
+            t.streams = streams;
+            t.fused = 2;
+            t.slab_planes = slab;
+            t.block_chunk = bc;
+            t.graph_steps = 64;
+            t.chunk_sweeps = kChunk;
             cand.push_back(t);
           }
       continue;

@@ -218,7 +218,7 @@ constexpr uint32_t kResidentStatic = 6144;  // static LDS reserved for a residen
 uint32_t resident_lds_limit();
 // resident workgroups of `block` threads and `lds_bytes` of dynamic LDS that
 // fit on one CU at once
-hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, bool fine);
+hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, bool fine, bool fast);
 // fine: the instantiation for plans of thin slabs (at most two planes):
 // in-plane half-sweeps whose quads fit half of a slab's lanes run two cells
 // per lane (one, below 64 quads), cube families whose cubes fit the lanes one cube per lane, and
@@ -229,6 +229,6 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
                      const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
-                     bool fine);
+                     bool fine, bool fast);
 
 }  // namespace cvf

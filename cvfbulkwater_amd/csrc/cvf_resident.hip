@@ -1,6 +1,7 @@
 // Resident Metropolis kernel: the lattice stays in LDS for a whole sequence
 // of MC steps (the reference schedule: eta cube sweep + 12 sigma
-// half-sweeps per step, gpu_water3D.cu:1346-1417, 1890-2008, 3374-3466).
+// half-sweeps per step, gpu_water3D.cu:1346-1417, 1890-2008, 3374-3466; or
+// the fast schedule: eta cube sweep + two colour passes).
 //
 // Each state point is cut into ns z-slabs (ns = 1: the whole lattice in one
 // window, periodic in LDS); slabs of one point may differ in thickness.
@@ -45,6 +46,11 @@
 // the launch's last step also publishes a version, which the neighbours
 // await before they write their planes back to `words`.
 //
+// In the fast schedule a cell of the second pass reads the cells of the
+// first on the neighbouring planes: a slab publishes its boundary planes'
+// moved quads in slot 0 of the step's half, and before the second pass takes
+// its neighbours' into its ghost planes.
+//
 // Coherence across the XCDs' L2 caches: every ring word and every version
 // is accessed with agent-scope relaxed atomics (single-location coherent
 // loads and stores that bypass the XCDs' non-coherent L2 caching), so no
@@ -64,6 +70,7 @@
 #include "cvf_kernels.h"
 
 #include <atomic>
+#include <type_traits>
 
 #include <hip/hip_ext.h>
 
@@ -395,13 +402,154 @@ __device__ __forceinline__ void eta_cube_item_q(uint32_t* lds, uint32_t B, uint3
   }
 }
 
+// One colour pass of the fast schedule (k_sigma_f) over a slab's T planes:
+// every cell of the colour (x + y + z) mod 2 = pass takes its six arms in
+// order.  Its neighbours have the other colour, so the order of the quads is
+// free: the boundary planes go first, and their moved quads to `ring` (lower
+// half the bottom plane, upper half the top plane; null: kept here) as tagged
+// words, so that the interior covers the way to the neighbours.  A quad's four
+// words stay in registers through its six arms.  Bound by VALU issue.
+__device__ __forceinline__ void colour_pass(uint32_t* lds, uint32_t li, uint32_t L, uint32_t T, uint32_t z0,
+                                            uint32_t pbase, bool whole, uint64_t seed, uint64_t step, uint32_t pass,
+                                            FastDiv dQ, uint32_t mP8, uint32_t dp8, uint32_t du8, const uint32_t* thr,
+                                            uint64_t* ring) {
+  const uint32_t hL = L / 2, qL = L / 4, LL = L * L, Q8 = LL / 8;
+  for (Walk it = walk_start(li, Q8, mP8); it.pi < T; advance(it, Q8, dp8, du8)) {
+    const uint32_t zr = it.pi == 0 ? 0u : it.pi == 1 ? T - 1 : it.pi - 1;
+    const uint32_t y = fdiv(it.u, dQ), x = 2 * (it.u - y * qL) + ((y + z0 + zr + pass) & 1u);
+    const uint32_t o4 = 4 * (y * hL + x), cw = pbase + zr * LL + o4, site = x + L * y + LL * (z0 + zr);
+    uint32_t w[4];
+    quad_load(lds, cw, w);
+#pragma unroll
+    for (int arm = 0; arm < 6; ++arm) {
+      const int ax = arm >> 1;
+      const bool up = (arm & 1) == 0;
+      uint32_t wn[4];
+      if (ax < 2) {
+        // across the edge the quad at the other end, halves along the axis
+        // exchanged
+        const uint32_t st = ax == 0 ? 4u : 4u * hL, c = ax == 0 ? x : y;
+        const bool wrap = c == (up ? hL - 1 : 0u);
+        const uint32_t d = up ? st : 0u - st, dw = up ? 0u - (hL - 1) * st : (hL - 1) * st;
+        quad_load(lds, cw + (wrap ? dw : d), wn);
+        swap_halves(wn, wrap ? ~0u : 0u, ax == 0 ? 2 : 1);
+      } else {
+        const bool wrap = whole && zr == (up ? T - 1 : 0u);
+        const uint32_t d = up ? LL : 0u - LL, dw = up ? 0u - (T - 1) * LL : (T - 1) * LL;
+        quad_load(lds, cw + (wrap ? dw : d), wn);
+      }
+      const U4 rq = draw_site(site, phase_draws(seed, kStSigmaF, step, 8 * pass + (uint32_t)arm));
+      sigma_quad_regs(w, wn, thr, arm, rq);
+    }
+    quad_store(lds, cw, w);
+    if (ring && it.pi < 2) {
+      const uint64_t tw = (uint64_t)end_tag(step) << 32;
+      if (zr == 0) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) ring_store64(ring + o4 + m, tw | w[m]);
+      }
+      if (zr == T - 1) {
+        uint64_t* hi = ring + (size_t)kRingHalf * LL;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) ring_store64(hi + o4 + m, tw | w[m]);
+      }
+    }
+  }
+}
+
+// (two trips a lane still beat quads on a quarter of the lanes: L = 48 / 64,
+// one-plane slabs of 1024 threads, 16.6 / 21.1 us per step, as quads 19.2 / 21.5)
+constexpr uint32_t kCellTrips = 2;
+
+// Lane q of every four lanes' x, in all four.
+template <int q>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, q * 0x55, 0xF, 0xF, true);
+}
+
+// The same pass where its cells fit the slab's lanes (thin slabs): one cell
+// per lane, cell li mod 4 of quad li div 4, so that a lane's chain is six
+// moves and not twenty-four.  The four lanes of a quad share its six Philox
+// blocks: lane m draws those of arms m and (m < 2) 4 + m, and passes word h to
+// lane h.  L = 16 / 32, one-plane slabs: 9.4 / 10.9 us per step, as quads 13.0 / 13.4.
+__device__ __forceinline__ void colour_pass_cells(uint32_t* lds, uint32_t li, uint32_t L, uint32_t T, uint32_t z0,
+                                                  uint32_t pbase, bool whole, uint64_t seed, uint64_t step,
+                                                  uint32_t pass, uint32_t lanes, FastDiv dQ, uint32_t mP8,
+                                                  const uint32_t* thr, uint64_t* ring) {
+  const uint32_t hL = L / 2, qL = L / 4, LL = L * L, Q8 = LL / 8, h = li & 3u;
+  for (uint32_t i = li >> 2; i < T * Q8; i += lanes / 4) {  // (the four lanes of a quad together)
+    const Walk it = walk_start(i, Q8, mP8);
+    const uint32_t zr = it.pi;
+    const uint32_t y = fdiv(it.u, dQ), x = 2 * (it.u - y * qL) + ((y + z0 + zr + pass) & 1u);
+    const uint32_t o = 4 * (y * hL + x), cw = pbase + zr * LL + o, site = x + L * y + LL * (z0 + zr);
+    uint32_t w = lds[cw + h], wn[6];
+#pragma unroll
+    for (int arm = 0; arm < 6; ++arm) {
+      const int ax = arm >> 1;
+      const bool up = (arm & 1) == 0;
+      if (ax < 2) {
+        const uint32_t st = ax == 0 ? 4u : 4u * hL, c = ax == 0 ? x : y;
+        const bool wrap = c == (up ? hL - 1 : 0u);
+        const uint32_t d = up ? st : 0u - st, dw = up ? 0u - (hL - 1) * st : (hL - 1) * st;
+        wn[arm] = lds[cw + (wrap ? dw : d) + (wrap ? h ^ (ax == 0 ? 2u : 1u) : h)];
+      } else {
+        const bool wrap = whole && zr == (up ? T - 1 : 0u);
+        const uint32_t d = up ? LL : 0u - LL, dw = up ? 0u - (T - 1) * LL : (T - 1) * LL;
+        wn[arm] = lds[cw + (wrap ? dw : d) + h];
+      }
+    }
+    const U4 a = draw(seed, kStSigmaF, site, step, 8 * pass + h);
+    const U4 b = draw(seed, kStSigmaF, site, step, 8 * pass + 4 + h);
+    const auto from = [&](const U4& r, auto lane) {
+      constexpr int m = decltype(lane)::value;
+      return pick4(U4{quad_lane<m>(r.x), quad_lane<m>(r.y), quad_lane<m>(r.z), quad_lane<m>(r.w)}, h);
+    };
+    w = sigma_cell(w, wn[0], thr, 0, from(a, std::integral_constant<int, 0>()));
+    w = sigma_cell(w, wn[1], thr, 1, from(a, std::integral_constant<int, 1>()));
+    w = sigma_cell(w, wn[2], thr, 2, from(a, std::integral_constant<int, 2>()));
+    w = sigma_cell(w, wn[3], thr, 3, from(a, std::integral_constant<int, 3>()));
+    w = sigma_cell(w, wn[4], thr, 4, from(b, std::integral_constant<int, 0>()));
+    w = sigma_cell(w, wn[5], thr, 5, from(b, std::integral_constant<int, 1>()));
+    lds[cw + h] = w;
+    if (ring) {
+      const uint64_t v = (uint64_t)end_tag(step) << 32 | w;
+      if (zr == 0) ring_store64(ring + o + h, v);
+      if (zr == T - 1) ring_store64(ring + (size_t)kRingHalf * LL + o + h, v);
+    }
+  }
+}
+
+// The quads of colour 0 of the planes above (`hi`) and below (`lo`) into the
+// slab's ghost planes (window W).  False on time-out or abort.
+__device__ __forceinline__ bool colour_ghosts(uint32_t* W, uint32_t li, uint32_t L, uint32_t T, uint32_t z0,
+                                              const uint64_t* hi, const uint64_t* lo, uint32_t tag, uint32_t lanes,
+                                              FastDiv dP8, FastDiv dQ, uint32_t* status) {
+  const uint32_t hL = L / 2, qL = L / 4, LL = L * L, Q8 = LL / 8;
+  bool ok = true;
+  for (uint32_t i = li; i < 2 * Q8; i += lanes) {
+    const bool above = i < Q8;
+    const uint32_t u = above ? i : i - Q8, y = fdiv(u, dQ);
+    const uint32_t z = above ? z0 + T : z0 + L - 1;  // (L is even: no wrap needed for the colour)
+    const uint32_t o4 = 4 * (y * hL + 2 * (u - y * qL) + ((y + z) & 1u));
+    const uint64_t* p = (above ? hi : lo) + o4;
+    const uint64_t* const src[4] = {p, p + 1, p + 2, p + 3};
+    uint64_t v[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) v[m] = ring_load64(src[m]);
+    ok = wait_tags(src, tag, v, status) && ok;
+    const uint32_t w[4] = {(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+    quad_store(W, (above ? (T + 1) * LL : 0u) + o4, w);
+  }
+  return __ballot(!ok) == 0;
+}
+
 }  // namespace
 
 // grid = one workgroup per RGroupEnt; dynamic LDS = the largest sum of
 // window sizes of one workgroup.  The slab records sit in LDS and each
 // phase reads the fields it uses (wave-uniform), so that they are not all
 // held in scalar registers through the step loop.
-template <bool FINE>
+template <bool FINE, bool FAST>
 __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__ grp, const RSlab* __restrict__ slabs,
                                                     const PointDev* __restrict__ pts, uint32_t* __restrict__ words,
                                                     uint32_t* __restrict__ rings, uint64_t* __restrict__ ver,
@@ -494,7 +642,7 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
       const uint64_t seed = ((uint64_t)F(seed_hi) << 32) | F(seed_lo);
       // the slab's first wave draws them and keeps them for every wave of
       // the slab
-      if (wave == F(w0)) {
+      if (!FAST && wave == F(w0)) {
         uint32_t schv = 0;
         if (lane < 12) {
           const U4 r = draw(seed, kStSched, 0, step, lane);
@@ -615,8 +763,41 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
       }
       __syncthreads();
     }
+    if (FAST) {
+      // ------------------------------------------------- two colour passes
+      for (uint32_t pass = 0; pass < 2; ++pass) {
+        if (run) {
+          const uint32_t L = F(L), T = F(T), LL = L * L, ns = F(ns);
+          const uint64_t seed = ((uint64_t)F(seed_hi) << 32) | F(seed_lo);
+          uint64_t* ring =
+              pass == 0 && ns > 1 ? reinterpret_cast<uint64_t*>(rings + F(ring) + half * LL) : nullptr;
+          const uint32_t pbase = F(lds) + (ns > 1 ? LL : 0u);
+          const FastDiv dQ{L / 4, F(mQ)};
+          const uint32_t lanes = 64 * F(nw);
+          if (FINE && T * (LL / 2) <= kCellTrips * lanes)
+            colour_pass_cells(lds, li, L, T, F(z0), pbase, ns == 1, seed, step, pass, lanes, dQ, F(mP8), thr_s[gs],
+                              ring);
+          else
+            colour_pass(lds, li, L, T, F(z0), pbase, ns == 1, seed, step, pass, dQ, F(mP8), F(dp8), F(du8),
+                        thr_s[gs], ring);
+        }
+        if (pass == 0) {
+          // the neighbours' boundary planes as the pass left them; the
+          // second pass reads them as ghosts
+          if (run && F(ns) > 1) {
+            const uint32_t L = F(L), LL = L * L;
+            if (!colour_ghosts(lds + F(lds), li, L, F(T), F(z0),
+                               reinterpret_cast<const uint64_t*>(rings + F(ring_hi) + half * LL),
+                               reinterpret_cast<const uint64_t*>(rings + F(ring_lo) + (2 * kRingHalf + half) * LL),
+                               end_tag(step), 64 * F(nw), FastDiv{LL / 8, F(mP8)}, FastDiv{L / 4, F(mQ)}, status))
+              abort_s = 1;
+          }
+        }
+        __syncthreads();
+      }
+    }
     // ----------------------------------------------------- 12 half-sweeps
-    for (uint32_t k = 0; k < 12; ++k) {
+    for (uint32_t k = 0; k < (FAST ? 0u : 12u); ++k) {
       const uint32_t sk = has ? uni(sch_s[gs][k]) : 0u;
       const bool wr = (sk >> 8) & 1u;
       const int arm = (int)(sk & 7u);
@@ -862,35 +1043,42 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
 
 uint32_t resident_lds_limit() { return 160 * 1024 - kResidentStatic; }
 
-static void set_resident_attribute() {
+namespace {
+using ResidentKernel = decltype(&k_resident<false, false>);
+ResidentKernel resident_kernel(bool fine, bool fast) {
+  return fast ? (fine ? &k_resident<true, true> : &k_resident<false, true>)
+              : (fine ? &k_resident<true, false> : &k_resident<false, false>);
+}
+
+void set_resident_attribute() {
   // the dynamic-LDS limit is a per-device function attribute
   static std::atomic<uint64_t> attr_set{0};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const uint64_t bit = 1ull << (dev & 63);
   if (!(attr_set.load(std::memory_order_acquire) & bit)) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_resident<false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)resident_lds_limit());
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_resident<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)resident_lds_limit());
+    for (int i = 0; i < 4; ++i)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(resident_kernel(i & 1, i & 2)),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)resident_lds_limit());
     attr_set.fetch_or(bit, std::memory_order_acq_rel);
   }
 }
+}  // namespace
 
-hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, bool fine) {
+hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, bool fine, bool fast) {
   set_resident_attribute();
-  return fine ? hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_resident<true>, (int)block, (size_t)lds_bytes)
-              : hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_resident<false>, (int)block, (size_t)lds_bytes);
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, resident_kernel(fine, fast), (int)block,
+                                                      (size_t)lds_bytes);
 }
 
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
                      const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
-                     bool fine) {
+                     bool fine, bool fast) {
   set_resident_attribute();
   hipEvent_t t0, t1;
   get_launch_timing(&t0, &t1);
-  auto* k = fine ? k_resident<true> : k_resident<false>;
+  const ResidentKernel k = resident_kernel(fine, fast);
   if (t0)
     hipExtLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, rings, ver,
                           stepp, step_off, nsteps, step_out, status);

@@ -156,9 +156,9 @@ typedef struct cvf_tuning {
                            LDS or would be one plane thick; 0: one kernel per half-sweep;
                            2: the resident kernel (every step of a graph in one launch, the
                            lattice held in LDS, one stream group) where the points allow it
-                           (reference schedule, one Metropolis sweep per step, chessboard
-                           rule), else as 1.  The default is 1, or 2 with one-plane slabs
-                           for small handles of one Metropolis sweep per step */
+                           (one Metropolis sweep per step, chessboard rule), else as 1.  The default is 1, or 2 with one-plane slabs
+                           for small handles of one Metropolis sweep per step, or with the
+                           fast schedule up to L = 64 */
   int32_t slab_planes;  /* planes per slab of the fused kernel (<= 16), or the thickest slab
                            of the resident kernel; 0 = automatic (tiles included) */
   int32_t block_chunk;  /* workgroup size of the fused kernel */
