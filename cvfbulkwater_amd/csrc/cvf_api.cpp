@@ -127,6 +127,7 @@ struct Group {
   DevBuf<uint64_t> rver;
   uint32_t r_ngroups = 0, r_lds = 0;
   bool r_fine = false;  // every slab at most two planes: the fine instantiation
+  uint32_t r_per = 0;   // one plane per workgroup: the plane kernel, this many half-sweeps at a time (0: not)
   // a second stream beside `stream` for the device volume chain of a
   // resident sequence, which never reads the lattice (fork / join events)
   hipStream_t side = nullptr;
@@ -740,7 +741,28 @@ int build_resident(cvf_sim* s, Group& g) {
                  (s->sched == CVF_SCHED_FAST && r.T * LL / 2 <= 128ull * r.nw);
   }
   const bool fine = thin && fine_phase;
-  HIPC(resident_occupancy(&occ, (uint32_t)s->tune.block_chunk, d.lds_bytes, fine, s->sched == CVF_SCHED_FAST));
+  // one plane per workgroup: the kernel for that, while its phases are short
+  // (one point of L = 12 / 32 / 48 / 56: 7.9 / 11.6 / 17.6 / 23.7 us per step, the
+  // general kernel 13.7 / 15.6 / 22.2 / 24.2; L = 64 25.9 and 24.4)
+  bool planes = s->sched == CVF_SCHED_REFERENCE;
+  uint32_t maxL = 0;
+  for (const auto& r : d.slabs) {
+    planes = planes && r.T == 1 && r.nw == wpg && r.L <= 56;
+    maxL = std::max(maxL, r.L);
+  }
+  // as many half-sweeps laid out at a time as a workgroup's share of LDS holds
+  // (its threads of the CU's 2048: the records take no CU from other launches)
+  uint32_t per = 12;
+  const uint32_t share = std::min<uint32_t>(4 * cap, 160 * 1024 / 2048 * (uint32_t)s->tune.block_chunk - 512);
+  for (uint32_t next : {6u, 4u, 3u, 2u, 1u})
+    if (plane_lds_bytes(maxL, per) > share) per = next;
+  planes = planes && plane_lds_bytes(maxL, per) <= 4 * cap;
+  if (planes) {
+    d.lds_bytes = plane_lds_bytes(maxL, per);
+    HIPC(plane_occupancy(&occ, (uint32_t)s->tune.block_chunk, d.lds_bytes));
+  } else {
+    HIPC(resident_occupancy(&occ, (uint32_t)s->tune.block_chunk, d.lds_bytes, fine, s->sched == CVF_SCHED_FAST));
+  }
   if (occ < per_cu) return CVF_OK;
   int rc;
   if ((rc = upload_vec(g.rslabs, d.slabs)) || (rc = upload_vec(g.rgroups, d.groups))) return rc;
@@ -754,6 +776,7 @@ int build_resident(cvf_sim* s, Group& g) {
   g.r_ngroups = (uint32_t)d.groups.size();
   g.r_lds = d.lds_bytes;
   g.r_fine = fine;
+  g.r_per = planes ? per : 0;
   if (!g.side) {
     HIPC(hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking));
     HIPC(hipEventCreateWithFlags(&g.fork, hipEventDisableTiming));
@@ -1283,6 +1306,20 @@ int build_groups(cvf_sim* s) {
   return CVF_OK;
 }
 
+// nsteps steps of resident group g in one launch (launch_resident's stepp,
+// step_off and step_out).
+void run_resident(cvf_sim* s, const Group& g, hipStream_t st, const uint64_t* stepp, uint64_t step_off,
+                  uint32_t nsteps, uint64_t* step_out) {
+  s->resident_used = true;
+  if (g.r_per)
+    launch_plane(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
+                 s->words.p, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_per);
+  else
+    launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
+                    s->words.p, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_fine,
+                    s->sched == CVF_SCHED_FAST);
+}
+
 // A fused launch of half-sweeps k0 .. k0 + nk - 1 of group g from src to dst.
 void launch_fused(cvf_sim* s, const Group& g, hipStream_t st, const uint64_t* stepp, uint32_t step_off,
                   const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk, int with_eta) {
@@ -1319,12 +1356,8 @@ void enqueue_lattice(cvf_sim* s, int gi, hipStream_t st, uint32_t step_off, Time
   const Launch lc{g.tab_cube.p, g.nb_cube, (uint32_t)s->tune.block_eta, stepp, step_off};
   const Launch ll{g.tab_cell.p, g.nb_cell, (uint32_t)s->tune.block_cell, stepp, step_off};
   if (g.resident) {
-    s->resident_used = true;
     // one step of the resident kernel, in place on `words`
-    timed(CVF_KCLASS_RESIDENT, [&] {
-      launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                      s->words.p, g.rings.p, g.rver.p, stepp, step_off, 1, nullptr, s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
-    });
+    timed(CVF_KCLASS_RESIDENT, [&] { run_resident(s, g, st, stepp, step_off, 1, nullptr); });
   } else if (s->sched == CVF_SCHED_FAST) {
     // eta cube sweep, then n_metropolis x the two colour passes (in place,
     // on the array holding the state)
@@ -1429,9 +1462,7 @@ int enqueue_resident(cvf_sim* s, int gi, hipStream_t st, int nsteps) {
                      s->dist.p, s->freq.p, s->precision, 1);
     HIPC(hipEventRecord(g.join, g.side));
   }
-  launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                  s->words.p, g.rings.p, g.rver.p, nullptr, (uint64_t)s->steps, (uint32_t)nsteps,
-                  s->cur_steps.p + gi, s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
+  run_resident(s, g, st, nullptr, (uint64_t)s->steps, (uint32_t)nsteps, s->cur_steps.p + gi);
   if (s->vol_device) HIPC(hipStreamWaitEvent(st, g.join, 0));
   HIPC(hipGetLastError());
   return CVF_OK;
@@ -1582,12 +1613,11 @@ cvf_tuning default_tuning(const cvf_sim* s) {
   }
   // a small handle of one Metropolis sweep per step, nothing between the
   // steps, whose planes can each have a workgroup: one-plane resident slabs
-  // in 64-step graphs (one point at L = 16 / 32 / 48 / 64: 13.7 / 16.9 /
-  // 23.6 / 26.6 us per step, against 18.4 / 20.9 / 32.4 / 38.2 for
-  // whole-pass fused launches), 256-thread workgroups up to L = 16 and
-  // 512-thread ones up to L = 32, whose fine phases then fill their waves
-  // (L = 16: 13.74 us per step at 256 threads, 13.96 at 512; L = 24: 15.26
-  // at 512, 15.52 at 256; L = 32: 15.24 at 512, 15.64 at 256)
+  // (one point at L = 16 / 32 / 48 / 64: 8.0 / 11.6 / 17.6 / 24.4 us per step, against
+  // 18.4 / 20.9 / 32.4 / 38.2 for whole-pass fused launches), 256-thread workgroups up
+  // to L = 16 and 512-thread ones up to L = 32 (L = 16: 8.0 us per step at 256
+  // threads, 8.2 at 512; L = 24: 10.3 at 512, 14.0 at 256; L = 32: 11.6 at 512, 11.3 at
+  // 1024, of which a CU holds half as many)
   uint64_t planes = 0;
   uint32_t maxL = 0;
   for (const auto& P : s->ph) {
@@ -2178,9 +2208,7 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     if (!g.resident || s->nc > 0 || n_steps == 0) continue;
     s->resident_used = true;
     timed(CVF_KCLASS_RESIDENT, [&] {
-      launch_resident(g.stream, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p,
-                      s->pts.p, s->words.p, g.rings.p, g.rver.p, s->cur_steps.p + gi, 0, (uint32_t)n_steps, nullptr,
-                      s->rstatus.p, g.r_fine, s->sched == CVF_SCHED_FAST);
+      run_resident(s, g, g.stream, s->cur_steps.p + gi, 0, (uint32_t)n_steps, nullptr);
     });
     timed(CVF_KCLASS_BEGIN, [&] {
       launch_vol_chain(g.stream, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,

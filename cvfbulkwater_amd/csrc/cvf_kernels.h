@@ -230,5 +230,14 @@ void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uin
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
                      const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
                      bool fine, bool fast);
+// The same for plans of the reference schedule whose workgroups hold one
+// one-plane slab each (cvf_plane.hip), the moves of `per` half-sweeps (a
+// divisor of 12) laid out at a time in plane_lds_bytes of dynamic LDS.
+uint32_t plane_lds_bytes(uint32_t L, uint32_t per);
+hipError_t plane_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes);
+void launch_plane(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
+                  const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
+                  const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                  uint32_t per);
 
 }  // namespace cvf
