@@ -10,9 +10,11 @@
 #include <string.h>
 
 #include <algorithm>
+#include <condition_variable>
 #include <map>
-#include <queue>
 #include <memory>
+#include <mutex>
+#include <queue>
 #include <string>
 #include <vector>
 
@@ -184,6 +186,92 @@ int set_error(int code, const char* fmt, ...) {
 }
 }  // namespace cvf
 
+// Resident launches of several handles.  A resident kernel's workgroups wait
+// for each other, so each launch needs all of its own on the card at once, and
+// two launches of which each has a part would wait until their limit.  Handles
+// of a process whose plans are resident therefore enter() before they
+// enqueue such launches and leave() after: those that surely fit together (half
+// of the device's room in all, none with workgroups of more than half a CU)
+// run side by side, any other one waits on the device for those before it.  A
+// handle that is alone only takes the lock.
+struct ResidentGate {
+  struct User {
+    int device = 0;
+    double share = 0;     // of the device's room for workgroups such as its
+    bool large = false;   // a CU holds one of them
+    bool launching = false, recorded = false;
+    hipEvent_t done = nullptr;
+  };
+  std::mutex mu;
+  std::condition_variable left;
+  std::vector<User*> users;
+
+  void add(User* u) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (std::find(users.begin(), users.end(), u) == users.end()) users.push_back(u);
+  }
+  void remove(User* u) {
+    std::lock_guard<std::mutex> lock(mu);
+    users.erase(std::remove(users.begin(), users.end(), u), users.end());
+  }
+  hipError_t enter(User* u, hipStream_t st) {
+    std::unique_lock<std::mutex> lock(mu);
+    for (;;) {
+      double sum = u->share;
+      bool large = u->large, launching = false;
+      std::vector<User*> before;
+      for (User* o : users) {
+        if (o == u || o->device != u->device) continue;
+        if (!o->launching && (!o->recorded || hipEventQuery(o->done) == hipSuccess)) {
+          o->recorded = false;
+          continue;
+        }
+        before.push_back(o);
+        sum += o->share;
+        large = large || o->large;
+        launching = launching || o->launching;
+      }
+      if (!before.empty() && (sum > 0.5 || large)) {
+        if (launching) {  // its event is not recorded yet
+          left.wait(lock);
+          continue;
+        }
+        for (User* o : before)
+          if (hipError_t e = hipStreamWaitEvent(st, o->done, 0)) return e;
+      }
+      u->launching = true;
+      return hipSuccess;
+    }
+  }
+  hipError_t leave(User* u, hipStream_t st) {
+    std::lock_guard<std::mutex> lock(mu);
+    hipError_t e = hipSuccess;
+    // (a handle added later has synchronized the device before its first
+    // launch, after this one's)
+    if (users.size() > 1) {
+      e = hipEventRecord(u->done, st);
+      u->recorded = e == hipSuccess;
+    }
+    u->launching = false;
+    left.notify_all();
+    return e;
+  }
+};
+ResidentGate g_resident_gate;
+
+struct ResidentTurn {
+  ResidentGate::User* u = nullptr;
+  hipStream_t st = nullptr;
+  hipError_t take(ResidentGate::User* user, hipStream_t stream) {
+    hipError_t e = g_resident_gate.enter(user, stream);
+    if (e == hipSuccess) u = user, st = stream;
+    return e;
+  }
+  ~ResidentTurn() {
+    if (u) (void)g_resident_gate.leave(u, st);
+  }
+};
+
 struct cvf_sim {
   int device = 0;
   hipStream_t stream = nullptr;  // main stream: uploads, observables, statistics
@@ -211,6 +299,7 @@ struct cvf_sim {
   DevBuf<uint64_t> hist_base;              // step count at the first recorded step
   DevBuf<uint32_t> rstatus;                // abort flag of the resident kernel
   bool resident_used = false;              // some launch ran the resident kernel
+  ResidentGate::User turn;                 // of its resident plan, if it has one
   uint64_t hist_base_host = 0;
   int rec_pt = -1;                         // point recorded by the groups' rec graphs
   uint32_t nb_cell_all = 0;
@@ -238,6 +327,8 @@ struct cvf_sim {
     for (auto& g : groups) g->drop_graphs();
   }
   ~cvf_sim() {
+    g_resident_gate.remove(&turn);
+    if (turn.done) (void)hipEventDestroy(turn.done);
     groups.clear();
     if (start_ev) (void)hipEventDestroy(start_ev);
     if (stream) (void)hipStreamDestroy(stream);
@@ -721,7 +812,7 @@ int build_resident(cvf_sim* s, Group& g) {
   int ncu = 0;
   HIPC(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, s->device));
   if (ncu <= 0) return CVF_OK;
-  const int per_cu = std::min(2, std::max(1, s->tune.streams));
+  const int per_cu = std::min(s->tune.slab_planes == 1 ? 4 : 2, std::max(1, s->tune.streams));
   const uint32_t cap = (resident_lds_limit() - (uint32_t)(per_cu - 1) * kResidentStatic) / (uint32_t)per_cu / 4u;
   const uint32_t wpg = (uint32_t)s->tune.block_chunk / 64u;
   RDeal d;
@@ -751,9 +842,10 @@ int build_resident(cvf_sim* s, Group& g) {
     maxL = std::max(maxL, r.L);
   }
   // as many half-sweeps laid out at a time as a workgroup's share of LDS holds
-  // (its threads of the CU's 2048: the records take no CU from other launches)
+  // (its threads of the 1024 that the kernels' registers allow a CU: the
+  // records take no CU from other launches)
   uint32_t per = 12;
-  const uint32_t share = std::min<uint32_t>(4 * cap, 160 * 1024 / 2048 * (uint32_t)s->tune.block_chunk - 512);
+  const uint32_t share = std::min<uint32_t>(4 * cap, 160 * (uint32_t)s->tune.block_chunk - 512);
   for (uint32_t next : {6u, 4u, 3u, 2u, 1u})
     if (plane_lds_bytes(maxL, per) > share) per = next;
   planes = planes && plane_lds_bytes(maxL, per) <= 4 * cap;
@@ -783,6 +875,11 @@ int build_resident(cvf_sim* s, Group& g) {
     HIPC(hipEventCreateWithFlags(&g.join, hipEventDisableTiming));
   }
   g.resident = true;
+  s->turn.device = s->device;
+  s->turn.share = (double)d.groups.size() / ((double)occ * ncu);
+  s->turn.large = occ < 2;
+  if (!s->turn.done) HIPC(hipEventCreateWithFlags(&s->turn.done, hipEventDisableTiming));
+  g_resident_gate.add(&s->turn);
   for (int p : g.points) s->ph[p].slab_T = 0;
   // the plan query reports a point's thickest slab
   for (const auto& r : d.slabs) s->ph[r.point].slab_T = std::max(s->ph[r.point].slab_T, r.T);
@@ -1205,6 +1302,7 @@ int build_tiles(cvf_sim* s, Group& g, const SlabTable& slabs) {
 // largest-first onto the group with the fewest cells.
 int build_groups(cvf_sim* s) {
   HIPC(hipDeviceSynchronize());
+  g_resident_gate.remove(&s->turn);
   s->groups.clear();
   // the resident kernel takes every point in one group (its workgroups must
   // all be resident at once, one per CU at most)
@@ -1611,25 +1709,53 @@ cvf_tuning default_tuning(const cvf_sim* s) {
       t.block_chunk = (int32_t)best.block;
     }
   }
-  // a small handle of one Metropolis sweep per step, nothing between the
-  // steps, whose planes can each have a workgroup: one-plane resident slabs
-  // (one point at L = 16 / 32 / 48 / 64: 8.0 / 11.6 / 17.6 / 24.4 us per step, against
-  // 18.4 / 20.9 / 32.4 / 38.2 for whole-pass fused launches), 256-thread workgroups up
-  // to L = 16 and 512-thread ones up to L = 32 (L = 16: 8.0 us per step at 256
-  // threads, 8.2 at 512; L = 24: 10.3 at 512, 14.0 at 256; L = 32: 11.6 at 512, 11.3 at
-  // 1024, of which a CU holds half as many)
+  // One Metropolis sweep per step up to L = 64: the resident kernels.  One-plane
+  // slabs while there are workgroups for the planes, one to four of them per CU:
+  // 256 threads up to L = 16 and 512 up to L = 32, fewer where more share a CU
+  // (one point of L = 16 / 32 / 48 / 64: 8.1 / 10.9 / 17.0 / 24.4 us per step, whole-pass
+  // fused launches 18.4 / 20.9 / 32.4 / 38.2; two per CU, 16 points of L = 32 / 32 of
+  // L = 16: 15.9 / 9.8, fused 29.2 / 19.6; three, 24 of L = 32 / 48 of L = 16: 21.3 /
+  // 11.0, fused 39.2 / 23.2; four, 40 of L = 24 / 64 of L = 16: 19.3 / 11.7, fused 32.8
+  // / 20.8).  Else thicker slabs, one workgroup per CU (32 points of L = 32 / 48, 96
+  // of L = 16 / 32 / 48: 23.0 / 35 / 57 us, fused 35.1 / 73 / 136), from L = 12 on
+  // (96 points of L = 12 18.9 and 21.8 us, 140 of L = 8 24.2 and 20.3).
   uint64_t planes = 0;
   uint32_t maxL = 0;
   for (const auto& P : s->ph) {
     planes += P.L;
     maxL = std::max(maxL, P.L);
   }
-  if (!any_nc && maxL <= 64 && s->sched == CVF_SCHED_REFERENCE && s->nm == 1 && s->nc == 0 && planes <= 256 &&
-      s->total_cells < (1u << 20)) {
-    t.fused = 2;
-    t.slab_planes = 1;
-    t.block_chunk = maxL <= 16 ? 256 : maxL <= 32 ? 512 : 1024;
-    t.graph_steps = 64;
+  // words of all CUs' LDS; windows hold ghost planes too
+  const uint64_t room = cu_count(s, ncu) == CVF_OK ? (uint64_t)ncu * resident_lds_limit() / 4 : 0;
+  const bool fits = s->total_cells <= room / 5 * 4;
+  if (!any_nc && maxL <= 64 && s->sched == CVF_SCHED_REFERENCE && s->nm == 1) {
+    const uint64_t per_cu = (planes + ncu - 1) / std::max(ncu, 1u);
+    int block = 0;
+    if (per_cu <= 1)
+      block = maxL <= 16 ? 256 : maxL <= 32 ? 512 : 1024;
+    else if (per_cu == 2 && maxL <= 40)
+      block = maxL <= 16 ? 256 : 512;
+    else if (per_cu == 3 && maxL <= 32)
+      block = 256;
+    else if (per_cu == 4 && maxL <= 24)
+      block = maxL <= 16 ? 128 : 256;
+    // with a cluster sweep, a launch per step, small lattices only (L = 8 / 16 /
+    // 32: 26.2 / 28.5 / 32.6 us per step, tiles 32.7 / 33.8 / 35.0; 24 of L = 32
+    // 72.9 and 77.8)
+    const bool one_plane =
+        block && (s->nc == 0 ? planes > ncu || s->total_cells < (1u << 20) : maxL <= 32 && per_cu <= 3);
+    if (one_plane) {
+      t.fused = 2;
+      t.streams = (int32_t)per_cu;
+      t.slab_planes = 1;
+      t.block_chunk = block;
+      t.graph_steps = s->nc == 0 ? 64 : 16;
+    } else if (s->nc == 0 && maxL >= 12 && fits) {
+      t.fused = 2;
+      t.slab_planes = 0;
+      t.block_chunk = maxL <= 24 ? 512 : 1024;
+      t.graph_steps = 64;
+    }
   }
   // the fast schedule's step of four phases with two exchanges between: the
   // resident kernel where it holds the points (one-plane slabs while there is
@@ -1639,10 +1765,9 @@ cvf_tuning default_tuning(const cvf_sim* s) {
   // L = 32 17.7 and 28.0, 128 of L = 16 .. 48 58.0 and 69.4).  With a cluster
   // sweep, a launch per step, only small ones gain (L = 16 / 32 / 64: 29.3 / 31.2 /
   // 47.3 and 35.4 / 35.0 / 43.0).
-  if (s->sched == CVF_SCHED_FAST && s->nm == 1 && cu_count(s, ncu) == CVF_OK) {
-    const bool planes_fit = planes <= 256, small = maxL <= 32 && s->total_cells < (1u << 21);
-    const uint64_t room = (uint64_t)ncu * resident_lds_limit() / 4;  // words; windows hold ghost planes too
-    if (s->nc == 0 ? maxL <= 64 && s->total_cells <= room / 5 * 4 : maxL <= 32 && planes_fit) {
+  if (s->sched == CVF_SCHED_FAST && s->nm == 1) {
+    const bool planes_fit = planes <= ncu, small = maxL <= 32 && s->total_cells < (1u << 21);
+    if (s->nc == 0 ? maxL <= 64 && fits : maxL <= 32 && planes_fit) {
       t.fused = 2;
       t.slab_planes = planes_fit ? 1 : 0;
       t.block_chunk = small ? 512 : 1024;
@@ -1846,6 +1971,8 @@ int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
 // n_steps MC steps as resident launches or graph launches; group rec_gi (if
 // >= 0) replays its recording sequences.
 int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
+  ResidentTurn turn;
+  if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
   if (rec_gi < 0 && s->groups.size() == 1 && resident_sequences(s, *s->groups[0])) {
     for (int64_t i = 0; i < n_steps;) {
       const int k = (int)std::min<int64_t>(s->tune.graph_steps, n_steps - i);
@@ -2198,6 +2325,8 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     set_launch_timing(nullptr, nullptr);
     recs.push_back(r);
   };
+  ResidentTurn turn;
+  if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
   int rc = fork_groups(s);
   if (rc) return rc;
   if (s->nc > 0 && n_steps > 0) s->sw_labels = true;

@@ -146,7 +146,8 @@ void cvf_destroy(cvf_sim *s);
  * is fixed at N/512 blocks of 512 threads (gpu_water3D.cu:68, 517-518). */
 typedef struct cvf_tuning {
   int32_t streams;      /* groups of state points, each on its own stream (1..8); with
-                           fused = 2, resident workgroups per CU (1 or 2) */
+                           fused = 2, resident workgroups per CU (1 or 2, to 4 with one-plane
+                           slabs) */
   int32_t block_sigma;  /* workgroup size of the sigma half-sweep (64..1024, power of 2) */
   int32_t block_eta;    /* workgroup size of the eta cube sweep */
   int32_t block_cell;   /* workgroup size of the per-cell kernels (SW, observables) */
@@ -156,9 +157,12 @@ typedef struct cvf_tuning {
                            LDS or would be one plane thick; 0: one kernel per half-sweep;
                            2: the resident kernel (every step of a graph in one launch, the
                            lattice held in LDS, one stream group) where the points allow it
-                           (one Metropolis sweep per step, chessboard rule), else as 1.  The default is 1, or 2 with one-plane slabs
-                           for small handles of one Metropolis sweep per step, or with the
-                           fast schedule up to L = 64 */
+                           (one Metropolis sweep per step, chessboard rule), else as 1.  Its
+                           workgroups wait for each other: launches of several handles of
+                           a process take turns where they might not fit together; two
+                           processes on one device should use 1.  The default is 2 for
+                           handles of one Metropolis sweep per step up to L = 64 that
+                           fit, else 1 */
   int32_t slab_planes;  /* planes per slab of the fused kernel (<= 16), or the thickest slab
                            of the resident kernel; 0 = automatic (tiles included) */
   int32_t block_chunk;  /* workgroup size of the fused kernel */
