@@ -1012,11 +1012,14 @@ __device__ __forceinline__ uint32_t uf_find(const uint32_t* par, uint32_t x) {
   return x;
 }
 
+// The components of a and b become one: the larger of the two is linked to the
+// smaller if it is a root, else its parent takes its place.  The smaller need
+// not be a root itself: it lies below every id of the other's component.  Nine
+// nodes in ten are alone, so one exchange usually does, where finding both
+// roots first took two loads before it (all three go to memory, past the XCDs'
+// caches).
 __device__ void uf_unite(uint32_t* par, uint32_t a, uint32_t b) {
-  while (true) {
-    a = uf_find(par, a);
-    b = uf_find(par, b);
-    if (a == b) return;
+  while (a != b) {
     if (a < b) {
       const uint32_t t = a;
       a = b;
@@ -1026,6 +1029,7 @@ __device__ void uf_unite(uint32_t* par, uint32_t a, uint32_t b) {
     if (__hip_atomic_compare_exchange_strong(par + a, &expected, b, __ATOMIC_RELAXED,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       return;
+    a = expected;
   }
 }
 
@@ -1052,7 +1056,7 @@ __global__ void k_sw_local(const BlockEnt* __restrict__ tab, uint32_t nb,
   const uint64_t seed = seed_of(e);
 #pragma unroll
   for (int g = 0; g < 5; ++g) {
-    const U4 r = draw(seed, kStSwBond, t, step, jc * 5 + g);
+    const U4 r = draw_site(t, phase_draws(seed, kStSwBond, step, jc * 5 + g));
     rw[4 * g] = r.x;
     rw[4 * g + 1] = r.y;
     rw[4 * g + 2] = r.z;
@@ -1135,13 +1139,17 @@ __global__ void k_sw_flip(const BlockEnt* __restrict__ tab, uint32_t nb,
   uint32_t* W = words + e.woff;
   uint32_t w = W[t];
   uint32_t nw = w & ~kSigmaBits;
+  const PhiloxFixed pf = phase_draws(seed, kStSwFlip, step, jc);
+  uint32_t p[6];  // the arms' parents, six loads at once
+#pragma unroll
+  for (int a = 0; a < 6; ++a) p[a] = uf_load(par, a * N + t);
 #pragma unroll
   for (int a = 0; a < 6; ++a) {
     const uint32_t node = a * N + t;
-    const uint32_t root = uf_find(par, node);
-    __hip_atomic_store(par + node, root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const U4 r = draw(seed, kStSwFlip, root, step, jc);
-    uint32_t s = sigma_of(w, a) + uniform_int(r.x, 6);
+    const uint32_t root = p[a] == node ? node : uf_find(par, p[a]);
+    // (most nodes hold their root already)
+    if (root != p[a]) __hip_atomic_store(par + node, root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t s = sigma_of(w, a) + uniform_int(draw_site(root, pf).x, 6);
     s = s >= 6 ? s - 6 : s;
     nw |= s << (3 * a);
   }
