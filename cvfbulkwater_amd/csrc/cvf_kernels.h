@@ -152,21 +152,29 @@ void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned l
 void launch_sigma_hist_slot(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* series,
                             const uint64_t* gstep, uint32_t step_off, const uint64_t* base, uint32_t span);
 // cluster statistics of one point (labels at `label`, 6N nodes)
-void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* size);
-// Cluster sizes size[0..nn) (zero: no cluster): the count into *total and
-// each workgroup's offset into bcount (compact_blocks(nn) words), and the
-// sizes' moments bmom[4 nb .. 4 nb + 3] = sum, sum of squares, largest |
-// second largest << 32 (bmom: 4 (compact_blocks(nn) + 1) words); then, with
-// those offsets, the non-zero sizes in label order into out[0..*total)
-constexpr uint32_t kCompactSpan = 1024;
+// Per cluster root the cluster's other nodes (others[0..nn) zero before).
+void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* others);
+// A labelling's clusters in host memory (pinned): their count, the sum and sum
+// of squares of their sizes, the largest two, the percolation slots taken and
+// the percolating ones.
+struct ClusterSums {
+  uint64_t sum, squares;
+  uint32_t largest, second, clusters, slots, percolating, pad;
+};
+// Counts and moments per workgroup of kCompactSpan nodes (bcount and 4 words
+// each of bmom, compact_blocks(nn) of them) and a slot for each cluster of at
+// least minsize nodes; then, after the percolation test, the counts' offsets
+// and the sums, and, with the offsets, the sizes in label order.
+constexpr uint32_t kCompactSpan = 4096;
 uint32_t compact_blocks(uint32_t nn);
-void launch_compact_count(hipStream_t st, const int32_t* size, uint32_t nn, uint32_t* bcount, uint32_t* total,
-                          uint64_t* bmom);
-void launch_compact_write(hipStream_t st, const int32_t* size, uint32_t nn, const uint32_t* bcount, int32_t* out);
-void launch_perc_slots(hipStream_t st, const uint32_t* label, uint32_t nn, const int32_t* size,
-                       int32_t minsize, int32_t* slot, uint32_t* nslot, uint32_t max_slots);
-void launch_perc_cover(hipStream_t st, const uint32_t* label, uint32_t nn, uint32_t L,
-                       const int32_t* size, int32_t minsize, const int32_t* slot, uint32_t* cover,
+void launch_compact_count(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn, uint32_t* bcount,
+                          uint64_t* bmom, uint32_t minsize, int32_t* slot, uint32_t* nslot, uint32_t max_slots);
+void launch_compact_scan(hipStream_t st, uint32_t* bcount, uint32_t nn, const uint64_t* bmom,
+                         const uint32_t* nslot_nperc, ClusterSums* out);
+void launch_compact_write(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn,
+                          const uint32_t* bcount, int32_t* out);
+void launch_perc_cover(hipStream_t st, const uint32_t* label, uint32_t nn, uint32_t L, const int32_t* others,
+                       uint32_t minsize, const int32_t* slot, const uint32_t* nslot, uint32_t* cover,
                        uint32_t max_slots);
 void launch_perc_count(hipStream_t st, const uint32_t* cover, const uint32_t* nslot, uint32_t L,
                        uint32_t max_slots, uint32_t* nperc);

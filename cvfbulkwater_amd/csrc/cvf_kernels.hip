@@ -1170,18 +1170,36 @@ __device__ __forceinline__ uint32_t run_end(uint64_t heads, uint32_t lane) {
   return above ? (uint32_t)__builtin_ctzll(above) : 64u;
 }
 
+// A cluster's nodes but its root, counted at its root (whose label is its own
+// id): most nodes are roots of one, and need no atomic.  Bound by the atomics
+// (L = 96: 430,000 of them, 17 us; all of 5.3 million 28).
 __global__ __launch_bounds__(256) void k_cluster_sizes(const uint32_t* __restrict__ label, uint32_t nn,
-                                                       int32_t* __restrict__ size) {
+                                                       int32_t* __restrict__ others) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
-  const uint32_t lab = i < nn ? label[i] : 0xFFFFFFFFu;  // no node has that label
+  uint32_t lab = i < nn ? label[i] : i;
+  if (lab == i) lab = 0xFFFFFFFFu;  // no node has that label
   const uint32_t prev = __shfl_up(lab, 1, 64);
   const bool head = lane == 0 || lab != prev;
   const uint64_t heads = __ballot(head);
-  if (head && i < nn) atomicAdd(&size[lab], (int32_t)(run_end(heads, lane) - lane));
+  if (head && lab != 0xFFFFFFFFu) atomicAdd(&others[lab], (int32_t)(run_end(heads, lane) - lane));
 }
 
-// Order-preserving compaction of the cluster sizes (non-zero entries of
-// size[], in label order): per workgroup of kCompactSpan labels the count
+// Sizes of the clusters whose roots are nodes i .. i + 3 (0: not a root).
+__device__ __forceinline__ void root_sizes(const uint32_t* label, const int32_t* others, uint32_t nn, uint32_t i,
+                                           uint32_t (&v)[4]) {
+  if (i + 3 < nn) {  // (nn, six lattices of a multiple of four cells, is a multiple of four)
+    const uint4 l = *reinterpret_cast<const uint4*>(label + i);
+    const int4 o = *reinterpret_cast<const int4*>(others + i);
+    v[0] = l.x == i ? 1u + (uint32_t)o.x : 0u;
+    v[1] = l.y == i + 1 ? 1u + (uint32_t)o.y : 0u;
+    v[2] = l.z == i + 2 ? 1u + (uint32_t)o.z : 0u;
+    v[3] = l.w == i + 3 ? 1u + (uint32_t)o.w : 0u;
+  } else {
+    v[0] = v[1] = v[2] = v[3] = 0;
+  }
+}
+
+// Order-preserving compaction of the cluster sizes (in label order): per workgroup of kCompactSpan labels the count
 // of clusters, one workgroup's exclusive scan of those counts, then every
 // workgroup writes its clusters at its offset.  The host then assembles the
 // cluster.out row from the clusters alone, in the same order.
@@ -1262,18 +1280,31 @@ __device__ __forceinline__ void mom_block_store(Mom m, uint64_t* sh, uint64_t* o
   }
 }
 
-__global__ __launch_bounds__(256) void k_compact_count(const int32_t* __restrict__ size, uint32_t nn,
-                                                       uint32_t* __restrict__ bcount, uint64_t* __restrict__ bmom) {
+// The clusters of kCompactSpan nodes: their count and moments, and a slot for
+// each of at least minsize nodes (*nslot of them so far).
+__global__ __launch_bounds__(256) void k_compact_count(const uint32_t* __restrict__ label,
+                                                       const int32_t* __restrict__ others, uint32_t nn,
+                                                       uint32_t* __restrict__ bcount, uint64_t* __restrict__ bmom,
+                                                       uint32_t minsize, int32_t* __restrict__ slot,
+                                                       uint32_t* __restrict__ nslot, uint32_t max_slots) {
   __shared__ uint32_t sh[4];
   __shared__ uint64_t shm[16];
-  const uint32_t base = blockIdx.x * kCompactSpan + threadIdx.x * 4;
   uint32_t c = 0;
   Mom m{0, 0, 0, 0};
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
-    const uint32_t v = base + k < nn ? (uint32_t)size[base + k] : 0u;
-    c += v != 0;
-    mom_add(m, v);
+  for (uint32_t r = 0; r < kCompactSpan; r += 1024) {
+    const uint32_t i = blockIdx.x * kCompactSpan + r + threadIdx.x * 4;
+    uint32_t v[4];
+    root_sizes(label, others, nn, i, v);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      c += v[k] != 0;
+      mom_add(m, v[k]);
+      if (v[k] >= minsize) {
+        const uint32_t s = atomicAdd(nslot, 1u);
+        slot[i + k] = s < max_slots ? (int32_t)s : -1;
+      }
+    }
   }
   uint32_t total;
   block_excl_scan256(c, sh, &total);
@@ -1281,12 +1312,15 @@ __global__ __launch_bounds__(256) void k_compact_count(const int32_t* __restrict
   mom_block_store(m, shm, bmom + 4 * blockIdx.x);
 }
 
-// one workgroup: bcount[0..nb) -> exclusive offsets, the sum into *total;
-// the workgroups' moments bmom[0..nb) into bmom[nb]
+// one workgroup: bcount[0..nb) -> exclusive offsets; the sums, the
+// workgroups' moments bmom[0..nb) together and the percolation counters to
+// host memory
 __global__ __launch_bounds__(256) void k_compact_scan(uint32_t* __restrict__ bcount, uint32_t nb,
-                                                      uint32_t* __restrict__ total, uint64_t* __restrict__ bmom) {
+                                                      const uint64_t* __restrict__ bmom,
+                                                      const uint32_t* __restrict__ nslot_nperc,
+                                                      ClusterSums* __restrict__ out) {
   __shared__ uint32_t sh[4];
-  __shared__ uint64_t shm[16];
+  __shared__ uint64_t shm[16], sums[4];
   uint32_t run = 0;
   Mom m{0, 0, 0, 0};
   for (uint32_t b0 = 0; b0 < nb; b0 += 256) {
@@ -1299,36 +1333,35 @@ __global__ __launch_bounds__(256) void k_compact_scan(uint32_t* __restrict__ bco
     run += sum;
     __syncthreads();  // sh is reused by the next round
   }
-  if (threadIdx.x == 0) *total = run;
-  mom_block_store(m, shm, bmom + 4 * nb);
+  mom_block_store(m, shm, sums);
+  if (threadIdx.x == 0) {
+    out->sum = sums[0];
+    out->squares = sums[1];
+    out->largest = (uint32_t)sums[2];
+    out->second = (uint32_t)(sums[2] >> 32);
+    out->clusters = run;
+    out->slots = nslot_nperc[0];
+    out->percolating = nslot_nperc[1];
+  }
 }
 
-__global__ __launch_bounds__(256) void k_compact_write(const int32_t* __restrict__ size, uint32_t nn,
+__global__ __launch_bounds__(256) void k_compact_write(const uint32_t* __restrict__ label,
+                                                       const int32_t* __restrict__ others, uint32_t nn,
                                                        const uint32_t* __restrict__ boff, int32_t* __restrict__ out) {
   __shared__ uint32_t sh[4];
-  const uint32_t base = blockIdx.x * kCompactSpan + threadIdx.x * 4;
-  int32_t v[4];
-  uint32_t c = 0;
+  uint32_t at = boff[blockIdx.x];
+  for (uint32_t r = 0; r < kCompactSpan; r += 1024) {
+    uint32_t v[4], c = 0;
+    root_sizes(label, others, nn, blockIdx.x * kCompactSpan + r + threadIdx.x * 4, v);
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
-    v[k] = base + k < nn ? size[base + k] : 0;
-    c += v[k] != 0;
-  }
-  uint32_t total;
-  uint32_t pos = boff[blockIdx.x] + block_excl_scan256(c, sh, &total);
+    for (uint32_t k = 0; k < 4; ++k) c += v[k] != 0;
+    uint32_t total;
+    uint32_t pos = at + block_excl_scan256(c, sh, &total);
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k)
-    if (v[k]) out[pos++] = v[k];
-}
-
-__global__ void k_perc_slots(const uint32_t* __restrict__ label, uint32_t nn,
-                             const int32_t* __restrict__ size, int32_t minsize,
-                             int32_t* __restrict__ slot, uint32_t* __restrict__ nslot,
-                             uint32_t max_slots) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nn && label[i] == i && size[i] >= minsize) {
-    const uint32_t s = atomicAdd(nslot, 1u);
-    slot[i] = s < max_slots ? (int32_t)s : -1;
+    for (uint32_t k = 0; k < 4; ++k)
+      if (v[k]) out[pos++] = (int32_t)v[k];
+    at += total;
+    __syncthreads();  // sh is reused by the next round
   }
 }
 
@@ -1339,14 +1372,16 @@ __global__ void k_perc_slots(const uint32_t* __restrict__ label, uint32_t nn,
 // (segmented butterfly over the wavefront) and its first lane makes three
 // atomics.
 __global__ __launch_bounds__(256) void k_perc_cover(const uint32_t* __restrict__ label, uint32_t nn, uint32_t L,
-                                                    const int32_t* __restrict__ size, int32_t minsize,
-                                                    const int32_t* __restrict__ slot, uint32_t* __restrict__ cover,
+                                                    const int32_t* __restrict__ others, uint32_t minsize,
+                                                    const int32_t* __restrict__ slot,
+                                                    const uint32_t* __restrict__ nslot, uint32_t* __restrict__ cover,
                                                     uint32_t max_slots) {
+  if (*nslot == 0) return;  // no cluster is large enough (uniform over the grid)
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
   uint32_t key = 0xFFFFFFFFu, bx = 0, by = 0, bz = 0, x = 0, y = 0, z = 0;
   if (i < nn) {
     const uint32_t r = label[i];
-    const int32_t s = size[r] >= minsize ? slot[r] : -1;
+    const int32_t s = 1u + (uint32_t)others[r] >= minsize ? slot[r] : -1;
     if (s >= 0 && (uint32_t)s < max_slots) {
       const uint32_t N = L * L * L;
       const uint32_t cell = i % N;
@@ -1634,28 +1669,27 @@ void launch_sigma_hist_slot(hipStream_t st, const uint32_t* W, uint32_t N, unsig
                             const uint64_t* gstep, uint32_t step_off, const uint64_t* base, uint32_t span) {
   launch(k_sigma_hist, hist_grid(N), dim3(256), st, W, N, series, gstep, step_off, base, span);
 }
-void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* size) {
-  launch(k_cluster_sizes, grid1(nn, 256), dim3(256), st, label, nn, size);
+void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* others) {
+  launch(k_cluster_sizes, grid1(nn, 256), dim3(256), st, label, nn, others);
 }
 uint32_t compact_blocks(uint32_t nn) { return (nn + kCompactSpan - 1) / kCompactSpan; }
-void launch_compact_count(hipStream_t st, const int32_t* size, uint32_t nn, uint32_t* bcount, uint32_t* total,
-                          uint64_t* bmom) {
-  const uint32_t nb = compact_blocks(nn);
-  launch(k_compact_count, dim3(nb), dim3(256), st, size, nn, bcount, bmom);
-  launch(k_compact_scan, dim3(1), dim3(256), st, bcount, nb, total, bmom);
+void launch_compact_count(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn, uint32_t* bcount,
+                          uint64_t* bmom, uint32_t minsize, int32_t* slot, uint32_t* nslot, uint32_t max_slots) {
+  launch(k_compact_count, dim3(compact_blocks(nn)), dim3(256), st, label, others, nn, bcount, bmom, minsize, slot,
+         nslot, max_slots);
 }
-void launch_compact_write(hipStream_t st, const int32_t* size, uint32_t nn, const uint32_t* bcount, int32_t* out) {
-  launch(k_compact_write, dim3(compact_blocks(nn)), dim3(256), st, size, nn, bcount, out);
+void launch_compact_scan(hipStream_t st, uint32_t* bcount, uint32_t nn, const uint64_t* bmom,
+                         const uint32_t* nslot_nperc, ClusterSums* out) {
+  launch(k_compact_scan, dim3(1), dim3(256), st, bcount, compact_blocks(nn), bmom, nslot_nperc, out);
 }
-void launch_perc_slots(hipStream_t st, const uint32_t* label, uint32_t nn, const int32_t* size,
-                       int32_t minsize, int32_t* slot, uint32_t* nslot, uint32_t max_slots) {
-  launch(k_perc_slots, grid1(nn, 256), dim3(256), st, label, nn, size, minsize, slot, nslot, max_slots);
+void launch_compact_write(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn,
+                          const uint32_t* bcount, int32_t* out) {
+  launch(k_compact_write, dim3(compact_blocks(nn)), dim3(256), st, label, others, nn, bcount, out);
 }
-void launch_perc_cover(hipStream_t st, const uint32_t* label, uint32_t nn, uint32_t L,
-                       const int32_t* size, int32_t minsize, const int32_t* slot, uint32_t* cover,
+void launch_perc_cover(hipStream_t st, const uint32_t* label, uint32_t nn, uint32_t L, const int32_t* others,
+                       uint32_t minsize, const int32_t* slot, const uint32_t* nslot, uint32_t* cover,
                        uint32_t max_slots) {
-  launch(k_perc_cover, grid1(nn, 256), dim3(256), st, label, nn, L, size, minsize, slot, cover,
-         max_slots);
+  launch(k_perc_cover, grid1(nn, 256), dim3(256), st, label, nn, L, others, minsize, slot, nslot, cover, max_slots);
 }
 void launch_perc_count(hipStream_t st, const uint32_t* cover, const uint32_t* nslot, uint32_t L,
                        uint32_t max_slots, uint32_t* nperc) {
