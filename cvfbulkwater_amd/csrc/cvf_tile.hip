@@ -89,7 +89,6 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   __shared__ uint32_t thr_s[33];
   __shared__ uint64_t thr_e[9];
   __shared__ uint64_t etab[9];
-  __shared__ uint32_t sch[kMaxChunk];
   // per axis and window position: its share of the quad's site (of its cube's
   // index), the exchange in the top bits
   __shared__ uint32_t site_t[3][kMaxTileWin], cube_t[3][kMaxTileWin];
@@ -108,11 +107,14 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   if (tid <= kMaxTileWin) magic[tid] = tid <= 1 ? 0u : 0xFFFFFFFFu / tid + 1u;
   const uint64_t step = *stepp + step_off;
   const uint64_t seed = ((uint64_t)e.seed_hi << 32) | e.seed_lo;
-  if (tid < nk) {
-    const U4 r = draw(seed, kStSched, 0, step, k0 + tid);
-    sch[tid] = uniform_int(r.x, 6) | (((r.y >> 31) ? 0u : 1u) << 3);  // arm, kept parity
+  // the launch's half-sweeps in lanes 0 .. nk - 1 of every wavefront (arm | kept
+  // parity << 3), so that no wavefront waits for another's draws
+  uint32_t sch;
+  {
+    const U4 r = draw(seed, kStSched, 0, step, k0 + (tid & 63u));
+    sch = uniform_int(r.x, 6) | (((r.y >> 31) ? 0u : 1u) << 3);
   }
-  __syncthreads();
+  const auto entry = [&](uint32_t k) { return (uint32_t)__builtin_amdgcn_readlane((int)sch, (int)k); };
   const int L = (int)e.L, hL = L / 2;
   const int org[3] = {(int)e.x0, (int)e.y0, (int)e.z0};
   const bool nc = kAnyNc && e.nc != 0;
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   int lo[3] = {0, 0, 0}, hi[3] = {(int)e.tx, (int)e.ty, (int)e.tz};
   uint32_t grow_lo = 0, grow_hi = 0;
   for (int k = (int)nk - 1; k >= 0; --k) {
-    const uint32_t s = uni(sch[k]), arm = s & 7u, q = s >> 3, down = arm & 1u;
+    const uint32_t s = entry((uint32_t)k), arm = s & 7u, q = s >> 3, down = arm & 1u;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
       if (a == (int)(arm >> 1)) {
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
     }
   }
   for (uint32_t k = 0; k < nk; ++k) {
-    const uint32_t sk = uni(sch[k]), q = sk >> 3;
+    const uint32_t sk = entry(k), q = sk >> 3;
     const int arm = (int)(sk & 7u), ax = arm >> 1;
     uint32_t f[3], cnt[3];
 #pragma unroll
