@@ -2519,6 +2519,7 @@ extern "C" int cvf_autotune(cvf_sim* s, int32_t steps_per_trial, cvf_tuning* cho
   // candidates
   std::vector<cvf_tuning> cand;
   const cvf_tuning base = default_tuning(s);
+  cand.push_back(base);
   for (int streams : {1, 2, 4}) {
     if (streams > s->npts) continue;
     if (s->sched == CVF_SCHED_FAST) {
