@@ -248,6 +248,9 @@ struct cvf_reweight {
   DMem<RwMixed> mix;
   DMem<uint32_t> plow, low;
   DMem<RwSim> sims;
+  bool tables_fit = false;  // the sweeps' exponentials come from tables (RwTables), allocated by the first solve
+  DMem<double> th, tkt;
+  DMem<double2> trow, tcol, tsc;
   int32_t cap_t = 0, n_t = 0;
   size_t cap_dens = 0;
   HMem<double> dist;  // [target][cell] densities of the last reweighting (pinned)
@@ -292,6 +295,33 @@ struct cvf_reweight {
     HIPR(lz.alloc(n));
     HIPR(norm.alloc(n));
     cap_t = n;
+    return CVF_OK;
+  }
+
+  RwTables tables() const { return RwTables{trow.p, tcol.p, tsc.p, tkt.p, th.p, dcell.p, nb}; }
+  // Whether the simulations are few and near enough to each other, and the
+  // histograms far enough from the ends of a double's range: kRwMaxShift,
+  // kRwMaxLogHist.
+  bool tables_apply(const std::vector<RwSim>& s, const std::vector<double>& lh) const {
+    if (n_sim < 2 || n_sim > kRwRow || !(rho_min > 0)) return false;
+    const auto bounds = std::minmax_element(lh.begin(), lh.end());
+    if (!(*bounds.first >= -kRwMaxLogHist && *bounds.second <= kRwMaxLogHist)) return false;
+    const auto volume = [&](int k) { return sl(0.018f) / (rho_min + ((k + 1) - 0.5) * drho) * N; };
+    const double dE = (0.5 * nb + 1) * de * N, v0 = volume(nb / 2);
+    const double dV = std::max(fabs(volume(0) - v0), fabs(volume(nb - 1) - v0));
+    for (const RwSim& q : s) {
+      const double x = fabs(q.beta - s[0].beta) * dE + fabs(q.beta * q.pres - s[0].beta * s[0].pres) * dV;
+      if (!(x <= kRwMaxShift)) return false;
+    }
+    return true;
+  }
+  int reserve_tables() {
+    if (tkt.p) return CVF_OK;
+    HIPR(trow.alloc((size_t)(n_sim + 1) / 2 * nb));
+    HIPR(tcol.alloc((size_t)(n_sim + 1) / 2 * nb));
+    HIPR(th.alloc(cell.size()));
+    HIPR(tsc.alloc(n_sim));
+    HIPR(tkt.alloc(3 * kRwRow));
     return CVF_OK;
   }
 
@@ -472,6 +502,7 @@ int cvf_rw_create(int32_t L, int32_t n_sim, const double* T_hat, const double* P
   HIPR(hipMemcpy(rw->vn.p, hvn.data(), nc * sizeof(double), hipMemcpyHostToDevice));
   HIPR(hipMemcpy(rw->lh.p, hlh.data(), nc * sizeof(double), hipMemcpyHostToDevice));
   HIPR(hipMemcpy(rw->sims.p, hs.data(), n_sim * sizeof(RwSim), hipMemcpyHostToDevice));
+  rw->tables_fit = rw->tables_apply(hs, hlh);
   *out = rw.release();
   return CVF_OK;
 }
@@ -508,9 +539,18 @@ int cvf_rw_solve_constants(cvf_reweight* rw, int32_t steps, double* ctes, double
   // first launch takes its constants from the partial sums of the one before
   if (int rc = rw->upload_inputs(nullptr, rw->n_sim, rw->T.data(), rw->P.data())) return rc;
   const RwTargets tg = rw->targets(rw->n_sim);
+  const bool tables = rw->tables_fit && steps > 0;
+  if (tables) {
+    if (int rc = rw->reserve_tables()) return rc;
+    HIPR(launch_rw_tables(rw->cells(), rw->sims.p, rw->n_sim, rw->geom(), rw->N, rw->tables(), rw->stream));
+  }
   for (int s = 0; s < steps; ++s)
-    HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), rw->geom(), kRwSweep,
-                        s > 0, rw->used.p, rw->stream));
+    if (tables)
+      HIPR(launch_rw_sweep(rw->tables(), (int64_t)rw->cell.size(), rw->n_sim, rw->work(tg.n), s > 0, rw->used.p,
+                           rw->stream));
+    else
+      HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), rw->geom(), kRwSweep,
+                          s > 0, rw->used.p, rw->stream));
   std::vector<double> z(rw->n_sim, 0.0), prev(rw->n_sim, 0.0);
   if (steps > 0) {
     HIPR(launch_rw_finish(tg, rw->work(tg.n), rw->geom(), kRwSweep, nullptr, rw->stream));

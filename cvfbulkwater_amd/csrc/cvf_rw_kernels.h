@@ -55,6 +55,23 @@ struct RwWork {
   int32_t rows, nblk, threads;  // rows of targets; launch shape (rw_shape)
 };
 
+// What the sweeps of the constants take from tables instead of exponentials.
+// With x_j(c) = -(beta_j - beta_0)(E - E0) - (beta_j p_j - beta_0 p_0)(V - V0),
+// E0 and V0 of the grid's middle, exp(x_j) is a factor of the cell's energy row
+// times one of its density column, and exp(u_j) = exp(x_j + w_j - t1_0) with
+// w_j = lm_j - g_j - c_j the same for all cells.
+struct RwTables {
+  double2 *row, *col;    // [pair of simulations][nb]
+  double2* sc;           // [simulation]: g_j = (beta_j - beta_0) E0 + (beta_j p_j - beta_0 p_0) V0, and lm_j
+  double* kt;            // [3][kRwRow] of a sweep: g_t + max w, and the bounds of the cut (k_rw_sweep_cells)
+  double* h;             // [cell]: summed normalized histograms
+  const uint32_t* cell;  // i << 16 | w
+  int32_t nb;
+};
+// The largest |x_j| that the tables serve, and the largest |log| of a cell's
+// histogram: no product or quotient of a sweep leaves the range of a double.
+constexpr double kRwMaxShift = 150, kRwMaxLogHist = 100;
+
 // Grid geometry for the projections: cell = i << 16 | w (nb < 2^16), energy
 // e_min + (i + 1/2) de (kJ/mol), density rho_min + (w + 1/2) drho (kg/m^3).
 struct RwGeom {
@@ -95,6 +112,12 @@ void rw_shape(int64_t n_cells, int32_t n_targets, RwWork* w);
 hipError_t launch_rw_pass(const RwCells& cells, const RwSim* sims, const double* ctes, int32_t n_sim,
                           const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, bool chain, double* used,
                           hipStream_t stream);
+// The tables of n_sim simulations (2 .. kRwRow) for molecules N, and a sweep
+// with them: chain as above, else from constants of zero.
+hipError_t launch_rw_tables(const RwCells& cells, const RwSim* sims, int32_t n_sim, const RwGeom& g, int32_t N,
+                            const RwTables& tb, hipStream_t st);
+hipError_t launch_rw_sweep(const RwTables& tb, int64_t n_cells, int32_t n_sim, const RwWork& w, bool chain,
+                           double* used, hipStream_t st);
 // log_Z, norm and (kRwScan) the Binder cumulants {energy, density} per target
 hipError_t launch_rw_finish(const RwTargets& tg, const RwWork& w, const RwGeom& g, int mode, double* binder_ed,
                             hipStream_t st);

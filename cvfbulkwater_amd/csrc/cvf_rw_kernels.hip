@@ -567,6 +567,237 @@ __global__ __launch_bounds__(64) void k_rw_finish(RwWork w, double de, double dr
   }
 }
 
+// ------------------------------------------------- sweeps of the constants
+// The tables of a solve (RwTables), the cells' histograms among them.
+__global__ __launch_bounds__(256) void k_rw_tables(RwCells cells, const RwSim* __restrict__ sims, int32_t n_sim,
+                                                   RwGeom g, int32_t N, RwTables tb) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < cells.n) {
+    tb.h[i] = exp(cells.lh[i]);
+    return;
+  }
+  i -= cells.n;
+  const auto energy = [&](int k) { return (g.e_min + ((k + 1) - 0.5) * g.de) * N; };
+  const auto volume = [&](int k) { return (double)0.018f / (g.rho_min + ((k + 1) - 0.5) * g.drho) * N; };
+  const double e0 = energy(g.nb / 2), v0 = volume(g.nb / 2);
+  const int64_t per = 2 * (int64_t)g.nb;
+  if (i >= n_sim * (per + 1)) return;
+  const int j = (int)(i / (per + 1)), k = (int)(i - j * (per + 1));
+  // beta p to twice the digits: the product's rounding would be the same in
+  // every cell
+  const double b0 = sims[0].beta, p0 = sims[0].pres, b = sims[j].beta, p = sims[j].pres;
+  const double q0 = b0 * p0, q = b * p;
+  const double db = b - b0, dq = (q - q0) + (__builtin_fma(b, p, -q) - __builtin_fma(b0, p0, -q0));
+  const auto put = [&](double2* t, int at, double x) {
+    (&t[(size_t)(j / 2) * g.nb + at].x)[j & 1] = exp(x);
+  };
+  if (k < g.nb)
+    put(tb.row, k, -(db * (energy(k) - e0)));
+  else if (k < per)
+    put(tb.col, k - g.nb, -(dq * (volume(k - g.nb) - v0)));
+  else
+    tb.sc[j] = double2{db * e0 + dq * v0, sims[j].lm};
+}
+
+constexpr double kExpM10 = 0x1.7cd79b5647c9bp-15;  // e^-10: the cut-offs of both sums
+
+template <int N>
+constexpr int kPad = N <= 2 ? 2 : N <= 4 ? 4 : N <= 8 ? 8 : 16;
+
+// exp(x_j) of a cell for each of N simulations, two to a load: a gather costs
+// by its lanes, not its bytes.
+template <int N>
+__device__ inline void cell_shifts(const RwTables& tb, uint32_t c, double (&D)[N]) {
+  const double2 *row = tb.row + (c >> 16), *col = tb.col + (c & 0xFFFFu);
+#pragma unroll
+  for (int j = 0; j < N; j += 2) {
+    const double2 r = row[(size_t)(j / 2 * tb.nb)], q = col[(size_t)(j / 2 * tb.nb)];
+    D[j] = r.x * q.x;
+    if (j + 1 < N) D[j + 1] = r.y * q.y;
+  }
+}
+
+// A sweep's first launch, as k_rw_cells, on the tables: with D_j = exp(x_j)
+// and W_j = exp(w_j - max w) a cell's terms are W_j D_j, its sum S over them
+// (all, or those above e^-10 of the largest) gives R = h / S, and exp(log_P)
+// of target t is R D_t exp(-(g_t + max w)), whose last factor no cell needs.
+// The targets are the simulations, so every D_j serves twice and a cell costs
+// N gathers of 16 bytes from tables in the L2s, a quotient and about 6 N FP64
+// instructions, instead of N exponentials here and N more in k_rw_sum.  The
+// exponents are differences between simulations, of order 1 to 100 where
+// beta E is 10^5: against 80-bit arithmetic (6 simulations, 24,000 cells, 15
+// sweeps) the constants are 3.5e-14 off, 1.1e-11 with exponentials.
+// Bound by the gathers (one value at a time, twice as many: 27.0 us a sweep)
+// and, for few cells, by the launches and their reductions.  A sweep of 11
+// simulations and 710,000 cells 41.8 -> 22.6 us; 5 and 31,000 14.1 -> 9.3;
+// 12 and 122,000 22.5 -> 11.8; 2 and 2,700 10.6 -> 8.2.  (In squares of 32 x 32
+// cells a wavefront's gathers share lines: 21.4 us, for a sort on the host
+// that costs more than a solve gains.)
+// Stores R, negative where the cell's targets use different sums (mix[cell]:
+// h / near, h / all, largest and smallest term).
+template <int N>
+__global__ __launch_bounds__(1024) void k_rw_sweep_cells(RwTables tb, int64_t n, RwWork w,
+                                                         const double* __restrict__ ps, double* __restrict__ used) {
+  constexpr int P = kPad<N>;
+  __shared__ double red[16][16];
+  __shared__ double lz[16], W[N], cut_hi[N], cut_lo[N];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t lanes = (int64_t)gridDim.x * blockDim.x, b0 = first_cell();
+  uint32_t cn = 0;
+  double hn = 0;
+  if (b0 < n) cn = tb.cell[b0], hn = tb.h[b0];
+  if (ps) {
+    const double m = w.mx[min((int)(threadIdx.x >> 2), N - 1)];
+    reduce_partials<P, false>(ps, w.nblk, red, [&](int k, double st) {
+      if (k < N) lz[k] = (st != 0 ? log(st) : 0.0) + m;
+    });
+    __syncthreads();
+  }
+  if (wave == 0) {
+    const int k = min(lane, N - 1);
+    const double c = ps ? lz[k] - lz[0] : 0.0;
+    const double2 s = tb.sc[k];
+    const double wk = (s.y - s.x) - c, top = wave_max(wk), K = s.x + top;
+    if (lane < N) {
+      // arg_j of target t is log(W_j D_j) + K_t - x_t: above 10 where
+      // W_j D_j > D_t exp(10 - K_t), below -10 where less than
+      // D_t exp(-10 - K_t).  (Beyond 700 the comparison with any term has the
+      // result that it has at 700: |x| <= kRwMaxShift, and the largest W is 1.)
+      const double hi = exp(fmin(fmax(10.0 - K, -700.0), 700.0)), lo = exp(fmin(fmax(-10.0 - K, -700.0), 700.0));
+      W[k] = exp(wk - top);
+      cut_hi[k] = hi;
+      cut_lo[k] = lo;
+      if (blockIdx.x == 0) {
+        used[k] = c;
+        tb.kt[k] = K;
+        tb.kt[kRwRow + k] = hi;
+        tb.kt[2 * kRwRow + k] = lo;
+      }
+    }
+  }
+  __syncthreads();
+  double top[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) top[k] = 0;
+  for (int64_t b = b0; b < n; b += lanes) {
+    const uint32_t c = cn;
+    const double h = hn;
+    if (b + lanes < n) cn = tb.cell[b + lanes], hn = tb.h[b + lanes];
+    double D[N];
+    cell_shifts<N>(tb, c, D);
+    const double* Wp = W + opaque_zero();
+    double M = 0, m = INFINITY, all = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const double t = D[j] * Wp[j];
+      M = max1(M, t);
+      m = min1(m, t);
+      all = all + t;
+    }
+    double S = all, near = all;
+    bool mixed = false;
+    const bool split = !(m > M * kExpM10);  // the sums differ
+    if (__ballot(split)) {
+      near = 0;
+      bool any_cut = false, any_all = false;
+      const double *hi = cut_hi + opaque_zero(), *lo = cut_lo + opaque_zero();
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const double t = D[j] * Wp[j];
+        if (t > M * kExpM10) near = near + t;
+        const bool cut = M > D[j] * hi[j] || m < D[j] * lo[j];
+        any_cut = any_cut || cut;
+        any_all = any_all || !cut;
+      }
+      S = any_cut ? near : all;
+      mixed = split && any_cut && any_all;
+    }
+    const double R = h / S;
+    if (__ballot(mixed)) {
+      const double Ra = h / all;
+      const double *hi = cut_hi + opaque_zero(), *lo = cut_lo + opaque_zero();
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const bool cut = M > D[k] * hi[k] || m < D[k] * lo[k];
+        top[k] = max1(top[k], D[k] * (!mixed || cut ? R : Ra));
+      }
+      if (mixed) w.mix[b] = RwMixed{R, Ra, M, m};
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; ++k) top[k] = max1(top[k], D[k] * R);
+    }
+    w.sum[b] = mixed ? -R : R;
+  }
+  wave_reduce<P, true>(top);
+  if (reduced_first<P>()) red[reduced_index<P>()][wave] = top[0];
+  __syncthreads();
+  if ((int)threadIdx.x < 4 * P) {
+    const double m = combine_waves<true>(red);
+    const int k = threadIdx.x >> 2;
+    if ((threadIdx.x & 3) == 0 && k < N) w.pmax[(int64_t)blockIdx.x * kRwRow + k] = m;
+  }
+}
+
+// Its second launch: per target the sum of R D_t over the cells within e^-10
+// of the largest; w.mx takes log of the factor left out.
+template <int N>
+__global__ __launch_bounds__(1024) void k_rw_sweep_sum(RwTables tb, int64_t n, RwWork w) {
+  constexpr int P = kPad<N>;
+  __shared__ double red[16][16];
+  __shared__ double low[N], cut_hi[N], cut_lo[N];
+  const int wave = threadIdx.x >> 6;
+  const int64_t lanes = (int64_t)gridDim.x * blockDim.x, b0 = first_cell();
+  uint32_t cn = 0;
+  double rn = 0;
+  if (b0 < n) cn = tb.cell[b0], rn = w.sum[b0];
+  if ((int)threadIdx.x < N) {
+    cut_hi[threadIdx.x] = tb.kt[kRwRow + threadIdx.x];
+    cut_lo[threadIdx.x] = tb.kt[2 * kRwRow + threadIdx.x];
+    if (blockIdx.x == 0) w.mx[threadIdx.x] = -tb.kt[threadIdx.x];
+  }
+  reduce_partials<P, true>(w.pmax, w.nblk, red, [&](int k, double m) {
+    if (k < N) low[k] = m * kExpM10;
+  });
+  __syncthreads();
+  double s[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) s[k] = 0;
+  for (int64_t b = b0; b < n; b += lanes) {
+    const uint32_t c = cn;
+    const double R = rn;
+    if (b + lanes < n) cn = tb.cell[b + lanes], rn = w.sum[b + lanes];
+    double D[N];
+    cell_shifts<N>(tb, c, D);
+    const double* lp = low + opaque_zero();
+    if (__ballot(R < 0)) {
+      const bool mixed = R < 0;
+      RwMixed m{R, R, 0, 0};
+      if (mixed) m = w.mix[b];
+      const double *hi = cut_hi + opaque_zero(), *lo = cut_lo + opaque_zero();
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const bool cut = m.umax > D[k] * hi[k] || m.umin < D[k] * lo[k];
+        const double x = D[k] * (cut ? m.near : m.all);
+        if (x > lp[k]) s[k] = s[k] + x;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const double x = D[k] * R;
+        if (x > lp[k]) s[k] = s[k] + x;
+      }
+    }
+  }
+  wave_reduce<P, false>(s);
+  if (reduced_first<P>()) red[reduced_index<P>()][wave] = s[0];
+  __syncthreads();
+  if ((int)threadIdx.x < 4 * P) {
+    const double x = combine_waves<false>(red);
+    const int k = threadIdx.x >> 2;
+    if ((threadIdx.x & 3) == 0 && k < N) w.ps[(int64_t)blockIdx.x * kRwRow + k] = x;
+  }
+}
+
 // densities exp(log_P - log_Z) / norm, one target per blockIdx.y
 __global__ __launch_bounds__(kRwBlock) void k_rw_dist(RwCells cells, RwTargets tg, RwWork w,
                                                       double* __restrict__ dens) {
@@ -947,6 +1178,16 @@ void sum_launch(const RwCells& cells, const RwTargets& tg, const RwWork& w, cons
                      st, cells, tg, w, g);
 }
 
+template <int N>
+void sweep_launch(const RwTables& tb, int64_t n, int32_t n_sim, const RwWork& w, bool chain, double* used,
+                  hipStream_t st) {
+  if constexpr (N < kRwRow)
+    if (n_sim > N) return sweep_launch<N + 1>(tb, n, n_sim, w, chain, used, st);
+  hipLaunchKernelGGL(k_rw_sweep_cells<N>, dim3((unsigned)w.nblk), dim3(w.threads), 0, st, tb, n, w,
+                     chain ? w.ps : nullptr, used);
+  hipLaunchKernelGGL(k_rw_sweep_sum<N>, dim3((unsigned)w.nblk), dim3(w.threads), 0, st, tb, n, w);
+}
+
 template <int NA>
 hipError_t xhist_launch(const RwGeom& g, const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwScan& sc,
                         hipStream_t st) {
@@ -1002,6 +1243,20 @@ hipError_t launch_rw_pass(const RwCells& cells, const RwSim* sims, const double*
     sum_launch<8, kRwDensity>(cells, tg, w, g, stream);
   else
     sum_launch<4, kRwScan>(cells, tg, w, g, stream);
+  return hipGetLastError();
+}
+
+hipError_t launch_rw_tables(const RwCells& cells, const RwSim* sims, int32_t n_sim, const RwGeom& g, int32_t N,
+                            const RwTables& tb, hipStream_t st) {
+  const int64_t items = cells.n + n_sim * (2 * (int64_t)g.nb + 1);
+  hipLaunchKernelGGL(k_rw_tables, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, cells, sims, n_sim, g, N,
+                     tb);
+  return hipGetLastError();
+}
+
+hipError_t launch_rw_sweep(const RwTables& tb, int64_t n_cells, int32_t n_sim, const RwWork& w, bool chain,
+                           double* used, hipStream_t st) {
+  sweep_launch<2>(tb, n_cells, n_sim, w, chain, used, st);
   return hipGetLastError();
 }
 
