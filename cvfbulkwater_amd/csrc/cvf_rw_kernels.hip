@@ -6,8 +6,8 @@
 // The reference's argument for cell c, target t and simulation j is
 //   arg_j = beta_t (E + p_t V) - beta_j (E + p_j V) - c_j + lm_j = t1 + u_j,
 // so the target only shifts a cell's sum: log sum_j exp(arg_j) =
-// t1 + log sum_j exp(u_j).  k_rw_logp evaluates the n_sim terms u_j once
-// per cell and then serves every target of its block with a few flops.
+// t1 + log sum_j exp(u_j).  k_rw_cells evaluates the n_sim terms u_j once
+// per cell and then serves every target of its row with a few flops.
 // The reference's two cut-offs are kept exactly:
 //  - a cell's sum switches to the max-shifted form that drops terms more
 //    than 10 below the largest once any |arg_j| > 10 (f90:1048-1078); the
@@ -22,7 +22,8 @@
 // pass forms it again from 33 bytes per cell (which stay in the caches)
 // instead of writing and reading 8 bytes per cell and target.  At the
 // production shape (710,000 cells, 11 simulations) a constants' sweep went
-// from three launches of 31.8 + 17.8 + 6.0 us to two of 26.0 + 17.7, and a
+// from three launches of 31.8 + 17.8 + 6.0 us to two of 26.0 + 17.7 (the sweeps
+// of few, near simulations now multiply tables, see k_rw_sweep_cells), and a
 // scan of 64 targets x 3 angles from 1.17 ms of kernels over 363 MB of
 // densities to 0.57 ms.
 #include <math.h>
