@@ -264,6 +264,7 @@ struct cvf_reweight {
   DMem<uint32_t> scode, scbin;
   HMem<double> sout;
   int32_t cap_pairs = 0, cap_angles = 0;
+  size_t cap_parts = 0;
 
   RwCells cells() const { return RwCells{en.p, vn.p, lh.p, (int64_t)cell.size()}; }
   RwWork work(int32_t n) const {
@@ -693,16 +694,22 @@ int cvf_rw_scan(cvf_reweight* rw, int32_t n_targets, const double* T_K, const do
   if (nta > rw->cap_pairs || n_angles > rw->cap_angles) {
     const size_t pairs = (size_t)std::max(nta, rw->cap_pairs), ang = (size_t)std::max(n_angles, rw->cap_angles);
     rw->cap_pairs = rw->cap_angles = 0;
-    HIPR(rw->srange.alloc((ang + pairs) * kRwProjBlocks));
     HIPR(rw->sbin.alloc(pairs + ang));
     HIPR(rw->scbin.alloc(ang * rw->cell.size()));  // at most a group per angle
-    HIPR(rw->shist.alloc(pairs * kRwProjBlocks * nm));
     HIPR(rw->scode.alloc(pairs));
     // 2 cumulants per target (at most one target per pair), 2 nm + 9 numbers
     // and a code per pair
     HIPR(rw->sout.resize(pairs * (2 * (size_t)nm + 12)));
     rw->cap_pairs = (int32_t)pairs;
     rw->cap_angles = (int32_t)ang;
+  }
+  const int32_t n_proj = rw_proj_blocks((int64_t)rw->cell.size(), n_targets);
+  const size_t parts = (size_t)(nta + n_angles) * n_proj;
+  if (parts > rw->cap_parts) {
+    rw->cap_parts = 0;
+    HIPR(rw->srange.alloc(parts));
+    HIPR(rw->shist.alloc(parts * nm));
+    rw->cap_parts = parts;
   }
   if (int rc = rw->upload_inputs(rw->ctes.data(), n_targets, T_K, P_bar, n_angles, alpha)) return rc;
   const RwTargets tg = rw->targets(n_targets);
@@ -718,7 +725,7 @@ int cvf_rw_scan(cvf_reweight* rw, int32_t n_targets, const double* T_K, const do
                       rw->stream));
   HIPR(launch_rw_finish(tg, rw->work(tg.n), g, kRwScan, out.binder_ed, rw->stream));
   const RwScan sc{rw->dev_angles(n_targets), n_angles, rw->srange.p, rw->sbin.p + n_angles, rw->sbin.p,
-                  rw->scbin.p, rw->shist.p, rw->scode.p};
+                  rw->scbin.p, rw->shist.p, rw->scode.p, n_proj};
   double peak2d, peak3d;
   ising_peaks(&peak2d, &peak3d);
   HIPR(launch_rw_project(rw->cells(), tg, rw->work(tg.n), g, sc, peak2d, peak3d, out, rw->stream));

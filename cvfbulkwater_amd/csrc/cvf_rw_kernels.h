@@ -10,7 +10,7 @@ namespace cvf {
 
 constexpr int kRwBlock = 256;
 constexpr int kRwRow = 16;          // targets that share one pass over the cells' simulation sums
-constexpr int kRwProjBlocks = 64;   // workgroups per target (or pair) of a projection
+constexpr int kRwProjBlocks = 64;   // the fewest workgroups per target (or pair) of a projection
 // what a pass is for: a sweep of the constants (log_Z alone), densities
 // (and the normalization), a scan (and the moments of the marginals)
 enum { kRwSweep = 0, kRwDensity = 1, kRwScan = 2 };
@@ -85,13 +85,19 @@ struct RwGeom {
 struct RwScan {
   const double2* angle;  // (sin, cos) per angle
   int32_t n_a;
-  double2* range;  // [n_a + pairs][kRwProjBlocks]: min and max of x
+  double2* range;  // [n_a + pairs][n_proj]: min and max of x
   double2* bin;    // [pair]: first bin's lower edge, bin width
   double2* gbin;   // [n_a]: the same over all the grid's cells
   uint32_t* cbin;  // [group of up to 4 angles][cell]: the cell's bins, a byte per angle
-  double* hist;    // [pair][kRwProjBlocks][nm]
+  double* hist;    // [pair][n_proj][nm]
   uint32_t* code;  // [pair]: kRwNoCell, kRwOutside
+  int32_t n_proj;  // workgroups per target (or pair) of a projection
 };
+// As many workgroups per target as fill the card with histograms (one
+// wavefront each, seven on a CU), a thousand cells each at least; 64 of them
+// left most CUs idle for a few targets.  One angle, 710,000 cells, 1 / 5 / 10 / 16
+// targets: 64 workgroups 217 / 235 / 248 / 262 us, so many 131 / 150 / 178 / 210.
+int32_t rw_proj_blocks(int64_t n_cells, int32_t n_targets);
 // What went wrong with a pair: no cell of positive density, an x outside its
 // bins, moments off before or after the axis stretch.
 enum : uint32_t { kRwNoCell = 1, kRwOutside = 2, kRwMoments = 4, kRwStretched = 8 };

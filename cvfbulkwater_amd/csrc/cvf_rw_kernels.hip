@@ -545,17 +545,18 @@ __global__ __launch_bounds__(64) void k_rw_finish(RwWork w, double de, double dr
   const int t = blockIdx.x, lane = threadIdx.x;
   double s[V];
 #pragma unroll
-  for (int v = 0; v < V; ++v) {
-    const double* p = w.ps + ((int64_t)v * w.rows + t / kRwRow) * w.nblk * kRwRow + t % kRwRow;
-    double x = 0;
-    for (int i = lane; i < w.nblk; i += 64) x += p[i * kRwRow];
-    s[v] = wave_sum(x);
-  }
+  for (int v = 0; v < V; ++v) s[v] = 0;
   uint32_t low = 0;
-  if (kMode == kRwScan) {
-    for (int i = lane; i < w.nblk; i += 64) low |= w.plow[(int64_t)t * w.nblk + i];
-    low = __ballot(low != 0) != 0;
+  // (all sums' loads of a round together)
+  for (int i = lane; i < w.nblk; i += 64) {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+      s[v] += w.ps[(((int64_t)v * w.rows + t / kRwRow) * w.nblk + i) * kRwRow + t % kRwRow];
+    if (kMode == kRwScan) low |= w.plow[(int64_t)t * w.nblk + i];
   }
+#pragma unroll
+  for (int v = 0; v < V; ++v) s[v] = wave_sum(s[v]);
+  low = __ballot(low != 0) != 0;
   if (lane) return;
   const double z = (s[0] != 0 ? log(s[0]) : 0.0) + w.mx[t];
   w.lz[t] = z;
@@ -858,9 +859,9 @@ __global__ __launch_bounds__(64) void k_rw_bins(RwWork w, RwScan sc, int32_t nm)
   const bool pair = (int)blockIdx.x >= sc.n_a;
   const int ta = (int)blockIdx.x - sc.n_a, t = pair ? ta / sc.n_a : 0;
   const int at = pair && !w.low[t] ? ta - t * sc.n_a : (int)blockIdx.x;  // whose range
-  const double2* r = sc.range + (int64_t)at * kRwProjBlocks;
+  const double2* r = sc.range + (int64_t)at * sc.n_proj;
   double xmin = (double)1E12f, xmax = (double)-1E12f;
-  for (int i = threadIdx.x; i < kRwProjBlocks; i += 64) {
+  for (int i = threadIdx.x; i < sc.n_proj; i += 64) {
     xmin = fmin(xmin, r[i].x);
     xmax = fmax(xmax, r[i].y);
   }
@@ -1072,7 +1073,8 @@ __global__ __launch_bounds__(64) void k_rw_order(RwScan sc, int32_t nm, double p
     const int k = lane + 64 * i;
     double s = 0;
     if (k < nm)
-      for (int b = 0; b < kRwProjBlocks; ++b) s += sc.hist[((int64_t)ta * kRwProjBlocks + b) * nm + k];
+#pragma unroll 32
+      for (int b = 0; b < sc.n_proj; ++b) s += sc.hist[((int64_t)ta * sc.n_proj + b) * nm + k];
     h.p[i] = s;
     h.x[i] = bin.x + ((k + 1) - 0.5) * bin.y;
     h.w[i] = k < nm ? bin.y : 0.0;
@@ -1201,7 +1203,7 @@ hipError_t xhist_launch(const RwGeom& g, const RwCells& cells, const RwTargets& 
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_rw_xhist<NA>, dim3(kRwProjBlocks, (unsigned)tg.n * groups), dim3(64), lds, st, g,
+  hipLaunchKernelGGL(k_rw_xhist<NA>, dim3((unsigned)sc.n_proj, (unsigned)tg.n * groups), dim3(64), lds, st, g,
                      cells, tg, w, sc);
   return hipGetLastError();
 }
@@ -1275,10 +1277,15 @@ hipError_t launch_rw_dist(const RwCells& cells, const RwTargets& tg, const RwWor
   return hipGetLastError();
 }
 
+int32_t rw_proj_blocks(int64_t n_cells, int32_t n_targets) {
+  const int64_t fill = std::min<int64_t>(1792 / n_targets, n_cells / 1024) / 32 * 32;
+  return (int32_t)std::max<int64_t>(kRwProjBlocks, std::min<int64_t>(kRwMaxBlocks, fill));
+}
+
 hipError_t launch_rw_project(const RwCells& cells, const RwTargets& tg, const RwWork& w, const RwGeom& g,
                              const RwScan& sc, double peak2d, double peak3d, const RwScanOut& out, hipStream_t st) {
   const unsigned nta = (unsigned)(tg.n * sc.n_a);
-  hipLaunchKernelGGL(k_rw_xrange, dim3(kRwProjBlocks, (unsigned)sc.n_a + nta), dim3(kRwBlock), 0, st, g, cells, tg, w,
+  hipLaunchKernelGGL(k_rw_xrange, dim3((unsigned)sc.n_proj, (unsigned)sc.n_a + nta), dim3(kRwBlock), 0, st, g, cells, tg, w,
                      sc);
   hipLaunchKernelGGL(k_rw_bins, dim3((unsigned)sc.n_a + nta), dim3(64), 0, st, w, sc, g.nm);
   // angles per wavefront: as many (up to 4) as keep five wavefronts on a CU
