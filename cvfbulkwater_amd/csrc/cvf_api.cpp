@@ -10,15 +10,13 @@
 #include <string.h>
 
 #include <algorithm>
-#include <condition_variable>
 #include <map>
 #include <memory>
-#include <mutex>
-#include <queue>
 #include <string>
 #include <vector>
 
 #include "cvf_core.h"
+#include "cvf_gate.h"
 #include "cvf_host.h"
 #include "cvf_kernels.h"
 
@@ -101,10 +99,14 @@ struct PointHost {
 
 // A group of state points advanced by its own stream: its own block tables,
 // step slot and captured graphs.  Groups share nothing mutable, so their
-// launch sequences overlap on separate hardware queues.
+// launch sequences overlap on separate hardware queues.  A handle's only group
+// uses the handle's main stream: the card has few hardware queues, and a stream
+// that is never used still takes one, so that the launches of two handles
+// end up in the same one, behind each other.
 struct Group {
   std::vector<int> points;
   hipStream_t stream = nullptr;
+  bool own_stream = false;
   hipEvent_t done = nullptr;
   DevBuf<BlockEnt> tab_half, tab_cube, tab_cell, tab_slab;
   DevBuf<int32_t> plist;
@@ -168,7 +170,7 @@ struct Group {
     if (fork) (void)hipEventDestroy(fork);
     if (join) (void)hipEventDestroy(join);
     if (side) (void)hipStreamDestroy(side);
-    if (stream) (void)hipStreamDestroy(stream);
+    if (own_stream) (void)hipStreamDestroy(stream);
   }
 };
 
@@ -186,84 +188,22 @@ int set_error(int code, const char* fmt, ...) {
 }
 }  // namespace cvf
 
-// Resident launches of several handles.  A resident kernel's workgroups wait
-// for each other, so each launch needs all of its own on the card at once, and
-// two launches of which each has a part would wait until their limit.  Handles
-// of a process whose plans are resident therefore enter() before they
-// enqueue such launches and leave() after: those that surely fit together (half
-// of the device's room in all, none with workgroups of more than half a CU)
-// run side by side, any other one waits on the device for those before it.  A
-// handle that is alone only takes the lock.
-struct ResidentGate {
-  struct User {
-    int device = 0;
-    double share = 0;     // of the device's room for workgroups such as its
-    bool large = false;   // a CU holds one of them
-    bool launching = false, recorded = false;
-    hipEvent_t done = nullptr;
-  };
-  std::mutex mu;
-  std::condition_variable left;
-  std::vector<User*> users;
-
-  void add(User* u) {
-    std::lock_guard<std::mutex> lock(mu);
-    if (std::find(users.begin(), users.end(), u) == users.end()) users.push_back(u);
-  }
-  void remove(User* u) {
-    std::lock_guard<std::mutex> lock(mu);
-    users.erase(std::remove(users.begin(), users.end(), u), users.end());
-  }
-  hipError_t enter(User* u, hipStream_t st) {
-    std::unique_lock<std::mutex> lock(mu);
-    for (;;) {
-      double sum = u->share;
-      bool large = u->large, launching = false;
-      std::vector<User*> before;
-      for (User* o : users) {
-        if (o == u || o->device != u->device) continue;
-        if (!o->launching && (!o->recorded || hipEventQuery(o->done) == hipSuccess)) {
-          o->recorded = false;
-          continue;
-        }
-        before.push_back(o);
-        sum += o->share;
-        large = large || o->large;
-        launching = launching || o->launching;
-      }
-      if (!before.empty() && (sum > 0.5 || large)) {
-        if (launching) {  // its event is not recorded yet
-          left.wait(lock);
-          continue;
-        }
-        for (User* o : before)
-          if (hipError_t e = hipStreamWaitEvent(st, o->done, 0)) return e;
-      }
-      u->launching = true;
-      return hipSuccess;
-    }
-  }
-  hipError_t leave(User* u, hipStream_t st) {
-    std::lock_guard<std::mutex> lock(mu);
-    hipError_t e = hipSuccess;
-    // (a handle added later has synchronized the device before its first
-    // launch, after this one's)
-    if (users.size() > 1) {
-      e = hipEventRecord(u->done, st);
-      u->recorded = e == hipSuccess;
-    }
-    u->launching = false;
-    left.notify_all();
-    return e;
-  }
+// Resident launches of several handles (cvf_gate.h).
+struct HipEvents {
+  using Event = hipEvent_t;
+  using Stream = hipStream_t;
+  static bool done(Event e) { return hipEventQuery(e) == hipSuccess; }
+  static int wait(Stream st, Event e) { return hipStreamWaitEvent(st, e, 0); }
+  static int record(Event e, Stream st) { return hipEventRecord(e, st); }
 };
-ResidentGate g_resident_gate;
+ResidentGate<HipEvents> g_resident_gate;
+using GateUser = ResidentGate<HipEvents>::User;
 
 struct ResidentTurn {
-  ResidentGate::User* u = nullptr;
+  GateUser* u = nullptr;
   hipStream_t st = nullptr;
-  hipError_t take(ResidentGate::User* user, hipStream_t stream) {
-    hipError_t e = g_resident_gate.enter(user, stream);
+  hipError_t take(GateUser* user, hipStream_t stream) {
+    const hipError_t e = (hipError_t)g_resident_gate.enter(user, stream);
     if (e == hipSuccess) u = user, st = stream;
     return e;
   }
@@ -300,7 +240,7 @@ struct cvf_sim {
   DevBuf<uint64_t> hist_base;              // step count at the first recorded step
   DevBuf<uint32_t> rstatus;                // abort flag of the resident kernel
   bool resident_used = false;              // some launch ran the resident kernel
-  ResidentGate::User turn;                 // of its resident plan, if it has one
+  GateUser turn;                           // of its resident plan, if it has one
   uint64_t hist_base_host = 0;
   int rec_pt = -1;                         // point recorded by the groups' rec graphs
   uint32_t nb_cell_all = 0;
@@ -897,9 +837,7 @@ int build_resident(cvf_sim* s, Group& g) {
     HIPC(hipEventCreateWithFlags(&g.join, hipEventDisableTiming));
   }
   g.resident = true;
-  s->turn.device = s->device;
-  s->turn.share = (double)d.groups.size() / ((double)occ * ncu);
-  s->turn.large = occ < 2;
+  s->turn.plan = ResidentPlan{s->device, (uint32_t)d.groups.size(), (uint32_t)occ, (uint32_t)ncu};
   if (!s->turn.done) HIPC(hipEventCreateWithFlags(&s->turn.done, hipEventDisableTiming));
   g_resident_gate.add(&s->turn);
   for (int p : g.points) s->ph[p].slab_T = 0;
@@ -1343,7 +1281,12 @@ int build_groups(cvf_sim* s) {
   }
   for (auto& g : s->groups) {
     std::sort(g->points.begin(), g->points.end());
-    HIPC(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
+    if (ng == 1) {
+      g->stream = s->stream;
+    } else {
+      HIPC(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
+      g->own_stream = true;
+    }
     HIPC(hipEventCreateWithFlags(&g->done, hipEventDisableTiming));
     const auto th = make_table(s->ph, g->points, (uint32_t)s->tune.block_sigma, cells_sigma);
     // k_eta runs four threads per cube quad: block_eta / 4 quads per workgroup

@@ -1,0 +1,116 @@
+// Turns of the resident launches of several handles of a process (host only).
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+#include <condition_variable>
+#include <mutex>
+#include <vector>
+
+namespace cvf {
+
+// Engines of workgroups on a card, 8 XCDs of 4: a launch's workgroups go round
+// them in turn.
+constexpr uint32_t kEngines = 32;
+
+// What a resident plan asks of its device: workgroups, how many of them a CU
+// holds at once, and the CUs.
+struct ResidentPlan {
+  int device = 0;
+  uint32_t groups = 0, per_cu = 1, cus = 1;
+  // workgroups on the busiest engine, times the engines
+  uint32_t spread() const { return (groups + kEngines - 1) / kEngines * kEngines; }
+};
+
+// Launches that are on one device at the same time.
+struct ResidentLoad {
+  uint32_t groups = 0;  // spread
+  double room = 0;      // share of the room for workgroups such as each plan's
+  bool large = false;   // some plan has one workgroup per CU
+  void add(const ResidentPlan& p) {
+    groups += p.spread();
+    room += (double)p.spread() / ((double)p.per_cu * p.cus);
+    large = large || p.per_cu < 2;
+  }
+  // Whether all their workgroups surely are on the card at once, wherever the
+  // dispatcher puts them: with no more workgroups than CUs on any engine there
+  // is an empty CU for the next one; with workgroups of at most half a CU, half
+  // of the room is free CUs or free halves of CUs.
+  bool fits(uint32_t cus) const { return groups <= cus || (!large && room <= 0.5); }
+};
+
+// A resident kernel's workgroups wait for each other, so each launch needs all
+// of its own on the card at once, and two launches of which each has a part
+// would wait until their limit.  Handles of a process whose plans are resident
+// therefore enter() before they enqueue such launches and leave() after: those
+// that surely fit together run side by side, any other one waits on the device
+// for those before it.  A handle that is alone only takes the lock.
+// Events: done(event), wait(stream, event), record(event, stream), the last
+// two with an error code, 0 for none.
+template <class Events>
+struct ResidentGate {
+  using Event = typename Events::Event;
+  using Stream = typename Events::Stream;
+  struct User {
+    ResidentPlan plan;
+    bool launching = false, recorded = false;
+    Event done = {};
+  };
+  std::mutex mu;
+  std::condition_variable left;
+  std::vector<User*> users;
+
+  void add(User* u) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (std::find(users.begin(), users.end(), u) == users.end()) users.push_back(u);
+  }
+  void remove(User* u) {
+    std::lock_guard<std::mutex> lock(mu);
+    users.erase(std::remove(users.begin(), users.end(), u), users.end());
+  }
+  int enter(User* u, Stream st) {
+    std::unique_lock<std::mutex> lock(mu);
+    for (;;) {
+      ResidentLoad load;
+      load.add(u->plan);
+      bool launching = false;
+      std::vector<User*> before;
+      for (User* o : users) {
+        if (o == u || o->plan.device != u->plan.device) continue;
+        if (!o->launching && (!o->recorded || Events::done(o->done))) {
+          o->recorded = false;
+          continue;
+        }
+        before.push_back(o);
+        load.add(o->plan);
+        launching = launching || o->launching;
+      }
+      if (!before.empty() && !load.fits(u->plan.cus)) {
+        if (launching) {  // its event is not recorded yet
+          left.wait(lock);
+          continue;
+        }
+        for (User* o : before)
+          if (int e = Events::wait(st, o->done)) return e;
+      }
+      u->launching = true;
+      return 0;
+    }
+  }
+  int leave(User* u, Stream st) {
+    std::lock_guard<std::mutex> lock(mu);
+    int e = 0;
+    // (a handle added later has synchronized the device before its first
+    // launch, after this one's)
+    if (users.size() > 1) {
+      e = Events::record(u->done, st);
+      u->recorded = e == 0;
+    }
+    u->launching = false;
+    left.notify_all();
+    return e;
+  }
+};
+
+}  // namespace cvf
