@@ -1937,12 +1937,14 @@ int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
 // n_steps MC steps as resident launches or graph launches; group rec_gi (if
 // >= 0) replays its recording sequences.
 int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
-  ResidentTurn turn;
-  if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
   if (rec_gi < 0 && s->groups.size() == 1 && resident_sequences(s, *s->groups[0])) {
     for (int64_t i = 0; i < n_steps;) {
       const int k = (int)std::min<int64_t>(s->tune.graph_steps, n_steps - i);
-      if (int rc = enqueue_resident(s, 0, s->stream, k)) return rc;
+      {
+        ResidentTurn turn;
+        HIPC(turn.take(&s->turn, s->stream));
+        if (int rc = enqueue_resident(s, 0, s->stream, k)) return rc;
+      }
       host_moves(s, k);
       i += k;
     }
@@ -1959,10 +1961,14 @@ int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
   for (int64_t i = 0; i < n_steps;) {
     size_t c = 0;
     while (sizes[c] > n_steps - i) ++c;  // the last size is 1
-    for (size_t gi = 0; gi < s->groups.size(); ++gi) {
-      Group& g = *s->groups[gi];
-      if (g.resident) s->resident_used = true;
-      HIPC(hipGraphLaunch((int)gi == rec_gi ? g.rgexecs[c] : g.gexecs[c], fork ? g.stream : s->stream));
+    {
+      ResidentTurn turn;
+      if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
+      for (size_t gi = 0; gi < s->groups.size(); ++gi) {
+        Group& g = *s->groups[gi];
+        if (g.resident) s->resident_used = true;
+        HIPC(hipGraphLaunch((int)gi == rec_gi ? g.rgexecs[c] : g.gexecs[c], fork ? g.stream : s->stream));
+      }
     }
     host_moves(s, sizes[c]);
     i += sizes[c];

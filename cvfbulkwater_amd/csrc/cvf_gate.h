@@ -43,9 +43,12 @@ struct ResidentLoad {
 // A resident kernel's workgroups wait for each other, so each launch needs all
 // of its own on the card at once, and two launches of which each has a part
 // would wait until their limit.  Handles of a process whose plans are resident
-// therefore enter() before they enqueue such launches and leave() after: those
-// that surely fit together run side by side, any other one waits on the device
-// for those before it.  A handle that is alone only takes the lock.
+// therefore enter() before they enqueue one such launch (a sequence of at most
+// graph_steps steps) and leave() after it: those that surely fit together run
+// side by side, any other one waits on the device for those before it.  They
+// get in in the order in which they came, so that a handle that steps on and on
+// lets the others in between its launches.  A handle that is alone only takes
+// the lock.
 // Events: done(event), wait(stream, event), record(event, stream), the last
 // two with an error code, 0 for none.
 template <class Events>
@@ -58,7 +61,8 @@ struct ResidentGate {
     Event done = {};
   };
   std::mutex mu;
-  std::condition_variable left;
+  std::condition_variable changed;
+  uint64_t came = 0, in = 0;  // calls of enter(), and those of them that have returned
   std::vector<User*> users;
 
   void add(User* u) {
@@ -71,32 +75,40 @@ struct ResidentGate {
   }
   int enter(User* u, Stream st) {
     std::unique_lock<std::mutex> lock(mu);
+    const uint64_t me = came++;
+    std::vector<User*> before;
     for (;;) {
-      ResidentLoad load;
-      load.add(u->plan);
       bool launching = false;
-      std::vector<User*> before;
-      for (User* o : users) {
-        if (o == u || o->plan.device != u->plan.device) continue;
-        if (!o->launching && (!o->recorded || Events::done(o->done))) {
-          o->recorded = false;
-          continue;
+      if (in == me) {
+        ResidentLoad load;
+        load.add(u->plan);
+        before.clear();
+        for (User* o : users) {
+          if (o == u || o->plan.device != u->plan.device) continue;
+          if (!o->launching && (!o->recorded || Events::done(o->done))) {
+            o->recorded = false;
+            continue;
+          }
+          before.push_back(o);
+          load.add(o->plan);
+          launching = launching || o->launching;
         }
-        before.push_back(o);
-        load.add(o->plan);
-        launching = launching || o->launching;
-      }
-      if (!before.empty() && !load.fits(u->plan.cus)) {
-        if (launching) {  // its event is not recorded yet
-          left.wait(lock);
-          continue;
+        if (before.empty() || load.fits(u->plan.cus)) {
+          before.clear();
+          break;
         }
-        for (User* o : before)
-          if (int e = Events::wait(st, o->done)) return e;
+        if (!launching) break;
       }
-      u->launching = true;
-      return 0;
+      // someone came earlier, or is launching: its event is not recorded yet
+      changed.wait(lock);
     }
+    int e = 0;
+    for (User* o : before)
+      if (!e) e = Events::wait(st, o->done);
+    u->launching = e == 0;
+    ++in;
+    changed.notify_all();
+    return e;
   }
   int leave(User* u, Stream st) {
     std::lock_guard<std::mutex> lock(mu);
@@ -108,7 +120,7 @@ struct ResidentGate {
       u->recorded = e == 0;
     }
     u->launching = false;
-    left.notify_all();
+    changed.notify_all();
     return e;
   }
 };

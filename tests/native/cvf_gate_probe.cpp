@@ -41,3 +41,33 @@ extern "C" int probe_together(int n, int groups, int per_cu, int cus) {
   }
   return n;
 }
+
+// Two whole-card handles, the first of which launches on and on: whether the
+// second, which came while the first was launching, gets in before the first
+// one's next launch
+extern "C" int probe_order() {
+  using namespace std::chrono;
+  g_done = {0, 1};
+  Gate gate;
+  Gate::User a, b;
+  a.plan = b.plan = ResidentPlan{0, 256, 1, 256};
+  b.done = 1;
+  gate.add(&a);
+  gate.add(&b);
+  std::string order;  // (written between enter and leave: one handle at a time)
+  gate.enter(&a, 0);
+  std::thread t([&] {
+    gate.enter(&b, 0);
+    order += 'b';
+    gate.leave(&b, 0);
+  });
+  std::this_thread::sleep_for(milliseconds(200));  // b waits
+  for (int i = 0; i < 3; ++i) {
+    order += 'a';
+    gate.leave(&a, 0);
+    gate.enter(&a, 0);
+  }
+  gate.leave(&a, 0);
+  t.join();
+  return order == "abaa";
+}

@@ -28,3 +28,8 @@ def test_handles_that_fit_run_together(probe, groups, per_cu, together):
     # they fit on every engine of workgroups: as many CUs, or half of the room
     busiest = -(-groups // ENGINES) * together
     assert busiest <= CUS // ENGINES or busiest <= per_cu * CUS // ENGINES // 2 or together == 1
+
+
+def test_handles_get_in_as_they_came(probe):
+    """A handle that launches on and on does not keep another one out."""
+    assert probe.probe_order()
