@@ -189,26 +189,27 @@ int set_error(int code, const char* fmt, ...) {
 }  // namespace cvf
 
 // Resident launches of several handles (cvf_gate.h).
-struct HipEvents {
+struct HipStreams {
   using Event = hipEvent_t;
   using Stream = hipStream_t;
-  static bool done(Event e) { return hipEventQuery(e) == hipSuccess; }
-  static int wait(Stream st, Event e) { return hipStreamWaitEvent(st, e, 0); }
-  static int record(Event e, Stream st) { return hipEventRecord(e, st); }
+  static bool idle(Stream st) { return hipStreamQuery(st) == hipSuccess; }
+  static int after(Stream st, Stream other, Event e) {
+    if (hipError_t err = hipEventRecord(e, other)) return err;
+    return hipStreamWaitEvent(st, e, 0);
+  }
 };
-ResidentGate<HipEvents> g_resident_gate;
-using GateUser = ResidentGate<HipEvents>::User;
+ResidentGate<HipStreams> g_resident_gate;
+using GateUser = ResidentGate<HipStreams>::User;
 
 struct ResidentTurn {
   GateUser* u = nullptr;
-  hipStream_t st = nullptr;
-  hipError_t take(GateUser* user, hipStream_t stream) {
-    const hipError_t e = (hipError_t)g_resident_gate.enter(user, stream);
-    if (e == hipSuccess) u = user, st = stream;
+  hipError_t take(GateUser* user) {
+    const hipError_t e = (hipError_t)g_resident_gate.enter(user);
+    if (e == hipSuccess) u = user;
     return e;
   }
   ~ResidentTurn() {
-    if (u) (void)g_resident_gate.leave(u, st);
+    if (u) g_resident_gate.leave(u);
   }
 };
 
@@ -269,7 +270,7 @@ struct cvf_sim {
   }
   ~cvf_sim() {
     g_resident_gate.remove(&turn);
-    if (turn.done) (void)hipEventDestroy(turn.done);
+    if (turn.event) (void)hipEventDestroy(turn.event);
     groups.clear();
     if (start_ev) (void)hipEventDestroy(start_ev);
     if (stream) (void)hipStreamDestroy(stream);
@@ -838,7 +839,8 @@ int build_resident(cvf_sim* s, Group& g) {
   }
   g.resident = true;
   s->turn.plan = ResidentPlan{s->device, (uint32_t)d.groups.size(), (uint32_t)occ, (uint32_t)ncu};
-  if (!s->turn.done) HIPC(hipEventCreateWithFlags(&s->turn.done, hipEventDisableTiming));
+  s->turn.stream = s->stream;
+  if (!s->turn.event) HIPC(hipEventCreateWithFlags(&s->turn.event, hipEventDisableTiming));
   g_resident_gate.add(&s->turn);
   for (int p : g.points) s->ph[p].slab_T = 0;
   // the plan query reports a point's thickest slab
@@ -1532,7 +1534,9 @@ int enqueue_resident(cvf_sim* s, int gi, hipStream_t st, int nsteps) {
 }
 
 int capture(cvf_sim* s, int gi, int nsteps, hipGraph_t* g, hipGraphExec_t* ge, bool rec = false) {
-  hipStream_t st = s->groups[gi]->stream;
+  // (not the stream of resident launches, on which another handle's thread may
+  // record an event)
+  hipStream_t st = s->groups[gi]->resident ? s->groups[gi]->side : s->groups[gi]->stream;
   HIPC(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   const int rc = enqueue_steps(s, gi, st, nsteps, rec);
   hipError_t e = hipStreamEndCapture(st, g);
@@ -1942,7 +1946,7 @@ int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
       const int k = (int)std::min<int64_t>(s->tune.graph_steps, n_steps - i);
       {
         ResidentTurn turn;
-        HIPC(turn.take(&s->turn, s->stream));
+        HIPC(turn.take(&s->turn));
         if (int rc = enqueue_resident(s, 0, s->stream, k)) return rc;
       }
       host_moves(s, k);
@@ -1963,7 +1967,7 @@ int run_steps(cvf_sim* s, int64_t n_steps, int rec_gi) {
     while (sizes[c] > n_steps - i) ++c;  // the last size is 1
     {
       ResidentTurn turn;
-      if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
+      if (s->groups[0]->resident) HIPC(turn.take(&s->turn));
       for (size_t gi = 0; gi < s->groups.size(); ++gi) {
         Group& g = *s->groups[gi];
         if (g.resident) s->resident_used = true;
@@ -2295,7 +2299,7 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     recs.push_back(r);
   };
   ResidentTurn turn;
-  if (s->groups[0]->resident) HIPC(turn.take(&s->turn, s->stream));
+  if (s->groups[0]->resident) HIPC(turn.take(&s->turn));
   int rc = fork_groups(s);
   if (rc) return rc;
   if (s->nc > 0 && n_steps > 0) s->sw_labels = true;

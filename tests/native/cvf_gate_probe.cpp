@@ -1,5 +1,5 @@
-// The gate of resident launches with events of this file's own: a launch is
-// done when the test says so.
+// The gate of resident launches with streams of this file's own: a launch has
+// ended when the test says so.
 #include <chrono>
 #include <set>
 #include <string>
@@ -10,14 +10,13 @@
 using namespace cvf;
 
 namespace {
-std::set<int> g_done;        // launches that have ended
-std::vector<int> g_waited;   // events that the streams were made to wait for
+std::set<int> g_idle;        // streams whose launches have ended
+std::vector<int> g_waited;   // streams that others were made to wait for
 struct Fake {
   using Event = int;
   using Stream = int;
-  static bool done(int e) { return g_done.count(e) != 0; }
-  static int wait(int, int e) { return g_waited.push_back(e), 0; }
-  static int record(int, int) { return 0; }
+  static bool idle(int st) { return g_idle.count(st) != 0; }
+  static int after(int, int other, int) { return g_waited.push_back(other), 0; }
 };
 using Gate = ResidentGate<Fake>;
 }  // namespace
@@ -25,19 +24,19 @@ using Gate = ResidentGate<Fake>;
 // n handles of `groups` workgroups, `per_cu` to a CU, launch one after the
 // other, none of which ends: how many of them run before one is made to wait
 extern "C" int probe_together(int n, int groups, int per_cu, int cus) {
-  g_done.clear();
+  g_idle.clear();
   g_waited.clear();
   Gate gate;
   std::vector<Gate::User> u((size_t)n);
   for (int i = 0; i < n; ++i) {
     u[i].plan = ResidentPlan{0, (uint32_t)groups, (uint32_t)per_cu, (uint32_t)cus};
-    u[i].done = i;
+    u[i].stream = i;
     gate.add(&u[i]);
   }
   for (int i = 0; i < n; ++i) {
-    gate.enter(&u[i], 0);
+    gate.enter(&u[i]);
     if (!g_waited.empty()) return i;
-    gate.leave(&u[i], 0);
+    gate.leave(&u[i]);
   }
   return n;
 }
@@ -47,27 +46,27 @@ extern "C" int probe_together(int n, int groups, int per_cu, int cus) {
 // one's next launch
 extern "C" int probe_order() {
   using namespace std::chrono;
-  g_done = {0, 1};
+  g_idle = {0, 1};
   Gate gate;
   Gate::User a, b;
   a.plan = b.plan = ResidentPlan{0, 256, 1, 256};
-  b.done = 1;
+  b.stream = 1;
   gate.add(&a);
   gate.add(&b);
   std::string order;  // (written between enter and leave: one handle at a time)
-  gate.enter(&a, 0);
+  gate.enter(&a);
   std::thread t([&] {
-    gate.enter(&b, 0);
+    gate.enter(&b);
     order += 'b';
-    gate.leave(&b, 0);
+    gate.leave(&b);
   });
   std::this_thread::sleep_for(milliseconds(200));  // b waits
   for (int i = 0; i < 3; ++i) {
     order += 'a';
-    gate.leave(&a, 0);
-    gate.enter(&a, 0);
+    gate.leave(&a);
+    gate.enter(&a);
   }
-  gate.leave(&a, 0);
+  gate.leave(&a);
   t.join();
   return order == "abaa";
 }

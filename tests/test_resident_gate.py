@@ -1,5 +1,5 @@
-"""Turns of resident launches of several handles, on the CPU with events of the
-test's own."""
+"""Turns of resident launches of several handles, on the CPU with streams of
+the test's own."""
 import ctypes
 import subprocess
 from pathlib import Path
