@@ -225,7 +225,7 @@ struct cvf_sim {
 
   DevBuf<uint32_t> words, words2, parent, cover, nslot_nperc;  // words2: ping-pong partner
   DevBuf<uint8_t> cov, cfg_bytes;
-  DevBuf<uint32_t> cfg_res;                 // first value out of range, inconsistent cubes
+  DevBuf<uint32_t> cfg_res;                 // first value out of range, inconsistent cubes, abort flag
   DevBuf<int32_t> csize, slot, cclusters;  // clusters' nodes but their roots, percolation slots, compacted sizes
   DevBuf<uint32_t> cblock;                  // per-workgroup cluster counts of the compaction
   DevBuf<uint64_t> cmom;                    // per-workgroup size moments (4 words each)
@@ -239,7 +239,7 @@ struct cvf_sim {
   DevBuf<unsigned long long> hist;     // sigma histogram of one point (6 counters)
   DevBuf<unsigned long long> hist_series;  // per-step histograms (6 counters per step)
   DevBuf<uint64_t> hist_base;              // step count at the first recorded step
-  DevBuf<uint32_t> rstatus;                // abort flag of the resident kernel
+  DevBuf<uint32_t> rstatus;                // abort flag of the resident kernel, launch_mark of the launch
   bool resident_used = false;              // some launch ran the resident kernel
   GateUser turn;                           // of its resident plan, if it has one
   uint64_t hist_base_host = 0;
@@ -386,21 +386,6 @@ void init_words(const PointHost& P, std::vector<uint32_t>& w) {
   });
 }
 
-// The resident kernel's abort flag: a neighbour wait that timed out leaves
-// the lattice invalid.  Call after the handle's stream has been synchronised.
-int resident_status(uint32_t v) {
-  if (v)
-    return fail(CVF_EDEVICE, "resident kernel: a workgroup's wait for its neighbour slab timed out; "
-                             "the lattice state is invalid");
-  return CVF_OK;
-}
-int check_resident(cvf_sim* s) {
-  if (!s->resident_used) return CVF_OK;
-  uint32_t v = 0;
-  HIPC(hipMemcpy(&v, s->rstatus.p, sizeof v, hipMemcpyDeviceToHost));
-  return resident_status(v);
-}
-
 int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
   HIPC(hipStreamSynchronize(s->stream));
   HIPC(hipMemcpyAsync(s->words.p + s->ph[pt].woff, w.data(), w.size() * 4, hipMemcpyHostToDevice,
@@ -413,7 +398,7 @@ int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
 // Device copy of a point's sigma and eta bytes, kept for the next call
 // (sized for the largest point that asked).
 int reserve_config(cvf_sim* s, size_t n6) {
-  if (!s->cfg_res.p) HIPC(s->cfg_res.alloc(2));
+  if (!s->cfg_res.p) HIPC(s->cfg_res.alloc(3));
   if (2 * n6 > s->cfg_bytes.n) HIPC(s->cfg_bytes.alloc(2 * n6));
   return CVF_OK;
 }
@@ -1372,16 +1357,19 @@ int build_groups(cvf_sim* s) {
 }
 
 // nsteps steps of resident group g in one launch (launch_resident's stepp,
-// step_off and step_out).
+// step_off and step_out).  A sequence of launches keeps the lattice before its
+// first one (24 points of L = 32 with a cluster sweep, a launch per step: 0.9 us
+// of 69 where every one does).
 void run_resident(cvf_sim* s, const Group& g, hipStream_t st, const uint64_t* stepp, uint64_t step_off,
                   uint32_t nsteps, uint64_t* step_out) {
   s->resident_used = true;
+  uint32_t* kept = stepp && step_off ? nullptr : s->words2.p;
   if (g.r_per)
     launch_plane(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                 s->words.p, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_per);
+                 s->words.p, kept, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_per);
   else
     launch_resident(st, g.rgroups.p, g.r_ngroups, (uint32_t)s->tune.block_chunk, g.r_lds, g.rslabs.p, s->pts.p,
-                    s->words.p, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_fine,
+                    s->words.p, kept, g.rings.p, g.rver.p, stepp, step_off, nsteps, step_out, s->rstatus.p, g.r_fine,
                     s->sched == CVF_SCHED_FAST);
 }
 
@@ -1478,7 +1466,8 @@ constexpr uint32_t kHistSpan = 4096;  // per-step histograms per copy back
 // array holding it, and the last step of a sequence takes its plain form
 // when the variant would end there in words2: every sequence ends with the
 // state in `words`.
-int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = false) {
+// Without moves the volume chain stays where it is.
+int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = false, bool moves = true) {
   Group& g = *s->groups[gi];
   const bool ok = g.fused && s->nm > 0;
   bool variant_ok = false;
@@ -1501,7 +1490,7 @@ int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = fal
     }
   }
   launch_vol_chain(st, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,
-                   (uint32_t)nsteps, s->dist.p, s->freq.p, s->precision, s->vol_device);
+                   (uint32_t)nsteps, s->dist.p, s->freq.p, s->precision, moves && s->vol_device);
   return CVF_OK;
 }
 
@@ -1640,7 +1629,8 @@ int check_tuning(const cvf_tuning& t) {
   return CVF_OK;
 }
 
-cvf_tuning default_tuning(const cvf_sim* s) {
+// (resident: with resident plans where they are the faster ones)
+cvf_tuning default_tuning(const cvf_sim* s, bool resident = true) {
   cvf_tuning t;
   t.streams = 1;
   t.block_sigma = s->total_cells < (1u << 20) ? 64 : 256;
@@ -1678,6 +1668,7 @@ cvf_tuning default_tuning(const cvf_sim* s) {
       t.block_chunk = (int32_t)best.block;
     }
   }
+  if (!resident) return t;
   // One Metropolis sweep per step up to L = 64: the resident kernels.  One-plane
   // slabs while there are workgroups for the planes, one to four of them per CU:
   // 256 threads up to L = 16 and 512 up to L = 32, fewer where more share a CU
@@ -1744,6 +1735,57 @@ cvf_tuning default_tuning(const cvf_sim* s) {
     }
   }
   return t;
+}
+
+// The steps since the aborted resident launch of this mark, again: from the
+// lattice that it started from, by launches that wait for nothing, which are
+// the handle's plan from now on.  (Its plan needs the card to itself, and
+// another process has a part of it.)  The volume chain, which never reads the
+// lattice, stands.  rec_base: the steps from there on are recorded again for
+// point rec_pt.  The handle's stream has been synchronised.
+int redo_steps(cvf_sim* s, uint32_t mark, int64_t rec_base = -1) {
+  const int64_t end = s->steps;
+  int64_t at = end - (int64_t)(((uint32_t)end + 1 - mark) & 0x7FFFFFFFu);
+  HIPC(hipMemcpy(s->words.p, s->words2.p, s->total_cells * 4, hipMemcpyDeviceToDevice));
+  s->tune = default_tuning(s, false);
+  s->steps = at;
+  int rc = build_groups(s);
+  s->steps = end;
+  if (rc) return rc;
+  if (rec_base >= 0) {
+    const size_t first = (size_t)(std::max(at, rec_base) - rec_base), n = (size_t)(end - rec_base);
+    launch_zero_u32(s->stream, (uint32_t*)(s->hist_series.p + kHistWords * first), 2 * kHistWords * (n - first));
+  }
+  if ((rc = fork_groups(s))) return rc;
+  while (at < end) {
+    const int64_t to = at < rec_base ? std::min(rec_base, end) : end;
+    const int n = (int)std::min<int64_t>(64, to - at);
+    for (size_t gi = 0; gi < s->groups.size(); ++gi) {
+      const bool rec = rec_base >= 0 && at >= rec_base && (int32_t)gi == s->ph[s->rec_pt].group;
+      if ((rc = enqueue_steps(s, (int)gi, s->groups[gi]->stream, n, rec, false))) return rc;
+    }
+    at += n;
+  }
+  if ((rc = join_groups(s))) return rc;
+  HIPC(hipGetLastError());
+  HIPC(hipStreamSynchronize(s->stream));
+  HIPC(hipMemset(s->rstatus.p, 0, 2 * sizeof(uint32_t)));
+  HIPC(hipDeviceSynchronize());
+  s->resident_used = false;
+  s->obs_at = -1;
+  return CVF_OK;
+}
+
+// A handle whose stream has been synchronised: steps that a resident launch
+// could not finish are done again.  (*done: whether there were any.)
+int settle(cvf_sim* s, int64_t rec_base = -1, bool* done = nullptr) {
+  if (done) *done = false;
+  if (!s->resident_used) return CVF_OK;
+  uint32_t status[2];
+  HIPC(hipMemcpy(status, s->rstatus.p, sizeof status, hipMemcpyDeviceToHost));
+  if (!status[0]) return CVF_OK;
+  if (done) *done = true;
+  return redo_steps(s, status[1], rec_base);
 }
 
 int create_impl(const cvf_params* pts, int32_t n, cvf_sim** out) {
@@ -1901,17 +1943,23 @@ int cvf_set_config(cvf_sim* s, int32_t pt, const uint8_t* sigma6N, const uint8_t
   const PointHost& P = s->ph[pt];
   const size_t n6 = 6 * (size_t)P.N;
   if ((rc = reserve_config(s, n6))) return rc;
-  // words2 is free between steps: the packed input, decoded into words
+  // words2 is free between steps (unless a resident launch was aborted): the
+  // packed input, decoded into words
   uint32_t* res = s->cfg_res.p;
-  HIPC(hipMemcpyAsync(s->cfg_bytes.p, sigma6N, n6, hipMemcpyHostToDevice, s->stream));
-  HIPC(hipMemcpyAsync(s->cfg_bytes.p + n6, eta6N, n6, hipMemcpyHostToDevice, s->stream));
-  HIPC(hipMemsetAsync(res, 0xFF, 2 * sizeof(uint32_t), s->stream));
-  launch_config_in(s->stream, s->cfg_bytes.p, s->cfg_bytes.p + n6, P.L, P.prm.flag_chessboard, s->words2.p + P.woff,
-                   s->words.p + P.woff, res, res + 1);
-  HIPC(hipGetLastError());
-  uint32_t out[2];
-  HIPC(hipMemcpyAsync(out, res, sizeof out, hipMemcpyDeviceToHost, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
+  uint32_t out[3];
+  for (;;) {
+    HIPC(hipMemcpyAsync(s->cfg_bytes.p, sigma6N, n6, hipMemcpyHostToDevice, s->stream));
+    HIPC(hipMemcpyAsync(s->cfg_bytes.p + n6, eta6N, n6, hipMemcpyHostToDevice, s->stream));
+    HIPC(hipMemsetAsync(res, 0xFF, 2 * sizeof(uint32_t), s->stream));
+    launch_config_in(s->stream, s->cfg_bytes.p, s->cfg_bytes.p + n6, P.L, P.prm.flag_chessboard,
+                     s->words2.p + P.woff, s->words.p + P.woff, res, res + 1, s->rstatus.p, res + 2);
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(out, res, sizeof out, hipMemcpyDeviceToHost, s->stream));
+    HIPC(hipStreamSynchronize(s->stream));
+    bool again = false;
+    if (out[2] && (rc = settle(s, -1, &again))) return rc;
+    if (!again) break;
+  }
   if (out[0] != 0xFFFFFFFFu) {
     const uint32_t i = out[0] / 2;
     if (out[0] & 1u)
@@ -1929,10 +1977,13 @@ int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
   const PointHost& P = s->ph[pt];
   const size_t n6 = 6 * (size_t)P.N;
   if ((rc = reserve_config(s, n6))) return rc;
-  launch_config_out(s->stream, s->words.p + P.woff, P.N, s->cfg_bytes.p, s->cfg_bytes.p + n6);
-  HIPC(hipGetLastError());
-  HIPC(hipStreamSynchronize(s->stream));
-  if ((rc = check_resident(s))) return rc;
+  bool again;
+  do {
+    launch_config_out(s->stream, s->words.p + P.woff, P.N, s->cfg_bytes.p, s->cfg_bytes.p + n6);
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(s->stream));
+    if ((rc = settle(s, -1, &again))) return rc;
+  } while (again);
   if (sigma6N) HIPC(hipMemcpy(sigma6N, s->cfg_bytes.p, n6, hipMemcpyDeviceToHost));
   if (eta6N) HIPC(hipMemcpy(eta6N, s->cfg_bytes.p + n6, n6, hipMemcpyDeviceToHost));
   return CVF_OK;
@@ -1992,7 +2043,18 @@ int cvf_sync(cvf_sim* s) {
   if (!s) return fail(CVF_EINVAL, "null handle");
   HIPC(hipSetDevice(s->device));
   HIPC(hipStreamSynchronize(s->stream));
-  return check_resident(s);
+  return settle(s);
+}
+
+// For the tests: the handle's next resident launch (of steps not yet enqueued)
+// finds itself aborted, as one of its waits that timed out leaves it.
+int cvf_abort_next_launch(cvf_sim* s) {
+  if (!s->groups[0]->resident) return fail(CVF_EINVAL, "no resident plan");
+  HIPC(hipSetDevice(s->device));
+  HIPC(hipStreamSynchronize(s->stream));
+  const uint32_t status[2] = {1u, launch_mark((uint64_t)s->steps)};
+  HIPC(hipMemcpy(s->rstatus.p, status, sizeof status, hipMemcpyHostToDevice));
+  return CVF_OK;
 }
 
 int cvf_get_volume(cvf_sim* s, int32_t pt, double* r_cell, double* V, double* E_vdw) {
@@ -2017,14 +2079,16 @@ int cvf_observe(cvf_sim* s, int32_t pt, cvf_obs* o) {
   if (rc) return rc;
   if (!o) return fail(CVF_EINVAL, "null output");
   HIPC(hipSetDevice(s->device));
-  if (s->obs_at != s->steps) {
+  while (s->obs_at != s->steps) {
     launch_observe(s->stream, s->tab_cell_all.p, s->nb_cell_all, s->words.p, observe_span(s->total_cells), s->pst.p,
                    s->rstatus.p, ObsOut{s->obs_part.p, s->obs_ps.p, s->obs_status.p}, s->bonds.p);
     if (s->n_capped)
       launch_capped_hb(s->stream, s->tab_capped.p, s->n_capped, s->capped_L, s->bonds.p, s->obs_capped.p);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
-    if ((rc = resident_status(*s->obs_status.p))) return rc;
+    bool again = false;
+    if (*s->obs_status.p && (rc = settle(s, -1, &again))) return rc;
+    if (again) continue;
     s->obs_nhb2.assign(s->npts, 0);
     s->obs_nsig.assign(s->npts, 0);
     for (size_t b = 0; b < s->obs_point.size(); ++b)
@@ -2122,7 +2186,7 @@ int cvf_get_labels(cvf_sim* s, int32_t pt, int32_t* labels6N) {
   if (rc) return rc;
   HIPC(hipSetDevice(s->device));
   HIPC(hipStreamSynchronize(s->stream));
-  if ((rc = check_resident(s))) return rc;
+  if ((rc = settle(s))) return rc;
   const PointHost& P = s->ph[pt];
   HIPC(hipMemcpy(labels6N, s->parent.p + P.loff, 6 * (size_t)P.N * 4, hipMemcpyDeviceToHost));
   return CVF_OK;
@@ -2352,7 +2416,7 @@ int cvf_profile_steps(cvf_sim* s, int64_t n_steps, double* kernel_ms, int64_t* l
     if (launches) launches[c] = cnt[c];
   }
   s->obs_at = -1;
-  return CVF_OK;
+  return settle(s);
 }
 
 int cvf_get_plan(cvf_sim* s, int32_t pt, int32_t* group, int32_t* slab_planes, int32_t* chunk_sweeps,
@@ -2392,6 +2456,7 @@ int cvf_set_tuning(cvf_sim* s, const cvf_tuning* t) {
   if (rc) return rc;
   HIPC(hipSetDevice(s->device));
   HIPC(hipStreamSynchronize(s->stream));
+  if ((rc = settle(s))) return rc;
   s->tune = *t;
   return build_groups(s);
 }
@@ -2478,6 +2543,7 @@ extern "C" int cvf_autotune(cvf_sim* s, int32_t steps_per_trial, cvf_tuning* cho
   }
   // snapshot of everything a step changes
   HIPC(hipStreamSynchronize(s->stream));
+  if ((rc = settle(s))) return rc;
   DevBuf<uint32_t> w0, l0;
   DevBuf<PointState> p0;
   HIPC(w0.alloc(s->total_cells));
@@ -2587,7 +2653,9 @@ extern "C" int cvf_autotune(cvf_sim* s, int32_t steps_per_trial, cvf_tuning* cho
     HIPC(hipEventSynchronize(b));
     float ms = 0;
     HIPC(hipEventElapsedTime(&ms, a, b));
-    if ((double)ms / n < best_ms) {
+    bool aborted = false;
+    if ((rc = settle(s, -1, &aborted))) break;
+    if (!aborted && (double)ms / n < best_ms) {
       best_ms = (double)ms / n;
       best = t;
     }
@@ -2596,6 +2664,7 @@ extern "C" int cvf_autotune(cvf_sim* s, int32_t steps_per_trial, cvf_tuning* cho
   (void)hipEventDestroy(b);
   // restore the snapshot and apply the winner
   HIPC(hipStreamSynchronize(s->stream));
+  if (!rc) rc = settle(s);
   HIPC(hipMemcpy(s->words.p, w0.p, s->total_cells * 4, hipMemcpyDeviceToDevice));
   HIPC(hipMemcpy(s->parent.p, l0.p, s->total_nodes * 4, hipMemcpyDeviceToDevice));
   HIPC(hipMemcpy(s->pst.p, p0.p, s->npts * sizeof(PointState), hipMemcpyDeviceToDevice));

@@ -136,8 +136,11 @@ void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* s
 // sigma and eta arrays to the words W through `scratch` (L^3 words): *first
 // (all ones before) tells the first value out of range, then W is not
 // written; *inconsistent counts up the cubes whose eta was not a solution.
+// *flag is the resident launches' abort flag: if it is set, neither scratch nor
+// W is written.
 void launch_config_in(hipStream_t st, const uint8_t* sigma, const uint8_t* eta, uint32_t L, int chessboard,
-                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent);
+                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent,
+                      const uint32_t* rstatus, uint32_t* flag);
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc);
 void launch_sw_union(hipStream_t st, Launch ln, uint32_t* parent, const uint8_t* cov);
@@ -234,9 +237,14 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 // does, instead of one quad (one four-cube item) per lane
 // The launch's first step is *stepp + step_off, or step_off itself without
 // stepp; with step_out (then no stepp) the step after its last goes there.
+// The lattice that it starts from stays in `kept` (null: that of an earlier
+// launch serves), for the steps to be done again if a wait times out: then
+// status[0] is not zero, and status[1] the launch_mark of the first step of the
+// launch whose start `kept` holds.  Launches after it leave `kept` alone.
+constexpr uint32_t launch_mark(uint64_t step) { return (uint32_t)(step + 1) | 0x80000000u; }
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
-                     const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                     const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                     const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* kept, uint32_t* rings,
+                     uint64_t* ver, const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
                      bool fine, bool fast);
 // The same for plans of the reference schedule whose workgroups hold one
 // one-plane slab each (cvf_plane.hip), the moves of `per` half-sweeps (a
@@ -244,8 +252,8 @@ void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uin
 uint32_t plane_lds_bytes(uint32_t L, uint32_t per);
 hipError_t plane_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes);
 void launch_plane(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
-                  const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                  const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                  const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* kept, uint32_t* rings,
+                  uint64_t* ver, const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
                   uint32_t per);
 
 }  // namespace cvf

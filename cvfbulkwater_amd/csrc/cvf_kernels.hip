@@ -866,11 +866,15 @@ __global__ __launch_bounds__(256) void k_config_out(const uint32_t* __restrict__
 }
 
 // The first value out of range (sigma above 5, eta above 1) in the order of
-// the arrays, sigma before eta at one index: *first = 2 i, or 2 i + 1.
+// the arrays, sigma before eta at one index: *first = 2 i, or 2 i + 1.  Nothing
+// is written but *flag if the resident launches' abort flag is set: W may hold
+// what their steps are done again from.
 __global__ __launch_bounds__(256) void k_config_in(const uint8_t* __restrict__ sigma, const uint8_t* __restrict__ eta,
-                                                  uint32_t N, uint32_t* __restrict__ W, uint32_t* __restrict__ first) {
-  const uint32_t t = 4 * (blockIdx.x * 256 + threadIdx.x);
-  if (t >= N) return;
+                                                  uint32_t N, uint32_t* __restrict__ W, uint32_t* __restrict__ first,
+                                                  const uint32_t* __restrict__ rstatus, uint32_t* __restrict__ flag) {
+  const uint32_t t = 4 * (blockIdx.x * 256 + threadIdx.x), f = *rstatus;
+  if (t == 0) *flag = f;
+  if (t >= N || f) return;
   uint32_t w[4] = {0, 0, 0, 0}, bad = 0xFFFFFFFFu;
 #pragma unroll
   for (int a = 0; a < 6; ++a) {
@@ -907,9 +911,10 @@ __device__ __forceinline__ uint32_t cube_state(Eta&& eta) {
 __global__ __launch_bounds__(256) void k_config_decode(const uint32_t* __restrict__ src, uint32_t L, FastDiv dL,
                                                       int chessboard, uint32_t* __restrict__ dst,
                                                       const uint32_t* __restrict__ first,
+                                                      const uint32_t* __restrict__ flag,
                                                       uint32_t* __restrict__ inconsistent) {
   const uint32_t t = blockIdx.x * 256 + threadIdx.x, N = L * L * L;
-  if (t >= N || *first != 0xFFFFFFFFu) return;
+  if (t >= N || *first != 0xFFFFFFFFu || *flag) return;
   const uint32_t r1 = fdiv(t, dL), x = t - r1 * L, z = fdiv(r1, dL), y = r1 - z * L;
   const uint32_t w = src[t];
   if (!chessboard) {
@@ -1641,11 +1646,12 @@ void launch_config_out(hipStream_t st, const uint32_t* W, uint32_t N, uint8_t* s
   launch(k_config_out, dim3((N / 4 + 255) / 256), dim3(256), st, W, N, sigma, eta);
 }
 void launch_config_in(hipStream_t st, const uint8_t* sigma, const uint8_t* eta, uint32_t L, int chessboard,
-                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent) {
+                      uint32_t* scratch, uint32_t* W, uint32_t* first, uint32_t* inconsistent,
+                      const uint32_t* rstatus, uint32_t* flag) {
   const uint32_t N = L * L * L;
-  launch(k_config_in, dim3((N / 4 + 255) / 256), dim3(256), st, sigma, eta, N, scratch, first);
+  launch(k_config_in, dim3((N / 4 + 255) / 256), dim3(256), st, sigma, eta, N, scratch, first, rstatus, flag);
   launch(k_config_decode, dim3((N + 255) / 256), dim3(256), st, (const uint32_t*)scratch, L, make_fastdiv(L),
-         chessboard, W, (const uint32_t*)first, inconsistent);
+         chessboard, W, (const uint32_t*)first, (const uint32_t*)flag, inconsistent);
 }
 void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t* parent, uint8_t* cov,
                      uint32_t jc) {

@@ -61,7 +61,8 @@ __device__ __forceinline__ uint32_t lane_push(uint32_t y, uint32_t to) {
 // planes of L^2 words, then the batch's records (plane_lds_bytes)
 __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ grp, const RSlab* __restrict__ slabs,
                                                  const PointDev* __restrict__ pts, uint32_t* __restrict__ words,
-                                                 uint32_t* __restrict__ rings, uint64_t* __restrict__ ver,
+                                                 uint32_t* __restrict__ kept, uint32_t* __restrict__ rings,
+                                                 uint64_t* __restrict__ ver,
                                                  const uint64_t* __restrict__ stepp, uint64_t step_off,
                                                  uint32_t nsteps, uint64_t* __restrict__ step_out,
                                                  uint32_t* __restrict__ status, uint32_t per) {
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ gr
   __shared__ uint64_t thr_e[9], etab[9];
   __shared__ uint32_t abort_s;
   const uint32_t tid = threadIdx.x, nt = blockDim.x, lane = tid & 63u, h = tid & 3u;
-  const uint32_t me = grp[blockIdx.x].first;
+  const uint32_t me = grp[blockIdx.x].first, flag = status[0];
   const RSlab S = slabs[me];
   const uint32_t L = S.L, hL = L / 2, qL = L / 4, LL = L * L, Q4 = LL / 4, Q8 = LL / 8, z0 = S.z0, par = z0 & 1u;
   const uint64_t seed = ((uint64_t)S.seed_hi << 32) | S.seed_lo;
@@ -84,6 +85,7 @@ __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ gr
     etab[tid] = eta_table_entry(tid);
   }
   if (tid == 0) abort_s = 0;
+  const uint64_t step0 = (stepp ? *stepp : 0) + step_off;
   for (uint32_t i = tid; i < 3 * Q4; i += nt) {
     const uint32_t p = fdiv(i, FastDiv{Q4, S.mP4}), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
     const uint32_t zp = z0 + L - 1 + p, z = zp >= 2 * L ? zp - 2 * L : zp >= L ? zp - L : zp;
@@ -91,7 +93,20 @@ __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ gr
     reinterpret_cast<uint4*>(lds)[i] = make_uint4(s[0], s[hL * L], s[hL], s[hL * L + hL]);
   }
   __syncthreads();
-  const uint64_t step0 = (stepp ? *stepp : 0) + step_off;
+  const auto store_plane = [&](uint32_t* to) {
+    for (uint32_t i = tid; i < Q4; i += nt) {
+      const uint32_t y = fdiv(i, dH), x = i - y * hL;
+      const uint4 v = reinterpret_cast<const uint4*>(lds + LL)[i];
+      uint32_t* d = to + S.woff + z0 * LL + x + L * y;
+      d[0] = v.x;
+      d[hL * L] = v.y;
+      d[hL] = v.z;
+      d[hL * L + hL] = v.w;
+    }
+  };
+  // (not as it is staged: the next loads would wait for these stores)
+  if (keeps_start(kept, flag, status, step0)) store_plane(kept);
+  leave_mark(kept, flag, status, step0);
   if (step_out && blockIdx.x == 0 && tid == 0) *step_out = step0 + nsteps;
   bool aborted = false;
   // lane 16 j + k: half-sweep k of the j-th of four steps, k | arm << 4 |
@@ -345,15 +360,7 @@ __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ gr
   }
   __syncthreads();
   if (abort_s) return;  // after the last barrier
-  for (uint32_t i = tid; i < Q4; i += nt) {
-    const uint32_t y = fdiv(i, dH), x = i - y * hL;
-    const uint4 v = reinterpret_cast<const uint4*>(lds + LL)[i];
-    uint32_t* d = words + S.woff + z0 * LL + x + L * y;
-    d[0] = v.x;
-    d[hL * L] = v.y;
-    d[hL] = v.z;
-    d[hL * L + hL] = v.w;
-  }
+  store_plane(words);
 }
 
 uint32_t plane_lds_bytes(uint32_t L, uint32_t per) { return 4 * 3 * L * L + 20 * 2 * per * (L * L / 8); }
@@ -379,18 +386,18 @@ hipError_t plane_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes) {
 }
 
 void launch_plane(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
-                  const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                  const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                  const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* kept, uint32_t* rings,
+                  uint64_t* ver, const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
                   uint32_t per) {
   set_plane_attribute();
   hipEvent_t t0, t1;
   get_launch_timing(&t0, &t1);
   if (t0)
-    hipExtLaunchKernelGGL(k_plane, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, rings, ver,
-                          stepp, step_off, nsteps, step_out, status, per);
+    hipExtLaunchKernelGGL(k_plane, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, kept,
+                          rings, ver, stepp, step_off, nsteps, step_out, status, per);
   else
-    hipLaunchKernelGGL(k_plane, dim3(ngroups), dim3(block), lds_bytes, st, grp, slabs, pts, words, rings, ver, stepp,
-                       step_off, nsteps, step_out, status, per);
+    hipLaunchKernelGGL(k_plane, dim3(ngroups), dim3(block), lds_bytes, st, grp, slabs, pts, words, kept, rings, ver,
+                       stepp, step_off, nsteps, step_out, status, per);
 }
 
 }  // namespace cvf

@@ -63,9 +63,12 @@
 // overwritten before they are read.
 //
 // Every wait is bounded: a wait that times out, or sees another workgroup's
-// abort, sets the abort flag in `status`; from then on every workgroup skips
-// its remaining work and waits (its barriers still run, uniformly), writes
-// nothing back, and the host reports the error.
+// abort, sets the abort flag in `status`; from then on every workgroup of a
+// split point skips its remaining work and waits (its barriers still run,
+// uniformly) and writes nothing back.  What other processes run on the card can
+// bring that about, so a launch first stores the planes that it starts from in
+// `kept`, and the host does the steps since then again with launches that wait
+// for nothing.
 #include "cvf_device.h"
 #include "cvf_kernels.h"
 #include "cvf_ring.h"
@@ -449,7 +452,8 @@ __device__ __forceinline__ bool colour_ghosts(uint32_t* W, uint32_t li, uint32_t
 template <bool FINE, bool FAST>
 __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__ grp, const RSlab* __restrict__ slabs,
                                                     const PointDev* __restrict__ pts, uint32_t* __restrict__ words,
-                                                    uint32_t* __restrict__ rings, uint64_t* __restrict__ ver,
+                                                    uint32_t* __restrict__ kept, uint32_t* __restrict__ rings,
+                                                    uint64_t* __restrict__ ver,
                                                     const uint64_t* __restrict__ stepp, uint64_t step_off,
                                                     uint32_t nsteps, uint64_t* __restrict__ step_out,
                                                     uint32_t* __restrict__ status) {
@@ -466,6 +470,7 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   // sits in the lower half of its ring only)
   __shared__ uint32_t below1_s[kMaxRSlabs];
   const RGroupEnt G = grp[blockIdx.x];
+  const uint32_t flag = status[0];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni(tid >> 6);
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(slabs + G.first);
@@ -524,7 +529,39 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
     }
   }
   __syncthreads();
+  // the slab's planes from its window to the array `to`, one quad per lane and item
+  const auto store_planes = [&](uint32_t* to) {
+    const uint32_t L = F(L), hL = L / 2, LL = L * L, Q4 = LL / 4, gofs = F(ns) > 1 ? 1u : 0u;
+    uint32_t* Wp = to + F(woff) + F(z0) * LL;
+    const uint4* Wl = reinterpret_cast<const uint4*>(lds + F(lds) + gofs * LL);
+    const FastDiv dq{Q4, F(mP4)}, dH{hL, F(mH)};
+    if ((hL & 3u) == 0) {
+      // four quads along x per lane and item: 16-byte rows of `words`
+      for (uint32_t i = 4 * li; i < F(T) * Q4; i += 256 * F(nw)) {
+        const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
+        const uint4 q0 = Wl[i], q1 = Wl[i + 1], q2 = Wl[i + 2], q3 = Wl[i + 3];
+        uint4* d = reinterpret_cast<uint4*>(Wp + p * LL + x + L * y);
+        d[0] = make_uint4(q0.x, q1.x, q2.x, q3.x);
+        d[hL * L / 4] = make_uint4(q0.y, q1.y, q2.y, q3.y);
+        d[hL / 4] = make_uint4(q0.z, q1.z, q2.z, q3.z);
+        d[(hL * L + hL) / 4] = make_uint4(q0.w, q1.w, q2.w, q3.w);
+      }
+    } else {
+      for (uint32_t i = li; i < F(T) * Q4; i += 64 * F(nw)) {
+        const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
+        const uint4 v = Wl[i];
+        uint32_t* d = Wp + p * LL + x + L * y;
+        d[0] = v.x;
+        d[hL * L] = v.y;
+        d[hL] = v.z;
+        d[hL * L + hL] = v.w;
+      }
+    }
+  };
   const uint64_t step0 = (stepp ? *stepp : 0) + step_off;
+  // (not as they are staged: the next loads would wait for these stores)
+  if (has && keeps_start(kept, flag, status, step0)) store_planes(kept);
+  leave_mark(kept, flag, status, step0);
   // (a launch that moves the counter on takes its first step by value, so
   // no workgroup of it reads the counter)
   if (step_out && blockIdx.x == 0 && tid == 0) *step_out = step0 + nsteps;
@@ -906,35 +943,7 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   }
   __syncthreads();
   if (abort_s || !has) return;  // after the last barrier
-  {
-    // the slab's planes back to `words`, one quad per lane and item
-    const uint32_t L = F(L), hL = L / 2, LL = L * L, Q4 = LL / 4, gofs = F(ns) > 1 ? 1u : 0u;
-    uint32_t* Wp = words + F(woff) + F(z0) * LL;
-    const uint4* Wl = reinterpret_cast<const uint4*>(lds + F(lds) + gofs * LL);
-    const FastDiv dq{Q4, F(mP4)}, dH{hL, F(mH)};
-    if ((hL & 3u) == 0) {
-      // four quads along x per lane and item: 16-byte rows of `words`
-      for (uint32_t i = 4 * li; i < F(T) * Q4; i += 256 * F(nw)) {
-        const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
-        const uint4 q0 = Wl[i], q1 = Wl[i + 1], q2 = Wl[i + 2], q3 = Wl[i + 3];
-        uint4* d = reinterpret_cast<uint4*>(Wp + p * LL + x + L * y);
-        d[0] = make_uint4(q0.x, q1.x, q2.x, q3.x);
-        d[hL * L / 4] = make_uint4(q0.y, q1.y, q2.y, q3.y);
-        d[hL / 4] = make_uint4(q0.z, q1.z, q2.z, q3.z);
-        d[(hL * L + hL) / 4] = make_uint4(q0.w, q1.w, q2.w, q3.w);
-      }
-    } else {
-      for (uint32_t i = li; i < F(T) * Q4; i += 64 * F(nw)) {
-        const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
-        const uint4 v = Wl[i];
-        uint32_t* d = Wp + p * LL + x + L * y;
-        d[0] = v.x;
-        d[hL * L] = v.y;
-        d[hL] = v.z;
-        d[hL * L + hL] = v.w;
-      }
-    }
-  }
+  store_planes(words);
 #undef F
 }
 
@@ -969,18 +978,18 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 }
 
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
-                     const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* rings, uint64_t* ver,
-                     const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
+                     const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* kept, uint32_t* rings,
+                     uint64_t* ver, const uint64_t* stepp, uint64_t step_off, uint32_t nsteps, uint64_t* step_out, uint32_t* status,
                      bool fine, bool fast) {
   set_resident_attribute();
   hipEvent_t t0, t1;
   get_launch_timing(&t0, &t1);
   const ResidentKernel k = resident_kernel(fine, fast);
   if (t0)
-    hipExtLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, rings, ver,
-                          stepp, step_off, nsteps, step_out, status);
+    hipExtLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, t0, t1, 0, grp, slabs, pts, words, kept, rings,
+                          ver, stepp, step_off, nsteps, step_out, status);
   else
-    hipLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, grp, slabs, pts, words, rings, ver, stepp,
+    hipLaunchKernelGGL(k, dim3(ngroups), dim3(block), lds_bytes, st, grp, slabs, pts, words, kept, rings, ver, stepp,
                        step_off, nsteps, step_out, status);
 }
 

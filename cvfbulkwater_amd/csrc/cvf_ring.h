@@ -7,7 +7,9 @@
 
 namespace cvf {
 
-constexpr uint32_t kSpinLimit = 1u << 24;  // polls of one wait (~1 s with s_sleep 2)
+// polls of one wait, of the order of a second: what the steps of a launch are
+// delayed before they are done again by other launches
+constexpr uint32_t kSpinLimit = 1u << 21;
 
 // The version a slab publishes after the last step of a launch.
 __device__ __forceinline__ uint64_t end_version(uint64_t step) { return step + 1; }
@@ -20,12 +22,31 @@ __device__ __forceinline__ uint64_t end_version(uint64_t step) { return step + 1
 constexpr uint32_t kEndSlot = kRingHalf - 2;
 // first ring slot (of two) of the publish after half-sweep k
 __device__ __forceinline__ uint32_t ring_slot(uint32_t k) { return 2 * k; }
-__device__ __forceinline__ uint32_t end_tag(uint64_t step) { return (uint32_t)(step + 1) | 0x80000000u; }
+__device__ __forceinline__ uint32_t end_tag(uint64_t step) { return launch_mark(step); }
 __device__ __forceinline__ uint64_t ring_load64(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void ring_store64(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Whether this launch, whose first step is step0, keeps the lattice that it
+// starts from: no launch before it was aborted.  `flag` is status[0], through
+// the caches (as of the launch's start, or newer), loaded ahead of the lattice.
+// The first workgroup of each XCD leaves the launch's mark, long before a wait
+// of one that started after it can time out, so that workgroups which start
+// after that know that the abort is theirs.  (One address for all: as an
+// uncached load in every wavefront and a store in every workgroup these took
+// 14 us of a launch of 512 workgroups.)
+static __device__ __forceinline__ bool keeps_start(const uint32_t* kept, uint32_t flag, const uint32_t* status,
+                                                   uint64_t step0) {
+  return kept && (!flag || __hip_atomic_load(status + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                               launch_mark(step0));
+}
+static __device__ __forceinline__ void leave_mark(const uint32_t* kept, uint32_t flag, uint32_t* status,
+                                                  uint64_t step0) {
+  if (kept && !flag && blockIdx.x < kNumXcd && threadIdx.x == 0)
+    __hip_atomic_store(status + 1, launch_mark(step0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Wait until *v >= want.  False on time-out or abort.

@@ -159,10 +159,13 @@ typedef struct cvf_tuning {
                            lattice held in LDS, one stream group) where the points allow it
                            (one Metropolis sweep per step, chessboard rule), else as 1.  Its
                            workgroups wait for each other: launches of several handles of
-                           a process take turns where they might not fit together; two
-                           processes on one device should use 1.  The default is 2 for
-                           handles of one Metropolis sweep per step up to L = 64 that
-                           fit, else 1 */
+                           a process take turns where they might not fit together.  Those
+                           of two processes on one device may keep each other waiting
+                           until their waits' limit, about a second: the steps are then
+                           done again by launches of kind 1, the handle's plan from then
+                           on, so processes that share a device are better off with 1 at
+                           once.  The default is 2 for handles of one Metropolis sweep
+                           per step up to L = 64 that fit, else 1 */
   int32_t slab_planes;  /* planes per slab of the fused kernel (<= 16), or the thickest slab
                            of the resident kernel; 0 = automatic (tiles included) */
   int32_t block_chunk;  /* workgroup size of the fused kernel */
