@@ -236,8 +236,9 @@ struct cvf_sim {
   DevBuf<int32_t> freq;
   DevBuf<uint64_t> cur_steps;          // one slot per group
   DevBuf<BlockEnt> tab_cell_all;       // every point's cells, for observables
-  DevBuf<unsigned long long> hist;     // sigma histogram of one point (6 counters)
-  DevBuf<unsigned long long> hist_series;  // per-step histograms (6 counters per step)
+  // sigma histogram of one point, per-step histograms (kHistWords counters
+  // each, the abort flag before them)
+  DevBuf<unsigned long long> hist, hist_series;
   DevBuf<uint64_t> hist_base;              // step count at the first recorded step
   DevBuf<uint32_t> rstatus;                // abort flag of the resident kernel, launch_mark of the launch
   bool resident_used = false;              // some launch ran the resident kernel
@@ -1485,8 +1486,8 @@ int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = fal
     enqueue_lattice(s, gi, st, (uint32_t)i, Untimed{}, par, variant);
     if (rec) {
       const PointHost& P = s->ph[s->rec_pt];
-      launch_sigma_hist_slot(st, (par ? s->words2.p : s->words.p) + P.woff, P.N, s->hist_series.p,
-                             s->cur_steps.p + gi, (uint32_t)i, s->hist_base.p, kHistSpan);
+      launch_sigma_hist_slot(st, (par ? s->words2.p : s->words.p) + P.woff, P.N, s->hist_series.p + 1, s->rstatus.p,
+                             s->hist_series.p, s->cur_steps.p + gi, (uint32_t)i, s->hist_base.p, kHistSpan);
     }
   }
   launch_vol_chain(st, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,
@@ -1754,7 +1755,7 @@ int redo_steps(cvf_sim* s, uint32_t mark, int64_t rec_base = -1) {
   if (rc) return rc;
   if (rec_base >= 0) {
     const size_t first = (size_t)(std::max(at, rec_base) - rec_base), n = (size_t)(end - rec_base);
-    launch_zero_u32(s->stream, (uint32_t*)(s->hist_series.p + kHistWords * first), 2 * kHistWords * (n - first));
+    launch_zero_u32(s->stream, (uint32_t*)(s->hist_series.p + 1 + kHistWords * first), 2 * kHistWords * (n - first));
   }
   if ((rc = fork_groups(s))) return rc;
   while (at < end) {
@@ -2128,15 +2129,20 @@ int cvf_sigma_histogram(cvf_sim* s, int32_t pt, int64_t counts6[6]) {
   if (!counts6) return fail(CVF_EINVAL, "null output");
   HIPC(hipSetDevice(s->device));
   const PointHost& P = s->ph[pt];
-  if (!s->hist.p) HIPC(s->hist.alloc(kHistWords));  // kept for the handle's life: called every step
-  launch_zero_u32(s->stream, (uint32_t*)s->hist.p, 2 * kHistWords);
-  launch_sigma_hist(s->stream, s->words.p + P.woff, P.N, s->hist.p);
-  unsigned long long out[kHistWords];
-  HIPC(hipMemcpyAsync(out, s->hist.p, sizeof out, hipMemcpyDeviceToHost, s->stream));
-  HIPC(hipStreamSynchronize(s->stream));
+  if (!s->hist.p) HIPC(s->hist.alloc(1 + kHistWords));  // kept for the handle's life: called every step
+  unsigned long long out[1 + kHistWords];
+  bool again;
+  do {
+    again = false;
+    launch_zero_u32(s->stream, (uint32_t*)s->hist.p, 2 * (1 + kHistWords));
+    launch_sigma_hist(s->stream, s->words.p + P.woff, P.N, s->hist.p + 1, s->rstatus.p, s->hist.p);
+    HIPC(hipMemcpyAsync(out, s->hist.p, sizeof out, hipMemcpyDeviceToHost, s->stream));
+    HIPC(hipStreamSynchronize(s->stream));
+    if (out[0] && (rc = settle(s, -1, &again))) return rc;
+  } while (again);
   for (int i = 0; i < 6; ++i) {
     counts6[i] = 0;
-    for (int r = 0; r < kHistReplicas; ++r) counts6[i] += (int64_t)out[6 * r + i];
+    for (int r = 0; r < kHistReplicas; ++r) counts6[i] += (int64_t)out[1 + 6 * r + i];
   }
   return CVF_OK;
 }
@@ -2148,33 +2154,33 @@ int cvf_step_histograms(cvf_sim* s, int32_t pt, int64_t n_steps, int64_t* counts
   if (n_steps == 0) return CVF_OK;
   if (!counts) return fail(CVF_EINVAL, "null output");
   HIPC(hipSetDevice(s->device));
-  if (!s->hist_series.p) HIPC(s->hist_series.alloc(kHistWords * (size_t)kHistSpan));
+  if (!s->hist_series.p) HIPC(s->hist_series.alloc(1 + kHistWords * (size_t)kHistSpan));
   if (!s->hist_base.p) HIPC(s->hist_base.alloc(1));
   if (s->rec_pt != pt) {
     for (auto& g : s->groups) g->drop_rec_graphs();
     s->rec_pt = pt;
   }
-  int rec_gi = -1;
-  for (size_t gi = 0; gi < s->groups.size() && rec_gi < 0; ++gi)
-    for (int q : s->groups[gi]->points)
-      if (q == pt) rec_gi = (int)gi;
-  if (rec_gi < 0) return fail(CVF_EINVAL, "point %d is in no stream group", pt);
   std::vector<unsigned long long> buf;
   for (int64_t i0 = 0; i0 < n_steps; i0 += kHistSpan) {
     const int64_t n = std::min<int64_t>(kHistSpan, n_steps - i0);
     // slots are counted from the step count before this span
     s->hist_base_host = (uint64_t)s->steps;
     HIPC(hipMemcpyAsync(s->hist_base.p, &s->hist_base_host, sizeof(uint64_t), hipMemcpyHostToDevice, s->stream));
-    launch_zero_u32(s->stream, (uint32_t*)s->hist_series.p, (size_t)2 * kHistWords * n);
-    if ((rc = run_steps(s, n, rec_gi))) return rc;
-    buf.resize(kHistWords * (size_t)n);
-    HIPC(hipMemcpyAsync(buf.data(), s->hist_series.p, buf.size() * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s->stream));
-    HIPC(hipStreamSynchronize(s->stream));
+    launch_zero_u32(s->stream, (uint32_t*)s->hist_series.p, 2 * (1 + kHistWords * (size_t)n));
+    if ((rc = run_steps(s, n, s->ph[pt].group))) return rc;
+    buf.resize(1 + kHistWords * (size_t)n);
+    bool again;
+    do {
+      again = false;
+      HIPC(hipMemcpyAsync(buf.data(), s->hist_series.p, buf.size() * sizeof(unsigned long long),
+                          hipMemcpyDeviceToHost, s->stream));
+      HIPC(hipStreamSynchronize(s->stream));
+      if (buf[0] && (rc = settle(s, (int64_t)s->hist_base_host, &again))) return rc;
+    } while (again);
     for (int64_t i = 0; i < n; ++i)
       for (int v = 0; v < 6; ++v) {
         int64_t c = 0;
-        for (int r = 0; r < kHistReplicas; ++r) c += (int64_t)buf[kHistWords * i + 6 * r + v];
+        for (int r = 0; r < kHistReplicas; ++r) c += (int64_t)buf[1 + kHistWords * i + 6 * r + v];
         counts[6 * (i0 + i) + v] = c;
       }
   }
@@ -2243,17 +2249,22 @@ int cvf_cluster_stats(cvf_sim* s, int32_t pt, cvf_cstat* c) {
   const uint32_t* label = s->parent.p + P.loff;
   const uint32_t minsize = 2 * L, nw = (L + 31) / 32;
   uint32_t* nslot = s->nslot_nperc.p;
-  launch_zero3_u32(s->stream, (uint32_t*)s->csize.p, nn, nslot, 2, s->cover.p, (size_t)s->max_slots * 3 * nw);
-  launch_cluster_sizes(s->stream, label, nn, s->csize.p);
-  // the clusters' counts, moments and slots, then the percolation test of
-  // those that have a slot
-  launch_compact_count(s->stream, label, s->csize.p, nn, s->cblock.p, s->cmom.p, minsize, s->slot.p, nslot,
-                       s->max_slots);
-  launch_perc_cover(s->stream, label, nn, L, s->csize.p, minsize, s->slot.p, nslot, s->cover.p, s->max_slots);
-  launch_perc_count(s->stream, s->cover.p, nslot, L, s->max_slots, nslot + 1);
-  launch_compact_scan(s->stream, s->cblock.p, nn, s->cmom.p, nslot, s->csums.p);
-  HIPC(hipGetLastError());
-  HIPC(hipStreamSynchronize(s->stream));
+  bool again;
+  do {
+    again = false;
+    launch_zero3_u32(s->stream, (uint32_t*)s->csize.p, nn, nslot, 2, s->cover.p, (size_t)s->max_slots * 3 * nw);
+    launch_cluster_sizes(s->stream, label, nn, s->csize.p);
+    // the clusters' counts, moments and slots, then the percolation test of
+    // those that have a slot
+    launch_compact_count(s->stream, label, s->csize.p, nn, s->cblock.p, s->cmom.p, minsize, s->slot.p, nslot,
+                         s->max_slots);
+    launch_perc_cover(s->stream, label, nn, L, s->csize.p, minsize, s->slot.p, nslot, s->cover.p, s->max_slots);
+    launch_perc_count(s->stream, s->cover.p, nslot, L, s->max_slots, nslot + 1);
+    launch_compact_scan(s->stream, s->cblock.p, nn, s->cmom.p, nslot, s->rstatus.p, s->csums.p);
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(s->stream));
+    if (s->csums.p->aborted && (rc = settle(s, -1, &again))) return rc;
+  } while (again);
   const ClusterSums& sums = *s->csums.p;
   const uint32_t np[2] = {sums.slots, sums.percolating}, ncl = sums.clusters;
   if (np[0] > s->max_slots) return fail(CVF_EDEVICE, "percolation slot overflow");

@@ -146,23 +146,26 @@ void launch_sw_local(hipStream_t st, Launch ln, const uint32_t* words, uint32_t*
 void launch_sw_union(hipStream_t st, Launch ln, uint32_t* parent, const uint8_t* cov);
 void launch_sw_flip(hipStream_t st, Launch ln, uint32_t* words, uint32_t* parent, uint32_t jc);
 // sigma histogram as kHistReplicas partial histograms of 6 counters
-// (kHistWords counters, zeroed by the caller) that the caller sums
+// (kHistWords counters, zeroed by the caller) that the caller sums; *flag: the
+// resident launches' abort flag
 constexpr int kHistReplicas = 8;
 constexpr int kHistWords = 6 * kHistReplicas;
-void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* counts);
+void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* counts,
+                       const uint32_t* rstatus, unsigned long long* flag);
 // the same into slot (*gstep + step_off - *base) of a per-step series of
 // `span` histograms (graph-replayable: the slot is read on the device)
 void launch_sigma_hist_slot(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* series,
-                            const uint64_t* gstep, uint32_t step_off, const uint64_t* base, uint32_t span);
+                            const uint32_t* rstatus, unsigned long long* flag, const uint64_t* gstep,
+                            uint32_t step_off, const uint64_t* base, uint32_t span);
 // cluster statistics of one point (labels at `label`, 6N nodes)
 // Per cluster root the cluster's other nodes (others[0..nn) zero before).
 void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* others);
 // A labelling's clusters in host memory (pinned): their count, the sum and sum
 // of squares of their sizes, the largest two, the percolation slots taken and
-// the percolating ones.
+// the percolating ones; the resident launches' abort flag.
 struct ClusterSums {
   uint64_t sum, squares;
-  uint32_t largest, second, clusters, slots, percolating, pad;
+  uint32_t largest, second, clusters, slots, percolating, aborted;
 };
 // Counts and moments per workgroup of kCompactSpan nodes (bcount and 4 words
 // each of bmom, compact_blocks(nn) of them) and a slot for each cluster of at
@@ -173,7 +176,7 @@ uint32_t compact_blocks(uint32_t nn);
 void launch_compact_count(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn, uint32_t* bcount,
                           uint64_t* bmom, uint32_t minsize, int32_t* slot, uint32_t* nslot, uint32_t max_slots);
 void launch_compact_scan(hipStream_t st, uint32_t* bcount, uint32_t nn, const uint64_t* bmom,
-                         const uint32_t* nslot_nperc, ClusterSums* out);
+                         const uint32_t* nslot_nperc, const uint32_t* rstatus, ClusterSums* out);
 void launch_compact_write(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn,
                           const uint32_t* bcount, int32_t* out);
 void launch_perc_cover(hipStream_t st, const uint32_t* label, uint32_t nn, uint32_t L, const int32_t* others,

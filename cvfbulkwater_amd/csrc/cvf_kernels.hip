@@ -965,8 +965,11 @@ __global__ __launch_bounds__(256) void k_config_decode(const uint32_t* __restric
 // written.
 __global__ __launch_bounds__(256) void k_sigma_hist(const uint32_t* __restrict__ W, uint32_t N,
                                                     unsigned long long* __restrict__ counts,
+                                                    const uint32_t* __restrict__ rstatus,
+                                                    unsigned long long* __restrict__ flag,
                                                     const uint64_t* __restrict__ gstep, uint32_t step_off,
                                                     const uint64_t* __restrict__ base, uint32_t span) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = *rstatus;
   if (gstep) {
     const uint64_t slot = *gstep + step_off - *base;
     if (slot >= span) return;  // uniform over the grid
@@ -1323,6 +1326,7 @@ __global__ __launch_bounds__(256) void k_compact_count(const uint32_t* __restric
 __global__ __launch_bounds__(256) void k_compact_scan(uint32_t* __restrict__ bcount, uint32_t nb,
                                                       const uint64_t* __restrict__ bmom,
                                                       const uint32_t* __restrict__ nslot_nperc,
+                                                      const uint32_t* __restrict__ rstatus,
                                                       ClusterSums* __restrict__ out) {
   __shared__ uint32_t sh[4];
   __shared__ uint64_t shm[16], sums[4];
@@ -1347,6 +1351,7 @@ __global__ __launch_bounds__(256) void k_compact_scan(uint32_t* __restrict__ bco
     out->clusters = run;
     out->slots = nslot_nperc[0];
     out->percolating = nslot_nperc[1];
+    out->aborted = *rstatus;
   }
 }
 
@@ -1667,13 +1672,15 @@ void launch_sw_flip(hipStream_t st, Launch ln, uint32_t* words, uint32_t* parent
 }
 // workgroups of the sigma histogram: about 4 cells per thread, at most 256
 static dim3 hist_grid(uint32_t N) { return dim3(std::max(1u, std::min(256u, (N + 1023) / 1024))); }
-void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* counts) {
-  launch(k_sigma_hist, hist_grid(N), dim3(256), st, W, N, counts, (const uint64_t*)nullptr, 0u,
+void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* counts,
+                       const uint32_t* rstatus, unsigned long long* flag) {
+  launch(k_sigma_hist, hist_grid(N), dim3(256), st, W, N, counts, rstatus, flag, (const uint64_t*)nullptr, 0u,
          (const uint64_t*)nullptr, 0u);
 }
 void launch_sigma_hist_slot(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* series,
-                            const uint64_t* gstep, uint32_t step_off, const uint64_t* base, uint32_t span) {
-  launch(k_sigma_hist, hist_grid(N), dim3(256), st, W, N, series, gstep, step_off, base, span);
+                            const uint32_t* rstatus, unsigned long long* flag, const uint64_t* gstep,
+                            uint32_t step_off, const uint64_t* base, uint32_t span) {
+  launch(k_sigma_hist, hist_grid(N), dim3(256), st, W, N, series, rstatus, flag, gstep, step_off, base, span);
 }
 void launch_cluster_sizes(hipStream_t st, const uint32_t* label, uint32_t nn, int32_t* others) {
   launch(k_cluster_sizes, grid1(nn, 256), dim3(256), st, label, nn, others);
@@ -1685,8 +1692,8 @@ void launch_compact_count(hipStream_t st, const uint32_t* label, const int32_t* 
          nslot, max_slots);
 }
 void launch_compact_scan(hipStream_t st, uint32_t* bcount, uint32_t nn, const uint64_t* bmom,
-                         const uint32_t* nslot_nperc, ClusterSums* out) {
-  launch(k_compact_scan, dim3(1), dim3(256), st, bcount, compact_blocks(nn), bmom, nslot_nperc, out);
+                         const uint32_t* nslot_nperc, const uint32_t* rstatus, ClusterSums* out) {
+  launch(k_compact_scan, dim3(1), dim3(256), st, bcount, compact_blocks(nn), bmom, nslot_nperc, rstatus, out);
 }
 void launch_compact_write(hipStream_t st, const uint32_t* label, const int32_t* others, uint32_t nn,
                           const uint32_t* bcount, int32_t* out) {

@@ -98,9 +98,21 @@ def profile(a, b):
     b.step(3)
 
 
+def read_clusters(a, b):
+    assert a.cluster_stats(1) == b.cluster_stats(1)
+
+
+def read_histogram(a, b):
+    assert np.array_equal(a.sigma_histogram(1), b.sigma_histogram(1))
+
+
+def record(a, b):
+    assert np.array_equal(a.step_histograms(21, 1), b.step_histograms(21, 1))
+
+
 # the first call after the aborted launch
-@pytest.mark.parametrize("call", [read_config, read_labels, load_config, refuse_config, retune, tune, profile],
-                         ids=lambda f: f.__name__)
+@pytest.mark.parametrize("call", [read_config, read_labels, load_config, refuse_config, retune, tune, profile,
+                                  read_clusters, read_histogram, record], ids=lambda f: f.__name__)
 def test_every_call_finds_the_steps_done(call):
     a, b = handles([16, 16], nc=1)
     for s in (a, b):
@@ -111,4 +123,17 @@ def test_every_call_finds_the_steps_done(call):
     call(a, b)
     for s in (a, b):
         s.step(2)
+    same_lattices(a, b)
+
+
+# aborted in the first and a later launch of the recorded steps (a launch per step)
+@pytest.mark.parametrize("Ls,nc", [([16], 1), ([12, 32], 0)])
+@pytest.mark.parametrize("n", [1, 40])
+def test_recorded_steps_are_done_again(Ls, nc, n):
+    a, b = handles(Ls, nc)
+    a.step(3)
+    b.step(3)
+    abort_next(a)
+    assert np.array_equal(a.step_histograms(n, 0), b.step_histograms(n, 0))
+    assert np.array_equal(a.step_histograms(5, 0), b.step_histograms(5, 0))
     same_lattices(a, b)
