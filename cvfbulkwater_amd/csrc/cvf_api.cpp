@@ -225,7 +225,6 @@ struct cvf_sim {
 
   DevBuf<uint32_t> words, words2, parent, cover, nslot_nperc;  // words2: ping-pong partner
   DevBuf<uint8_t> cov, cfg_bytes;
-  DevBuf<uint32_t> cfg_res;                 // first value out of range, inconsistent cubes, abort flag
   DevBuf<int32_t> csize, slot, cclusters;  // clusters' nodes but their roots, percolation slots, compacted sizes
   DevBuf<uint32_t> cblock;                  // per-workgroup cluster counts of the compaction
   DevBuf<uint64_t> cmom;                    // per-workgroup size moments (4 words each)
@@ -396,11 +395,20 @@ int upload_point_words(cvf_sim* s, int pt, const std::vector<uint32_t>& w) {
   return CVF_OK;
 }
 
+// Configurations of fewer cells than this are brought to the host as words and
+// unpacked there, and their arrays go down in one copy: the runtime takes about
+// 1 us per KB for copies of less than 64 KB, so the 12 bytes per cell of the
+// arrays cost more than the host's work.  get_config of L = 8 / 16 / 24 / 28: 30 / 40 / 68
+// / 90 us (first call of a handle 43 / 50 / 79 / 103), unpacked on the device 55 / 74 / 130 /
+// 65 - 170 (63 / 90 / 137 / 180); L = 32 / 40: 122 / 106 (137 / 214) and 71 / 87 (80 / 124).
+constexpr uint32_t kSmallConfig = 1u << 15;
+
 // Device copy of a point's sigma and eta bytes, kept for the next call
-// (sized for the largest point that asked).
+// (sized for the largest point that asked), and after them what becomes of an
+// input: first value out of range, inconsistent cubes, abort flag.
+constexpr size_t kConfigResults = 3 * sizeof(uint32_t);
 int reserve_config(cvf_sim* s, size_t n6) {
-  if (!s->cfg_res.p) HIPC(s->cfg_res.alloc(3));
-  if (2 * n6 > s->cfg_bytes.n) HIPC(s->cfg_bytes.alloc(2 * n6));
+  if (2 * n6 + kConfigResults > s->cfg_bytes.n) HIPC(s->cfg_bytes.alloc(2 * n6 + kConfigResults));
   return CVF_OK;
 }
 
@@ -1944,16 +1952,27 @@ int cvf_set_config(cvf_sim* s, int32_t pt, const uint8_t* sigma6N, const uint8_t
   const PointHost& P = s->ph[pt];
   const size_t n6 = 6 * (size_t)P.N;
   if ((rc = reserve_config(s, n6))) return rc;
-  // words2 is free between steps (unless a resident launch was aborted): the
-  // packed input, decoded into words
-  uint32_t* res = s->cfg_res.p;
+  uint8_t* dev = s->cfg_bytes.p;
+  uint32_t* res = reinterpret_cast<uint32_t*>(dev + 2 * n6);
+  std::vector<uint8_t> in;  // both arrays and the results' initial bits, of a small point
+  if (P.N < kSmallConfig) {
+    in.assign(2 * n6 + kConfigResults, 0xFF);
+    memcpy(in.data(), sigma6N, n6);
+    memcpy(in.data() + n6, eta6N, n6);
+  }
   uint32_t out[3];
   for (;;) {
-    HIPC(hipMemcpyAsync(s->cfg_bytes.p, sigma6N, n6, hipMemcpyHostToDevice, s->stream));
-    HIPC(hipMemcpyAsync(s->cfg_bytes.p + n6, eta6N, n6, hipMemcpyHostToDevice, s->stream));
-    HIPC(hipMemsetAsync(res, 0xFF, 2 * sizeof(uint32_t), s->stream));
-    launch_config_in(s->stream, s->cfg_bytes.p, s->cfg_bytes.p + n6, P.L, P.prm.flag_chessboard,
-                     s->words2.p + P.woff, s->words.p + P.woff, res, res + 1, s->rstatus.p, res + 2);
+    if (!in.empty()) {
+      HIPC(hipMemcpyAsync(dev, in.data(), in.size(), hipMemcpyHostToDevice, s->stream));
+    } else {
+      HIPC(hipMemcpyAsync(dev, sigma6N, n6, hipMemcpyHostToDevice, s->stream));
+      HIPC(hipMemcpyAsync(dev + n6, eta6N, n6, hipMemcpyHostToDevice, s->stream));
+      HIPC(hipMemsetAsync(res, 0xFF, kConfigResults, s->stream));
+    }
+    // words2 is free between steps (unless a resident launch was aborted): the
+    // packed input, decoded into words
+    launch_config_in(s->stream, dev, dev + n6, P.L, P.prm.flag_chessboard, s->words2.p + P.woff, s->words.p + P.woff,
+                     res, res + 1, s->rstatus.p, res + 2);
     HIPC(hipGetLastError());
     HIPC(hipMemcpyAsync(out, res, sizeof out, hipMemcpyDeviceToHost, s->stream));
     HIPC(hipStreamSynchronize(s->stream));
@@ -1976,7 +1995,20 @@ int cvf_get_config(cvf_sim* s, int32_t pt, uint8_t* sigma6N, uint8_t* eta6N) {
   if (rc) return rc;
   HIPC(hipSetDevice(s->device));
   const PointHost& P = s->ph[pt];
-  const size_t n6 = 6 * (size_t)P.N;
+  const size_t N = P.N, n6 = 6 * N;
+  if (N < kSmallConfig) {
+    HIPC(hipStreamSynchronize(s->stream));
+    if ((rc = settle(s))) return rc;
+    std::vector<uint32_t> w(N);
+    HIPC(hipMemcpy(w.data(), s->words.p + P.woff, N * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    for (int a = 0; a < 6; ++a) {
+      if (sigma6N)
+        for (size_t c = 0; c < N; ++c) sigma6N[a * N + c] = (uint8_t)sigma_of(w[c], a);
+      if (eta6N)
+        for (size_t c = 0; c < N; ++c) eta6N[a * N + c] = (uint8_t)eta_of(w[c], a);
+    }
+    return CVF_OK;
+  }
   if ((rc = reserve_config(s, n6))) return rc;
   bool again;
   do {
