@@ -228,7 +228,6 @@ struct cvf_sim {
   DevBuf<int32_t> csize, slot, cclusters;  // clusters' nodes but their roots, percolation slots, compacted sizes
   DevBuf<uint32_t> cblock;                  // per-workgroup cluster counts of the compaction
   DevBuf<uint64_t> cmom;                    // per-workgroup size moments (4 words each)
-  PinBuf<ClusterSums> csums;
   DevBuf<PointDev> pts;
   DevBuf<PointState> pst;
   DevBuf<float> dist;
@@ -253,15 +252,17 @@ struct cvf_sim {
   bool sw_labels = false;  // the labels hold a Swendsen-Wang step's (all zero before the first)
   // the sample of step obs_at: written by k_observe, the partial sums added
   // up per point
-  PinBuf<uint2> obs_part;
-  PinBuf<PointState> obs_ps;
-  PinBuf<uint32_t> obs_status;
+  // (one allocation, which is most of what they cost: 70 us each)
+  PinBuf<uint64_t> pinned;
+  ClusterSums* csums = nullptr;
+  uint2* obs_part = nullptr;
+  PointState* obs_ps = nullptr;
+  uint32_t *obs_status = nullptr, *obs_capped = nullptr;
   // non-chessboard points: their table, bond bytes (one per cell of the
   // handle) and capped counts (by point)
   DevBuf<CappedEnt> tab_capped;
   uint32_t n_capped = 0, capped_L = 0;
   DevBuf<uint8_t> bonds;
-  PinBuf<uint32_t> obs_capped;
   std::vector<int32_t> obs_point;  // point of each k_observe workgroup (-1: padding)
   std::vector<int64_t> obs_nhb2, obs_nsig;
 
@@ -1338,15 +1339,12 @@ int build_groups(cvf_sim* s) {
   if (rc0) return rc0;
   std::vector<int> all(s->npts);
   for (int i = 0; i < s->npts; ++i) all[i] = i;
-  if (!s->obs_part.p) {  // the observables' table does not depend on the tuning
+  if (!s->pinned.p) {  // the observables' table does not depend on the tuning
     const auto ta = make_table(s->ph, all, observe_span(s->total_cells), cells_all);
     int rc = upload_vec(s->tab_cell_all, ta);
     if (rc) return rc;
     s->nb_cell_all = (uint32_t)ta.size();
     for (const BlockEnt& en : ta) s->obs_point.push_back(en.point);
-    HIPC(s->obs_ps.alloc(s->npts));
-    HIPC(s->obs_status.alloc(1));
-    HIPC(s->obs_part.alloc(ta.size()));
     std::vector<CappedEnt> tc;
     for (int p = 0; p < s->npts; ++p) {
       const PointHost& P = s->ph[p];
@@ -1357,9 +1355,16 @@ int build_groups(cvf_sim* s) {
     if (!tc.empty()) {
       if ((rc = upload_vec(s->tab_capped, tc))) return rc;
       HIPC(s->bonds.alloc(s->total_cells));
-      HIPC(s->obs_capped.alloc(s->npts));
       s->n_capped = (uint32_t)tc.size();
     }
+    static_assert(sizeof(ClusterSums) % 8 == 0 && sizeof(PointState) % 8 == 0 && sizeof(uint2) == 8, "8-byte words");
+    const size_t n = (size_t)s->npts, ps_at = sizeof(ClusterSums) / 8, part_at = ps_at + n * (sizeof(PointState) / 8);
+    HIPC(s->pinned.alloc(part_at + ta.size() + 1 + (n + 1) / 2));
+    s->csums = reinterpret_cast<ClusterSums*>(s->pinned.p);
+    s->obs_ps = reinterpret_cast<PointState*>(s->pinned.p + ps_at);
+    s->obs_part = reinterpret_cast<uint2*>(s->pinned.p + part_at);
+    s->obs_status = reinterpret_cast<uint32_t*>(s->pinned.p + part_at + ta.size());
+    s->obs_capped = reinterpret_cast<uint32_t*>(s->pinned.p + part_at + ta.size() + 1);
   }
   HIPC(hipDeviceSynchronize());
   return CVF_OK;
@@ -1878,7 +1883,6 @@ int create_impl(const cvf_params* pts, int32_t n, cvf_sim** out) {
   HIPC(s->cclusters.alloc(6 * (size_t)maxN));
   HIPC(s->cblock.alloc(compact_blocks(6 * maxN)));
   HIPC(s->cmom.alloc(4 * (size_t)compact_blocks(6 * maxN)));
-  HIPC(s->csums.alloc(1));
   s->max_slots = 3 * maxL * maxL + 1;  // a cluster of >= 2L nodes: at most 6N/(2L)
   HIPC(s->cover.alloc((size_t)s->max_slots * 3 * ((maxL + 31) / 32)));
   HIPC(s->nslot_nperc.alloc(2));
@@ -2114,28 +2118,28 @@ int cvf_observe(cvf_sim* s, int32_t pt, cvf_obs* o) {
   HIPC(hipSetDevice(s->device));
   while (s->obs_at != s->steps) {
     launch_observe(s->stream, s->tab_cell_all.p, s->nb_cell_all, s->words.p, observe_span(s->total_cells), s->pst.p,
-                   s->rstatus.p, ObsOut{s->obs_part.p, s->obs_ps.p, s->obs_status.p}, s->bonds.p);
+                   s->rstatus.p, ObsOut{s->obs_part, s->obs_ps, s->obs_status}, s->bonds.p);
     if (s->n_capped)
-      launch_capped_hb(s->stream, s->tab_capped.p, s->n_capped, s->capped_L, s->bonds.p, s->obs_capped.p);
+      launch_capped_hb(s->stream, s->tab_capped.p, s->n_capped, s->capped_L, s->bonds.p, s->obs_capped);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
     bool again = false;
-    if (*s->obs_status.p && (rc = settle(s, -1, &again))) return rc;
+    if (*s->obs_status && (rc = settle(s, -1, &again))) return rc;
     if (again) continue;
     s->obs_nhb2.assign(s->npts, 0);
     s->obs_nsig.assign(s->npts, 0);
     for (size_t b = 0; b < s->obs_point.size(); ++b)
       if (s->obs_point[b] >= 0) {
-        s->obs_nhb2[s->obs_point[b]] += s->obs_part.p[b].x;
-        s->obs_nsig[s->obs_point[b]] += s->obs_part.p[b].y;
+        s->obs_nhb2[s->obs_point[b]] += s->obs_part[b].x;
+        s->obs_nsig[s->obs_point[b]] += s->obs_part[b].y;
       }
     s->obs_at = s->steps;
   }
   // the volume chain as of the same step
-  const VolState& vol = s->vol_device ? s->obs_ps.p[pt].vol : s->ph[pt].vol;
+  const VolState& vol = s->vol_device ? s->obs_ps[pt].vol : s->ph[pt].vol;
   const double r_cell = vol.r_cell, E_vdw = vol.E_vdw;
   const PointHost& P = s->ph[pt];
-  const int64_t nhb2 = P.prm.flag_chessboard ? s->obs_nhb2[pt] : (int64_t)s->obs_capped.p[pt];
+  const int64_t nhb2 = P.prm.flag_chessboard ? s->obs_nhb2[pt] : (int64_t)s->obs_capped[pt];
   const int64_t nsig = s->obs_nsig[pt];
   // measure(), gpu_water3D.cu:2138-2152
   const double n_hb = 0.5 * (double)nhb2;
@@ -2292,12 +2296,12 @@ int cvf_cluster_stats(cvf_sim* s, int32_t pt, cvf_cstat* c) {
                          s->max_slots);
     launch_perc_cover(s->stream, label, nn, L, s->csize.p, minsize, s->slot.p, nslot, s->cover.p, s->max_slots);
     launch_perc_count(s->stream, s->cover.p, nslot, L, s->max_slots, nslot + 1);
-    launch_compact_scan(s->stream, s->cblock.p, nn, s->cmom.p, nslot, s->rstatus.p, s->csums.p);
+    launch_compact_scan(s->stream, s->cblock.p, nn, s->cmom.p, nslot, s->rstatus.p, s->csums);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));
-    if (s->csums.p->aborted && (rc = settle(s, -1, &again))) return rc;
+    if (s->csums->aborted && (rc = settle(s, -1, &again))) return rc;
   } while (again);
-  const ClusterSums& sums = *s->csums.p;
+  const ClusterSums& sums = *s->csums;
   const uint32_t np[2] = {sums.slots, sums.percolating}, ncl = sums.clusters;
   if (np[0] > s->max_slots) return fail(CVF_EDEVICE, "percolation slot overflow");
   if (ncl == 0 || ncl > nn) return fail(CVF_EDEVICE, "cluster compaction overflow");
