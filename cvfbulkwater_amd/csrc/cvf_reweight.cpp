@@ -264,7 +264,7 @@ struct cvf_reweight {
   DMem<uint32_t> scode, scbin;
   HMem<double> sout;
   int32_t cap_pairs = 0, cap_angles = 0;
-  size_t cap_parts = 0;
+  size_t cap_parts = 0, cap_cbin = 0;
 
   RwCells cells() const { return RwCells{en.p, vn.p, lh.p, (int64_t)cell.size()}; }
   RwWork work(int32_t n) const {
@@ -704,13 +704,18 @@ int cvf_rw_scan(cvf_reweight* rw, int32_t n_targets, const double* T_K, const do
     const size_t pairs = (size_t)std::max(nta, rw->cap_pairs), ang = (size_t)std::max(n_angles, rw->cap_angles);
     rw->cap_pairs = rw->cap_angles = 0;
     HIPR(rw->sbin.alloc(pairs + ang));
-    HIPR(rw->scbin.alloc(ang * rw->cell.size()));  // at most a group per angle
     HIPR(rw->scode.alloc(pairs));
     // 2 cumulants per target (at most one target per pair), 2 nm + 9 numbers
     // and a code per pair
     HIPR(rw->sout.resize(pairs * (2 * (size_t)nm + 12)));
     rw->cap_pairs = (int32_t)pairs;
     rw->cap_angles = (int32_t)ang;
+  }
+  const size_t n_cbin = (size_t)rw_angle_groups(nm, n_angles) * rw->cell.size();
+  if (n_cbin > rw->cap_cbin) {
+    rw->cap_cbin = 0;
+    HIPR(rw->scbin.alloc(n_cbin));
+    rw->cap_cbin = n_cbin;
   }
   const int32_t n_proj = rw_proj_blocks((int64_t)rw->cell.size(), n_targets);
   const size_t parts = (size_t)(nta + n_angles) * n_proj;

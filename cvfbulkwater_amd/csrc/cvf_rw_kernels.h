@@ -98,6 +98,8 @@ struct RwScan {
 // left most CUs idle for a few targets.  One angle, 710,000 cells, 1 / 5 / 10 / 16
 // targets: 64 workgroups 217 / 235 / 248 / 262 us, so many 131 / 150 / 178 / 210.
 int32_t rw_proj_blocks(int64_t n_cells, int32_t n_targets);
+// Groups of angles that a pass over the cells takes together (RwScan::cbin).
+int32_t rw_angle_groups(int32_t nm, int32_t n_a);
 // What went wrong with a pair: no cell of positive density, an x outside its
 // bins, moments off before or after the axis stretch.
 enum : uint32_t { kRwNoCell = 1, kRwOutside = 2, kRwMoments = 4, kRwStretched = 8 };

@@ -1198,17 +1198,24 @@ hipError_t xhist_launch(const RwGeom& g, const RwCells& cells, const RwTargets& 
   hipLaunchKernelGGL(k_rw_cell_bins<NA>, dim3((unsigned)((g.n + kRwBlock - 1) / kRwBlock), groups), dim3(kRwBlock), 0,
                      st, g, sc);
   const size_t lds = sizeof(double) * NA * kRwRows * (size_t)(g.nm | 1);
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rw_xhist<NA>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-  }
   hipLaunchKernelGGL(k_rw_xhist<NA>, dim3((unsigned)sc.n_proj, (unsigned)tg.n * groups), dim3(64), lds, st, g,
                      cells, tg, w, sc);
   return hipGetLastError();
 }
 
+// Angles per wavefront: as many (up to 4) as keep five wavefronts on a CU, one
+// at least (27 KB of LDS for 215 bins).
+int angles_per_wave(int nm, int n_a) {
+  const int fit = (int)(32 * 1024 / (sizeof(double) * kRwRows * (size_t)(nm | 1)));
+  return std::max(1, std::min({fit, n_a, 4}));
+}
+
 }  // namespace
+
+int32_t rw_angle_groups(int32_t nm, int32_t n_a) {
+  const int per = angles_per_wave(nm, n_a);
+  return (n_a + per - 1) / per;
+}
 
 // At most 256 workgroups per row of targets, since every workgroup of the
 // next launch reduces their partial results for itself, and at most one of
@@ -1288,9 +1295,7 @@ hipError_t launch_rw_project(const RwCells& cells, const RwTargets& tg, const Rw
   hipLaunchKernelGGL(k_rw_xrange, dim3((unsigned)sc.n_proj, (unsigned)sc.n_a + nta), dim3(kRwBlock), 0, st, g, cells, tg, w,
                      sc);
   hipLaunchKernelGGL(k_rw_bins, dim3((unsigned)sc.n_a + nta), dim3(64), 0, st, w, sc, g.nm);
-  // angles per wavefront: as many (up to 4) as keep five wavefronts on a CU
-  const int fit = (int)(32 * 1024 / (sizeof(double) * kRwRows * (size_t)(g.nm | 1)));
-  const int na = fit < sc.n_a ? fit : sc.n_a;
+  const int na = angles_per_wave(g.nm, sc.n_a);
   const hipError_t e = na >= 4   ? xhist_launch<4>(g, cells, tg, w, sc, st)
                        : na == 3 ? xhist_launch<3>(g, cells, tg, w, sc, st)
                        : na == 2 ? xhist_launch<2>(g, cells, tg, w, sc, st)

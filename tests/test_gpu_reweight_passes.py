@@ -131,3 +131,16 @@ def test_scan_refuses_what_has_no_density(ctes, P):
             eng.scan([200.4], [P], [1.5])
         assert not np.any(eng.reweight([200.4], [P]) == 0.0)
         assert not np.any(eng.density(0) > 0)
+
+
+def test_buffers_of_one_handle_grow_and_serve_smaller_calls():
+    """Scans with more angles, more targets (also than the buffers have room
+    for at first) and fewer of both on one handle, its constants solved between."""
+    Ts, data = isobar(3, 1500)
+    with Reweighting(8, Ts, [0.5] * 3, data, 0.5) as eng:
+        first, _, _ = eng.solve_constants(40)
+        for n_t, n_a in ((2, 1), (1, 9), (70, 1), (3, 6), (66, 3), (1, 1)):
+            T = np.array([(0.1055 + 0.0015 * k / n_t) * 140.5678 + 185.4676 for k in range(n_t)])
+            P = np.array([(0.5 + 0.001 * (k % 3)) * 4694.59 - 2111.5552 for k in range(n_t)])
+            scan_matches_targets(eng, T, P, np.array([1.5 + 0.03 * a for a in range(n_a)]))
+            assert np.array_equal(eng.solve_constants(40)[0], first)
