@@ -217,10 +217,10 @@ int main(int argc, char** argv) {
   for (double S = in.Smin; S < in.Smax; S = S + in.dS) angles.push_back(S);
   const int na = (int)angles.size();
   if (na > 4096) return fprintf(stderr, "more than 4096 angles\n"), 2;
-  // targets per pass: at most 4096 (target, angle) pairs and about 2 GiB of
-  // densities, reduced on the device
+  // targets per pass: at most 4096 (target, angle) pairs and about 2 GiB of the
+  // cells' sums, nine bytes per cell for every 16 targets
   const int64_t chunk = std::max<int64_t>(
-      1, std::min<int64_t>(4096 / na, (int64_t(1) << 28) / info.n_occupied));
+      1, std::min<int64_t>(4096 / na, 16 * std::max<int64_t>(1, (int64_t(1) << 31) / (9 * info.n_occupied))));
   std::vector<double> ued, xs, ps, sts, scs;
   for (size_t t0 = 0; t0 < TK.size(); t0 += chunk) {
     const int nt = (int)std::min<size_t>(chunk, TK.size() - t0);
