@@ -423,7 +423,6 @@ struct RDeal {
   std::vector<RGroupEnt> groups;
   uint32_t lds_bytes = 0;
   size_t ring_words = 0;
-  double makespan = 0;  // largest cells per wave
 };
 
 // Waves of a workgroup for slabs of the given cells: one each, the rest by
@@ -676,7 +675,6 @@ bool plan_resident(const cvf_sim* s, const Group& g, int nwg, uint32_t wpg, uint
         ring += 4 * (size_t)kRingHalf * L * L;
       }
       out.slabs.push_back(r);
-      out.makespan = std::max(out.makespan, (double)x.T * L * L / nw[j]);
     }
     if (lds > cap) return false;
     out.lds_bytes = std::max(out.lds_bytes, lds * 4);
@@ -1178,10 +1176,10 @@ TilePlan best_tiles(const TilePoints& points, uint32_t nk, uint32_t block, uint3
 }
 
 // Fused launches can run on tiles: the reference schedule, no slab thickness
-// asked for, and the workgroups the kernel's tables need.
+// asked for, and workgroups as the kernel needs.
 bool tiles_possible(const cvf_sim* s, const cvf_tuning& t) {
   return s->sched == CVF_SCHED_REFERENCE && s->nm > 0 && t.fused != 0 && t.slab_planes == 0 &&
-         t.block_chunk >= 256;
+         t.block_chunk >= (int32_t)kTileMinBlock;
 }
 
 int cu_count(const cvf_sim* s, uint32_t& ncu) {

@@ -96,13 +96,14 @@ struct TileEnt {
 };
 constexpr int kMaxTileWin = 64;  // quads along one axis of a window
 constexpr uint32_t kMaxTile = kMaxTileWin - 2 * kMaxChunk - 2;
+constexpr uint32_t kTileMinBlock = 64 + 3 * kMaxTileWin;  // threads: a wavefront, and one per entry of the axes' tables
 // quads of the largest window of a tile for nk half-sweeps (and the cube
 // sweep; nc: of a non-chessboard point)
 uint32_t tile_window_quads(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t nk, bool nc);
 // largest dynamic LDS of a tile workgroup
 constexpr uint32_t tile_lds_limit() { return 160 * 1024 - 4096; }
 // As launch_chunk, on the ntiles (a multiple of kNumXcd) boxes of `tab`;
-// workgroups of at least 3 kMaxTileWin threads.
+// workgroups of at least kTileMinBlock threads.
 void launch_tile(hipStream_t st, const TileEnt* tab, uint32_t ntiles, uint32_t block, const uint64_t* stepp,
                  uint32_t step_off, const PointDev* pts, const uint32_t* src, uint32_t* dst, uint32_t k0, uint32_t nk,
                  int with_eta, uint32_t lds_bytes, bool any_nc);

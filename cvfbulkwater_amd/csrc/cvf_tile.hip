@@ -147,7 +147,7 @@ __global__ __launch_bounds__(1024) void k_tile(const TileEnt* __restrict__ tab, 
   }
   const uint32_t nx = (uint32_t)wn[0], ny = (uint32_t)wn[1], nz = (uint32_t)wn[2];
   const uint32_t sy = 4 * nx, sz = 4 * nx * ny;  // words per step along y and z
-  if (tid >= 64 && tid < 64 + 3 * kMaxTileWin) {
+  if (tid >= 64 && tid < kTileMinBlock) {
     const uint32_t a = (tid - 64) / kMaxTileWin, i = (tid - 64) % kMaxTileWin;
     uint32_t sw = 0;
     if (a == 0 && i < nx) {
