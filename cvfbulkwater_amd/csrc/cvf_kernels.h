@@ -244,7 +244,7 @@ hipError_t resident_occupancy(int* per_cu, uint32_t block, uint32_t lds_bytes, b
 // The lattice that it starts from stays in `kept` (null: that of an earlier
 // launch serves), for the steps to be done again if a wait times out: then
 // status[0] is not zero, and status[1] the launch_mark of the first step of the
-// launch whose start `kept` holds.  Launches after it leave `kept` alone.
+// launch whose start `kept` holds.  Launches after it with `kept` do nothing.
 constexpr uint32_t launch_mark(uint64_t step) { return (uint32_t)(step + 1) | 0x80000000u; }
 void launch_resident(hipStream_t st, const RGroupEnt* grp, uint32_t ngroups, uint32_t block, uint32_t lds_bytes,
                      const RSlab* slabs, const PointDev* pts, uint32_t* words, uint32_t* kept, uint32_t* rings,

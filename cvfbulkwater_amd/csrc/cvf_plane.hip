@@ -105,7 +105,12 @@ __global__ __launch_bounds__(1024) void k_plane(const RGroupEnt* __restrict__ gr
     }
   };
   // (not as it is staged: the next loads would wait for these stores)
-  if (keeps_start(kept, flag, status, step0)) store_plane(kept);
+  if (kept) {
+    // (the same in all threads: no workgroup of this launch was waited for in
+    // vain before its mark was there)
+    if (!keeps_start(flag, status, step0)) return;
+    store_plane(kept);
+  }
   leave_mark(kept, flag, status, step0);
   if (step_out && blockIdx.x == 0 && tid == 0) *step_out = step0 + nsteps;
   bool aborted = false;

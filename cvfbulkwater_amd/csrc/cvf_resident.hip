@@ -560,7 +560,12 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   };
   const uint64_t step0 = (stepp ? *stepp : 0) + step_off;
   // (not as they are staged: the next loads would wait for these stores)
-  if (has && keeps_start(kept, flag, status, step0)) store_planes(kept);
+  if (kept) {
+    // (the same in all threads: no workgroup of this launch was waited for in
+    // vain before its mark was there)
+    if (!keeps_start(flag, status, step0)) return;
+    if (has) store_planes(kept);
+  }
   leave_mark(kept, flag, status, step0);
   // (a launch that moves the counter on takes its first step by value, so
   // no workgroup of it reads the counter)

@@ -30,18 +30,18 @@ __device__ __forceinline__ void ring_store64(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Whether this launch, whose first step is step0, keeps the lattice that it
-// starts from: no launch before it was aborted.  `flag` is status[0], through
-// the caches (as of the launch's start, or newer), loaded ahead of the lattice.
+// Whether this launch, whose first step is step0, runs and keeps the lattice
+// that it starts from: no launch before it was aborted.  `flag` is status[0],
+// through the caches (as of the launch's start, or newer), loaded ahead of the
+// lattice.
 // The first workgroup of each XCD leaves the launch's mark, long before a wait
 // of one that started after it can time out, so that workgroups which start
 // after that know that the abort is theirs.  (One address for all: as an
 // uncached load in every wavefront and a store in every workgroup these took
 // 14 us of a launch of 512 workgroups.)
-static __device__ __forceinline__ bool keeps_start(const uint32_t* kept, uint32_t flag, const uint32_t* status,
-                                                   uint64_t step0) {
-  return kept && (!flag || __hip_atomic_load(status + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                               launch_mark(step0));
+static __device__ __forceinline__ bool keeps_start(uint32_t flag, const uint32_t* status, uint64_t step0) {
+  return !flag ||
+         __hip_atomic_load(status + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch_mark(step0);
 }
 static __device__ __forceinline__ void leave_mark(const uint32_t* kept, uint32_t flag, uint32_t* status,
                                                   uint64_t step0) {
