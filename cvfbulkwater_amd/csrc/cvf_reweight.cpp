@@ -242,7 +242,7 @@ struct cvf_reweight {
   bool have_ctes = false;
 
   hipStream_t stream = nullptr;
-  DMem<double> en, vn, lh, used, dens, sum, pmax, mx, ps, lz, norm;
+  DMem<double> en, vn, lh, used, sum, pmax, mx, ps, lz, norm;
   DMem<uint32_t> dcell;  // the occupied cells as i << 16 | w, for the projections
   DMem<uint8_t> mixed;
   DMem<RwMixed> mix;
@@ -252,8 +252,7 @@ struct cvf_reweight {
   DMem<double> th, tkt;
   DMem<double2> trow, tcol, tsc;
   int32_t cap_t = 0, n_t = 0;
-  size_t cap_dens = 0;
-  HMem<double> dist;  // [target][cell] densities of the last reweighting (pinned)
+  HMem<double> dist;  // [target][cell] densities of the last reweighting (pinned, written by the kernel)
   // a call's inputs (constants, targets, angles) go down in one copy
   HMem<double> hin;
   DMem<double> din;
@@ -589,26 +588,18 @@ int cvf_rw_reweight(cvf_reweight* rw, int32_t n_targets, const double* T_K, cons
     if (!(T_K[t] > 0)) return set_error(CVF_EINVAL, "target %d: T = %g K", t, T_K[t]);
   HIPR(hipSetDevice(rw->device));
   if (int rc = rw->reserve_targets(n_targets)) return rc;
-  const size_t nc = rw->cell.size();
-  if ((size_t)n_targets * nc > rw->cap_dens) {
-    rw->cap_dens = 0;
-    HIPR(rw->dens.alloc((size_t)n_targets * nc));
-    rw->cap_dens = (size_t)n_targets * nc;
-  }
+  rw->n_t = 0;
+  HIPR(rw->dist.resize((size_t)n_targets * rw->cell.size()));
   if (int rc = rw->upload_inputs(rw->ctes.data(), n_targets, T_K, P_bar)) return rc;
   const RwTargets tg = rw->targets(n_targets);
   HIPR(launch_rw_pass(rw->cells(), rw->sims.p, rw->dev_ctes(), rw->n_sim, tg, rw->work(tg.n), rw->geom(), kRwDensity,
                       false, nullptr, rw->stream));
   HIPR(launch_rw_finish(tg, rw->work(tg.n), rw->geom(), kRwDensity, nullptr, rw->stream));
-  HIPR(launch_rw_dist(rw->cells(), tg, rw->work(tg.n), rw->dens.p, rw->stream));
-  rw->n_t = 0;
-  HIPR(rw->dist.resize((size_t)n_targets * nc));
-  rw->n_t = n_targets;
-  HIPR(hipMemcpyAsync(rw->dist.data(), rw->dens.p, rw->dist.size() * sizeof(double), hipMemcpyDeviceToHost,
-                      rw->stream));
+  HIPR(launch_rw_dist(rw->cells(), tg, rw->work(tg.n), rw->dist.data(), rw->stream));
   std::vector<double> z(n_targets);
   HIPR(hipMemcpyAsync(z.data(), rw->lz.p, n_targets * sizeof(double), hipMemcpyDeviceToHost, rw->stream));
   HIPR(hipStreamSynchronize(rw->stream));
+  rw->n_t = n_targets;
   if (log_z) std::copy(z.begin(), z.end(), log_z);
   return CVF_OK;
 }
