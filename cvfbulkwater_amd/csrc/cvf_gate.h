@@ -83,24 +83,25 @@ struct ResidentGate {
     for (;;) {
       bool launching = false;
       if (in == me) {
-        ResidentLoad load;
-        load.add(u->plan);
-        before.clear();
-        for (User* o : users) {
-          if (o == u || o->plan.device != u->plan.device) continue;
-          if (!o->launching && (!o->pending || Streams::idle(o->stream))) {
-            o->pending = false;
-            continue;
-          }
-          before.push_back(o);
-          load.add(o->plan);
-          launching = launching || o->launching;
-        }
-        if (before.empty() || load.fits(u->plan.cus)) {
+        // with all that may be running, then (if need be) with what is
+        bool fits = false;
+        for (int look = 0; look < 2 && !fits; ++look) {
+          ResidentLoad load;
+          load.add(u->plan);
           before.clear();
-          break;
+          launching = false;
+          for (User* o : users) {
+            if (o == u || o->plan.device != u->plan.device) continue;
+            if (look && !o->launching && o->pending && Streams::idle(o->stream)) o->pending = false;
+            if (!o->launching && !o->pending) continue;
+            before.push_back(o);
+            load.add(o->plan);
+            launching = launching || o->launching;
+          }
+          fits = before.empty() || load.fits(u->plan.cus);
         }
-        if (!launching) break;
+        if (fits) before.clear();
+        if (fits || !launching) break;
       }
       // someone came earlier, or has not enqueued its launch yet
       changed.wait(lock);
