@@ -133,7 +133,8 @@ struct Group {
   bool r_fine = false;  // every slab at most two planes: the fine instantiation
   uint32_t r_per = 0;   // one plane per workgroup: the plane kernel, this many half-sweeps at a time (0: not)
   // a second stream beside `stream` for the device volume chain of a
-  // resident sequence, which never reads the lattice (fork / join events)
+  // resident sequence, which never reads the lattice (fork / join events), and
+  // for the capture of a resident group's graphs
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
   // captured step sequences, longest first: graph_steps, then the powers of
@@ -758,6 +759,11 @@ bool resident_plan_valid(const cvf_sim* s, const Group& g, const RDeal& d, uint3
 template <class T>
 int upload_vec(DevBuf<T>& buf, const std::vector<T>& v);
 
+int side_stream(Group& g) {
+  if (!g.side) HIPC(hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking));
+  return CVF_OK;
+}
+
 // With fused = 2, `streams` is the number of resident workgroups per CU (1
 // or 2) and slab_planes caps the slab thickness (0: automatic): every
 // workgroup of the launch must be resident at once, so the plan is checked
@@ -789,8 +795,8 @@ int build_resident(cvf_sim* s, Group& g) {
   }
   const bool fine = thin && fine_phase;
   // one plane per workgroup: the kernel for that, while its phases are short
-  // (one point of L = 12 / 32 / 48 / 56: 7.9 / 11.6 / 17.6 / 23.7 us per step, the
-  // general kernel 13.7 / 15.6 / 22.2 / 24.2; L = 64 25.9 and 24.4)
+  // (one point of L = 12 / 32 / 48 / 56: 7.2 / 10.3 / 16.5 / 21.0 us per step of a long run,
+  // the general kernel 13.7 / 15.8 / 22.3 / 23.6; L = 64, 64 steps a call: 25.9 and 24.4)
   bool planes = s->sched == CVF_SCHED_REFERENCE;
   uint32_t maxL = 0;
   for (const auto& r : d.slabs) {
@@ -825,8 +831,8 @@ int build_resident(cvf_sim* s, Group& g) {
   g.r_lds = d.lds_bytes;
   g.r_fine = fine;
   g.r_per = planes ? per : 0;
-  if (!g.side) {
-    HIPC(hipStreamCreateWithFlags(&g.side, hipStreamNonBlocking));
+  if (s->vol_device) {
+    if ((rc = side_stream(g))) return rc;
     HIPC(hipEventCreateWithFlags(&g.fork, hipEventDisableTiming));
     HIPC(hipEventCreateWithFlags(&g.join, hipEventDisableTiming));
   }
@@ -1537,9 +1543,11 @@ int enqueue_resident(cvf_sim* s, int gi, hipStream_t st, int nsteps) {
 int capture(cvf_sim* s, int gi, int nsteps, hipGraph_t* g, hipGraphExec_t* ge, bool rec = false) {
   // (not the stream of resident launches, on which another handle's thread may
   // record an event)
+  int rc = CVF_OK;
+  if (s->groups[gi]->resident && (rc = side_stream(*s->groups[gi]))) return rc;
   hipStream_t st = s->groups[gi]->resident ? s->groups[gi]->side : s->groups[gi]->stream;
   HIPC(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_steps(s, gi, st, nsteps, rec);
+  rc = enqueue_steps(s, gi, st, nsteps, rec);
   hipError_t e = hipStreamEndCapture(st, g);
   if (rc) return rc;
   if (e != hipSuccess) return fail(CVF_EDEVICE, "graph capture failed: %s", hipGetErrorString(e));
