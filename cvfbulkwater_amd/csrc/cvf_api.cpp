@@ -1503,8 +1503,9 @@ int enqueue_steps(cvf_sim* s, int gi, hipStream_t st, int nsteps, bool rec = fal
     enqueue_lattice(s, gi, st, (uint32_t)i, Untimed{}, par, variant);
     if (rec) {
       const PointHost& P = s->ph[s->rec_pt];
-      launch_sigma_hist_slot(st, (par ? s->words2.p : s->words.p) + P.woff, P.N, s->hist_series.p + 1, s->rstatus.p,
-                             s->hist_series.p, s->cur_steps.p + gi, (uint32_t)i, s->hist_base.p, kHistSpan);
+      launch_sigma_hist_slot(st, (par ? s->words2.p : s->words.p) + P.woff, P.N, s->hist_series.p + 1,
+                             i == nsteps - 1 ? s->rstatus.p : nullptr, s->hist_series.p, s->cur_steps.p + gi,
+                             (uint32_t)i, s->hist_base.p, kHistSpan);
     }
   }
   launch_vol_chain(st, s->pts.p, g.plist.p, (int)g.points.size(), s->pst.p, s->cur_steps.p + gi,

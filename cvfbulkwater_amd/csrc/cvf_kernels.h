@@ -148,7 +148,7 @@ void launch_sw_union(hipStream_t st, Launch ln, uint32_t* parent, const uint8_t*
 void launch_sw_flip(hipStream_t st, Launch ln, uint32_t* words, uint32_t* parent, uint32_t jc);
 // sigma histogram as kHistReplicas partial histograms of 6 counters
 // (kHistWords counters, zeroed by the caller) that the caller sums; *flag: the
-// resident launches' abort flag
+// resident launches' abort flag (with rstatus)
 constexpr int kHistReplicas = 8;
 constexpr int kHistWords = 6 * kHistReplicas;
 void launch_sigma_hist(hipStream_t st, const uint32_t* W, uint32_t N, unsigned long long* counts,

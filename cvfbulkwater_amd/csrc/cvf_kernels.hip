@@ -969,7 +969,7 @@ __global__ __launch_bounds__(256) void k_sigma_hist(const uint32_t* __restrict__
                                                     unsigned long long* __restrict__ flag,
                                                     const uint64_t* __restrict__ gstep, uint32_t step_off,
                                                     const uint64_t* __restrict__ base, uint32_t span) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = *rstatus;
+  if (rstatus && blockIdx.x == 0 && threadIdx.x == 0) *flag = *rstatus;
   if (gstep) {
     const uint64_t slot = *gstep + step_off - *base;
     if (slot >= span) return;  // uniform over the grid

@@ -22,11 +22,11 @@
 //     moving phase, the cells which rest in it alongside, and the next step's
 //     schedule, first records and cube draws are made while the neighbours'
 //     planes are on the way.
-// L = 12 / 16 / 24 / 32 / 48: 7.9 / 8.0 / 10.3 / 11.6 / 17.6 us per step, the general
-// kernel 13.7 / 13.7 / 15.2 / 15.6 / 22.2; of 18050 clocks at L = 12, 740 a phase in
-// the plane, 3500 from a step's start to its neighbours' planes, 2800 the cubes.
-// With the moves of all twelve half-sweeps at once L = 32 / 48 take 11.0 / 16.9, in
-// twice the LDS.
+// L = 12 / 16 / 24 / 32 / 48: 7.2 / 7.4 / 9.4 / 10.3 / 16.5 us per step of a long run, the
+// general kernel 13.7 / 13.6 / 15.8 / 15.8 / 22.3; of 18050 clocks at L = 12, 740 a phase
+// in the plane, 3500 from a step's start to its neighbours' planes, 2800 the cubes.
+// The moves of all twelve half-sweeps are made at once up to L = 32 (512 threads),
+// of six from L = 48 on: as a workgroup's share of LDS holds them.
 #include "cvf_device.h"
 #include "cvf_kernels.h"
 #include "cvf_ring.h"

@@ -470,7 +470,6 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   // sits in the lower half of its ring only)
   __shared__ uint32_t below1_s[kMaxRSlabs];
   const RGroupEnt G = grp[blockIdx.x];
-  const uint32_t flag = status[0];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni(tid >> 6);
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(slabs + G.first);
@@ -529,15 +528,16 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
     }
   }
   __syncthreads();
-  // the slab's planes from its window to the array `to`, one quad per lane and item
-  const auto store_planes = [&](uint32_t* to) {
-    const uint32_t L = F(L), hL = L / 2, LL = L * L, Q4 = LL / 4, gofs = F(ns) > 1 ? 1u : 0u;
-    uint32_t* Wp = to + F(woff) + F(z0) * LL;
-    const uint4* Wl = reinterpret_cast<const uint4*>(lds + F(lds) + gofs * LL);
-    const FastDiv dq{Q4, F(mP4)}, dH{hL, F(mH)};
+  // the slab's planes from its window to the array `to`, one quad per lane and
+  // item; f: its fields as scalars (or, where they cost the step loop's, not)
+  const auto store_planes = [&](uint32_t* to, auto f) {
+    const uint32_t L = f(S.L), hL = L / 2, LL = L * L, Q4 = LL / 4, gofs = f(S.ns) > 1 ? 1u : 0u;
+    uint32_t* Wp = to + f(S.woff) + f(S.z0) * LL;
+    const uint4* Wl = reinterpret_cast<const uint4*>(lds + f(S.lds) + gofs * LL);
+    const FastDiv dq{Q4, f(S.mP4)}, dH{hL, f(S.mH)};
     if ((hL & 3u) == 0) {
       // four quads along x per lane and item: 16-byte rows of `words`
-      for (uint32_t i = 4 * li; i < F(T) * Q4; i += 256 * F(nw)) {
+      for (uint32_t i = 4 * li; i < f(S.T) * Q4; i += 256 * f(S.nw)) {
         const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
         const uint4 q0 = Wl[i], q1 = Wl[i + 1], q2 = Wl[i + 2], q3 = Wl[i + 3];
         uint4* d = reinterpret_cast<uint4*>(Wp + p * LL + x + L * y);
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
         d[(hL * L + hL) / 4] = make_uint4(q0.w, q1.w, q2.w, q3.w);
       }
     } else {
-      for (uint32_t i = li; i < F(T) * Q4; i += 64 * F(nw)) {
+      for (uint32_t i = li; i < f(S.T) * Q4; i += 64 * f(S.nw)) {
         const uint32_t p = fdiv(i, dq), r = i - p * Q4, y = fdiv(r, dH), x = r - y * hL;
         const uint4 v = Wl[i];
         uint32_t* d = Wp + p * LL + x + L * y;
@@ -563,10 +563,11 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   if (kept) {
     // (the same in all threads: no workgroup of this launch was waited for in
     // vain before its mark was there)
+    const uint32_t flag = status[0];
     if (!keeps_start(flag, status, step0)) return;
-    if (has) store_planes(kept);
+    if (has) store_planes(kept, [](auto v) { return (uint32_t)v; });
+    leave_mark(kept, flag, status, step0);
   }
-  leave_mark(kept, flag, status, step0);
   // (a launch that moves the counter on takes its first step by value, so
   // no workgroup of it reads the counter)
   if (step_out && blockIdx.x == 0 && tid == 0) *step_out = step0 + nsteps;
@@ -948,7 +949,7 @@ __global__ __launch_bounds__(1024) void k_resident(const RGroupEnt* __restrict__
   }
   __syncthreads();
   if (abort_s || !has) return;  // after the last barrier
-  store_planes(words);
+  store_planes(words, [](auto v) { return uni((uint32_t)v); });
 #undef F
 }
 
