@@ -150,11 +150,13 @@ typedef struct cvf_tuning {
                            slabs) */
   int32_t block_sigma;  /* workgroup size of the sigma half-sweep (64..1024, power of 2) */
   int32_t block_eta;    /* workgroup size of the eta cube sweep */
-  int32_t block_cell;   /* workgroup size of the per-cell kernels (SW, observables) */
+  int32_t block_cell;   /* workgroup size of the per-cell kernels (SW) */
   int32_t graph_steps;  /* MC steps per replayed hipGraph, or per resident launch (1..64) */
   int32_t fused;        /* 1: eta sweep + 6 half-sweeps per kernel on LDS-staged z-slabs, or
                            on boxes short along all axes (tiles) where slabs do not fit in
-                           LDS or would be one plane thick; 0: one kernel per half-sweep;
+                           LDS or a model of both says that they take longer (reference
+                           schedule, slab_planes = 0, block_chunk of 256 at least);
+                           0: one kernel per half-sweep;
                            2: the resident kernel (every step of a graph in one launch, the
                            lattice held in LDS, one stream group) where the points allow it
                            (one Metropolis sweep per step, chessboard rule), else as 1.  Its
@@ -171,8 +173,8 @@ typedef struct cvf_tuning {
   int32_t block_chunk;  /* workgroup size of the fused kernel */
   int32_t chunk_sweeps; /* half-sweeps per fused launch: 6, or 12 (a whole Metropolis pass per
                            launch where the wider window still fits in LDS); 0 = 6.  The default
-                           is 12 for handles under 2^20 cells with the chessboard rule, what
-                           the tiles' model gives when every point's L exceeds 64, else 6 */
+                           is what the tiles' model gives where it prefers them, else 12 for
+                           handles under 2^20 cells with the chessboard rule, else 6 */
 } cvf_tuning;
 
 int cvf_get_tuning(cvf_sim *s, cvf_tuning *t);
