@@ -372,7 +372,7 @@ int cvf_rw_create(int32_t L, int32_t n_sim, const double* T_hat, const double* P
                   const double* h_rho, double bin_factor, int32_t device, cvf_reweight** out) {
   if (!out || !T_hat || !P_hat || !counts || !h_rho) return set_error(CVF_EINVAL, "null argument");
   *out = nullptr;
-  // n_sim <= 1024: the kernels hold 32 bytes per simulation in LDS
+  // n_sim <= 1024: the kernels hold 40 bytes per simulation in LDS
   if (L < 1 || L > 1024 || n_sim < 1 || n_sim > 1024) return set_error(CVF_EINVAL, "L=%d, n_sim=%d", L, n_sim);
   if (!(bin_factor > 0)) return set_error(CVF_EINVAL, "bin_factor must be > 0");
   int64_t total = 0, mmax = 0;
